@@ -47,6 +47,10 @@ class LinearArgs(C.Structure):
                 ("batch", c_int), ("a_stride", c_int64), ("w_stride", c_int64), ("c_stride", c_int64), ("w_tiled_batch", c_void_p)]
 
 
+class NormChain(C.Structure):
+    _fields_ = [("post_ss", c_void_p), ("row_ss", c_void_p), ("row_ss_parts", c_int), ("row_eps", c_float)]
+
+
 class LinearFp8Args(C.Structure):
     _fields_ = [("a8", c_void_p), ("a_scale", c_void_p), ("w8", c_void_p), ("w_scale", c_void_p), ("bias", c_void_p), ("resid", c_void_p),
                 ("c", c_void_p), ("m", c_int), ("n", c_int), ("k", c_int), ("lda8", c_int), ("ldw8", c_int), ("ldc", c_int),
@@ -295,6 +299,8 @@ SIGNATURES = {
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "chatts_linear_workspace": (c_size_t, [c_int, c_int, c_int]),
     "chatts_linear_workspace_batch": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "chatts_linear_chain": (c_int, [c_void_p, c_void_p, c_void_p]),
+    "chatts_linear_post_ss_parts": (c_int, [c_void_p]),
     "chatts_gemv_ksplit": (c_int, [c_int, c_int, c_int, c_int]),
     "chatts_linear": (c_int, [C.POINTER(LinearArgs), c_void_p]),
     "chatts_quantize_rows_fp8": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_void_p]),

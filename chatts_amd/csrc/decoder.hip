@@ -14,7 +14,9 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s);
 int launch_gemm_f32(const ChattsLinearArgs* a, hipStream_t s);
 bool gemm_batched_stream(const ChattsLinearArgs* a);
 size_t gemm_workspace_batch(int m, int n, int k, int batch);
-int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope = nullptr, bool* rope_done = nullptr);
+int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope = nullptr, bool* rope_done = nullptr, const ChattsNormChain* chain = nullptr);
+int gemm_takes_rows(const ChattsLinearArgs* a);
+int rows_grid(int n, int epilogue);
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w,
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
@@ -38,6 +40,8 @@ struct ChattsDecoder {
   bool x_in_xn = false;     // batched step: o_proj left the residual stream in b.xn (ping-pong, see layer_part_batched); down_proj brings it back
   bool normed = false;      // planes 0 already hold RMSNorm(x) for the projection that comes next (written by the previous
                             // projection's fused epilogue): norm_into only binds them
+  int ss_parts = 0;         // > 0, with normed: ... planes 1 hold norm_w * x without the factor 1 / rms; its sums of squares are that many parts in
+                            // b.delta (free without tensor parallelism): a step of 2 .. 16 sequences whose projections hold whole columns
   bool sampling = false;    // token selection of the decode steps: greedy argmax, or the sampler with `sa`
   ChattsSamplingArgs sa{};
   ChattsTpComm* tp = nullptr;   // tensor-parallel exchange (borrowed); required by the whole-step entry points when tp_world > 1
@@ -51,18 +55,35 @@ struct ChattsDecoder {
 static int64_t embed_rows(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_rows : d->cfg.vocab_local; }
 static int64_t embed_offset(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_offset : d->cfg.vocab_offset; }
 
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain = nullptr);
+extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream) {
+  CHATTS_REQUIRE(a && ch, CHATTS_E_BADARG, "linear_chain: null args");
+  CHATTS_REQUIRE(!ch->row_ss || (((uintptr_t)ch->row_ss % 16) == 0 && a->a_hi && a->a_lo && a->m >= 2 && a->m <= 16 && a->batch <= 1 && !a->exact_f32 && ch->row_ss_parts >= 1 &&
+                                 ch->row_ss_parts <= 256), CHATTS_E_SHAPE,
+                 "linear_chain: row_ss takes 2 <= M <= 16 on planes and 1 .. 256 parts (M=%d, %d parts)", a->m, ch->row_ss_parts);
+  CHATTS_REQUIRE(!ch->post_ss || (((uintptr_t)ch->post_ss % 16) == 0 && a->batch <= 1 && !a->exact_f32 && chatts_linear_post_ss_parts(a) > 0), CHATTS_E_SHAPE,
+                 "linear_chain: post_ss needs post_norm_w and a shape of chatts_linear_post_ss_parts (M=%d N=%d K=%d)", a->m, a->n, a->k);
+  return linear_impl(a, stream, nullptr, nullptr, ch);
+}
+extern "C" int chatts_linear_post_ss_parts(const ChattsLinearArgs* a) {
+  const bool ok = a && a->w && a->m >= 2 && a->m <= 16 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && a->ldc >= a->n && a->ldw >= a->k && (!a->w8 || a->ldw8 >= a->k) &&
+                  a->post_norm_w && ((uintptr_t)a->post_norm_w % 16) == 0 && a->post_hi && a->post_lo && a->ld_post >= a->n && a->ld_post % 4 == 0 &&
+                  ((uintptr_t)a->post_hi % 8) == 0 && ((uintptr_t)a->post_lo % 8) == 0 && a->post_hi != a->a_hi && a->c && !a->c_hi &&
+                  (a->epilogue == CHATTS_EPI_NONE || a->epilogue == CHATTS_EPI_RESID) && gemm_takes_rows(a);
+  const int parts = ok ? rows_grid(a->n, a->epilogue) : 0;
+  return parts <= 256 ? parts : 0;
+}
 extern "C" size_t chatts_linear_workspace(int m, int n, int k) { return gemm_workspace(m, n, k); }
 extern "C" size_t chatts_linear_workspace_batch(int m, int n, int k, int batch) {
   const size_t one = gemm_workspace(m, n, k), all = gemm_workspace_batch(m, n, k, batch);
   return all > one ? all : one;
 }
 
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done);
 extern "C" int chatts_linear(const ChattsLinearArgs* a, chatts_stream_t stream) { return linear_impl(a, stream, nullptr, nullptr); }
 
 // rope / rope_done: the qkv projection of a prefill chunk may carry rope_kv_kernel's work in its split-K epilogue (*rope_done says
 // whether it did; otherwise the caller launches chatts_rope_kv_write as before)
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done) {
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain) {
   CHATTS_REQUIRE(a != nullptr, CHATTS_E_BADARG, "linear: null args");
   CHATTS_REQUIRE(a->m >= 0 && a->n > 0 && a->k > 0, CHATTS_E_BADARG, "linear: bad sizes m=%d n=%d k=%d", a->m, a->n, a->k);
   if (a->m == 0) return CHATTS_OK;
@@ -125,7 +146,7 @@ static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const 
     return launch_gemm_f32(a, as_stream(stream));
   }
   CHATTS_REQUIRE(a->norm_w == nullptr, CHATTS_E_BADARG, "linear: fused RMSNorm is only available for M == 1");
-  return launch_gemm(a, as_stream(stream), rope, rope_done);
+  return launch_gemm(a, as_stream(stream), rope, rope_done, chain);
 }
 
 extern "C" int chatts_split_bf16x2(const float* x, int m, int k, int ldx, chatts_bf16* hi, chatts_bf16* lo, int ld_planes,
@@ -218,20 +239,40 @@ static bool planes_path(const ChattsDecoder* d, int m, int k, bool fp8 = false) 
   return m >= 96 && !fp8;
 }
 
-// x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.
-static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream) {
+// x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.  chain: where the projection before may have left the
+// factor 1 / rms to this one (batched steps)
+static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream, ChattsNormChain* chain = nullptr) {
   if (planes_path(d, la->m, la->k, la->w8 != nullptr)) {
     la->a = nullptr; la->a_hi = d->b.planes_hi; la->a_lo = d->b.planes_lo; la->ld_planes = la->k;
+    if (d->normed && d->ss_parts && chain) {
+      la->a_hi = d->b.planes2_hi; la->a_lo = d->b.planes2_lo;
+      chain->row_ss = d->b.delta; chain->row_ss_parts = d->ss_parts; chain->row_eps = d->cfg.rms_eps;
+      d->normed = false; d->ss_parts = 0;
+      return CHATTS_OK;
+    }
     if (d->normed) { d->normed = false; return CHATTS_OK; }
     return chatts_rmsnorm_planes(d->b.x, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, stream);
   }
-  d->normed = false;
+  d->normed = false; d->ss_parts = 0;
   la->a = d->b.xn;
   return chatts_rmsnorm(d->b.x, norm_w, d->b.xn, la->m, la->k, d->cfg.rms_eps, stream);
 }
 
 // The residual-updating projection (o_proj / down_proj, tp_world == 1) also produces the NEXT projection's operand:
 // RMSNorm(x) with `next_norm_w` as planes 0, when that projection will take the plane path for the same M.
+// The same for few rows (layer_part_batched), without the norm's own launch: the projection writes norm_w * x as planes 1 and the sums of squares,
+// and the next projection multiplies by 1 / rms.  Planes 1, because workgroups that are done write them while others still read A (planes 0).
+static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormChain* chain, const float* next_norm_w, bool next_fp8) {
+  if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || !d->b.delta || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;
+  ChattsLinearArgs t = *la;
+  t.post_norm_w = next_norm_w; t.post_hi = d->b.planes2_hi; t.post_lo = d->b.planes2_lo; t.ld_post = la->n;
+  const int parts = chatts_linear_post_ss_parts(&t);
+  if (parts < 1 || 16 * 256 > (size_t)d->b.t_max * d->cfg.hidden || ((uintptr_t)d->b.delta % 16) != 0) return false;
+  *la = t;
+  chain->post_ss = d->b.delta;
+  d->normed = true; d->ss_parts = parts;
+  return true;
+}
 static bool gemm_post_norm_small_m() { return opt_get(OPT_POST_NORM_SMALL_M, 1) != 0; }
 static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const float* next_norm_w, bool next_fp8) {
   if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || la->epilogue != CHATTS_EPI_RESID) return;
@@ -617,6 +658,7 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
   const int H = c.hidden;
   int rc;
   ChattsLinearArgs la;
+  ChattsNormChain chain{};
   if (part == 0) {
     const int qkv_n = (c.n_q + 2 * c.n_kv) * kHeadDim;
     la = ChattsLinearArgs{};
@@ -624,8 +666,8 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
     la.lda = H; la.ldw = H; la.ldc = qkv_n; la.epilogue = CHATTS_EPI_NONE;
     la.w8 = lw.qkv8; la.w8_scale = lw.qkv8_scale; la.ldw8 = H; la.w8_format = d->cfg.w8_format;
     la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
-    if ((rc = norm_into(d, lw.input_norm, &la, stream)) != 0) return rc;
-    if ((rc = chatts_linear(&la, stream)) != 0) return rc;
+    if ((rc = norm_into(d, lw.input_norm, &la, stream, &chain)) != 0) return rc;
+    if ((rc = chatts_linear_chain(&la, &chain, stream)) != 0) return rc;
     ChattsKvCache kc = layer_cache(d, layer, 0);
     const bool attn_planes = planes_path(d, batch, c.n_q * kHeadDim, lw.o8 != nullptr);   // the combine writes o_proj's operand format
     if ((rc = attention_decode_batched_impl(d->b.qkv, batch, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, 0,
@@ -644,6 +686,8 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
     // The residual stream ping-pongs x -> xn (here) -> x (down_proj) inside a chained step, so that the post-norm epilogue may use
     // several workgroups per row (they read resid columns other workgroups update: c must not alias resid).
     d->x_in_xn = false;
+    chain = ChattsNormChain{};
+    if (request_post_ss(d, &la, &chain, lw.post_norm, lw.gate_up8 != nullptr)) return chatts_linear_chain(&la, &chain, stream);
     if (!tp && d->chain && d->b.xn && batch <= 16 && planes_path(d, batch, H, lw.gate_up8 != nullptr)) {
       la.c = d->b.xn;
       d->x_in_xn = true;
@@ -657,23 +701,27 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
   la.lda = H; la.ldw = H; la.ldc = c.inter; la.epilogue = CHATTS_EPI_SWIGLU;
   la.w8 = lw.gate_up8; la.w8_scale = lw.gate_up8_scale; la.ldw8 = H; la.w8_format = d->cfg.w8_format;
   la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
-  if ((rc = norm_into(d, lw.post_norm, &la, stream)) != 0) return rc;
+  if ((rc = norm_into(d, lw.post_norm, &la, stream, &chain)) != 0) return rc;
   const bool act_planes = planes_path(d, batch, c.inter, lw.down8 != nullptr) && planes_path(d, batch, H, lw.gate_up8 != nullptr);
-  if (act_planes) { la.c = nullptr; la.c_hi = d->b.planes2_hi; la.c_lo = d->b.planes2_lo; la.ld_cplanes = c.inter; }
-  if ((rc = chatts_linear(&la, stream)) != 0) return rc;
+  const bool in1 = la.a_hi == d->b.planes2_hi;       // (the other pair than the one that is being read)
+  chatts_bf16 *act_hi = in1 ? d->b.planes_hi : d->b.planes2_hi, *act_lo = in1 ? d->b.planes_lo : d->b.planes2_lo;
+  if (act_planes) { la.c = nullptr; la.c_hi = act_hi; la.c_lo = act_lo; la.ld_cplanes = c.inter; }
+  if ((rc = chatts_linear_chain(&la, &chain, stream)) != 0) return rc;
   la = ChattsLinearArgs{};
   la.a = d->b.act; la.w = lw.down; la.w_tiled = lw.down_t; la.m = batch; la.n = H; la.k = c.inter;
   la.lda = c.inter; la.ldw = c.inter; la.ldc = H;
   la.w8 = lw.down8; la.w8_scale = lw.down8_scale; la.ldw8 = c.inter; la.w8_format = d->cfg.w8_format;
   la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
-  if (act_planes) { la.a = nullptr; la.a_hi = d->b.planes2_hi; la.a_lo = d->b.planes2_lo; la.ld_planes = c.inter; }
+  if (act_planes) { la.a = nullptr; la.a_hi = act_hi; la.a_lo = act_lo; la.ld_planes = c.inter; }
   d->tp_fused = false;
   if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
   else { la.c = d->b.x; la.resid = d->x_in_xn ? d->b.xn : d->b.x; la.epilogue = CHATTS_EPI_RESID; }
   d->x_in_xn = false;
-  request_post_norm(d, &la, layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : d->w.final_norm,
-                    (layer + 1 < c.n_layers ? d->layers[layer + 1].qkv8 : d->w.lm_head8) != nullptr);
-  return chatts_linear(&la, stream);
+  const float* next_norm = layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : d->w.final_norm;
+  const bool next_fp8 = (layer + 1 < c.n_layers ? d->layers[layer + 1].qkv8 : d->w.lm_head8) != nullptr;
+  chain = ChattsNormChain{};
+  if (!request_post_ss(d, &la, &chain, next_norm, next_fp8)) request_post_norm(d, &la, next_norm, next_fp8);
+  return chatts_linear_chain(&la, &chain, stream);
 }
 
 // final norm + lm_head for rows 0 .. batch-1 of x (cache slots 0 .. batch-1) -> logits_all [batch, vocab_local]: the tail of a
@@ -689,10 +737,11 @@ extern "C" int chatts_decoder_logits_batched(ChattsDecoder* d, int batch, float*
   la.lda = c.hidden; la.ldw = c.hidden; la.ldc = (int)c.vocab_local; la.epilogue = CHATTS_EPI_NONE;
   la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
   la.w8 = d->w.lm_head8; la.w8_scale = d->w.lm_head8_scale; la.ldw8 = c.hidden; la.w8_format = d->cfg.w8_format;
-  int rc = norm_into(d, d->w.final_norm, &la, stream);      // binds planes a fused epilogue already wrote (d->normed), or launches the norm
-  d->normed = false; d->normed_q = false;
+  ChattsNormChain chain{};
+  int rc = norm_into(d, d->w.final_norm, &la, stream, &chain);      // binds planes a fused epilogue already wrote (d->normed), or launches the norm
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   if (rc) return rc;
-  return chatts_linear(&la, stream);
+  return chatts_linear_chain(&la, &chain, stream);
 }
 
 // One greedy step for `batch` sequences (TP = 1): all layers, final norm + lm_head for every row, per-sequence
@@ -716,7 +765,7 @@ extern "C" int chatts_decoder_decode_step_batched(ChattsDecoder* d, int batch, i
   if ((rc = chatts_embed_token_batched(token_dev, batch, d->w.embed, embed_offset(d), embed_rows(d), c.hidden, d->b.x,
                                        stream)) != 0) return rc;
   d->chain = true;               // layers run back to back: a projection may write the next one's normed operand
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   const int64_t nx = (int64_t)batch * c.hidden;
   for (int l = 0; l < c.n_layers && rc == CHATTS_OK; ++l) {
     rc = chatts_decoder_layer_part_batched(d, l, 0, batch, pos_dev, n_splits, stream);
@@ -725,7 +774,7 @@ extern "C" int chatts_decoder_decode_step_batched(ChattsDecoder* d, int batch, i
     if (tp && rc == CHATTS_OK && !d->tp_fused) rc = chatts_allreduce(d->tp, d->b.delta, d->b.x, d->b.x, nx, stream);     // ... and down_proj
   }
   d->chain = false;
-  if (rc) { d->normed = false; d->normed_q = false; return rc; }
+  if (rc) { d->normed = false; d->ss_parts = 0; d->normed_q = false; return rc; }
   if ((rc = chatts_decoder_logits_batched(d, batch, logits_all, stream)) != 0) return rc;
   return chatts_decoder_select_tokens(d, logits_all, batch, c.vocab_local, token_dev, token_logit_dev, out_tokens, out_stride, step_dev,
                                       pos_dev, c.max_ctx - 1, nullptr, stream);
@@ -752,7 +801,7 @@ extern "C" int chatts_decoder_prefill(ChattsDecoder* d, int t, int pos0, chatts_
   StageRange stage("chatts.prefill");
   const bool tp = d->cfg.tp_world > 1;
   d->chain = true;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   int rc = CHATTS_OK;
   for (int l = 0; l < d->cfg.n_layers && rc == CHATTS_OK; ++l) {
     rc = chatts_decoder_layer_part(d, l, 0, t, pos0, nullptr, 1, stream);
@@ -761,7 +810,7 @@ extern "C" int chatts_decoder_prefill(ChattsDecoder* d, int t, int pos0, chatts_
     if (tp && rc == CHATTS_OK) rc = tp_sum_into_x(d, t, stream);
   }
   d->chain = false;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   return rc;
 }
 
@@ -821,7 +870,7 @@ extern "C" int chatts_decoder_prefill_last(ChattsDecoder* d, int t, int pos0, ch
   StageRange stage("chatts.prefill_last");
   const bool tp = d->cfg.tp_world > 1;
   d->chain = true;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   int rc = CHATTS_OK;
   const int L = d->cfg.n_layers;
   for (int l = 0; l + 1 < L && rc == CHATTS_OK; ++l) {
@@ -842,7 +891,7 @@ extern "C" int chatts_decoder_prefill_last(ChattsDecoder* d, int t, int pos0, ch
     }
   } else if (rc == CHATTS_OK) rc = layer_last_row(d, L - 1, t, pos0, stream);
   d->chain = false;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   // the last row's o_proj / down_proj carried their exchange without advancing the device-side call counter (host-counted epochs):
   // settle it here, so that whatever runs next on this communicator - a replayed decode graph above all - starts from a flushed count
   if (tp && d->tp) { const int frc = chatts_tp_flush_epochs(d->tp, stream); if (rc == CHATTS_OK) rc = frc; }
@@ -863,7 +912,7 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
   const bool f8 = d->prefill_fp8 && t >= 16;          // speed mode: qkv and o_proj as fp8 x fp8 GEMMs (layer_part_fp8's arithmetic)
   ChattsLinearArgs la{};
   if (f8) {
-    d->normed = false; d->normed_q = false;
+    d->normed = false; d->ss_parts = 0; d->normed_q = false;
     uint8_t* a8 = reinterpret_cast<uint8_t*>(d->b.planes_hi);
     if ((rc = chatts_quantize_rows_fp8(d->b.x, t, H, H, lw.input_norm, c.rms_eps, a8, H, d->b.xn, stream)) != 0) return rc;
     ChattsLinearFp8Args f{};
@@ -925,14 +974,14 @@ extern "C" int chatts_decoder_prefill_packed(ChattsDecoder* d, const ChattsPrefi
   CHATTS_REQUIRE(t <= d->b.t_max, CHATTS_E_SHAPE, "decoder_prefill_packed: %d rows exceed buffers (%d)", t, d->b.t_max);
   StageRange stage("chatts.prefill_packed");
   d->chain = true;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   int rc = CHATTS_OK;
   for (int l = 0; l < d->cfg.n_layers && rc == CHATTS_OK; ++l) {
     rc = layer_part0_packed(d, l, t, segs, n_segs, stream);
     if (rc == CHATTS_OK) rc = chatts_decoder_layer_part(d, l, 1, t, 0, nullptr, 1, stream);
   }
   d->chain = false;
-  d->normed = false; d->normed_q = false;
+  d->normed = false; d->ss_parts = 0; d->normed_q = false;
   return rc;
 }
 

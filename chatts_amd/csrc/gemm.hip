@@ -366,6 +366,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
   for (int b = 0; b < MBW; ++b)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[b][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  f32x4 rs_part[16 / NW];
+  if constexpr (MB == 1) row_rstd_load(p, wave, NW, lane, rs_part);
 #pragma unroll
   for (int s = 0; s < NSTAGE - 1; ++s)
     if (s < nk) issue(s);
@@ -386,21 +388,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
         const int r = wn * (16 * FN) + j * 16 + frow;
         if (W8) {   // 8 fp8 = 8 bytes at byte 32 h + 8 q of the row: 16-byte chunk 2 h + (q >> 1), half q & 1
           const u32x2 q8 = *reinterpret_cast<const u32x2*>(base + W_OFF + lds_off128(r, 2 * h + (fchunk >> 1)) + (fchunk & 1) * 8);
-          typedef float f32x2_t __attribute__((ext_vector_type(2)));
-          const f32x2_t f0 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, true);
-          const f32x2_t f2 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, true);
-          bf16x8_t bv;
-          if (I8) {   // int8 copy: eight sign-extended bytes, exactly representable in bf16 (|q| <= 127)
-            const int a0 = (int)q8.x, a1 = (int)q8.y;
-            bv[0] = (__bf16)(float)((a0 << 24) >> 24); bv[1] = (__bf16)(float)((a0 << 16) >> 24);
-            bv[2] = (__bf16)(float)((a0 << 8) >> 24);  bv[3] = (__bf16)(float)(a0 >> 24);
-            bv[4] = (__bf16)(float)((a1 << 24) >> 24); bv[5] = (__bf16)(float)((a1 << 16) >> 24);
-            bv[6] = (__bf16)(float)((a1 << 8) >> 24);  bv[7] = (__bf16)(float)(a1 >> 24);
-          } else {
-            bv[0] = (__bf16)f0.x; bv[1] = (__bf16)f0.y; bv[2] = (__bf16)f1.x; bv[3] = (__bf16)f1.y;
-            bv[4] = (__bf16)f2.x; bv[5] = (__bf16)f2.y; bv[6] = (__bf16)f3.x; bv[7] = (__bf16)f3.y;
-          }
-          bfrag[h][j] = bv;
+          bfrag[h][j] = I8 ? widen_i8(q8) : widen_fp8(q8);      // (int8: |q| <= 127 is a bf16 number)
         } else {
           bfrag[h][j] = *reinterpret_cast<const bf16x8_t*>(base + W_OFF + lds_off128(r, h * 4 + fchunk));
         }
@@ -421,6 +409,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
         for (int j = 0; j < FN; ++j) acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[h], bfrag[h][j], acc[b][j], 0, 0, 0);
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[h], bfrag[h][j], acc[b][j], 0, 0, 0);
+      }
+    }
+  }
+  if constexpr (MB == 1) {
+    if (p.row_ss) {                              // (uniform; the factors take the ring's place: 80 KB of LDS a workgroup let two share a CU)
+      float* rstd_s = reinterpret_cast<float*>(smem);
+      __syncthreads();
+      row_rstd_store(p, wave, NW, lane, rs_part, rstd_s);
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float f = rstd_s[(lane >> 4) * 4 + r];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[0][j][r] *= f;
       }
     }
   }
@@ -923,6 +925,18 @@ bool gemm_batched_stream(const ChattsLinearArgs* a) {
   return a->m >= 2 && a->m <= 16 && use_stream(a) && !a->w8 && a->c && !a->c_hi && a->epilogue == CHATTS_EPI_NONE && a->n % 4 == 0 && a->ldc % 4 == 0 && a->c_stride % 4 == 0 &&
          a->a_stride % 8 == 0 && a->w_stride % 8 == 0 && ((uintptr_t)a->c % 16) == 0 && opt_get(OPT_EPI_V4, 1) != 0 && pick_stream_sk(a->n * a->batch, a->k, false) <= 8;
 }
+// K ranges of gemm_stream_kernel for these arguments if launch_gemm hands them to gemm_rows_kernel, which takes the same ranges (bit-identical) and
+// alone writes post_ss; 0: it does not.  Line: where K is split at all, and up to 8 rows; 8-bit weights beyond 4 rows only with eight K ranges (use_rows).
+// A workgroup of it reads all of X (~55 KB a us and CU), which beyond that costs more than the launch it saves.  us with the epilogue launch / in
+// one: bf16, 5 rows, 4096 x 4096: 9.9 / 9.0, 6144 x 4096: 12.8 / 11.2, 4096 x 12288: 19.9 / 20.5; 8 rows: 10.4 / 9.7, 12.9 / 11.9, 20.1 / 23.5.  fp8: 5120 x
+// 13824 (six ranges) 2 / 5 / 8 rows: 15.7 / 16.1 / 16.1 against 17.9 / 19.7 / 22.8.  On top of that comes the RMSNorm that moves into the launch (3 - 4 us
+// of a chain).  Whole steps: 8B bf16, 2 / 5 sequences 3.90 -> 3.59 / 4.24 -> 4.04 ms, 14B bf16, 8: 6.53 -> 6.21, 8B int8, 7: 3.20 -> 2.92, 14B fp8, 2 / 6 / 8:
+// 4.20 -> 3.95 / 4.47 -> 4.47 / 4.53 -> 4.68 (hence the line).
+int gemm_takes_rows(const ChattsLinearArgs* a) {
+  if (a->m > 8 || a->batch > 1 || opt_get(OPT_GEMM_SK, 0) != 0 || !use_stream(a)) return 0;
+  const int kps = k_per_split(a->k, pick_stream_sk(a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr)), sk = (a->k + kps - 1) / kps;
+  return sk > 1 && use_rows(a, sk) ? sk : 0;
+}
 size_t gemm_workspace_batch(int m, int n, int k, int batch) {
   if (batch <= 1 || m < 2 || m > 16 || k % 64) return 0;
   const int sk = pick_stream_sk(n * batch, k, false);
@@ -944,7 +958,7 @@ size_t gemm_workspace(int m, int n, int k) {
   return sk > 1 ? (size_t)sk * m * n * sizeof(float) : 0;
 }
 
-int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, bool* rope_done) {
+int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain) {
   int bm, sk;
   ChattsLinearArgs a_copy;
   const ChattsLinearArgs* a = a_in;
@@ -997,6 +1011,19 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     p.c_stride = a->c_stride;
   }
   p.a_stride = a->a_stride; p.w_stride = a->w_stride;
+  const ChattsNormChain none{}, &ch = chain ? *chain : none;
+  p.row_ss = ch.row_ss; p.row_ss_parts = ch.row_ss_parts; p.row_eps = ch.row_eps;
+  p.post_ss = nullptr;
+  CHATTS_REQUIRE(!ch.row_ss || (stream && a->m <= 16 && batch == 1), CHATTS_E_SHAPE, "linear: row_ss is for 2 <= M <= 16 on planes (M=%d K=%d take another kernel)", a->m, a->k);
+  if (stream && gemm_takes_rows(a)) {      // (at the same sk)
+    p.c = a->c;
+    p.post_w = a->post_norm_w; p.post_ss = ch.post_ss; p.post_hi = a->post_hi; p.post_lo = a->post_lo; p.ld_post = a->ld_post;
+    if (const int rc = launch_rows(p, a, sk, s)) return rc;
+    if (a->post_norm_w && !ch.post_ss)
+      return chatts_rmsnorm_planes(a->c, a->post_norm_w, a->post_hi, a->post_lo, a->ld_post, a->m, a->n, a->post_norm_eps, reinterpret_cast<chatts_stream_t>(s));
+    return CHATTS_OK;
+  }
+  CHATTS_REQUIRE(!ch.post_ss, CHATTS_E_SHAPE, "linear: post_ss is written by the few-rows kernel only (M=%d N=%d K=%d take another one)", a->m, a->n, a->k);
   const int nt_count = (a->n + 127) / 128, mt_count = (a->m + bm - 1) / bm;
   dim3 grid(8 * ((nt_count + 7) / 8) * mt_count, 1, sk), block(256);
   if (stream) {

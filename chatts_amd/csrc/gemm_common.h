@@ -26,6 +26,15 @@ struct GemmParams {
   int planes_tiled;      // a_hi / a_lo are in that layout too
   float glu_limit, glu_alpha;
   int64_t a_stride, w_stride, c_stride;   // several products of one shape (gemm_stream_kernel, grid y)
+  // RMSNorm split over two projections of few rows (gemm_rows.hip): the row factor 1 / rms comes from the producer's partial sums of squares
+  const float* row_ss;   // [16][256], or NULL
+  int row_ss_parts;
+  float row_eps;
+  const float* post_w;   // with post_ss: planes of post_w * c beside c, and the sums of squares of this launch's columns
+  float* post_ss;
+  uint16_t* post_hi;
+  uint16_t* post_lo;
+  int ld_post;
 };
 
 __device__ __forceinline__ void store_planes(uint16_t* hi, uint16_t* lo, size_t off, float v) {
@@ -36,6 +45,40 @@ __device__ __forceinline__ void store_planes(uint16_t* hi, uint16_t* lo, size_t 
   const __bf16 l = (__bf16)(v - (float)h);
   hi[off] = __builtin_bit_cast(uint16_t, h);
   lo[off] = __builtin_bit_cast(uint16_t, l);
+}
+
+__device__ __forceinline__ void store_planes4(uint16_t* hi, uint16_t* lo, f32x4 v) {      // the same for four neighbours, 8 bytes a store
+#pragma clang fp contract(off)
+  typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+  bf16x4_t hv, lv;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const __bf16 h = (__bf16)v[j];
+    hv[j] = h;
+    lv[j] = (__bf16)(v[j] - (float)h);
+  }
+  *reinterpret_cast<bf16x4_t*>(hi) = hv;
+  *reinterpret_cast<bf16x4_t*>(lo) = lv;
+}
+
+// eight 8-bit weights as bf16: both steps are exact
+__device__ __forceinline__ bf16x8_t widen_fp8(u32x2 q8) {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  const f32x2_t f0 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, true);
+  const f32x2_t f2 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, true);
+  bf16x8_t bv;
+  bv[0] = (__bf16)f0.x; bv[1] = (__bf16)f0.y; bv[2] = (__bf16)f1.x; bv[3] = (__bf16)f1.y;
+  bv[4] = (__bf16)f2.x; bv[5] = (__bf16)f2.y; bv[6] = (__bf16)f3.x; bv[7] = (__bf16)f3.y;
+  return bv;
+}
+__device__ __forceinline__ bf16x8_t widen_i8(u32x2 q8) {
+  const int a0 = (int)q8.x, a1 = (int)q8.y;
+  bf16x8_t bv;
+  bv[0] = (__bf16)(float)((a0 << 24) >> 24); bv[1] = (__bf16)(float)((a0 << 16) >> 24);
+  bv[2] = (__bf16)(float)((a0 << 8) >> 24);  bv[3] = (__bf16)(float)(a0 >> 24);
+  bv[4] = (__bf16)(float)((a1 << 24) >> 24); bv[5] = (__bf16)(float)((a1 << 16) >> 24);
+  bv[6] = (__bf16)(float)((a1 << 8) >> 24);  bv[7] = (__bf16)(float)(a1 >> 24);
+  return bv;
 }
 
 __device__ __forceinline__ float gelu_erf_f(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f)); }
@@ -67,6 +110,34 @@ struct RingGroup {
 constexpr int kRingTile = 160;
 int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGroup& g, int most_tiles, hipStream_t s);
 int launch_ring(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, bool single, hipStream_t s);
+
+// 1 / rms of the rows of A from the sums of squares that its producer left (GemmParams.row_ss: row r's parts at r * kSsStride): wave w takes rows
+// w, w + waves, .. (ROWS of them).  Requested before anything else of the kernel and used at its end: a wait at the start would drain the first weights.
+constexpr int kSsStride = 256;
+template <int ROWS>
+__device__ __forceinline__ void row_rstd_load(const GemmParams& p, int wave, int waves, int lane, f32x4 (&part)[ROWS]) {
+  if (!p.row_ss) return;
+#pragma unroll
+  for (int t = 0; t < ROWS; ++t) part[t] = *reinterpret_cast<const f32x4*>(p.row_ss + ((wave + t * waves) & 15) * kSsStride + lane * 4);
+}
+template <int ROWS>
+__device__ __forceinline__ void row_rstd_store(const GemmParams& p, int wave, int waves, int lane, const f32x4 (&part)[ROWS], float* rstd) {
+  if (!p.row_ss) return;
+#pragma unroll
+  for (int t = 0; t < ROWS; ++t) {
+    const int row = wave + t * waves;
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += lane * 4 + j < p.row_ss_parts ? part[t][j] : 0.f;
+    s = wave_sum(s);
+    if (lane == 0 && row < 16) rstd[row] = rsqrtf(s / (float)p.k + p.row_eps);
+  }
+}
+
+// gemm_rows.hip: few rows, whole K per workgroup
+bool use_rows(const ChattsLinearArgs* a, int sk);      // sk: K ranges of gemm_stream_kernel
+int rows_grid(int n, int epilogue);      // workgroups = parts of post_ss
+int launch_rows(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s);
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
