@@ -665,6 +665,7 @@ int gemv_pick_ksplit(int tasks, int nchunks, bool norm, double w_bytes, int cus)
   return ks;
 }
 
+int launch_gemv4(const ChattsLinearArgs* a, hipStream_t s, bool* done);      // gemv4.hip
 int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
   GemvParams p;
   p.tp = TpParams{};
@@ -721,7 +722,12 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
   const int pad = opt_get(OPT_GEMV_LDSPAD, 0);
   if (pad >= 1 && (size_t)(160 * 1024 / pad) / 16 * 16 > lds) lds_launch = (size_t)(160 * 1024 / pad) / 16 * 16;
   if (lds_launch > 64 * 1024 && lds <= 64 * 1024) lds_launch = 64 * 1024;      // default dynamic-LDS cap (still 2 per CU)
-  if (a->w4 != nullptr) {                       // 4-bit codes: 2 rows x 4 chunks of 1024 elements (8-byte loads) in flight
+  if (a->w4 != nullptr) {
+    bool done = false;
+    const int rc = launch_gemv4(a, s, &done);
+    if (rc || done) return rc;
+  }
+  if (a->w4 != nullptr) {                       // 4-bit codes that gemv4.hip does not take: 2 rows x 4 chunks of 1024 elements (8-byte loads) in flight
     const int nchunks4 = (a->k + 1023) / 1024;
     const size_t lds4 = (size_t)nchunks4 * 1024 * 4 + 64 * 4;
     p.tasks = (units + (swiglu ? 1 : 2) - 1) / (swiglu ? 1 : 2);

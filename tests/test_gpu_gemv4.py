@@ -1,0 +1,78 @@
+"""The batch-1 projection on 4-bit codes (csrc/gemv4.hip): every weight it rebuilds is the stored bf16 value bit for bit, sums against float64; rows that deal
+unevenly over the CUs, K that ends inside a unit of 512, all group sizes it takes, gated rows, the fused norm."""
+import ctypes as C
+
+import pytest
+import torch
+
+from chatts_amd import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def problem(n, k, group, seed):
+    from chatts_amd.modeling import pack_int4, quantize_int4_rows
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    w = (r(n, k) * k ** -0.5 * 10.0 ** (3 * torch.rand((n, 1), generator=g, device=DEV) - 2)).bfloat16()
+    codes, scale, zero, deq = quantize_int4_rows(w, group)
+    return r(1, k), pack_int4(codes, scale, zero), deq, r(n), r(1, n), 1 + 0.1 * r(k)
+
+
+def run(x, w4, sz, deq, group, epi, bias=None, resid=None, norm=None):
+    n, k = deq.shape
+    out = torch.full((1, n // 2 if epi == _lib.EPI_SWIGLU else n), float("nan"), device=DEV)
+    a = _lib.LinearArgs(a=x.data_ptr(), w=deq.data_ptr(), bias=_lib.ptr(bias), resid=_lib.ptr(resid), c=out.data_ptr(), norm_w=_lib.ptr(norm), norm_eps=1e-6, m=1, n=n, k=k,
+                        lda=k, ldw=k, ldc=out.shape[1], epilogue=epi, w4=w4.data_ptr(), w4_sz=sz.data_ptr(), ldw4=k // 2, w4_group=group)
+    _lib.check(_lib.load().chatts_linear(C.byref(a), _lib.stream_ptr()))
+    torch.cuda.synchronize()
+    return out
+
+
+# the smallest of K, of N, of both; K that ends inside a unit; a row of units for some workgroups only; the largest K; both sides of the line to the old kernel
+SHAPES = [(16, 2560, 128), (16, 2080, 32), (1040, 2112, 64), (5120, 5120, 128), (7168, 5120, 128), (96, 13824, 128), (13200, 640, 64), (98304, 96, 32), (4096, 12288, 64),
+          (320, 16384, 128), (4096, 2048, 1024), (4112, 2048, 1024), (32, 4096, 256), (48, 96, 32), (1040, 1024, 32)]
+
+
+@pytest.mark.parametrize("n,k,group", SHAPES)
+def test_rebuilt_weights_are_the_stored_ones(n, k, group):
+    _, (w4, sz), deq, *_ = problem(n, k, group, n + k)
+    for at in [0, 1, 4, 7, 31, 32, k // 2 + 5, k - 1]:
+        x = torch.zeros((1, k), device=DEV)
+        x[0, at] = 1.0
+        assert torch.equal(run(x, w4, sz, deq, group, _lib.EPI_NONE)[0], deq[:, at].float())
+
+
+@pytest.mark.parametrize("epi", [_lib.EPI_NONE, _lib.EPI_RESID, _lib.EPI_SWIGLU])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("n,k,group", SHAPES + [(27648, 5120, 128)])
+def test_sums(n, k, group, norm, epi):
+    if epi == _lib.EPI_SWIGLU and n % 32:
+        n += 16
+    x, (w4, sz), deq, bias, resid, nw = problem(n, k, group, n * k)
+    xd = x.double()
+    if norm:
+        xd = xd * torch.rsqrt((xd * xd).mean() + 1e-6) * nw.double()
+    want = xd @ deq.double().T + bias.double()
+    # x = hi + lo loses 2^-18 of each term; float32 sums of K / 16 terms a lane and 16 more: 2^-24 a step, at most (K / 16 + 32) of them
+    bound = xd.abs() @ deq.double().abs().T * (2.0 ** -18 + (k / 16 + 32) * 2.0 ** -24) + want.abs() * 2.0 ** -20
+    if epi == _lib.EPI_RESID:
+        want = want + resid.double()
+        bound = bound + want.abs() * 2.0 ** -24
+    if epi == _lib.EPI_SWIGLU:
+        z, dz = want.view(-1, 2, 16), bound.view(-1, 2, 16)
+        gate = torch.nn.functional.silu(z[:, 0])
+        want = (gate * z[:, 1]).reshape(1, -1)
+        bound = (1.1 * dz[:, 0] * (z[:, 1].abs() + dz[:, 1]) + gate.abs() * dz[:, 1]).reshape(1, -1) + want.abs() * 2.0 ** -20      # (silu's slope is below 1.1)
+    out = run(x, w4, sz, deq, group, epi, bias, resid, nw if norm else None)
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("k", [2592, 2560, 5088])
+def test_rows_do_not_read_each_other(k):
+    x, (w4, sz), deq, *_ = problem(128, k, 32, k)
+    clean = run(x, w4, sz, deq, 32, _lib.EPI_NONE)
+    sz = sz.clone()
+    sz[1::2] = float("nan")
+    assert torch.equal(run(x, w4, sz, deq, 32, _lib.EPI_NONE)[:, ::2], clean[:, ::2])
