@@ -31,7 +31,7 @@ constexpr unsigned kRowsFar = 0x7ffffff0u, kRowsNoToken = 0x40000000u;
 constexpr int rows_ring(int np, int la) { return (la + 1) * np * 1024 + 1024; }
 
 template <bool W8, bool I8, int NP, int LA, int MAXW>
-__global__ __launch_bounds__(64 * MAXW) void gemm_rows_kernel(GemmParams p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp) {
+__global__ __launch_bounds__(64 * MAXW) void gemm_rows_kernel(GemmParams p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, int groups_each, int groups_more) {
 #ifdef __HIP_DEVICE_COMPILE__      // (buffer resources are a type of the device pass)
   constexpr int FN = (NP + 1) / 2, BK = W8 ? 128 : 64, KS = BK / 32, NX = KS, NB = LA + 1;
   constexpr int RING = rows_ring(NP, LA);
@@ -41,9 +41,8 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_rows_kernel(GemmParams p, cons
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool glu = epi_is_glu(p.epilogue);
-  const int gran = glu ? 8 : 4, groups = p.n / gran;
-  const int g0 = (int)((long long)blockIdx.x * groups / gridDim.x), g1 = (int)((long long)(blockIdx.x + 1) * groups / gridDim.x);
-  const int rows = (g1 - g0) * 4, r0 = g0 * 4;         // columns of this workgroup (gated: gates), the first of them
+  const int b0 = (int)blockIdx.x, more = b0 < groups_more;
+  const int rows = (groups_each + more) * 4, r0 = (b0 * groups_each + (more ? b0 : groups_more)) * 4;      // columns of this workgroup (gated: gates), the first of them
   constexpr int FG = FN > 1 ? FN / 2 : 1;              // gated: fragments 0 .. FG - 1 are gates, the others their up rows
 
   // rows of W behind logical row i of fragment f (rows past the end repeat the last one; their sums are dropped)
@@ -263,8 +262,9 @@ static int launch_rows_t(const GemmParams& p, const ChattsLinearArgs* a, int wav
     CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_rows: cannot reserve 156 KB of LDS: %s", hipGetErrorString(e));
     configured = true;
   }
-  hipLaunchKernelGGL((gemm_rows_kernel<W8, I8, NP, LA, MAXW>), dim3(rows_grid(a->n, a->epilogue)), dim3(64 * waves), rows_lds(NP, LA, waves), s, p, a->a_hi, a->a_lo,
-                     a->ld_planes);
+  const int groups = a->n / (epi_is_glu(a->epilogue) ? 8 : 4), grid = rows_grid(a->n, a->epilogue);
+  hipLaunchKernelGGL((gemm_rows_kernel<W8, I8, NP, LA, MAXW>), dim3(grid), dim3(64 * waves), rows_lds(NP, LA, waves), s, p, a->a_hi, a->a_lo, a->ld_planes, groups / grid,
+                     groups % grid);
   CHATTS_CHECK_LAUNCH("gemm_rows");
   return CHATTS_OK;
 }
