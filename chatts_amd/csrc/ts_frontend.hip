@@ -147,58 +147,32 @@ __global__ __launch_bounds__(256) void ts_normalise_kernel(const double* __restr
 
 }  // namespace chatts
 
-// ---- patchify + the first MLP layer in ONE launch (round 6) -------------------------------------------------------
-// out0[p, n] = GELU(feat[p, :] . W0[n, :] + b0[n]) written as bf16 hi / lo planes - the operand of layer 1.  The separate form cost a
-// patchify launch (5.5 us) plus a 20-workgroup run of the prefill kernel for 3 MB of weights (13 us: K = 320 is ten half-steps of
-// pipeline fill).  Here a one-wave workgroup owns 16 patch rows x 64 output columns; it builds the activation fragments of its
-// 16-row block IN REGISTERS, straight from the series / position table (the feature row never exists in memory), loads its W0
-// fragments straight from L2 (3 MB, shared by everybody) and issues the same MFMAs in the same order as the prefill kernel does
-// (per 32 K-values: lo pass, then hi pass; operands swapped, D = W . A^T): bit-identical planes.  No LDS, no barrier.
+// ---- patchify + the first MLP layer in ONE launch --------------------------------------------------------------------------------------
+// out0[p, n] = GELU(feat[p, :] . W0[n, :] + b0[n]) written as bf16 hi / lo planes - the operand of layer 1.  A wave owns 16 patch rows: it builds
+// and splits their features in registers, straight from the series and the position table (the feature row never exists in memory), and walks over
+// steps of 32 columns; W0 of a step comes to LDS once for the four waves of a workgroup, two steps ahead.  The MFMAs and their order are the prefill
+// kernel's (per 32 K-values: lo pass, then hi pass; operands swapped, D = W . A^T): bit-identical planes.
+// What bounds it: few patches - the chain offsets -> series -> MFMA -> store; many - vector operations, the 60 to 90 of an exact-erf GELU per output and the splits.
+// It used to be a wave per 16 rows x 32 columns that built its features anew and read its W0 fragments (64-byte pieces of lines) from L2: 7.5 TB/s of
+// those at many patches, and the features' loads one group after the other at few.  us before -> after: 1036 patches of 30 series, 5120 columns 64 -> 30
+// (the loop over columns with W0 in registers alone: 39), 128 patches 14.6 -> 13.1, 16 patches, 4096 columns 10 -> 6.6.
 namespace chatts {
-__device__ __forceinline__ float ts_feature(const ChattsPatchifyArgs& a, const float2* row, int vl, float last, int t0, int k) {
-  const int ps = a.patch_size;
-  if (a.mode == 1) {
-    if (k < ps) { const int t = t0 + k; return t < vl ? row[t].x : last; }
-    const int q = k - ps;
-    if (q >= ps * a.emb_dim) return 0.f;
-    const int j = q / a.emb_dim, e = q - j * a.emb_dim;
-    const int t = t0 + j;
-    return a.pos_table[(size_t)(t < vl ? t : a.max_seq_len) * a.emb_dim + e];
-  }
-  if (a.mode == 2) {
-    if (k >= 2 * ps) return 0.f;
-    const int t = t0 + (k >> 1);
-    if (!(k & 1)) return t < vl ? row[t].x : last;
-    const int den = a.max_valid_len - 1 > 1 ? a.max_valid_len - 1 : 1;
-    return t < vl ? (float)t / (float)den : -1.0f;
-  }
-  if (k >= ps) return 0.f;
-  const int t = t0 + k;
-  return t < vl ? row[t].x : last;
-}
-
-// the 8 consecutive features k0 .. k0 + 7 of one patch row (k0 % 8 == 0), LOADS ONLY and branch-free per lane: the tail value "last valid
-// value" is row[vl - 1], i.e. the load index is clamped instead of selecting afterwards; out-of-range groups load a valid address and
-// are zeroed.  MODE is compile time (the generic per-element form of ts_feature would put every mode's code, with its divisions, into each
-// of the 18 groups of a lane).  Mode 1 needs patch size and embedding width multiples of 8 (every shipped config: 16 / 16): a group then
-// lies wholly inside the value part or inside ONE position's embedding row - two 16-byte loads, one division per group.
+// the 8 consecutive features k0 .. k0 + 7 (k0 = 32 s + 8 kc) of one patch row.  Every load is unconditional, at a clamped address (the tail value is row[vl - 1], a group
+// past the features reads what another one reads), and selected afterwards: under a condition of the lane the compiler waits for each group before it
+// asks for the next one, nine round trips in a row.  MODE is compile time.  Mode 1 needs patch size and embedding width multiples of 8 (every shipped
+// config: 16 / 16): a group then lies wholly inside the value part or inside ONE position's embedding row, and with at most ten K-steps the
+// value part lies inside the first (patch * (1 + emb) <= 320, emb >= 8).  emb8_inv = ceil(2^32 / (emb_dim / 8)), 0 for 1.
 template <int MODE>
-__device__ __forceinline__ void ts_feature8(const ChattsPatchifyArgs& a, const float2* row, int vl, int t0, int k0, float (&v)[8]) {
-  const int ps = a.patch_size;
+__device__ __forceinline__ void ts_feature8(const ChattsPatchifyArgs& a, unsigned emb8_inv, const float2* row, int vl, int t0, int s, int kc, float (&v)[8]) {
+  const int ps = a.patch_size, k0 = s * 32 + kc * 8;
   if constexpr (MODE == 1) {
-    if (k0 < ps) {
+    const bool ok = k0 >= ps && k0 < ps + ps * a.emb_dim;
+    const int q0 = ok ? k0 - ps : 0, j = emb8_inv ? (int)__umulhi((unsigned)q0 >> 3, emb8_inv) : q0 >> 3;
+    const int t = t0 + j;
+    const float* src = a.pos_table + (size_t)(t < vl ? t : a.max_seq_len) * a.emb_dim + (q0 - j * a.emb_dim);
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(src), x1 = *reinterpret_cast<const f32x4*>(src + 4);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) { const int t = t0 + k0 + q; v[q] = row[t < vl ? t : vl - 1].x; }
-    } else {
-      const int q0 = k0 - ps;
-      const bool ok = q0 < ps * a.emb_dim;
-      const int j = ok ? q0 / a.emb_dim : 0, e0 = ok ? q0 - j * a.emb_dim : 0;
-      const int t = t0 + j;
-      const float* src = a.pos_table + (size_t)(t < vl ? t : a.max_seq_len) * a.emb_dim + e0;
-      const f32x4 x0 = *reinterpret_cast<const f32x4*>(src), x1 = *reinterpret_cast<const f32x4*>(src + 4);
-      const float m = ok ? 1.f : 0.f;
-      v[0] = x0.x * m; v[1] = x0.y * m; v[2] = x0.z * m; v[3] = x0.w * m; v[4] = x1.x * m; v[5] = x1.y * m; v[6] = x1.z * m; v[7] = x1.w * m;
-    }
+    for (int q = 0; q < 8; ++q) v[q] = ok ? (q < 4 ? x0[q & 3] : x1[q & 3]) : 0.f;      // (the value part: the caller's)
   } else if constexpr (MODE == 2) {      // (value, position) pairs: k even = value of t0 + k / 2, k odd = t / max(1, max_vl - 1) or -1
     const bool ok = k0 < 2 * ps;
     const int den = a.max_valid_len - 1 > 1 ? a.max_valid_len - 1 : 1;
@@ -216,26 +190,32 @@ __device__ __forceinline__ void ts_feature8(const ChattsPatchifyArgs& a, const f
   }
 }
 
-template <int KSTEPS, int MODE, int NJ = 2>      // NJ: 16-column fragments per wave;  K-steps of 32 (feature count rounded up) and the feature mode: compiled in, so that every load is in flight at once
-__global__ __launch_bounds__(64) void ts_layer0_kernel(ChattsPatchifyArgs a, const uint16_t* __restrict__ w0, int ldw, const float* __restrict__ b0,
-                                                         int hidden, uint16_t* __restrict__ out_hi, uint16_t* __restrict__ out_lo, int ld_out) {
+constexpr int kL0Waves = 4, kL0Cols = 32;      // waves (16 rows each) of a workgroup, columns of a step
+
+template <int KSTEPS, int MODE>      // K-steps of 32 (feature count rounded up) and the feature mode: compiled in, so that every load is in flight at once
+__global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatchifyArgs a, unsigned emb8_inv, const uint16_t* w0, int ldw, const float* b0, int hidden, int steps_each,
+                                                                     uint16_t* out_hi, uint16_t* out_lo, int ld_out) {
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-  // workgroup = ONE wave = 16 patch rows x 64 output columns (no LDS, no barrier: nothing to share): it builds (and splits) one activation
-  // fragment per K-step and re-uses it for four W fragments; P = 128, H = 5120: 640 independent waves over 256 CUs
-  const int lane = threadIdx.x & 63;
-  const int n0 = blockIdx.x * (16 * NJ), r0 = blockIdx.y * 16;
+  // W0 of a step: 32 rows of 4 KSTEPS 16-byte chunks, twice.  Chunk c of a K-step of row r lies at place c ^ (r >> turn): eight rows' chunks then meet
+  // different banks whatever KSTEPS makes of the row's length
+  constexpr int ROW = 4 * KSTEPS, PIECES = 2 * KSTEPS, TURN = KSTEPS % 2 ? 2 : (KSTEPS % 4 ? 1 : 0);
+  __shared__ __attribute__((aligned(1024))) char smem[2][PIECES * 1024];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r0 = ((int)blockIdx.y * kL0Waves + wave) * 16;
+  const bool mine = r0 < a.total_patches;                      // (else a wave that only fetches W0)
   const int frow = lane & 15, kc = lane >> 4;                  // this lane's row of a 16-row block, and its 8 K-values of a 32-deep step
-  if (r0 >= a.total_patches) return;                           // (wave-uniform: a block wholly beyond the last patch row)
-  // W0 fragments first: rows n0 + 16 j + frow, K-values 32 s + 8 kc ..; all KSTEPS x 4 loads are independent of everything else
-  bf16x8_t wf[KSTEPS][NJ];
+  int n0 = (int)blockIdx.x * steps_each * kL0Cols;
+  const int n_end = n0 + steps_each * kL0Cols < hidden ? n0 + steps_each * kL0Cols : hidden;
+  auto fetch = [&](int n, int b) __attribute__((always_inline)) {        // (rows past the end of W0 repeat its last one; their sums are dropped)
 #pragma unroll
-  for (int s = 0; s < KSTEPS; ++s)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      int wr = n0 + j * 16 + frow;
-      if (wr > hidden - 1) wr = hidden - 1;
-      wf[s][j] = *reinterpret_cast<const bf16x8_t*>(w0 + (size_t)wr * ldw + s * 32 + kc * 8);
+    for (int q = 0; q < (PIECES + kL0Waves - 1) / kL0Waves; ++q) {
+      const int piece = q * kL0Waves + wave;
+      if (q * kL0Waves + kL0Waves > PIECES && piece >= PIECES) continue;
+      const int c = piece * 64 + lane, r = c / ROW, x = c - r * ROW;
+      const int row = n + r < hidden ? n + r : hidden - 1;
+      __builtin_amdgcn_global_load_lds((gptr_t)(w0 + (size_t)row * ldw + ((x & ~3) | ((x & 3) ^ ((r >> TURN) & 3))) * 8), (lptr_t)(smem[b] + piece * 1024), 16, 0, 0);
     }
+  };
   // the patch row this lane feeds, clamped to the last real row (stores are masked).  Its series: up to 63 series - lane i holds
   // row_off[i] / valid_len[i] (ONE round trip), the search is a wave-uniform walk over lanes and two ds_bpermute; more series - the
   // binary search of ts_patchify_kernel (log2 N dependent round trips)
@@ -261,50 +241,84 @@ __global__ __launch_bounds__(64) void ts_layer0_kernel(ChattsPatchifyArgs a, con
   }
   const int t0 = (p - off) * a.patch_size;
   const float2* rowp = reinterpret_cast<const float2*>(a.series) + (size_t)sidx * a.lmax;
-  // every feature load of the block before the first use
+  // every feature load of the block before the first use, and the first two steps of W0 behind them
   float raw[KSTEPS][8];
 #pragma unroll
-  for (int s = 0; s < KSTEPS; ++s) ts_feature8<MODE>(a, rowp, vl, t0, s * 32 + kc * 8, raw[s]);
-  f32x4 acc[NJ];
+  for (int s = 0; s < KSTEPS; ++s) ts_feature8<MODE>(a, emb8_inv, rowp, vl, t0, s, kc, raw[s]);
+  float val[8];
+  if constexpr (MODE == 1) {
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < KSTEPS; ++s) {
-    bf16x8_t ahi, alo;
+    for (int q = 0; q < 8; ++q) { const int t = t0 + kc * 8 + q; val[q] = rowp[t < vl ? t : vl - 1].x; }
+  }
+  fetch(n0, 0);
+  if (n0 + kL0Cols < n_end) fetch(n0 + kL0Cols, 1);
+  if constexpr (MODE == 1) {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      uint16_t h, l;
-      split_bf16x2(raw[s][q], h, l);
-      ahi[q] = __builtin_bit_cast(__bf16, h);
-      alo[q] = __builtin_bit_cast(__bf16, l);
+      asm volatile("" : "+v"(val[q]));                         // (keeps the loads out of the condition)
+      if (kc * 8 < a.patch_size) raw[0][q] = val[q];
     }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][j], alo, acc[j], 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][j], ahi, acc[j], 0, 0, 0);
   }
-  // lane holds D[feature n0 + 16 j + 4 kc + r][token r0 + frow]: bias, exact-erf GELU, split, 8-byte stores (ring_store's arithmetic)
-  const int tok = r0 + frow;
+  bf16x8_t ahi[KSTEPS], alo[KSTEPS];
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int fb = n0 + j * 16 + kc * 4;
-    const int fbc = fb < hidden ? fb : 0;
-    const f32x4 bias = b0 ? *reinterpret_cast<const f32x4*>(b0 + fbc) : (f32x4){0.f, 0.f, 0.f, 0.f};
-    bf16x4_t hv, lv;
-    {
+  for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const __bf16 h = (__bf16)raw[s][q];
+      ahi[s][q] = h;
+      alo[s][q] = (__bf16)(raw[s][q] - (float)h);
+    }
+  const int tok = r0 + frow;
+  const bool live = tok < a.total_patches;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  for (int b = 0; n0 < n_end; n0 += kL0Cols, b ^= 1) {
+    // lane holds D[feature n0 + 16 j + 4 kc + r][token r0 + frow]: bias, exact-erf GELU, split, 8-byte stores (ring_store's arithmetic)
+    bf16x4_t hv[2], lv[2];
+    if (mine) {
+      f32x4 bias[2], acc[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int fb = n0 + j * 16 + kc * 4;
+        bias[j] = b0 ? *reinterpret_cast<const f32x4*>(b0 + (fb < hidden ? fb : 0)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+        acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+      const char* w = smem[b] + (frow * ROW + (kc ^ ((frow >> TURN) & 3))) * 16;      // (16 rows on: the same place, 16 >> TURN is a multiple of 4)
+#pragma unroll
+      for (int s = 0; s < KSTEPS; ++s) {
+        bf16x8_t wf[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wf[j] = *reinterpret_cast<const bf16x8_t*>(w + j * 16 * ROW * 16 + s * 64);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], alo[s], acc[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], ahi[s], acc[j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
 #pragma clang fp contract(off)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = gelu_erf_f(acc[j][r] + bias[r]);
-        const __bf16 h = (__bf16)v;
-        hv[r] = h;
-        lv[r] = (__bf16)(v - (float)h);
+        for (int r = 0; r < 4; ++r) {
+          const float v = gelu_erf_f(acc[j][r] + bias[j][r]);
+          const __bf16 h = (__bf16)v;
+          hv[j][r] = h;
+          lv[j][r] = (__bf16)(v - (float)h);
+        }
       }
     }
-    if (tok < a.total_patches && fb < hidden) {
-      *reinterpret_cast<bf16x4_t*>(out_hi + (size_t)tok * ld_out + fb) = hv;
-      *reinterpret_cast<bf16x4_t*>(out_lo + (size_t)tok * ld_out + fb) = lv;
-    }
+    // what is waited for: the next step's pieces of this wave, and the stores of the step before; then all waves are through with this step's W0 and have the next one's
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (live)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int fb = n0 + j * 16 + kc * 4;
+        if (fb < hidden) {
+          *reinterpret_cast<bf16x4_t*>(out_hi + (size_t)tok * ld_out + fb) = hv[j];
+          *reinterpret_cast<bf16x4_t*>(out_lo + (size_t)tok * ld_out + fb) = lv[j];
+        }
+      }
+    if (n0 + 2 * kL0Cols < n_end) fetch(n0 + 2 * kL0Cols, b);
   }
 }
 }  // namespace chatts
@@ -393,10 +407,16 @@ extern "C" int chatts_ts_encode(const float* series, const int32_t* row_off, con
       ((uintptr_t)w->w[0] % 16) == 0 && ((uintptr_t)w->b[0] % 16) == 0 && ((uintptr_t)w->pos_table % 16) == 0 && opt_get(OPT_TS_L0_FUSED, 1) != 0) {
     CHATTS_REQUIRE(pa.series && pa.row_off && pa.valid_len && (w->mode != 1 || (pa.pos_table && w->emb_dim > 0 && w->max_seq_len > 0)), CHATTS_E_BADARG,
                    "ts_encode: null series / offsets / position table");
-    const dim3 grid((H + 31) / 32, (P + 15) / 16), block(64);      // (NJ = 2: 32 columns per wave)
+    // four row blocks a workgroup; the columns in as many parts as three workgroups per CU ask for
+    const int groups = (P + 16 * kL0Waves - 1) / (16 * kL0Waves), steps = (H + kL0Cols - 1) / kL0Cols;
+    int parts = 3 * device_cus() / groups;
+    parts = parts < 1 ? 1 : (parts > steps ? steps : parts);
+    const int steps_each = (steps + parts - 1) / parts, emb8 = w->mode == 1 ? w->emb_dim / 8 : 1;
+    const unsigned emb8_inv = emb8 > 1 ? (unsigned)((0x100000000ull + emb8 - 1) / emb8) : 0u;      // (exact for the at most 40 groups of a row)
+    const dim3 grid((steps + steps_each - 1) / steps_each, groups), block(64 * kL0Waves);
     uint16_t* oh = hi_of(h0);
     uint16_t* ol = lo_of(h0, H);
-#define CHATTS_TS_L0(KS, MD) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD>), grid, block, 0, as_stream(stream), pa, w->w[0], w->in_features_pad, w->b[0], H, oh, ol, H)
+#define CHATTS_TS_L0(KS, MD) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD>), grid, block, 0, as_stream(stream), pa, emb8_inv, w->w[0], w->in_features_pad, w->b[0], H, steps_each, oh, ol, H)
     if (w->mode == 1) {
       switch (ksteps) {
         case 1: CHATTS_TS_L0(1, 1); break;
