@@ -625,12 +625,14 @@ __global__ __launch_bounds__(256) void splitk_epilogue_norm_kernel(const float* 
   }
 }
 
-// The same kernel with every memory round trip of a thread taken ONCE (round 5): sk <= 4 slabs, rows of <= 1024 kIt columns.  The kernel
+// The same kernel with every memory round trip of a thread taken ONCE: sk <= SLABS (4 or 8) slabs, rows of <= 1024 kIt columns.  The kernel
 // above walks a row in kIt dependent iterations - slab loads, wait, store - and then re-reads its own stores for the planes: ~2 kIt round
 // trips per workgroup, 16.5 us per 798 x 5120 epilogue (two per layer in a prefill chunk).  Here a thread requests all slabs, the residual,
 // bias and norm weights of all its kIt column groups up front, keeps the row values in registers, and writes c and the planes from them.
 // Same sums in the same order (split order per element, the row's sum of squares in column-group order per thread): bit-identical.
-template <int kIt>
+// Eight slabs (o / down of a short prompt) fit the registers up to kIt = 5; us of projection and epilogue, walking / here, 100 rows: 4096 x 4096 28.8 / 22.6,
+// 5120 x 5120 34.4 / 28.5, 4096 x 12288 44.7 / 40.2; 223 rows 61.6 / 57.8 (more columns or slabs than that keep the walking form).
+template <int kIt, int SLABS>
 __global__ __launch_bounds__(256) void splitk_epilogue_norm_reg_kernel(const float* __restrict__ ws, int sk, int m, int n,
                                                                       const float* __restrict__ bias, const float* __restrict__ resid,
                                                                       float* __restrict__ c, int ldc, int epilogue,
@@ -640,13 +642,13 @@ __global__ __launch_bounds__(256) void splitk_epilogue_norm_reg_kernel(const flo
   const int row = blockIdx.x;
   const size_t plane = (size_t)m * n;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 t[kIt][4], rs[kIt], gw[kIt], sc4[kIt], b4[kIt];
+  f32x4 t[kIt][SLABS], rs[kIt], gw[kIt], sc4[kIt], b4[kIt];
 #pragma unroll
   for (int it = 0; it < kIt; ++it) {
     const int col = threadIdx.x * 4 + it * 1024;
     const bool live = col < n;
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < SLABS; ++s)
       t[it][s] = live ? *reinterpret_cast<const f32x4*>(ws + (s < sk ? s : sk - 1) * plane + (size_t)row * n + col) : zero;
     rs[it] = (live && epilogue == CHATTS_EPI_RESID) ? *reinterpret_cast<const f32x4*>(resid + (size_t)row * ldc + col) : zero;
     gw[it] = live ? *reinterpret_cast<const f32x4*>(norm_w + col) : zero;
@@ -661,7 +663,7 @@ __global__ __launch_bounds__(256) void splitk_epilogue_norm_reg_kernel(const flo
     f32x4 v = zero;
     if (col < n) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < SLABS; ++s)
         if (s < sk) { v.x += t[it][s].x; v.y += t[it][s].y; v.z += t[it][s].z; v.w += t[it][s].w; }
       if (scale) { v.x *= sc4[it].x; v.y *= sc4[it].y; v.z *= sc4[it].z; v.w *= sc4[it].w; }
       if (bias) { v.x += b4[it].x; v.y += b4[it].y; v.z += b4[it].z; v.w += b4[it].w; }
@@ -1088,17 +1090,22 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     const float* ws_f = reinterpret_cast<const float*>(a->workspace);
     const float* sc = a->w8 ? a->w8_scale : nullptr;
     const int its = (a->n + 1023) / 1024;
-    if (sk <= 4 && its <= 8 && opt_get(OPT_EPI_NORM_REG, 1) != 0) {      // all round trips of a thread at once (bit-identical; 13.5)
-#define CHATTS_EPI_REG(K) hipLaunchKernelGGL((splitk_epilogue_norm_reg_kernel<K>), dim3(a->m), dim3(256), 0, s, ws_f, sk, a->m, a->n, a->bias, \
-                                             a->resid, a->c, a->ldc, a->epilogue, sc, a->post_norm_w, a->post_norm_eps, a->post_hi, a->post_lo, a->ld_post)
-      switch (its) {
-        case 1: CHATTS_EPI_REG(1); break;
-        case 2: CHATTS_EPI_REG(2); break;
-        case 3: CHATTS_EPI_REG(3); break;
-        case 4: CHATTS_EPI_REG(4); break;
-        case 5: CHATTS_EPI_REG(5); break;
-        case 6: CHATTS_EPI_REG(6); break;
-        default: CHATTS_EPI_REG(8); break;
+    if ((sk <= 4 ? its <= 8 : sk <= 8 && its <= 5) && opt_get(OPT_EPI_NORM_REG, 1) != 0) {      // all round trips of a thread at once (bit-identical)
+#define CHATTS_EPI_REG(K, S) hipLaunchKernelGGL((splitk_epilogue_norm_reg_kernel<K, S>), dim3(a->m), dim3(256), 0, s, ws_f, sk, a->m, a->n, a->bias, \
+                                                a->resid, a->c, a->ldc, a->epilogue, sc, a->post_norm_w, a->post_norm_eps, a->post_hi, a->post_lo, a->ld_post)
+      switch (sk <= 4 ? its : 8 + its) {
+        case 1: CHATTS_EPI_REG(1, 4); break;
+        case 2: CHATTS_EPI_REG(2, 4); break;
+        case 3: CHATTS_EPI_REG(3, 4); break;
+        case 4: CHATTS_EPI_REG(4, 4); break;
+        case 5: CHATTS_EPI_REG(5, 4); break;
+        case 6: CHATTS_EPI_REG(6, 4); break;
+        case 7: case 8: CHATTS_EPI_REG(8, 4); break;
+        case 9: CHATTS_EPI_REG(1, 8); break;
+        case 10: CHATTS_EPI_REG(2, 8); break;
+        case 11: CHATTS_EPI_REG(3, 8); break;
+        case 12: CHATTS_EPI_REG(4, 8); break;
+        default: CHATTS_EPI_REG(5, 8); break;
       }
 #undef CHATTS_EPI_REG
       CHATTS_CHECK_LAUNCH("splitk_epilogue_norm_reg");
