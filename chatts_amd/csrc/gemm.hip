@@ -891,7 +891,7 @@ static bool use_stream(const ChattsLinearArgs* a) {
   return stream_multiblock(a->m, a->n, a->k, a->w8 != nullptr);
 }
 
-static int pick_stream_sk(int n, int k, bool w8) {
+static int pick_stream_sk(int m, int n, int k, bool w8) {
   const int tiles = (n + kStreamBN - 1) / kStreamBN, nk = k / stream_bk(w8);
   // ~one workgroup per CU (tools/stream_sweep.py: gate_up / lm_head want no split, qkv 4, o / down ~6); each split costs a
   // partials round trip and the epilogue launch
@@ -899,7 +899,8 @@ static int pick_stream_sk(int n, int k, bool w8) {
   int sk = 4 * tiles >= 3 * cus ? 1 : (cus + tiles / 2) / tiles;
   // fp8 W: a workgroup's 4 x 24 KB ring leaves room for ONE per CU, so a grid beyond the CU count runs a second, nearly empty round
   // (qkv, 56 tiles: 5 splits = 280 workgroups 19.3 us, 4 = 224 workgroups 13.9 us - profiles/r3_stream_sweep_fp8.txt)
-  if (w8 && sk > 1 && tiles * sk > cus) sk = cus / tiles;
+  // ... and so do several row blocks (96 to 144 KB of stages): 7168 x 5120, 100 rows, 5 splits 44.2 us, 4 splits 32.2
+  if ((w8 || m > 16) && sk > 1 && tiles * sk > cus) sk = cus / tiles;
   if (sk > nk / 4) sk = nk / 4;
   if (sk < 1) sk = 1;
   const int force_sk = opt_get(OPT_GEMM_SK, 0);
@@ -925,7 +926,7 @@ static int launch_stream_t(const GemmParams& p, const ChattsLinearArgs* a, int s
 // can the weight-streaming kernel run all members of ChattsLinearArgs.batch at once (and the plain split-K epilogue finish them)?
 bool gemm_batched_stream(const ChattsLinearArgs* a) {
   return a->m >= 2 && a->m <= 16 && use_stream(a) && !a->w8 && a->c && !a->c_hi && a->epilogue == CHATTS_EPI_NONE && a->n % 4 == 0 && a->ldc % 4 == 0 && a->c_stride % 4 == 0 &&
-         a->a_stride % 8 == 0 && a->w_stride % 8 == 0 && ((uintptr_t)a->c % 16) == 0 && opt_get(OPT_EPI_V4, 1) != 0 && pick_stream_sk(a->n * a->batch, a->k, false) <= 8;
+         a->a_stride % 8 == 0 && a->w_stride % 8 == 0 && ((uintptr_t)a->c % 16) == 0 && opt_get(OPT_EPI_V4, 1) != 0 && pick_stream_sk(a->m, a->n * a->batch, a->k, false) <= 8;
 }
 // K ranges of gemm_stream_kernel for these arguments if launch_gemm hands them to gemm_rows_kernel, which takes the same ranges (bit-identical) and
 // alone writes post_ss; 0: it does not.  Line: where K is split at all, and up to 8 rows; 8-bit weights beyond 4 rows only with eight K ranges (use_rows).
@@ -936,12 +937,12 @@ bool gemm_batched_stream(const ChattsLinearArgs* a) {
 // 4.20 -> 3.95 / 4.47 -> 4.47 / 4.53 -> 4.68 (hence the line).
 int gemm_takes_rows(const ChattsLinearArgs* a) {
   if (a->m > 8 || a->batch > 1 || opt_get(OPT_GEMM_SK, 0) != 0 || !use_stream(a)) return 0;
-  const int kps = k_per_split(a->k, pick_stream_sk(a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr)), sk = (a->k + kps - 1) / kps;
+  const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr)), sk = (a->k + kps - 1) / kps;
   return sk > 1 && use_rows(a, sk) ? sk : 0;
 }
 size_t gemm_workspace_batch(int m, int n, int k, int batch) {
   if (batch <= 1 || m < 2 || m > 16 || k % 64) return 0;
-  const int sk = pick_stream_sk(n * batch, k, false);
+  const int sk = pick_stream_sk(m, n * batch, k, false);
   return sk > 1 ? (size_t)batch * sk * m * n * sizeof(float) : 0;
 }
 
@@ -954,7 +955,7 @@ size_t gemm_workspace(int m, int n, int k) {
     if (g.sk > sk) sk = g.sk;
   }
   if ((m <= 16 && k % 64 == 0) || stream_multiblock(m, n, k, false)) {
-    sk2 = pick_stream_sk(n, k, false);         // (the fp8 variant's K-steps are twice as long: never more splits)
+    sk2 = pick_stream_sk(m, n, k, false);         // (the fp8 variant's K-steps are twice as long: never more splits)
     if (sk2 > sk) sk = sk2;
   }
   return sk > 1 ? (size_t)sk * m * n * sizeof(float) : 0;
@@ -976,7 +977,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   CHATTS_REQUIRE(!a->planes_tiled || ring, CHATTS_E_SHAPE, "linear: tiled planes are the prefill kernel's operand format (M=%d K=%d take another kernel)", a->m, a->k);
   CHATTS_REQUIRE(!ring || !a->w_tiled || (((uintptr_t)a->w_tiled % 16) == 0 && a->ldw == a->k), CHATTS_E_SHAPE, "linear: w_tiled needs 16-byte alignment and ldw == K");
   if (stream) {
-    sk = pick_stream_sk(a->n * batch, a->k, a->w8 != nullptr);
+    sk = pick_stream_sk(a->m, a->n * batch, a->k, a->w8 != nullptr);
     bm = 16;
   } else if (ring) {
     if (const int rc = check_ring_operands(a)) return rc;
