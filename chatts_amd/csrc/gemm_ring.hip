@@ -285,10 +285,12 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------------------------
-// (T, sk) per shape: a cost model in cycles of the slowest workgroup - rounds x (K-steps x step + a per-unit constant) + the split-K
-// epilogue launch.  Fitted to the probe build's numbers (profiles/r5_ring_probe_first.txt): a 64-deep step of a tile with f fragments
-// takes ~235 f + 900 cycles (f = 6: 2330, 7-8: 2650-2680, 9: 3020 - the 16 f MFMAs per SIMD and the (32 f + 256) x 128 bytes of LDS-DMA
-// overlap only partly), a unit costs ~9000 cycles of prologue + epilogue, a split-K epilogue ~6 us + its slab traffic at ~5 TB/s.
+// (T, sk) per shape: a cost model in cycles of the slowest workgroup - rounds x (K-steps x step + a per-unit constant) + the split-K epilogue launch.  Fitted to
+// 4500 measurements of every (T, sk) for 14 projections (K 2048 .. 13824, N 1536 .. 27648) at 100 .. 1300 rows: a 64-deep step of a tile with f fragments
+// takes 253 f + 1069 cycles (the 16 f MFMAs per SIMD and the (32 f + 256) x 128 bytes of LDS-DMA overlap only partly), a unit 4800 of prologue and stores, a
+// split-K epilogue 5 us (8 from five slabs on, more where its threads cannot ask for all slabs at once) and its slab traffic at ~4.5 to 5 TB/s, less
+// where the slabs outgrow 64 MB.  Over these shapes its pick is 0.8 % slower than the best pair in the mean; the constants before (235 f + 900, 9000 a unit, a
+// row-walking epilogue from five slabs on) gave 1.4 % and up to 17 %: 5120 x 13824 at 223 rows (3, 4) 80.3 us, now (2, 6) 72.5; 4096 x 4096 at 900 rows 80.8 / 71.4.
 void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, RingGeom& g) {
   const int F = (m + 15) / 16, P = (n + kRingBN - 1) / kRingBN, nk = k / 64;
   g.F = F; g.P = P;
@@ -300,17 +302,17 @@ void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, RingGeom
   if (tmax < tmin) tmax = tmin;
   for (int T = tmin; T <= tmax; ++T) {
     const int fmax = (F + T - 1) / T;
-    const double step = 235.0 * fmax + 900.0;
+    const double step = 253.0 * fmax + 1069.0;
     for (int sk = 1; sk <= 16; ++sk) {
       if (sk > 1 && nk / sk < 4) break;
       const long long units = (long long)T * P * sk;
       const long long rounds = (units + slots - 1) / slots;
       const int steps = (nk + sk - 1) / sk;
-      double t = (double)rounds * (steps * step + 9000.0);
-      // split-K epilogue: <= 4 slabs take the all-round-trips-at-once form (splitk_epilogue_norm_reg_kernel), more the row-walking one -
-      // measured at down_proj, M = 798 (profiles/r6_ring_geometry_sweep.txt): (T, sk) = (6, 2) 210 us against 224-227 for the (5, 5) the
-      // flat estimate used to pick
-      if (sk > 1) t += sk <= 4 ? 12000.0 + (double)(sk + 2) * m * n * 4.0 / 2500.0 : 24000.0 + (double)(sk + 2) * m * n * 4.0 / 1800.0;
+      double t = (double)rounds * (steps * step + 4800.0);
+      if (sk > 1) {
+        const double slabs = (double)m * n * 4.0;
+        t += (sk <= 4 ? 10200.0 : sk <= 8 ? 17600.0 : 30000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1840.0 : sk <= 4 ? 2200.0 : 2480.0);
+      }
       if (t < best) { best = t; bt = T; bs = sk; }
     }
   }
