@@ -96,8 +96,9 @@ struct RingGeom {
   int F, P;           // 16-row fragments of M, W panels
   int units;          // T * P * sk, ordered (split, panel, M-tile): the M-tiles of a panel are adjacent
   int wpx;            // workgroups per XCD (grid = 8 * wpx)
+  int nf;             // a panel is 64 nf rows (3 or 4)
 };
-void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, RingGeom& g);
+void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int force_nf, RingGeom& g);
 // the same kernel over lists of rows with weights of their own (experts): tiles [count][4] = {matrix, first place, places, -}, places of a tile
 // at most kRingTile; order != nullptr: place -> row of A = order[place] / top, else A is packed by place.  C is packed by place; p.m: rows of A - 1 at most
 struct RingGroup {

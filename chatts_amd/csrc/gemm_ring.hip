@@ -19,7 +19,7 @@
 //     fragments evenly over the two wave rows, and (T, split-K) are chosen per shape so that the units fill whole rounds
 //     (o / down: 6 x 20 x 2 = 240 units; qkv: 9 x 28 = 252; gate_up: 7 x 108 = 756 = 2.95 rounds).
 //
-// Geometry: unit = (K split, W panel of 256 rows, M-tile of f <= 10 fragments); 12 waves = 8 compute (2 x 4: wave row r holds
+// Geometry: unit = (K split, W panel of 256 rows (or 192: NF), M-tile of f <= 10 fragments); 12 waves = 8 compute (2 x 4: wave row r holds
 // ceil / floor of f / 2 fragments x 64 columns) + 4 loaders.  Half-stage slot (36 KB): A_hi [160][64 B] | A_lo | W [256][64 B]; 16-byte
 // chunk c of row r lives at chunk c ^ (((r >> 3) & 1) << 1) (conflict-free for the ds_read_b128 fragment reads; applied on the SOURCE
 // side of the DMA: lane l of a 16-row piece fetches global chunk (l & 3) ^ ((l >> 5) << 1)).
@@ -57,10 +57,12 @@ __device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const R
 }
 
 // SINGLE: the "bf16" speed mode - the lo plane is neither staged nor multiplied (activations rounded to bf16: NOT parity grade)
-template <bool SINGLE, bool GROUPED = false>
+// NF: column fragments of a compute wave - a panel is 64 NF rows of W
+template <bool SINGLE, bool GROUPED = false, int NF = 4>
 __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, const uint16_t* __restrict__ a_hi,
                                                                  const uint16_t* __restrict__ a_lo, int ldp, RingGeom g, RingGroup gr) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr int BN = 64 * NF;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // this workgroup's units: XCD x (= blockIdx % 8, observed; speed only) owns a contiguous eighth of the unit sequence and its
@@ -93,31 +95,35 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     // order - whole cache lines per request instead of 16 half lines (profiles/r6_feed_probe.txt)
     const bool wtiled = p.wt != nullptr, atiled = p.planes_tiled != 0;
     const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64, astep = atiled ? 1024 : 64;
-    const char* src[9];
-    int dst[9];
+    // three fragments do not hold whole (gate, up) pairs of 16 columns: there a gated product's W block is 8 gates and their 8 up rows
+    const bool mixed = NF == 3 && p.direct && epi_is_glu(p.epilogue);
+    const char* src[NF + 5];
+    int dst[NF + 5];
     int np = 0, nh_cur = 0, hh = 0, ucur = u0;
     auto setup = [&](int u) {
       int matrix = 0, places = 0;
       const RingUnit r = unit(u, matrix, places);
       nh_cur = r.nh;
       np = 0;
-      const int n0 = r.panel * kRingBN;
+      const int n0 = r.panel * BN;
       const size_t skip = GROUPED ? (size_t)matrix * gr.w_stride : 0;
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
+      for (int h = 0; h < NF; ++h) {
+        int wr = n0 + (L + 4 * h) * 16 + prow;
+        if (mixed) {
+          const int u = (n0 >> 1) + (L + 4 * h) * 8;
+          wr = (u >> 4) * 32 + (u & 15) + (prow & 7) + (prow >> 3) * 16;
+        }
+        if (wr > p.n - 1) wr = p.n - 1;
         if (wtiled) {
-          int rb = (n0 >> 4) + L + 4 * h;
-          const int rbmax = ((p.n + 15) >> 4) - 1;
-          if (rb > rbmax) rb = rbmax;
-          src[h] = reinterpret_cast<const char*>(p.wt + skip + ((size_t)rb * nkt + (r.kbeg >> 5)) * 512) + lane * 16;
+          const int rr = wr & 15;
+          src[h] = reinterpret_cast<const char*>(p.wt + skip + ((size_t)(wr >> 4) * nkt + (r.kbeg >> 5)) * 512) + (rr * 4 + (gchunk ^ ((rr >> 3) << 1))) * 16;
         } else {
-          int wr = n0 + (L + 4 * h) * 16 + prow;
-          if (wr > p.n - 1) wr = p.n - 1;
           src[h] = reinterpret_cast<const char*>(p.w + skip + (size_t)wr * p.ldw + r.kbeg + gchunk * 8);
         }
         dst[h] = kRingWOff + (L + 4 * h) * 1024;
       }
-      np = 4;
+      np = NF;
       const int na = SINGLE ? r.f : 2 * r.f;
 #pragma unroll
       for (int h = 0; h < 5; ++h) {
@@ -125,7 +131,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
         if (q < na) {
           const int plane = q >= r.f, frag = plane ? q - r.f : q;
           if (atiled) {
-            src[4 + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + ((size_t)((r.m0 >> 4) + frag) * nkt + (r.kbeg >> 5)) * 512) + lane * 16;
+            src[NF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + ((size_t)((r.m0 >> 4) + frag) * nkt + (r.kbeg >> 5)) * 512) + lane * 16;
           } else {
             int am = r.m0 + frag * 16 + prow;
             if constexpr (GROUPED) {
@@ -134,10 +140,10 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
             } else if (am > p.m - 1) {
               am = p.m - 1;
             }
-            src[4 + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + (size_t)am * ldp + r.kbeg + gchunk * 8);
+            src[NF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + (size_t)am * ldp + r.kbeg + gchunk * 8);
           }
-          dst[4 + h] = plane * kRingAPlane + frag * 1024;
-          np = 5 + h;
+          dst[NF + h] = plane * kRingAPlane + frag * 1024;
+          np = NF + 1 + h;
         }
       }
     };
@@ -147,8 +153,8 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
       char* base = smem + (gi & (kRingSlots - 1)) * kRingHalf;
       const size_t koffw = (size_t)hh * wstep, koffa = (size_t)hh * astep;
 #pragma unroll
-      for (int h = 0; h < 9; ++h)
-        if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < 4 ? koffw : koffa)), (lptr_t)(base + dst[h]), 16, 0, 0);
+      for (int h = 0; h < NF + 5; ++h)
+        if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < NF ? koffw : koffa)), (lptr_t)(base + dst[h]), 16, 0, 0);
       const int n = np;
       ++gi;
       if (++hh == nh_cur) {
@@ -190,33 +196,33 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
       gh += r.nh;
       continue;
     }
-    f32x4 acc[5][4];
+    f32x4 acc[5][NF];
 #pragma unroll
     for (int i = 0; i < 5; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NF; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     auto k_loop = [&](auto fml_c) {
       constexpr int FML = decltype(fml_c)::value;
-      bf16x8_t wf[2][4], alo[FML], ahi[FML];
-      const int a_off = rowblk * 1024 + lane_off, w_off = kRingWOff + wn * 4096 + lane_off;
+      bf16x8_t wf[2][NF], alo[FML], ahi[FML];
+      const int a_off = rowblk * 1024 + lane_off, w_off = kRingWOff + wn * NF * 1024 + lane_off;
       auto slot = [&](int h) { return smem + ((gh + h) & (kRingSlots - 1)) * kRingHalf; };
-      auto read_w = [&](const char* base, bf16x8_t (&dst)[4]) {
+      auto read_w = [&](const char* base, bf16x8_t (&dst)[NF]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[j] = *reinterpret_cast<const bf16x8_t*>(base + w_off + j * 1024);
+        for (int j = 0; j < NF; ++j) dst[j] = *reinterpret_cast<const bf16x8_t*>(base + w_off + j * 1024);
       };
       auto read_a = [&](const char* base, int plane, bf16x8_t (&dst)[FML]) {
 #pragma unroll
         for (int i = 0; i < FML; ++i) dst[i] = *reinterpret_cast<const bf16x8_t*>(base + plane * kRingAPlane + a_off + i * 1024);
       };
-      auto sweep = [&](const bf16x8_t (&af)[FML], const bf16x8_t (&wfr)[4]) {      // D = W . A^T: operands swapped
+      auto sweep = [&](const bf16x8_t (&af)[FML], const bf16x8_t (&wfr)[NF]) {      // D = W . A^T: operands swapped
 #pragma unroll
         for (int i = 0; i < FML; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wfr[j], af[i], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < NF; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wfr[j], af[i], acc[i][j], 0, 0, 0);
       };
       // half-step h (operands in registers) with the fragments of h + 1 requested behind the barrier
-      auto half = [&](int h, const bf16x8_t (&wcur)[4], bf16x8_t (&wnxt)[4], bool more) {
+      auto half = [&](int h, const bf16x8_t (&wcur)[NF], bf16x8_t (&wnxt)[NF], bool more) {
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!SINGLE) sweep(alo, wcur);
         __builtin_amdgcn_sched_barrier(0);
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     }
     gh += r.nh;
 
-    const int tok0 = r.m0 + rowblk * 16, fb0 = r.panel * kRingBN + wn * 64;
+    const int tok0 = r.m0 + rowblk * 16, fb0 = r.panel * BN + wn * 16 * NF;
     const bool planes = p.c_hi != nullptr;
     if (!p.direct) ring_store<kStRaw, false>(p, acc, fml, tok0, fb0, lane, r.split);
     else if (p.epilogue == CHATTS_EPI_SWIGLU) {
@@ -291,50 +297,59 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 // split-K epilogue 5 us (8 from five slabs on, more where its threads cannot ask for all slabs at once) and its slab traffic at ~4.5 to 5 TB/s, less
 // where the slabs outgrow 64 MB.  Over these shapes its pick is 0.8 % slower than the best pair in the mean; the constants before (235 f + 900, 9000 a unit, a
 // row-walking epilogue from five slabs on) gave 1.4 % and up to 17 %: 5120 x 13824 at 223 rows (3, 4) 80.3 us, now (2, 6) 72.5; 4096 x 4096 at 900 rows 80.8 / 71.4.
-void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, RingGeom& g) {
-  const int F = (m + 15) / 16, P = (n + kRingBN - 1) / kRingBN, nk = k / 64;
-  g.F = F; g.P = P;
+// Panels of 192 rows are the second width: a step costs 215 f + 1080 there, dearer per column, but where panels of 256 leave CUs without a unit it fills them:
+// 24576 x 4096 gated, 223 rows: 96 panels x 2 tiles on 192 CUs 94.5 us, 128 x 2 on 256 CUs 90.3; 6144 x 4096 at 223 rows 36.4 / 34.2, 5120 x 5120 at 150 rows
+// 36.9 / 34.4, 6144 x 2048 at 380 rows 31.5 / 26.6; 27648 x 5120 (108 panels; 144 would need two rounds) stays at 256: 125.7 / 162.
+void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int force_nf, RingGeom& g) {
+  const int F = (m + 15) / 16, nk = k / 64;
+  g.F = F;
   const int slots = cus >= 8 ? (cus / 8) * 8 : 8;
   double best = 1e30;
   const int tmin = (F + kRingMaxF - 1) / kRingMaxF;
-  int bt = tmin, bs = 1;
+  int bt = tmin, bs = 1, bf = 4;
   int tmax = (F + 2) / 3;                              // >= 3 fragments per tile
   if (tmax < tmin) tmax = tmin;
-  for (int T = tmin; T <= tmax; ++T) {
-    const int fmax = (F + T - 1) / T;
-    const double step = 253.0 * fmax + 1069.0;
-    for (int sk = 1; sk <= 16; ++sk) {
-      if (sk > 1 && nk / sk < 4) break;
-      const long long units = (long long)T * P * sk;
-      const long long rounds = (units + slots - 1) / slots;
-      const int steps = (nk + sk - 1) / sk;
-      double t = (double)rounds * (steps * step + 4800.0);
-      if (sk > 1) {
-        const double slabs = (double)m * n * 4.0;
-        t += (sk <= 4 ? 10200.0 : sk <= 8 ? 17600.0 : 30000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1840.0 : sk <= 4 ? 2200.0 : 2480.0);
+  for (int nf = 4; nf >= 3; --nf) {
+    if (force_nf && nf != force_nf) continue;
+    const int P = (n + 64 * nf - 1) / (64 * nf);
+    for (int T = tmin; T <= tmax; ++T) {
+      const int fmax = (F + T - 1) / T;
+      const double step = nf == 4 ? 253.0 * fmax + 1069.0 : 215.0 * fmax + 1080.0;
+      if ((double)T * P * nk * step > best * slots) break;      // (the work itself, evenly spread: more tiles only add to it)
+      for (int sk = 1; sk <= 16; ++sk) {
+        if (sk > 1 && nk / sk < 4) break;
+        const long long units = (long long)T * P * sk;
+        const long long rounds = (units + slots - 1) / slots;
+        const int steps = (nk + sk - 1) / sk;
+        double t = (double)rounds * (steps * step + 4800.0);
+        if (sk > 1) {
+          const double slabs = (double)m * n * 4.0;
+          t += (sk <= 4 ? 10200.0 : sk <= 8 ? 17600.0 : 30000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1840.0 : sk <= 4 ? 2200.0 : 2480.0);
+        }
+        if (t < best) { best = t; bt = T; bs = sk; bf = nf; }
       }
-      if (t < best) { best = t; bt = T; bs = sk; }
     }
   }
   if (force_t >= tmin && force_t <= F) bt = force_t;
   if (force_sk >= 1 && force_sk <= 16 && nk / force_sk >= 1) bs = force_sk;
-  g.T = bt; g.sk = bs;
-  g.units = bt * P * bs;
+  g.T = bt; g.sk = bs; g.nf = bf;
+  g.P = (n + 64 * bf - 1) / (64 * bf);
+  g.units = bt * g.P * bs;
   int wpx = (g.units + 7) / 8;
   if (wpx > slots / 8) wpx = slots / 8;
   g.wpx = wpx;
 }
 
-template <bool SINGLE>
+template <bool SINGLE, int NF>
 static int launch_ring_t(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, hipStream_t s) {
   static bool configured = false;     // > 64 KB of dynamic LDS must be opted into once
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<SINGLE>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<SINGLE, false, NF>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                              kRingLds);
     CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_ring: cannot reserve %d bytes of LDS: %s", kRingLds, hipGetErrorString(e));
     configured = true;
   }
-  hipLaunchKernelGGL(gemm_ring_kernel<SINGLE>, dim3(8 * g.wpx), dim3(kRingThreads), kRingLds, s, p, a_hi, a_lo, ldp, g, RingGroup{});
+  hipLaunchKernelGGL((gemm_ring_kernel<SINGLE, false, NF>), dim3(8 * g.wpx), dim3(kRingThreads), kRingLds, s, p, a_hi, a_lo, ldp, g, RingGroup{});
   return CHATTS_OK;
 }
 int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGroup& gr, int most_tiles, hipStream_t s) {
@@ -355,7 +370,8 @@ int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t*
   return CHATTS_OK;
 }
 int launch_ring(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, bool single, hipStream_t s) {
-  return single ? launch_ring_t<true>(p, a_hi, a_lo, ldp, g, s) : launch_ring_t<false>(p, a_hi, a_lo, ldp, g, s);
+  if (g.nf == 3) return single ? launch_ring_t<true, 3>(p, a_hi, a_lo, ldp, g, s) : launch_ring_t<false, 3>(p, a_hi, a_lo, ldp, g, s);
+  return single ? launch_ring_t<true, 4>(p, a_hi, a_lo, ldp, g, s) : launch_ring_t<false, 4>(p, a_hi, a_lo, ldp, g, s);
 }
 
 // bf16 [rows, k] row-major -> the tiled layout: block (b = row / 16, t = k / 32) is 1 KB at ((b * k / 32) + t) * 1 KB; inside it the 16-byte

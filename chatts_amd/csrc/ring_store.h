@@ -37,10 +37,11 @@ __device__ __forceinline__ RingUnit ring_unit(const GemmParams& p, const RingGeo
   return r;
 }
 
-// The epilogue of one wave: acc[i][j] = D[feature = fb .. fb + 3][token] of fragment pair (i, j), fb = n0 + wn * 64 + j * 16 + (lane >> 4) * 4,
+// The epilogue of one wave: acc[i][j] = D[feature = fb .. fb + 3][token] of fragment pair (i, j), fb = fb0 + j * 16 + (lane >> 4) * 4,
 // token = m0 + rowbase + i * 16 + (lane & 15).  MODE / PLANES are compile-time: no branches, all loads of a row block in flight at once.
-template <int MODE, bool PLANES>
-__device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&acc)[5][4], int fml, int tok0, int fb0, int lane, int split) {
+// Three column fragments and a gated epilogue: a fragment is 8 gates (lanes 0 - 31) and their 8 up rows (lanes 32 - 63), fragment j the units fb0 / 2 + 8 j ..
+template <int MODE, bool PLANES, int NF>
+__device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&acc)[5][NF], int fml, int tok0, int fb0, int lane, int split) {
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
   const int tl = lane & 15, fq = (lane >> 4) * 4;
   auto put = [&](size_t row_off_c, size_t row_off_p, int col, const float (&v)[4]) __attribute__((always_inline)) {
@@ -66,9 +67,36 @@ __device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&ac
       if (i < fml) {
         const int tok = tok0 + i * 16 + tl;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NF; ++j) {
           const int fb = fb0 + j * 16 + fq;
           if (tok < p.m && fb < p.n) *reinterpret_cast<f32x4*>(ws + (size_t)tok * p.n + fb) = acc[i][j];
+        }
+      }
+    }
+  } else if constexpr ((MODE == kStSwiglu || MODE == kStClampGlu || MODE == kStGeglu) && NF == 3) {
+    constexpr int kEpi = MODE == kStSwiglu ? CHATTS_EPI_SWIGLU : (MODE == kStGeglu ? CHATTS_EPI_GEGLU : CHATTS_EPI_CLAMPGLU);
+    const int uq = (lane >> 4 & 1) * 4;           // this lane's units within a fragment; lanes 32 - 63 hand theirs over
+    f32x4 bg[NF], bu[NF];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      const int u = (fb0 >> 1) + j * 8 + uq, fb = 2 * u < p.n ? (u >> 4) * 32 + (u & 15) : 0;
+      bg[j] = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + fb) : (f32x4){0.f, 0.f, 0.f, 0.f};
+      bu[j] = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + fb + 16) : (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      if (i < fml) {
+        const int tok = tok0 + i * 16 + tl;
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+          const int u = (fb0 >> 1) + j * 8 + uq;
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float up = __shfl_xor(acc[i][j][r], 32, 64);
+            v[r] = glu_value(kEpi, acc[i][j][r] + bg[j][r], up + bu[j][r], p.glu_limit, p.glu_alpha);
+          }
+          if (lane < 32 && tok < p.m && 2 * u < p.n) put((size_t)tok * p.ldc, (size_t)tok * p.ldcp, u, v);
         }
       }
     }
@@ -99,9 +127,9 @@ __device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&ac
       }
     }
   } else {
-    f32x4 b4[4];
+    f32x4 b4[NF];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NF; ++j) {
       int fb = fb0 + j * 16 + fq;
       if (fb >= p.n) fb = 0;
       b4[j] = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + fb) : (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -111,17 +139,17 @@ __device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&ac
       if (i < fml) {
         const int tok = tok0 + i * 16 + tl;
         const int tokc = tok < p.m ? tok : p.m - 1;      // clamped: the loads are unconditional, the stores masked
-        f32x4 rs[4];
+        f32x4 rs[NF];
         if constexpr (MODE == kStResid) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+          for (int j = 0; j < NF; ++j) {
             int fb = fb0 + j * 16 + fq;
             if (fb >= p.n) fb = 0;
             rs[j] = *reinterpret_cast<const f32x4*>(p.resid + (size_t)tokc * p.ldc + fb);
           }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NF; ++j) {
           const int fb = fb0 + j * 16 + fq;
           float v[4];
 #pragma unroll
