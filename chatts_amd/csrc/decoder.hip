@@ -15,8 +15,7 @@ int launch_gemm_f32(const ChattsLinearArgs* a, hipStream_t s);
 bool gemm_batched_stream(const ChattsLinearArgs* a);
 size_t gemm_workspace_batch(int m, int n, int k, int batch);
 int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope = nullptr, bool* rope_done = nullptr, const ChattsNormChain* chain = nullptr);
-int gemm_takes_rows(const ChattsLinearArgs* a);
-int rows_grid(int n, int epilogue);
+int gemm_post_ss_parts(const ChattsLinearArgs* a);
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w,
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
@@ -69,8 +68,8 @@ extern "C" int chatts_linear_post_ss_parts(const ChattsLinearArgs* a) {
   const bool ok = a && a->w && a->m >= 2 && a->m <= 16 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && a->ldc >= a->n && a->ldw >= a->k && (!a->w8 || a->ldw8 >= a->k) &&
                   a->post_norm_w && ((uintptr_t)a->post_norm_w % 16) == 0 && a->post_hi && a->post_lo && a->ld_post >= a->n && a->ld_post % 4 == 0 &&
                   ((uintptr_t)a->post_hi % 8) == 0 && ((uintptr_t)a->post_lo % 8) == 0 && a->post_hi != a->a_hi && a->c && !a->c_hi &&
-                  (a->epilogue == CHATTS_EPI_NONE || a->epilogue == CHATTS_EPI_RESID) && gemm_takes_rows(a);
-  const int parts = ok ? rows_grid(a->n, a->epilogue) : 0;
+                  (a->epilogue == CHATTS_EPI_NONE || a->epilogue == CHATTS_EPI_RESID);
+  const int parts = ok ? gemm_post_ss_parts(a) : 0;
   return parts <= 256 ? parts : 0;
 }
 extern "C" size_t chatts_linear_workspace(int m, int n, int k) { return gemm_workspace(m, n, k); }
@@ -260,7 +259,7 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
 
 // The residual-updating projection (o_proj / down_proj, tp_world == 1) also produces the NEXT projection's operand:
 // RMSNorm(x) with `next_norm_w` as planes 0, when that projection will take the plane path for the same M.
-// The same for few rows (layer_part_batched), without the norm's own launch: the projection writes norm_w * x as planes 1 and the sums of squares,
+// The same for few rows (layer_part_batched), without waiting for a row's sum: the projection writes norm_w * x as planes 1 and the sums of squares,
 // and the next projection multiplies by 1 / rms.  Planes 1, because workgroups that are done write them while others still read A (planes 0).
 static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormChain* chain, const float* next_norm_w, bool next_fp8) {
   if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || !d->b.delta || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;

@@ -793,6 +793,51 @@ __global__ __launch_bounds__(256) void splitk_epilogue_norm_q_kernel(const float
   }
 }
 
+// The epilogue of few rows (2 .. 16) that leaves the factor 1 / rms of the norm behind it to the projection that reads the planes (row_ss): with no row's sum to
+// wait for, a wave takes 256 columns of a row, all its round trips at once, and writes c, the planes of norm_w * c and its part of the sum of squares.
+// splitk_epilogue_norm_q_kernel, which ran here, has each of its eight workgroups of a row sum the whole row (16 MB of slabs from L2): 2.8 us more a launch inside a
+// step; 14B fp8, 16 / 8 / 6 sequences 5.79 -> 5.52 / 4.42 -> 4.16 / 4.42 -> 4.06 ms, 8B bf16, 12: 4.20 -> 3.97, 14B int8, 10: 5.32 -> 5.05.
+constexpr int kEpiSsCols = 256;
+__global__ __launch_bounds__(64) void splitk_epilogue_ss_kernel(const float* ws, int sk, int m, int n, const float* bias, const float* resid, float* c, int ldc, int epilogue, const float* scale,
+                                                                const float* norm_w, float* post_ss, uint16_t* hi, uint16_t* lo, int ldp) {
+  const int row = blockIdx.y, col = blockIdx.x * kEpiSsCols + threadIdx.x * 4;
+  const bool live = col < n;
+  const int at = live ? col : 0;
+  const size_t plane = (size_t)m * n;
+  f32x4 t[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) t[s] = *reinterpret_cast<const f32x4*>(ws + (s < sk ? s : sk - 1) * plane + (size_t)row * n + at);
+  const f32x4 g = *reinterpret_cast<const f32x4*>(norm_w + at);
+  f32x4 r = {0.f, 0.f, 0.f, 0.f}, sc = r, b = r, v = r;
+  if (epilogue == CHATTS_EPI_RESID) r = *reinterpret_cast<const f32x4*>(resid + (size_t)row * ldc + at);
+  if (scale) sc = *reinterpret_cast<const f32x4*>(scale + at);
+  if (bias) b = *reinterpret_cast<const f32x4*>(bias + at);
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+    if (s < sk) { v.x += t[s].x; v.y += t[s].y; v.z += t[s].z; v.w += t[s].w; }
+  if (scale) { v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w; }
+  if (bias) { v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+  if (epilogue == CHATTS_EPI_RESID) { v.x = r.x + v.x; v.y = r.y + v.y; v.z = r.z + v.z; v.w = r.w + v.w; }
+  const float ss = wave_sum(live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f);
+  if (threadIdx.x == 0) post_ss[row * kSsStride + blockIdx.x] = ss;
+  if (!live) return;
+  *reinterpret_cast<f32x4*>(c + (size_t)row * ldc + col) = v;
+  const float o[4] = {g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w};
+  typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+  bf16x4_t hv, lv;
+  {
+#pragma clang fp contract(off)   // lo must be the split of the ROUNDED product
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const __bf16 h = (__bf16)o[j];
+      hv[j] = h;
+      lv[j] = (__bf16)(o[j] - (float)h);
+    }
+  }
+  *reinterpret_cast<bf16x4_t*>(hi + (size_t)row * ldp + col) = hv;
+  *reinterpret_cast<bf16x4_t*>(lo + (size_t)row * ldp + col) = lv;
+}
+
 // The qkv projection's split-K epilogue that also does rope_kv_kernel's work (prefill): one wave per (token, head) sums the head's
 // 128 columns over the slabs in split order, adds the bias - splitk_epilogue_kernel's arithmetic - and hands the two values per lane
 // to rope_kv_head: q rotated into c, K / V rows into the cache.  One pass over the [T, 7168] rows less per layer.
@@ -929,16 +974,28 @@ bool gemm_batched_stream(const ChattsLinearArgs* a) {
          a->a_stride % 8 == 0 && a->w_stride % 8 == 0 && ((uintptr_t)a->c % 16) == 0 && opt_get(OPT_EPI_V4, 1) != 0 && pick_stream_sk(a->m, a->n * a->batch, a->k, false) <= 8;
 }
 // K ranges of gemm_stream_kernel for these arguments if launch_gemm hands them to gemm_rows_kernel, which takes the same ranges (bit-identical) and
-// alone writes post_ss; 0: it does not.  Line: where K is split at all, and up to 8 rows; 8-bit weights beyond 4 rows only with eight K ranges (use_rows).
+// writes post_ss in the same launch; 0: it does not.  Line: where K is split at all, and up to 8 rows; 8-bit weights beyond 4 rows only with eight K ranges (use_rows).
 // A workgroup of it reads all of X (~55 KB a us and CU), which beyond that costs more than the launch it saves.  us with the epilogue launch / in
 // one: bf16, 5 rows, 4096 x 4096: 9.9 / 9.0, 6144 x 4096: 12.8 / 11.2, 4096 x 12288: 19.9 / 20.5; 8 rows: 10.4 / 9.7, 12.9 / 11.9, 20.1 / 23.5.  fp8: 5120 x
 // 13824 (six ranges) 2 / 5 / 8 rows: 15.7 / 16.1 / 16.1 against 17.9 / 19.7 / 22.8.  On top of that comes the RMSNorm that moves into the launch (3 - 4 us
 // of a chain).  Whole steps: 8B bf16, 2 / 5 sequences 3.90 -> 3.59 / 4.24 -> 4.04 ms, 14B bf16, 8: 6.53 -> 6.21, 8B int8, 7: 3.20 -> 2.92, 14B fp8, 2 / 6 / 8:
 // 4.20 -> 3.95 / 4.47 -> 4.47 / 4.53 -> 4.68 (hence the line).
+static int stream_ranges(const ChattsLinearArgs* a) {
+  const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr));
+  return (a->k + kps - 1) / kps;
+}
 int gemm_takes_rows(const ChattsLinearArgs* a) {
   if (a->m > 8 || a->batch > 1 || opt_get(OPT_GEMM_SK, 0) != 0 || !use_stream(a)) return 0;
-  const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr)), sk = (a->k + kps - 1) / kps;
+  const int sk = stream_ranges(a);
   return sk > 1 && use_rows(a, sk) ? sk : 0;
+}
+// parts of post_ss that launch_gemm would write for these arguments (post_norm_w and planes are there), 0: it would not
+int gemm_post_ss_parts(const ChattsLinearArgs* a) {
+  if (gemm_takes_rows(a)) return rows_grid(a->n, a->epilogue);
+  if (a->m > 16 || a->batch > 1 || !use_stream(a) || a->ldc % 4 || ((uintptr_t)a->c % 16) || ((uintptr_t)a->resid % 16) || ((uintptr_t)a->bias % 16) ||
+      (a->w8 && ((uintptr_t)a->w8_scale % 16)) || ((uintptr_t)a->workspace % 16)) return 0;
+  const int sk = stream_ranges(a);
+  return sk > 1 && sk <= 8 ? (a->n + kEpiSsCols - 1) / kEpiSsCols : 0;
 }
 size_t gemm_workspace_batch(int m, int n, int k, int batch) {
   if (batch <= 1 || m < 2 || m > 16 || k % 64) return 0;
@@ -1026,7 +1083,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
       return chatts_rmsnorm_planes(a->c, a->post_norm_w, a->post_hi, a->post_lo, a->ld_post, a->m, a->n, a->post_norm_eps, reinterpret_cast<chatts_stream_t>(s));
     return CHATTS_OK;
   }
-  CHATTS_REQUIRE(!ch.post_ss, CHATTS_E_SHAPE, "linear: post_ss is written by the few-rows kernel only (M=%d N=%d K=%d take another one)", a->m, a->n, a->k);
+  CHATTS_REQUIRE(!ch.post_ss || gemm_post_ss_parts(a) > 0, CHATTS_E_SHAPE, "linear: post_ss is written where K is split over few rows (M=%d N=%d K=%d is not)", a->m, a->n, a->k);
   const int nt_count = (a->n + 127) / 128, mt_count = (a->m + bm - 1) / bm;
   dim3 grid(8 * ((nt_count + 7) / 8) * mt_count, 1, sk), block(256);
   if (stream) {
@@ -1072,6 +1129,12 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     }
   }
   CHATTS_CHECK_LAUNCH("gemm_bf16x2");
+  if (ch.post_ss) {
+    hipLaunchKernelGGL(splitk_epilogue_ss_kernel, dim3((a->n + kEpiSsCols - 1) / kEpiSsCols, a->m), dim3(64), 0, s, reinterpret_cast<const float*>(a->workspace), sk, a->m, a->n, a->bias,
+                       a->resid, a->c, a->ldc, a->epilogue, a->w8 ? a->w8_scale : nullptr, a->post_norm_w, ch.post_ss, a->post_hi, a->post_lo, a->ld_post);
+    CHATTS_CHECK_LAUNCH("splitk_epilogue_ss");
+    return CHATTS_OK;
+  }
   const bool post_norm = a->post_norm_w != nullptr;
   if (sk > 1 && post_norm) {        // epilogue + the consumer's RMSNorm in one row-wise launch
     const int qsplit = opt_get(OPT_EPI_NORM_Q, 8);

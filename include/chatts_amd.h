@@ -246,9 +246,9 @@ typedef struct ChattsLinearArgs {
 #define CHATTS_W8_FP8 0
 #define CHATTS_W8_INT8 1
 /* chatts_linear with an RMSNorm whose producer and consumer are both projections of few rows (decoding for several sequences), without a launch
- * between them.  Producer (2 <= M <= 8): post_ss, with the call's post_norm_w, post_hi, post_lo and where chatts_linear_post_ss_parts() > 0 - the planes
- * are post_norm_w * c WITHOUT the factor 1 / rms, and post_ss (float [16][256], 16-byte aligned) receives the sums of squares of c's rows, one part per
- * workgroup.  Consumer (2 <= M <= 16 on planes): row_ss, the same array, row_ss_parts of each row's 256 places in use, and row_eps - row m of the product is
+ * of its own between them.  Producer (2 <= M <= 16): post_ss, with the call's post_norm_w, post_hi, post_lo and where chatts_linear_post_ss_parts() > 0 - the planes
+ * are post_norm_w * c WITHOUT the factor 1 / rms, and post_ss (float [16][256], 16-byte aligned) receives the sums of squares of c's rows, in
+ * parts.  Consumer (2 <= M <= 16 on planes): row_ss, the same array, row_ss_parts of each row's 256 places in use, and row_eps - row m of the product is
  * multiplied by 1 / sqrt(sum of its parts / K + row_eps) before scale, bias and epilogue. */
 typedef struct ChattsNormChain {
   float* post_ss;
@@ -257,7 +257,7 @@ typedef struct ChattsNormChain {
   float row_eps;
 } ChattsNormChain;
 int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* chain, chatts_stream_t stream);
-/* Host-only query: parts that this call would write to post_ss, 0 = it cannot (other shapes take kernels that do not hold whole columns). */
+/* Host-only query: parts that this call would write to post_ss, 0 = it cannot (K is not split, or the operands are not aligned). */
 int chatts_linear_post_ss_parts(const ChattsLinearArgs* a);
 size_t chatts_linear_workspace(int m, int n, int k);
 size_t chatts_linear_workspace_batch(int m, int n, int k, int batch);

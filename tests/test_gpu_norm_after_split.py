@@ -1,0 +1,46 @@
+"""The RMSNorm between two projections of few rows where K of the first is split over workgroups (splitk_epilogue_ss_kernel): c bit for bit what the call without
+the norm gives, and the second projection against float64; rows that end inside a wave's 256 columns, in place, rows of very different size."""
+import ctypes as C
+
+import pytest
+import torch
+
+from chatts_amd import _lib
+from tests.test_gpu_rows import DEV, args, planes, problem, rel, run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def lib():
+    return _lib.load()
+
+
+@pytest.mark.parametrize("form", ["bf16", "fp8", "int8"])
+@pytest.mark.parametrize("m,h,k,n2", [(9, 5120, 5120, 7168), (16, 4096, 4096, 6144), (12, 1152, 2048, 512), (16, 5120, 13824, 27648), (6, 5120, 5120, 7168), (16, 384, 1536, 4096)])
+def test_norm_after_a_split(lib, form, m, h, k, n2):
+    x, w1, _, resid, q1, s1 = problem(m, h, k, form, h)
+    _, w2, _, _, q2, s2 = problem(m, n2, h, form, n2)
+    resid *= 10.0 ** torch.linspace(-3, 3, m, device=DEV)[:, None]
+    nw = 1 + 0.1 * torch.randn(h, device=DEV)
+    hi, lo = planes(lib, x)
+    new = resid.double() + x.double() @ w1.double().T
+    want = (new * torch.rsqrt((new * new).mean(1, keepdim=True) + 1e-6) * nw.double()) @ w2.double().T
+    plain = torch.empty_like(resid)
+    run(lib, args(m, h, k, hi, lo, w1, q1, s1, form, plain, resid=resid.data_ptr(), ldc=h, epilogue=_lib.EPI_RESID), m, h, k)
+    ph, pl = (torch.empty((m, h), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ss = torch.full((16, 256), float("nan"), device=DEV)
+    c = resid.clone()
+    a = args(m, h, k, hi, lo, w1, q1, s1, form, c, resid=c.data_ptr(), ldc=h, epilogue=_lib.EPI_RESID, post_norm_w=nw.data_ptr(), post_hi=ph.data_ptr(), post_lo=pl.data_ptr(), ld_post=h)
+    parts = int(lib.chatts_linear_post_ss_parts(C.byref(a)))
+    assert 1 <= parts <= 256
+    run(lib, a, m, h, k, _lib.NormChain(post_ss=ss.data_ptr()))
+    assert torch.equal(c, plain) and bool((rel(c, new) < 1e-5))
+    prod = c * nw
+    assert torch.equal(ph, prod.bfloat16()) and torch.equal(pl, (prod - prod.bfloat16().float()).bfloat16())
+    # at most 4 + 6 roundings of positive float32 terms
+    assert bool(((ss[:m, :parts].double().sum(1) / (c.double() ** 2).sum(1) - 1).abs() < 10 * 2.0 ** -24).all())
+    out = torch.full((m, n2), float("nan"), device=DEV)
+    run(lib, args(m, n2, h, ph, pl, w2, q2, s2, form, out, ldc=n2, epilogue=_lib.EPI_NONE), m, n2, h, _lib.NormChain(row_ss=ss.data_ptr(), row_ss_parts=parts, row_eps=1e-6))
+    for i in range(m):
+        assert rel(out[i], want[i]) < 2e-5                # (x to 2^-17, sums in 32 bits)
