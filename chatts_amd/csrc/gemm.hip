@@ -794,48 +794,50 @@ __global__ __launch_bounds__(256) void splitk_epilogue_norm_q_kernel(const float
 }
 
 // The epilogue of few rows (2 .. 16) that leaves the factor 1 / rms of the norm behind it to the projection that reads the planes (row_ss): with no row's sum to
-// wait for, a wave takes 256 columns of a row, all its round trips at once, and writes c, the planes of norm_w * c and its part of the sum of squares.
-// splitk_epilogue_norm_q_kernel, which ran here, has each of its eight workgroups of a row sum the whole row (16 MB of slabs from L2): 2.8 us more a launch inside a
-// step; 14B fp8, 16 / 8 / 6 sequences 5.79 -> 5.52 / 4.42 -> 4.16 / 4.42 -> 4.06 ms, 8B bf16, 12: 4.20 -> 3.97, 14B int8, 10: 5.32 -> 5.05.
-constexpr int kEpiSsCols = 256;
-__global__ __launch_bounds__(64) void splitk_epilogue_ss_kernel(const float* ws, int sk, int m, int n, const float* bias, const float* resid, float* c, int ldc, int epilogue, const float* scale,
-                                                                const float* norm_w, float* post_ss, uint16_t* hi, uint16_t* lo, int ldp) {
-  const int row = blockIdx.y, col = blockIdx.x * kEpiSsCols + threadIdx.x * 4;
-  const bool live = col < n;
-  const int at = live ? col : 0;
+// wait for, every wave takes the columns of one part, a round trip for all slabs of 4 columns a lane, and writes c, the planes of norm_w * c and its part of the
+// sums of squares.  Parts and the order within them are gemm_rows_kernel's: a row's bits do not depend on which of the two ran.
+// splitk_epilogue_norm_q_kernel, which ran here, has each of its eight workgroups of a row sum the whole row (16 MB of slabs from L2): 2 us more a launch inside a
+// step; 14B fp8, 16 / 8 / 6 sequences 5.86 -> 5.68 / 4.46 -> 4.22 / 4.41 -> 4.14 ms, 8B bf16, 12: 4.15 -> 4.00.  (Parts of 256 columns a wave, whose last bits differ
+// from the few-rows kernel's, took 0.8 us less a launch.)
+__global__ __launch_bounds__(1024) void splitk_epilogue_ss_kernel(const float* ws, int sk, int m, int n, const float* bias, const float* resid, float* c, int ldc, int epilogue, const float* scale,
+                                                                const float* norm_w, float* post_ss, uint16_t* hi, uint16_t* lo, int ldp, int groups_each, int groups_more) {
+  __shared__ float ss_s[16][16];
+  const int b0 = (int)blockIdx.x, more = b0 < groups_more, lane = threadIdx.x & 63, tok = lane & 15, kc = lane >> 4, f = threadIdx.x >> 6;
+  const int groups = groups_each + more, g0 = b0 * groups_each + (more ? b0 : groups_more);
   const size_t plane = (size_t)m * n;
-  f32x4 t[8];
+  const int row = tok < m ? tok : 0;
+  {                                                    // a wave: 4 groups of 4 columns, 16 rows
+    const bool live = tok < m && 4 * f + kc < groups;
+    const int col = (live ? g0 + 4 * f + kc : g0) * 4;
+    f32x4 t[8];
 #pragma unroll
-  for (int s = 0; s < 8; ++s) t[s] = *reinterpret_cast<const f32x4*>(ws + (s < sk ? s : sk - 1) * plane + (size_t)row * n + at);
-  const f32x4 g = *reinterpret_cast<const f32x4*>(norm_w + at);
-  f32x4 r = {0.f, 0.f, 0.f, 0.f}, sc = r, b = r, v = r;
-  if (epilogue == CHATTS_EPI_RESID) r = *reinterpret_cast<const f32x4*>(resid + (size_t)row * ldc + at);
-  if (scale) sc = *reinterpret_cast<const f32x4*>(scale + at);
-  if (bias) b = *reinterpret_cast<const f32x4*>(bias + at);
+    for (int s = 0; s < 8; ++s) t[s] = *reinterpret_cast<const f32x4*>(ws + (s < sk ? s : sk - 1) * plane + (size_t)row * n + col);
+    const f32x4 g = *reinterpret_cast<const f32x4*>(norm_w + col);
+    f32x4 r = {0.f, 0.f, 0.f, 0.f}, sc = r, b = r, v = r;
+    if (epilogue == CHATTS_EPI_RESID) r = *reinterpret_cast<const f32x4*>(resid + (size_t)row * ldc + col);
+    if (scale) sc = *reinterpret_cast<const f32x4*>(scale + col);
+    if (bias) b = *reinterpret_cast<const f32x4*>(bias + col);
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
-    if (s < sk) { v.x += t[s].x; v.y += t[s].y; v.z += t[s].z; v.w += t[s].w; }
-  if (scale) { v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w; }
-  if (bias) { v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
-  if (epilogue == CHATTS_EPI_RESID) { v.x = r.x + v.x; v.y = r.y + v.y; v.z = r.z + v.z; v.w = r.w + v.w; }
-  const float ss = wave_sum(live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f);
-  if (threadIdx.x == 0) post_ss[row * kSsStride + blockIdx.x] = ss;
-  if (!live) return;
-  *reinterpret_cast<f32x4*>(c + (size_t)row * ldc + col) = v;
-  const float o[4] = {g.x * v.x, g.y * v.y, g.z * v.z, g.w * v.w};
-  typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-  bf16x4_t hv, lv;
-  {
-#pragma clang fp contract(off)   // lo must be the split of the ROUNDED product
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const __bf16 h = (__bf16)o[j];
-      hv[j] = h;
-      lv[j] = (__bf16)(o[j] - (float)h);
+    for (int s = 0; s < 8; ++s)
+      if (s < sk) { v.x += t[s].x; v.y += t[s].y; v.z += t[s].z; v.w += t[s].w; }
+    if (scale) { v.x *= sc.x; v.y *= sc.y; v.z *= sc.z; v.w *= sc.w; }
+    if (bias) { v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+    if (epilogue == CHATTS_EPI_RESID) { v.x = r.x + v.x; v.y = r.y + v.y; v.z = r.z + v.z; v.w = r.w + v.w; }
+    float ss = live ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f;
+    if (live) {
+      *reinterpret_cast<f32x4*>(c + (size_t)row * ldc + col) = v;
+      store_planes4(hi + (size_t)row * ldp + col, lo + (size_t)row * ldp + col, g * v);
     }
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    if (lane < 16) ss_s[f][lane] = ss;
   }
-  *reinterpret_cast<bf16x4_t*>(hi + (size_t)row * ldp + col) = hv;
-  *reinterpret_cast<bf16x4_t*>(lo + (size_t)row * ldp + col) = lv;
+  __syncthreads();
+  if ((int)threadIdx.x < m) {
+    float sum = ss_s[0][threadIdx.x];
+    for (int j = 1; j < (int)(blockDim.x >> 6); ++j) sum += ss_s[j][threadIdx.x];
+    post_ss[threadIdx.x * kSsStride + b0] = sum;
+  }
 }
 
 // The qkv projection's split-K epilogue that also does rope_kv_kernel's work (prefill): one wave per (token, head) sums the head's
@@ -995,7 +997,8 @@ int gemm_post_ss_parts(const ChattsLinearArgs* a) {
   if (a->m > 16 || a->batch > 1 || !use_stream(a) || a->ldc % 4 || ((uintptr_t)a->c % 16) || ((uintptr_t)a->resid % 16) || ((uintptr_t)a->bias % 16) ||
       (a->w8 && ((uintptr_t)a->w8_scale % 16)) || ((uintptr_t)a->workspace % 16)) return 0;
   const int sk = stream_ranges(a);
-  return sk > 1 && sk <= 8 ? (a->n + kEpiSsCols - 1) / kEpiSsCols : 0;
+  const int parts = rows_grid(a->n, a->epilogue);
+  return sk > 1 && sk <= 8 && (a->n / 4 + parts - 1) / parts <= 64 ? parts : 0;      // (16 waves of 4 groups)
 }
 size_t gemm_workspace_batch(int m, int n, int k, int batch) {
   if (batch <= 1 || m < 2 || m > 16 || k % 64) return 0;
@@ -1130,8 +1133,10 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   }
   CHATTS_CHECK_LAUNCH("gemm_bf16x2");
   if (ch.post_ss) {
-    hipLaunchKernelGGL(splitk_epilogue_ss_kernel, dim3((a->n + kEpiSsCols - 1) / kEpiSsCols, a->m), dim3(64), 0, s, reinterpret_cast<const float*>(a->workspace), sk, a->m, a->n, a->bias,
-                       a->resid, a->c, a->ldc, a->epilogue, a->w8 ? a->w8_scale : nullptr, a->post_norm_w, ch.post_ss, a->post_hi, a->post_lo, a->ld_post);
+    const int groups = a->n / 4, parts = rows_grid(a->n, a->epilogue);
+    hipLaunchKernelGGL(splitk_epilogue_ss_kernel, dim3(parts), dim3(64 * (((groups + parts - 1) / parts + 3) / 4)), 0, s, reinterpret_cast<const float*>(a->workspace), sk, a->m, a->n, a->bias, a->resid, a->c, a->ldc,
+                       a->epilogue,
+                       a->w8 ? a->w8_scale : nullptr, a->post_norm_w, ch.post_ss, a->post_hi, a->post_lo, a->ld_post, groups / parts, groups % parts);
     CHATTS_CHECK_LAUNCH("splitk_epilogue_ss");
     return CHATTS_OK;
   }
