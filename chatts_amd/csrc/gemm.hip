@@ -1078,13 +1078,11 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   p.row_ss = ch.row_ss; p.row_ss_parts = ch.row_ss_parts; p.row_eps = ch.row_eps;
   p.post_ss = nullptr;
   CHATTS_REQUIRE(!ch.row_ss || (stream && a->m <= 16 && batch == 1), CHATTS_E_SHAPE, "linear: row_ss is for 2 <= M <= 16 on planes (M=%d K=%d take another kernel)", a->m, a->k);
-  if (stream && gemm_takes_rows(a)) {      // (at the same sk)
+  // (at the same sk; a whole norm behind the product stays with the split, whose epilogue writes it: a launch of its own here)
+  if (stream && (!a->post_norm_w || ch.post_ss) && gemm_takes_rows(a)) {
     p.c = a->c;
     p.post_w = a->post_norm_w; p.post_ss = ch.post_ss; p.post_hi = a->post_hi; p.post_lo = a->post_lo; p.ld_post = a->ld_post;
-    if (const int rc = launch_rows(p, a, sk, s)) return rc;
-    if (a->post_norm_w && !ch.post_ss)
-      return chatts_rmsnorm_planes(a->c, a->post_norm_w, a->post_hi, a->post_lo, a->ld_post, a->m, a->n, a->post_norm_eps, reinterpret_cast<chatts_stream_t>(s));
-    return CHATTS_OK;
+    return launch_rows(p, a, sk, s);
   }
   CHATTS_REQUIRE(!ch.post_ss || gemm_post_ss_parts(a) > 0, CHATTS_E_SHAPE, "linear: post_ss is written where K is split over few rows (M=%d N=%d K=%d is not)", a->m, a->n, a->k);
   const int nt_count = (a->n + 127) / 128, mt_count = (a->m + bm - 1) / bm;
@@ -1212,8 +1210,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     CHATTS_CHECK_LAUNCH("splitk_epilogue");
   }
   if (post_norm)                  // no split-K epilogue to fuse into: the contract still holds, as its own launch
-    return chatts_rmsnorm_planes(a->c, a->post_norm_w, a->post_hi, a->post_lo, a->ld_post, a->m, a->n, a->post_norm_eps,
-                                 reinterpret_cast<chatts_stream_t>(s));
+    return launch_rmsnorm_planes(a->c, a->ldc, a->post_norm_w, a->post_hi, a->post_lo, a->ld_post, a->m, a->n, a->post_norm_eps, s);
   return CHATTS_OK;
 }
 

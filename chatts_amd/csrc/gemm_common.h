@@ -139,6 +139,8 @@ __device__ __forceinline__ void row_rstd_store(const GemmParams& p, int wave, in
 bool use_rows(const ChattsLinearArgs* a, int sk);      // sk: K ranges of gemm_stream_kernel
 int rows_grid(int n, int epilogue);      // workgroups = parts of post_ss
 int launch_rows(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s);
+// chatts_rmsnorm_planes on rows that lie ldx apart (elementwise.hip)
+int launch_rmsnorm_planes(const float* x, int ldx, const float* w, uint16_t* hi, uint16_t* lo, int ld_planes, int t, int hidden, float eps, hipStream_t s);
 
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
