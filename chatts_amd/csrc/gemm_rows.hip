@@ -15,8 +15,8 @@
 //
 // RMSNorm across the launch: the columns of a row lie in all workgroups, so the projection that updates the residual stream writes
 // norm_w * x as planes, WITHOUT the factor 1 / rms, and each workgroup's sum of squares per row (post_ss); the projection that reads these planes
-// sums the parts while its first weights travel and multiplies its rows by 1 / rms at the end (row_ss).  Products are linear in the row, so this
-// is the same value with one rounding moved.
+// sums the parts while its first weights travel and multiplies every K range's sums by 1 / rms at the end (row_ss), as gemm_stream_kernel does with what
+// goes to its slabs.  Products are linear in the row, so this is the same value with one rounding moved.
 #include <type_traits>
 
 #include "gemm_common.h"
@@ -169,18 +169,21 @@ __global__ __launch_bounds__(64 * MAXW) void gemm_rows_kernel(GemmParams p, cons
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (requests past the end of a range, too: the partial sums take their place in LDS)
   __syncthreads();
   f32x4* part = reinterpret_cast<f32x4*>(smem);        // [wave][fragment][lane]
+  if (p.row_ss) {                                      // (each range's sum, as gemm_stream_kernel's slabs have it; columns 8 .. 15 are nobody's)
+    const float inv = rstd_s[xrow];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[j] *= inv;
+  }
 #pragma unroll
   for (int j = 0; j < FN; ++j) part[(wave * FN + j) * 64 + lane] = acc[j];
   __syncthreads();
   float ss = 0.f;
   if (live) {
-    const float inv = p.row_ss ? rstd_s[tok] : 1.f;
     auto total = [&](int frag, f32x4 scale, f32x4 bias) __attribute__((always_inline)) {      // the waves' sums in wave order, scale and bias
       f32x4 s = part[frag * 64 + lane];
 #pragma unroll
       for (int w = 1; w < MAXW; ++w)
         if (w < kwaves) s += part[(w * FN + frag) * 64 + lane];
-      if (p.row_ss) s *= inv;
       if (W8) s *= scale;
       if (p.bias) s += bias;
       return s;

@@ -61,3 +61,38 @@ def test_a_row_does_not_depend_on_the_number_of_rows(lib, form, few, h, k):
         run(lib, a, m, h, k, _lib.NormChain(post_ss=ss.data_ptr()))
         got.append((c[:few], ph[:few], pl[:few], ss[:few]))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+# consumers with K in ranges (qkv, with a bias), in one piece (gate_up, the head), gated with K in ranges; the few-rows kernel beside the stream
+@pytest.mark.parametrize("form,few", [("bf16", 8), ("bf16", 3), ("fp8", 4), ("int8", 2)])
+@pytest.mark.parametrize("n,k,epi", [(6144, 4096, _lib.EPI_NONE), (7168, 5120, _lib.EPI_NONE), (24576, 4096, _lib.EPI_SWIGLU), (2048, 2048, _lib.EPI_SWIGLU), (1152, 2048, _lib.EPI_RESID)])
+def test_a_product_behind_the_norm_does_not_depend_on_the_number_of_rows(lib, form, few, n, k, epi):
+    x, w, bias, resid, q, s = problem(16, n, k, form, n + k)
+    x *= 10.0 ** torch.linspace(-2, 2, 16, device=DEV)[:, None]
+    ss = torch.full((16, 256), float("nan"), device=DEV)
+    ss[:, :200] = (x.double() ** 2).reshape(16, 64, -1).sum(2).float().repeat_interleave(4, 1)[:, :200] / 4      # (parts of any kind; what lies behind the last one is not read)
+    rstd = torch.rsqrt(ss[:, :200].double().sum(1, keepdim=True) / k + 1e-6)
+    z = (x.double() @ w.double().T) * rstd + bias.double()
+    gated = epi == _lib.EPI_SWIGLU
+    if gated:
+        z = z.view(16, -1, 2, 16)
+        want = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(16, n // 2)
+    else:
+        want = z + resid.double() if epi == _lib.EPI_RESID else z
+    got = []
+    for m in (16, few):
+        hi, lo = planes(lib, x[:m].contiguous())
+        chain = _lib.NormChain(row_ss=ss.data_ptr(), row_ss_parts=200, row_eps=1e-6)
+        cols = n // 2 if gated else n
+        if gated:                                         # (what the decoder's gate_up writes)
+            ph, pl = torch.full((2, m, cols), float("nan"), dtype=torch.bfloat16, device=DEV)
+            run(lib, args(m, n, k, hi, lo, w, q, s, form, None, bias=bias.data_ptr(), epilogue=epi, c_hi=ph.data_ptr(), c_lo=pl.data_ptr(), ld_cplanes=cols, ldc=cols), m, n, k, chain)
+            got.append((ph[:few], pl[:few]))
+            out = ph.double() + pl.double()
+        else:
+            out = torch.full((m, n), float("nan"), device=DEV)
+            run(lib, args(m, n, k, hi, lo, w, q, s, form, out, bias=bias.data_ptr(), resid=resid.data_ptr(), ldc=n, epilogue=epi), m, n, k, chain)
+            got.append((out[:few],))
+        for i in range(m):
+            assert rel(out[i], want[i]) < 2e-5            # (x to 2^-17, sums in 32 bits)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
