@@ -203,6 +203,20 @@ __device__ __forceinline__ float gelu_tanh_glu(float g, float u) { return g * si
 __host__ __device__ constexpr bool epi_is_glu(int epilogue) {
   return epilogue == CHATTS_EPI_SWIGLU || epilogue == CHATTS_EPI_CLAMPGLU || epilogue == CHATTS_EPI_GEGLU;
 }
+// Does a result of `rows` rows share memory with one of A's planes?  (from the first to behind the last element that is read or written)
+struct Range {
+  const char* at;
+  size_t bytes;
+  bool meets(const Range& o) const { return at && o.at && at < o.at + o.bytes && o.at < at + bytes; }
+};
+inline Range matrix_range(const void* p, int rows, int ld, int cols, int elem) { return {static_cast<const char*>(p), ((size_t)(rows - 1) * ld + cols) * elem}; }
+inline bool meets_planes(const ChattsLinearArgs* a, const Range& r) {
+  return r.meets(matrix_range(a->a_hi, a->m, a->ld_planes, a->k, 2)) || r.meets(matrix_range(a->a_lo, a->m, a->ld_planes, a->k, 2));
+}
+inline Range result_range(const ChattsLinearArgs* a, int i) {      // i 0: c (NULL where planes are written), 1 / 2: the planes
+  const int cols = epi_is_glu(a->epilogue) ? a->n / 2 : a->n;
+  return i ? matrix_range(i == 1 ? a->c_hi : a->c_lo, a->m, a->ld_cplanes, cols, 2) : matrix_range(a->c_hi ? nullptr : a->c, a->m, a->ldc, cols, 4);
+}
 inline hipStream_t as_stream(chatts_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ---- stage ranges for traces (api.hip): roctx push / pop around the host-side enqueue of a stage, resolved with dlopen at first use

@@ -16,6 +16,7 @@ bool gemm_batched_stream(const ChattsLinearArgs* a);
 size_t gemm_workspace_batch(int m, int n, int k, int batch);
 int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope = nullptr, bool* rope_done = nullptr, const ChattsNormChain* chain = nullptr);
 int gemm_post_ss_parts(const ChattsLinearArgs* a);
+int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w,
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
@@ -62,15 +63,31 @@ extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormCh
                  "linear_chain: row_ss takes 2 <= M <= 16 on planes and 1 .. 256 parts (M=%d, %d parts)", a->m, ch->row_ss_parts);
   CHATTS_REQUIRE(!ch->post_ss || (((uintptr_t)ch->post_ss % 16) == 0 && a->batch <= 1 && !a->exact_f32 && chatts_linear_post_ss_parts(a) > 0), CHATTS_E_SHAPE,
                  "linear_chain: post_ss needs post_norm_w and a shape of chatts_linear_post_ss_parts (M=%d N=%d K=%d)", a->m, a->n, a->k);
+  // sums of squares are read by every workgroup and written as each of them finishes
+  const Range in{reinterpret_cast<const char*>(ch->row_ss), sizeof(float) * 16 * 256}, out{reinterpret_cast<const char*>(ch->post_ss), sizeof(float) * 16 * 256};
+  bool meet = in.meets(out) || (ch->post_ss && meets_planes(a, out));
+  for (int i = 0; i < 3; ++i) meet = meet || in.meets(result_range(a, i)) || out.meets(result_range(a, i));
+  if (ch->post_ss || ch->row_ss)
+    for (const chatts_bf16* plane : {a->post_hi, a->post_lo}) meet = meet || in.meets(matrix_range(plane, a->m, a->ld_post, a->n, 2)) || out.meets(matrix_range(plane, a->m, a->ld_post, a->n, 2));
+  CHATTS_REQUIRE(!meet, CHATTS_E_SHAPE, "linear_chain: the sums of squares overlap each other, a result or A (M=%d N=%d K=%d)", a->m, a->n, a->k);
   return linear_impl(a, stream, nullptr, nullptr, ch);
 }
 extern "C" int chatts_linear_post_ss_parts(const ChattsLinearArgs* a) {
   const bool ok = a && a->w && a->m >= 2 && a->m <= 16 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && a->ldc >= a->n && a->ldw >= a->k && (!a->w8 || a->ldw8 >= a->k) &&
                   a->post_norm_w && ((uintptr_t)a->post_norm_w % 16) == 0 && a->post_hi && a->post_lo && a->ld_post >= a->n && a->ld_post % 4 == 0 &&
-                  ((uintptr_t)a->post_hi % 8) == 0 && ((uintptr_t)a->post_lo % 8) == 0 && a->post_hi != a->a_hi && a->c && !a->c_hi &&
+                  ((uintptr_t)a->post_hi % 8) == 0 && ((uintptr_t)a->post_lo % 8) == 0 && a->c && !a->c_hi &&
                   (a->epilogue == CHATTS_EPI_NONE || a->epilogue == CHATTS_EPI_RESID);
-  const int parts = ok ? gemm_post_ss_parts(a) : 0;
+  if (!ok) return 0;
+  // the planes are written while other workgroups still read A, c's own place included (c may be resid)
+  for (const chatts_bf16* plane : {a->post_hi, a->post_lo}) {
+    const Range r = matrix_range(plane, a->m, a->ld_post, a->n, 2);
+    if (meets_planes(a, r) || r.meets(matrix_range(a->c, a->m, a->ldc, a->n, 4)) || r.meets(matrix_range(a->resid, a->m, a->ldc, a->n, 4))) return 0;
+  }
+  const int parts = gemm_post_ss_parts(a);
   return parts <= 256 ? parts : 0;
+}
+extern "C" int chatts_linear_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* ch) {
+  return a && a->w && a->m >= 2 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && !a->exact_f32 ? gemm_few_rows(a, ch) : 0;
 }
 extern "C" size_t chatts_linear_workspace(int m, int n, int k) { return gemm_workspace(m, n, k); }
 extern "C" size_t chatts_linear_workspace_batch(int m, int n, int k, int batch) {

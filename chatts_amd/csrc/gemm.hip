@@ -986,10 +986,14 @@ static int stream_ranges(const ChattsLinearArgs* a) {
   const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr));
   return (a->k + kps - 1) / kps;
 }
-int gemm_takes_rows(const ChattsLinearArgs* a) {
+static int gemm_takes_rows(const ChattsLinearArgs* a) {
   if (a->m > 8 || a->batch > 1 || opt_get(OPT_GEMM_SK, 0) != 0 || !use_stream(a)) return 0;
   const int sk = stream_ranges(a);
   return sk > 1 && use_rows(a, sk) ? sk : 0;
+}
+// the same for a call of chatts_linear or chatts_linear_chain: a whole norm behind the product stays with the split, whose epilogue writes it (a launch of its own here)
+int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain) {
+  return a->post_norm_w && !(chain && chain->post_ss) ? 0 : gemm_takes_rows(a);
 }
 // parts of post_ss that launch_gemm would write for these arguments (post_norm_w and planes are there), 0: it would not
 int gemm_post_ss_parts(const ChattsLinearArgs* a) {
@@ -1078,8 +1082,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   p.row_ss = ch.row_ss; p.row_ss_parts = ch.row_ss_parts; p.row_eps = ch.row_eps;
   p.post_ss = nullptr;
   CHATTS_REQUIRE(!ch.row_ss || (stream && a->m <= 16 && batch == 1), CHATTS_E_SHAPE, "linear: row_ss is for 2 <= M <= 16 on planes (M=%d K=%d take another kernel)", a->m, a->k);
-  // (at the same sk; a whole norm behind the product stays with the split, whose epilogue writes it: a launch of its own here)
-  if (stream && (!a->post_norm_w || ch.post_ss) && gemm_takes_rows(a)) {
+  if (stream && gemm_few_rows(a, chain)) {      // (at the same sk)
     p.c = a->c;
     p.post_w = a->post_norm_w; p.post_ss = ch.post_ss; p.post_hi = a->post_hi; p.post_lo = a->post_lo; p.ld_post = a->ld_post;
     return launch_rows(p, a, sk, s);

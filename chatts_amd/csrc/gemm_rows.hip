@@ -246,6 +246,9 @@ static int rows_waves(int np, int sk) { return sk > (np + 1) / 2 ? sk : (np + 1)
 static int rows_ahead(bool w8, int np, int waves) { return waves > 8 ? 3 : (w8 ? (np > 6 ? 3 : 4) : 5); }
 
 bool use_rows(const ChattsLinearArgs* a, int sk) {
+  // a workgroup stores its result while others still read A (the split's epilogue is a launch behind them)
+  for (int i = 0; i < 3; ++i)
+    if (meets_planes(a, result_range(a, i))) return false;
   auto al = [](const void* q) { return ((uintptr_t)q % 16) == 0; };
   const bool w8 = a->w8 != nullptr;
   const size_t wbytes = w8 ? (size_t)a->n * a->ldw8 : (size_t)a->n * a->ldw * 2;

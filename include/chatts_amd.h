@@ -249,7 +249,8 @@ typedef struct ChattsLinearArgs {
  * of its own between them.  Producer (2 <= M <= 16): post_ss, with the call's post_norm_w, post_hi, post_lo and where chatts_linear_post_ss_parts() > 0 - the planes
  * are post_norm_w * c WITHOUT the factor 1 / rms, and post_ss (float [16][256], 16-byte aligned) receives the sums of squares of c's rows, in
  * parts.  Consumer (2 <= M <= 16 on planes): row_ss, the same array, row_ss_parts of each row's 256 places in use, and row_eps - row m of the product is
- * multiplied by 1 / sqrt(sum of its parts / K + row_eps) before scale, bias and epilogue. */
+ * multiplied by 1 / sqrt(sum of its parts / K + row_eps) before scale, bias and epilogue.  Neither array may overlap the other, a result or (post_ss) A: refused;
+ * post_hi / post_lo that overlap A, c or resid have no parts. */
 typedef struct ChattsNormChain {
   float* post_ss;
   const float* row_ss;
@@ -259,6 +260,9 @@ typedef struct ChattsNormChain {
 int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* chain, chatts_stream_t stream);
 /* Host-only query: parts that this call would write to post_ss, 0 = it cannot (K is not split, or the operands are not aligned). */
 int chatts_linear_post_ss_parts(const ChattsLinearArgs* a);
+/* Host-only query: K ranges if this call (chain may be NULL) runs on the few-rows kernel, which holds whole columns and has no second launch; 0 = another kernel
+ * runs.  Lets a test pin which shapes take which kernel. */
+int chatts_linear_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
 size_t chatts_linear_workspace(int m, int n, int k);
 size_t chatts_linear_workspace_batch(int m, int n, int k, int batch);
 /* Host-only query (no device work): how many waves share a row group of the M == 1 bf16 GEMV for this shape on the current device

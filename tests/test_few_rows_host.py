@@ -1,0 +1,69 @@
+"""Which projections of few rows write their result while other workgroups still read A: never one whose outputs share memory with A (host-side decisions for 256 CUs, no
+pointer is followed)."""
+import ctypes as C
+
+import pytest
+
+from chatts_amd import _lib
+
+M, N, K = 6, 4096, 4096
+PLANE = M * K * 2                                      # bytes of a plane of A
+A_HI, A_LO, OUT = 0x10000000, 0x10000000 + PLANE, 0x40000000
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _lib.load()
+
+
+def args(**kw):
+    base = dict(w=0x7f0000000000, c=OUT, m=M, n=N, k=K, lda=K, ldw=K, ldc=N, a_hi=A_HI, a_lo=A_LO, ld_planes=K, epilogue=_lib.EPI_NONE, workspace=0x50000000, workspace_bytes=1 << 28)
+    return _lib.LinearArgs(**{**base, **kw})
+
+
+def few_rows(lib, a, chain=None):
+    return int(lib.chatts_linear_few_rows(C.byref(a), C.byref(chain) if chain else None))
+
+
+@pytest.mark.parametrize("at,takes", [(OUT, True), (A_HI, False), (A_LO, False), (A_LO + PLANE, True), (A_LO + PLANE - 16, False), (A_HI - M * N * 4, True), (A_HI - M * N * 4 + 16, False)])
+def test_float_result(lib, at, takes):
+    assert (few_rows(lib, args(c=at)) > 1) == takes
+
+
+@pytest.mark.parametrize("hi,lo,takes", [(OUT, OUT + PLANE, True), (A_HI, A_LO, False), (A_LO, A_HI, False), (OUT, A_LO, False), (A_LO + PLANE - 16, OUT, False), (A_HI - M * N * 2, OUT, True),
+                                         (OUT, A_HI - M * N * 2 + 16, False)])
+def test_planes_as_the_result(lib, hi, lo, takes):
+    assert (few_rows(lib, args(c=None, c_hi=hi, c_lo=lo, ld_cplanes=N)) > 1) == takes
+
+
+def test_strides_count(lib):
+    assert few_rows(lib, args(ldc=2 * N, c=A_HI - (M * 2 - 1) * N * 4)) > 1               # (nothing lies behind the last row)
+    assert few_rows(lib, args(ldc=2 * N, c=A_HI - (M * 2 - 1) * N * 4 + 16)) == 0
+    assert few_rows(lib, args(ld_planes=2 * K, a_lo=A_HI + K * 2, c=A_HI + (2 * M * K) * 2)) > 1      # planes row by row in turn
+    assert few_rows(lib, args(ld_planes=2 * K, a_lo=A_HI + K * 2, c=A_HI + (2 * M * K) * 2 - 16)) == 0
+
+
+@pytest.mark.parametrize("m", [6, 12])                 # the few-rows kernel; the split's epilogue, which keeps to the same rule
+@pytest.mark.parametrize("hi,lo,takes", [(OUT + (1 << 24), OUT + (2 << 24), True), (A_HI, A_LO, False), (A_LO, A_HI, False), (OUT + (1 << 24), A_LO, False), (A_HI + 16, OUT + (1 << 24), False),
+                                         (OUT + (1 << 24), A_HI + 32, False)])
+def test_planes_for_the_norm(lib, m, hi, lo, takes):
+    a = args(m=m, a_lo=A_HI + m * K * 2, post_norm_w=0x60000000, post_hi=hi, post_lo=lo, ld_post=N)
+    assert (int(lib.chatts_linear_post_ss_parts(C.byref(a))) > 0) == takes
+
+
+@pytest.mark.parametrize("over", ["a_hi", "a_lo", "c", "post_hi", "row_ss"])
+def test_sums_of_squares_have_their_own_memory(lib, over):
+    """refused before anything is launched"""
+    a = args(post_norm_w=0x60000000, post_hi=OUT + (1 << 24), post_lo=OUT + (2 << 24), ld_post=N)
+    chain = _lib.NormChain(row_ss=0x70000000, row_ss_parts=256, row_eps=1e-6)
+    chain.post_ss = {"a_hi": A_HI, "a_lo": A_LO + 64, "c": OUT + 32, "post_hi": OUT + (1 << 24) + 16, "row_ss": 0x70000000 + 16}[over]
+    assert int(lib.chatts_linear_chain(C.byref(a), C.byref(chain), None)) == _lib.E_SHAPE
+    assert b"overlap" in lib.chatts_last_error()
+
+
+@pytest.mark.parametrize("over", ["c", "c_hi", "c_lo"])
+def test_results_leave_the_sums_that_are_read_alone(lib, over):
+    a = args() if over == "c" else args(c=None, c_hi=OUT, c_lo=OUT + (1 << 24), ld_cplanes=N)
+    chain = _lib.NormChain(row_ss={"c": OUT + 64, "c_hi": OUT - 16 * 256 * 4 + 16, "c_lo": OUT + (1 << 24)}[over], row_ss_parts=256, row_eps=1e-6)
+    assert int(lib.chatts_linear_chain(C.byref(a), C.byref(chain), None)) == _lib.E_SHAPE
+    assert b"overlap" in lib.chatts_last_error()

@@ -131,3 +131,19 @@ def test_norm_between_two_projections(lib, form, m, h, k, n2):
         assert rel(out[i], want[i]) < 2e-5
     a.post_hi = hi.data_ptr()                             # planes that the same launch still reads
     assert int(lib.chatts_linear_post_ss_parts(C.byref(a))) == 0
+
+
+@pytest.mark.parametrize("form", ["bf16", "fp8"])
+@pytest.mark.parametrize("m", [2, 4, 8])
+@pytest.mark.parametrize("as_planes", [True, False])
+def test_a_result_in_the_place_of_its_own_input(lib, form, m, as_planes):
+    n = k = 2048
+    x, w, bias, _, q, scale = problem(m, n, k, form, m)
+    hi, lo = planes(lib, x)
+    want = x.double() @ w.double().T + bias.double()
+    more = dict(c_hi=hi.data_ptr(), c_lo=lo.data_ptr(), ld_cplanes=n) if as_planes else {}
+    a = args(m, n, k, hi, lo, w, q, scale, form, None if as_planes else hi, bias=bias.data_ptr(), ldc=n, epilogue=_lib.EPI_NONE, **more)      # (both planes lie in a row: m x n floats)
+    run(lib, a, m, n, k)
+    assert lo.data_ptr() == hi.data_ptr() + m * k * 2
+    out = hi.double() + lo.double() if as_planes else torch.as_strided(hi, (m, 2 * n), (2 * n, 1)).view(torch.float32)
+    assert rel(out, want) < 1e-5
