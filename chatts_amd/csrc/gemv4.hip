@@ -59,7 +59,8 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
 
   // lane: row r of the quad, part kap of K within the unit, k group kq of 32 codes within the part
   const int r = lane & 3, kap = (lane >> 2) & 3, kq = lane >> 4, pos = kap * 4 + kq;
-  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.w4, 0, (int)((unsigned)p.n * (unsigned)p.ldw4), 0x00020000);
+  // (up to the last code of the last row: units of 512 codes run past the end of a row)
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.w4, 0, (int)((unsigned)(p.n - 1) * (unsigned)p.ldw4 + (unsigned)K / 2u), 0x00020000);
   const unsigned lane_off = (unsigned)(GLU ? (r >> 1) + (r & 1) * 16 : r) * (unsigned)p.ldw4 + pos * 16;
   auto first_row = [&](int q) __attribute__((always_inline)) {           // of quad q of this workgroup (gated: gates 2 u, 2 u + 1 and their up rows, 16 further on)
     const int at = (q0 + q) * (GLU ? 2 : 4);

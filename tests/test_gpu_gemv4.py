@@ -76,3 +76,20 @@ def test_rows_do_not_read_each_other(k):
     sz = sz.clone()
     sz[1::2] = float("nan")
     assert torch.equal(run(x, w4, sz, deq, 32, _lib.EPI_NONE)[:, ::2], clean[:, ::2])
+
+
+@pytest.mark.parametrize("at", [0, 1])                # the first columns of a wider matrix, and the last ones: the last row ends where the memory ends
+@pytest.mark.parametrize("k,group", [(2592, 32), (4096 + 64, 64), (5088, 32), (5120, 128)])
+def test_columns_of_a_wider_matrix(at, k, group):
+    n = 96
+    x, (w4, sz), deq, *_ = problem(n, k, group, k)
+    want = run(x, w4, sz, deq, group, _lib.EPI_NONE)
+    wide = torch.full((n, k), 0xff, dtype=torch.uint8, device=DEV)
+    part = wide[:, k // 2 * at:][:, :k // 2]
+    part.copy_(w4)
+    out = torch.full((1, n), float("nan"), device=DEV)
+    a = _lib.LinearArgs(a=x.data_ptr(), w=deq.data_ptr(), c=out.data_ptr(), m=1, n=n, k=k, lda=k, ldw=k, ldc=n, epilogue=_lib.EPI_NONE, w4=part.data_ptr(), w4_sz=sz.data_ptr(), ldw4=k,
+                        w4_group=group)
+    _lib.check(_lib.load().chatts_linear(C.byref(a), _lib.stream_ptr()))
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
