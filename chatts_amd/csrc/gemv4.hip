@@ -4,7 +4,7 @@
 // by HBM at about the same time, and gains from doing less per code and from doing both at once.  gemv4_ldsx_kernel (gemv.hip) spends 3.75
 // operations a code and waits for a batch of loads before it computes on it.  Here:
 //   * conversion: nibbles 0 and 4 (1 and 5, ...) of a word masked in place ARE two float16 denormals, code * 2^-24 (or * 2^-20), so one v_fma_mix each
-//     with scale * 2^24 gives code * scale - scale * zero with a single rounding (exact for every finite scale), and v_cvt_pk rounds two of them:
+//     with scale * 2^24 gives code * scale - scale * zero with a single rounding (scales below 2^104; sums that are not finite are done again code by code), and v_cvt_pk rounds two of them:
 //     2.1 operations a code; the order of k that falls out (0 4 1 5 2 6 3 7) is x's order in LDS;
 //   * products on the matrix pipe: a wave's unit is FOUR rows ("quad") x 512 k, one 16-byte load per lane = 256 consecutive bytes of each row.  The 16
 //     rows of an MFMA operand are 4 rows x 4 parts of K; x comes as columns (part, hi / lo), and the wanted sums are the blocks where the parts
@@ -15,6 +15,8 @@
 // 3.7 TB/s; v_fma_mix and v_cvt_pk issue at half rate, so the conversion alone is 13 us of it), down 5120 x 13824 17.0 -> 11.7.  16 waves instead of 8: 1 us
 // more everywhere (the prologue is serial per SIMD); scales staged in LDS: 1 to 2 us more.
 // x = hi + lo bf16 (2^-17), products exact, float32 sums: the accuracy of the kernel it replaces.
+#include <type_traits>
+
 #include "common.h"
 #include "gemv_common.h"
 
@@ -72,7 +74,8 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
   const unsigned lane_sz_end = (S - 1) * 512 + pos * 32 < K ? lane_sz : kQ4Far;      // past K: scale and zero read as 0, so weights of 0 (the codes are the next row's)
   u32x4 cv[kQ4Bufs];
   u32x2 zv[kQ4Bufs];
-  int rq = p.parts_inv ? (int)__umulhi((unsigned)i0, p.parts_inv) : i0, rs = i0 - rq * S, ri = 0;      // the unit to request next
+  const int first_q = p.parts_inv ? (int)__umulhi((unsigned)i0, p.parts_inv) : i0;
+  int rq = first_q, rs = i0 - rq * S, ri = 0;                            // the unit to request next
   int q = rq, s = rs;                                                    // ... and the one to compute next
   auto request = [&](int b) __attribute__((always_inline)) {
     const unsigned row = (unsigned)first_row(rq);
@@ -137,13 +140,18 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const int col = lane & 15;
+  bool finite = true;                                                    // of all sums so far
   auto flush = [&]() __attribute__((always_inline)) {                    // rows 4 kq .. of the product belong to part kq: columns 2 kq and 2 kq + 1 are theirs
     if ((col >> 1) == kq) part[(q * kQ4Waves + wave) * 8 + col] = acc;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) finite &= __builtin_isfinite(acc[j]);
     acc = (f32x4){0.f, 0.f, 0.f, 0.f};
   };
-  auto unit = [&](int b) __attribute__((always_inline)) {
+  auto unit = [&](int b, auto plain_c) __attribute__((always_inline)) {
+    constexpr bool PLAIN = decltype(plain_c)::value;                     // the code itself times the scale: two operations more a code, no scale * 2^24
     const char* xp = xs + s * 4 * kQ4Piece + (kq * 8 + (lane & 7)) * 16;
-    const float sc0 = __uint_as_float(zv[b].x) * 16777216.f, sc4 = sc0 * 0.0625f, nz = -__uint_as_float(zv[b].y);
+    const float sc = __uint_as_float(zv[b].x), sc0 = PLAIN ? sc : sc * 16777216.f, sc4 = PLAIN ? sc : sc0 * 0.0625f, nz = -__uint_as_float(zv[b].y);
+    const float c0 = PLAIN ? 16777216.f : 1.f, c4 = PLAIN ? 1048576.f : 1.f;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const uint32_t v = cv[b][m], u = v >> 8;
@@ -152,8 +160,8 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
       bf16x8_t w;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        w[2 * e] = (__bf16)fmaf((float)h[e].x, e & 1 ? sc4 : sc0, nz);
-        w[2 * e + 1] = (__bf16)fmaf((float)h[e].y, e & 1 ? sc4 : sc0, nz);
+        w[2 * e] = (__bf16)fmaf((float)h[e].x * (e & 1 ? c4 : c0), e & 1 ? sc4 : sc0, nz);
+        w[2 * e + 1] = (__bf16)fmaf((float)h[e].y * (e & 1 ? c4 : c0), e & 1 ? sc4 : sc0, nz);
       }
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, *reinterpret_cast<const bf16x8_t*>(xp + m * kQ4Piece), acc, 0, 0, 0);
     }
@@ -165,10 +173,19 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
     for (int b = 0; b < kQ4Bufs; ++b) {
       request((b + kQ4Ahead) % kQ4Bufs);
       __builtin_amdgcn_sched_barrier(0);
-      if (t + b < cnt) unit(b);
+      if (t + b < cnt) unit(b, std::false_type{});
     }
   }
   if (cnt > 0 && s > 0) flush();
+  if (__ballot(!finite)) {                 // scale * 2^24 overflows from 2^104 on, and its products are infinite or NaN: this wave's share once more, code by code
+    rq = q = first_q; rs = s = i0 - first_q * S; ri = 0;
+#pragma unroll 1
+    for (int t = 0; t < cnt; ++t) {
+      request(0);
+      unit(0, std::true_type{});
+    }
+    if (cnt > 0 && s > 0) flush();
+  }
   __syncthreads();
 
   float rstd = 1.f;
@@ -228,7 +245,7 @@ static int launch4_e(const Gemv4Params& p, int grid, size_t lds, hipStream_t s) 
   return p.norm_w ? launch4_t<EPI, true>(p, grid, lds, s) : launch4_t<EPI, false>(p, grid, lds, s);
 }
 
-// Which 4-bit projections run here: 16-byte pieces of a row (ldw4 and the pointer in 16 bytes), groups of at least the 32 codes of a lane, x in two turns of a
+// Which 4-bit projections run here: 16-byte pieces of a row (ldw4 and the pointer in 16 bytes), groups of at least the 32 codes of a lane, x in four turns of a
 // workgroup and everything in LDS.  The rest keeps gemv4_ldsx_kernel.  *done: whether this call launched.
 int launch_gemv4(const ChattsLinearArgs* a, hipStream_t s, bool* done) {
   Gemv4Params p;

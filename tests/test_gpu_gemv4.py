@@ -93,3 +93,22 @@ def test_columns_of_a_wider_matrix(at, k, group):
     _lib.check(_lib.load().chatts_linear(C.byref(a), _lib.stream_ptr()))
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("power", [-140, -100, 100, 103, 104, 110, 120])
+def test_scales_of_any_size(power):
+    n, k, group = 96, 4096 + 96, 32
+    x, _, _, *_ = problem(n, k, group, power)
+    g = torch.Generator(device=DEV).manual_seed(power)
+    from chatts_amd.modeling import pack_int4
+    codes = torch.randint(0, 16, (n, k), generator=g, device=DEV, dtype=torch.uint8)
+    scale = (1 + torch.rand((n, k // group), generator=g, device=DEV)) * 2.0 ** -6
+    scale[5::7, 3::11] = 1.5 * 2.0 ** power               # in some groups only: the others' weights must not suffer
+    zero = torch.randint(0, 16, scale.shape, generator=g, device=DEV).float()
+    deq = (codes.float() * scale.repeat_interleave(group, 1) - (scale * zero).repeat_interleave(group, 1)).bfloat16()
+    w4, sz = pack_int4(codes, scale, zero)
+    x = x * 2.0 ** min(0, 60 - power)                     # sums stay finite
+    out = run(x, w4, sz, deq, group, _lib.EPI_NONE)
+    want = x.double() @ deq.double().T
+    bound = x.double().abs() @ deq.double().abs().T * (2.0 ** -18 + (k / 16 + 32) * 2.0 ** -24) + 2.0 ** -126
+    assert bool(((out.double() - want).abs() <= bound).all())
