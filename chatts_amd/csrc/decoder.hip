@@ -274,12 +274,12 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
   return chatts_rmsnorm(d->b.x, norm_w, d->b.xn, la->m, la->k, d->cfg.rms_eps, stream);
 }
 
-// The residual-updating projection (o_proj / down_proj, tp_world == 1) also produces the NEXT projection's operand:
-// RMSNorm(x) with `next_norm_w` as planes 0, when that projection will take the plane path for the same M.
-// The same for few rows (layer_part_batched), without waiting for a row's sum: the projection writes norm_w * x as planes 1 and the sums of squares,
-// and the next projection multiplies by 1 / rms.  Planes 1, because workgroups that are done write them while others still read A (planes 0).
+// Few rows (layer_part_batched, tp_world == 1): the residual-updating projection (o_proj / down_proj) writes norm_w * x as planes 1 and the sums of squares,
+// without waiting for a row's sum, and the next projection multiplies by 1 / rms.  Planes 1, because workgroups that are done write them while others still read A
+// (planes 0).  POST_NORM_SMALL_M=0: every norm of a batched step in a launch of its own (other roundings: there the row is normed before it is split).
+static bool gemm_post_norm_small_m() { return opt_get(OPT_POST_NORM_SMALL_M, 1) != 0; }
 static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormChain* chain, const float* next_norm_w, bool next_fp8) {
-  if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || !d->b.delta || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;
+  if (!gemm_post_norm_small_m() || !d->chain || d->cfg.tp_world > 1 || !next_norm_w || !d->b.delta || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;
   ChattsLinearArgs t = *la;
   t.post_norm_w = next_norm_w; t.post_hi = d->b.planes2_hi; t.post_lo = d->b.planes2_lo; t.ld_post = la->n;
   const int parts = chatts_linear_post_ss_parts(&t);
@@ -289,7 +289,8 @@ static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormCh
   d->normed = true; d->ss_parts = parts;
   return true;
 }
-static bool gemm_post_norm_small_m() { return opt_get(OPT_POST_NORM_SMALL_M, 1) != 0; }
+// The residual-updating projection also produces the NEXT projection's operand: RMSNorm(x) with `next_norm_w` as planes 0, when that projection will take the
+// plane path for the same M.
 static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const float* next_norm_w, bool next_fp8) {
   if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || la->epilogue != CHATTS_EPI_RESID) return;
   // the fused epilogue runs one workgroup per row - fine for a prefill chunk; at batched-decode M it needs several workgroups per row,

@@ -1,4 +1,5 @@
-"""A whole batched decode step: a sequence's logits are the same bits however many sequences share the step."""
+"""A whole batched decode step: a sequence's logits are the same bits however many sequences share the step, and the norm that the projections hand on between them
+agrees with norms in launches of their own."""
 import pytest
 import torch
 
@@ -36,6 +37,18 @@ def step(m, positions, tokens, batch):
     return b["logits_all"][:batch].clone()
 
 
+def step_in_parts(m, positions, tokens, batch):
+    """the same step through the calls for one part of a layer, which leave every norm to a launch of its own"""
+    b, lib = start(m, positions, tokens), m.lib
+    _lib.check(lib.chatts_embed_token_batched(_lib.ptr(b["token_all"]), batch, _lib.ptr(m._tensors["embed"]), 0, 4096, m.config.hidden_size, _lib.ptr(b["x"]), _lib.stream_ptr()))
+    for layer in range(m.config.num_hidden_layers):
+        for part in (0, 1):
+            _lib.check(lib.chatts_decoder_layer_part_batched(m._decoder, layer, part, batch, _lib.ptr(b["pos_all"]), SPLITS, _lib.stream_ptr()))
+    _lib.check(lib.chatts_decoder_logits_batched(m._decoder, batch, _lib.ptr(b["logits_all"]), _lib.stream_ptr()))
+    torch.cuda.synchronize()
+    return b["logits_all"][:batch].clone()
+
+
 FORMS = [("chatts-8b", "bf16"), ("chatts-14b", "bf16"), ("chatts-14b", "fp8"), ("chatts-8b", "int8"), ("tiny-qwen3", "bf16")]
 
 
@@ -45,3 +58,15 @@ def test_the_number_of_sequences(name, form):
     all16 = step(m, positions, tokens, 16)
     for batch in (2, 3, 4, 5, 8, 9, 15):
         assert torch.equal(step(m, positions, tokens, batch), all16[:batch]), batch
+
+
+@pytest.mark.parametrize("name,form", FORMS)
+def test_separate_norms(monkeypatch, name, form):
+    m, positions, tokens = model_of(name, form)
+    for batch in (3, 8, 16):
+        parts, handed_on = step_in_parts(m, positions, tokens, batch), step(m, positions, tokens, batch)
+        # the factor 1 / rms is applied behind the products instead of in front of them: roundings, a few of 2^-17 a layer where planes hold the row
+        assert float((parts - handed_on).norm() / parts.norm()) < 1e-4
+        monkeypatch.setenv("CHATTS_POST_NORM_SMALL_M", "0")
+        assert torch.equal(step(m, positions, tokens, batch), parts)
+        monkeypatch.delenv("CHATTS_POST_NORM_SMALL_M")
