@@ -40,8 +40,8 @@ struct ChattsDecoder {
   bool x_in_xn = false;     // batched step: o_proj left the residual stream in b.xn (ping-pong, see layer_part_batched); down_proj brings it back
   bool normed = false;      // planes 0 already hold RMSNorm(x) for the projection that comes next (written by the previous
                             // projection's fused epilogue): norm_into only binds them
-  int ss_parts = 0;         // > 0, with normed: ... planes 1 hold norm_w * x without the factor 1 / rms; its sums of squares are that many parts in
-                            // b.delta (free without tensor parallelism): a step of 2 .. 16 sequences whose projections hold whole columns
+  int ss_parts = 0;         // > 0, with normed: ... planes 1 hold norm_w * x without the factor 1 / rms; each row's sum of squares is that many parts in
+                            // b.attn: a step of 2 .. 16 sequences behind a projection that hands its norm on (request_post_ss)
   bool sampling = false;    // token selection of the decode steps: greedy argmax, or the sampler with `sa`
   ChattsSamplingArgs sa{};
   ChattsTpComm* tp = nullptr;   // tensor-parallel exchange (borrowed); required by the whole-step entry points when tp_world > 1
@@ -262,7 +262,7 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
     la->a = nullptr; la->a_hi = d->b.planes_hi; la->a_lo = d->b.planes_lo; la->ld_planes = la->k;
     if (d->normed && d->ss_parts && chain) {
       la->a_hi = d->b.planes2_hi; la->a_lo = d->b.planes2_lo;
-      chain->row_ss = d->b.delta; chain->row_ss_parts = d->ss_parts; chain->row_eps = d->cfg.rms_eps;
+      chain->row_ss = d->b.attn; chain->row_ss_parts = d->ss_parts; chain->row_eps = d->cfg.rms_eps;
       d->normed = false; d->ss_parts = 0;
       return CHATTS_OK;
     }
@@ -279,13 +279,14 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
 // (planes 0).  POST_NORM_SMALL_M=0: every norm of a batched step in a launch of its own (other roundings: there the row is normed before it is split).
 static bool gemm_post_norm_small_m() { return opt_get(OPT_POST_NORM_SMALL_M, 1) != 0; }
 static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormChain* chain, const float* next_norm_w, bool next_fp8) {
-  if (!gemm_post_norm_small_m() || !d->chain || d->cfg.tp_world > 1 || !next_norm_w || !d->b.delta || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;
+  if (!gemm_post_norm_small_m() || !d->chain || d->cfg.tp_world > 1 || !next_norm_w || la->a_hi == d->b.planes2_hi || !planes_path(d, la->m, la->n, next_fp8)) return false;
   ChattsLinearArgs t = *la;
   t.post_norm_w = next_norm_w; t.post_hi = d->b.planes2_hi; t.post_lo = d->b.planes2_lo; t.ld_post = la->n;
   const int parts = chatts_linear_post_ss_parts(&t);
-  if (parts < 1 || 16 * 256 > (size_t)d->b.t_max * d->cfg.hidden || ((uintptr_t)d->b.delta % 16) != 0) return false;
+  // the sums of squares lie in b.attn: the attention's result in 32 bits, which a step on planes does not have, and which is over when they are written
+  if (parts < 1 || !d->b.attn || 16 * 256 > (size_t)d->b.t_max * d->cfg.n_q * kHeadDim || ((uintptr_t)d->b.attn % 16) != 0) return false;
   *la = t;
-  chain->post_ss = d->b.delta;
+  chain->post_ss = d->b.attn;
   d->normed = true; d->ss_parts = parts;
   return true;
 }

@@ -664,7 +664,7 @@ typedef struct ChattsDecoderBuffers {
   float* x;           /* [T_max, H] residual stream */
   float* xn;          /* [T_max, H] normed scratch (prefill) */
   float* qkv;         /* [T_max, (n_q+2n_kv)*128] */
-  float* attn;        /* [T_max, n_q*128] */
+  float* attn;        /* [T_max, n_q*128]; batched steps also keep the sums of squares of a norm that is under way here */
   float* act;         /* [T_max, inter] */
   float* delta;       /* [T_max, H] partial sums when tp_world > 1 */
   float* logits;      /* [vocab_local] */
@@ -674,7 +674,8 @@ typedef struct ChattsDecoderBuffers {
   int max_batch;      /* KV caches are [max_batch, n_layers, n_kv, max_ctx, 128]; 0 or 1 = single sequence */
   /* optional: two pairs of bf16 hi / lo planes, each plane [T_max, max(H, n_q*128, inter)] (ChattsLinearArgs.a_hi /
    * a_lo / c_hi / c_lo).  When all four are set, prefill chunks of >= 96 rows run the LDS-DMA GEMM: the RMSNorms and
-   * the SwiGLU epilogue write planes directly (pair 0 = projection input, pair 1 = gate_up output). */
+   * the SwiGLU epilogue write planes directly (pair 0 = projection input, pair 1 = gate_up output).  Batched steps of 2 .. 16 sequences use both pairs in
+   * turn: what a projection hands on lies in the pair that it does not read. */
   chatts_bf16* planes_hi;
   chatts_bf16* planes_lo;
   chatts_bf16* planes2_hi;

@@ -70,3 +70,12 @@ def test_separate_norms(monkeypatch, name, form):
         monkeypatch.setenv("CHATTS_POST_NORM_SMALL_M", "0")
         assert torch.equal(step(m, positions, tokens, batch), parts)
         monkeypatch.delenv("CHATTS_POST_NORM_SMALL_M")
+
+
+@pytest.mark.parametrize("batch", [3, 16])
+def test_one_gpu_leaves_delta_alone(batch):
+    """buffers.delta belongs to tensor parallelism: a program on one GPU may keep other things there"""
+    m, positions, tokens = model_of("chatts-8b", "bf16")
+    want = step(m, positions, tokens, batch)
+    m.buf["delta"].fill_(7.0)
+    assert torch.equal(step(m, positions, tokens, batch), want) and bool((m.buf["delta"] == 7.0).all())
