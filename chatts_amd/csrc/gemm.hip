@@ -976,12 +976,8 @@ bool gemm_batched_stream(const ChattsLinearArgs* a) {
          a->a_stride % 8 == 0 && a->w_stride % 8 == 0 && ((uintptr_t)a->c % 16) == 0 && opt_get(OPT_EPI_V4, 1) != 0 && pick_stream_sk(a->m, a->n * a->batch, a->k, false) <= 8;
 }
 // K ranges of gemm_stream_kernel for these arguments if launch_gemm hands them to gemm_rows_kernel, which takes the same ranges (bit-identical) and
-// writes post_ss in the same launch; 0: it does not.  Line: where K is split at all, and up to 8 rows; 8-bit weights beyond 4 rows only with eight K ranges (use_rows).
-// A workgroup of it reads all of X (~55 KB a us and CU), which beyond that costs more than the launch it saves.  us with the epilogue launch / in
-// one: bf16, 5 rows, 4096 x 4096: 9.9 / 9.0, 6144 x 4096: 12.8 / 11.2, 4096 x 12288: 19.9 / 20.5; 8 rows: 10.4 / 9.7, 12.9 / 11.9, 20.1 / 23.5.  fp8: 5120 x
-// 13824 (six ranges) 2 / 5 / 8 rows: 15.7 / 16.1 / 16.1 against 17.9 / 19.7 / 22.8.  On top of that comes the RMSNorm that moves into the launch (3 - 4 us
-// of a chain).  Whole steps: 8B bf16, 2 / 5 sequences 3.90 -> 3.59 / 4.24 -> 4.04 ms, 14B bf16, 8: 6.53 -> 6.21, 8B int8, 7: 3.20 -> 2.92, 14B fp8, 2 / 6 / 8:
-// 4.20 -> 3.95 / 4.47 -> 4.47 / 4.53 -> 4.68 (hence the line).
+// writes post_ss in the same launch; 0: it does not.  Line: where K is split at all, up to 8 rows (8-bit weights beyond 4 rows only with eight K ranges) and as
+// rows_pay (gemm_rows.hip) says.
 static int stream_ranges(const ChattsLinearArgs* a) {
   const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr));
   return (a->k + kps - 1) / kps;

@@ -245,6 +245,28 @@ static int rows_waves(int np, int sk) { return sk > (np + 1) / 2 ? sk : (np + 1)
 // K-steps ahead: ~16 KB a step of a workgroup, five of them in flight cover the latency; 8-bit weights have twice the X registers a step
 static int rows_ahead(bool w8, int np, int waves) { return waves > 8 ? 3 : (w8 ? (np > 6 ? 3 : 4) : 5); }
 
+// Is the launch that the split's epilogue costs worth more than X read by every workgroup (M x K x 4 bytes at ~55 KB a us and CU; the split reads a K range of it)?
+// Both sides measured back to back in a graph, 380 shapes N 1024 .. 10240, K 2048 .. 16384, residual epilogue, us split / here:
+//   * X up to 168 KB where K has five to eight ranges: 4096 x 4096 bf16, 8 rows 10.7 / 9.6; 5120 x 5120, 6 rows 13.0 / 12.5; but 4096 x 12288, 8 rows 20.1 / 23.5;
+//   * up to 256 KB with four ranges or fewer, whose split reads a larger part of X itself: 8192 x 8192, 8 rows 32.9 / 31.2; int8 7168 x 11264, 4 rows 18 % less here;
+//   * fp8 128 KB with eight ranges, 72 KB with five to seven: 4096 x 9216, 3 rows 13 % less; 4096 x 12288, 4 / 8 rows 13.1 / 13.8 and 13.2 / 17.7; 6144 x 4096, 4 rows
+//     13 % less, 6144 x 10240 15 % more.  Its waves spend their time widening W: five to seven waves load the four SIMDs unevenly;
+//   * and 8-bit not at all with five to seven ranges where more than a third of the fragments is rows that are not there: fp8 5120 x 13824, 2 rows 15.6 / 17.2;
+//   * rows of W 32 KB apart: 4096 x 16384 bf16, 2 rows 33.3 / 37.6;
+//   * a split of more than eight ranges (an epilogue that asks for one slab after the other) or of more workgroups than CUs has lost already: 2048 x 6144, 8 rows 13.2 /
+//     10.7; 7168 x 5120 20.6 / 15.7.
+// Beyond the line it would still win up to 14 % at K = 8192 with 5 to 8 rows and up to 11 % at 5120 or 6144 columns with K of 9216 to 12288; within it, it loses up to 3 %
+// at a few (5120 x 5120, 8 rows; fp8 4096 x 10240, 3 rows: 5 %).
+static bool rows_pay(const ChattsLinearArgs* a, int sk, int np) {
+  const int groups = a->n / (epi_is_glu(a->epilogue) ? 8 : 4), grid = rows_grid(a->n, a->epilogue), wrows = (groups + grid - 1) / grid * (epi_is_glu(a->epilogue) ? 8 : 4);
+  const bool w8 = a->w8 != nullptr, fp8 = w8 && a->w8_format != CHATTS_W8_INT8;
+  if (sk > 8 || (a->n + 127) / 128 * sk > device_cus()) return true;
+  if (sk > 4 && (w8 ? (size_t)a->ldw8 : 2 * (size_t)a->ldw) >= 32768) return false;
+  if (sk > 4 && sk < 8 && w8 && 16 * ((np + 1) / 2) * 2 > 3 * wrows) return false;
+  const int kb = sk <= 4 ? 256 : (!fp8 ? 168 : (sk == 8 ? 128 : 72));
+  return (size_t)a->m * a->k * 4 <= (size_t)kb * 1024;
+}
+
 bool use_rows(const ChattsLinearArgs* a, int sk) {
   // a workgroup stores its result while others still read A (the split's epilogue is a launch behind them)
   for (int i = 0; i < 3; ++i)
@@ -254,7 +276,7 @@ bool use_rows(const ChattsLinearArgs* a, int sk) {
   const size_t wbytes = w8 ? (size_t)a->n * a->ldw8 : (size_t)a->n * a->ldw * 2;
   const int np = rows_pieces(a->n, a->epilogue), waves = rows_waves(np, sk);
   const ptrdiff_t apart = reinterpret_cast<const char*>(a->a_lo) - reinterpret_cast<const char*>(a->a_hi);
-  return a->m >= 2 && a->m <= 8 && a->n % 16 == 0 && !a->planes_tiled && np <= 2 * kRowsMaxFN && waves <= (np == 1 && !w8 ? 16 : 8) && (!w8 || a->m <= 4 || waves == 8) &&
+  return a->m >= 2 && a->m <= 8 && a->n % 16 == 0 && rows_pay(a, sk, np) && !a->planes_tiled && np <= (w8 ? 2 * kRowsMaxFN : 6) && waves <= (np == 1 && !w8 ? 16 : 8) && (!w8 || a->m <= 4 || waves == 8) &&
          rows_lds(np, rows_ahead(w8, np, waves), waves) <= 156 * 1024 && wbytes < kRowsFar && (size_t)(apart < 0 ? -apart : apart) + (size_t)a->m * a->ld_planes * 2 < kRowsNoToken && a->ldc % 4 == 0 &&
          al(a->c) && al(a->resid) && al(a->bias) && al(a->w8_scale) &&
          (!a->c_hi || (a->ld_cplanes % 4 == 0 && ((uintptr_t)a->c_hi % 8) == 0 && ((uintptr_t)a->c_lo % 8) == 0));
@@ -288,8 +310,9 @@ static int launch_rows_w(const GemmParams& p, const ChattsLinearArgs* a, int sk,
     case 4: return launch_rows_t<W8, I8, 4, LA>(p, a, waves, s);
     case 5: return launch_rows_t<W8, I8, 5, LA>(p, a, waves, s);
     case 6: return launch_rows_t<W8, I8, 6, LA>(p, a, waves, s);
-    case 7: return launch_rows_t<W8, I8, 7, W8 ? 3 : LA>(p, a, waves, s);
-    default: return launch_rows_t<W8, I8, 8, W8 ? 3 : LA>(p, a, waves, s);
+    default:                                           // (bf16: use_rows has refused)
+      if constexpr (W8) return np == 7 ? launch_rows_t<true, I8, 7, 3>(p, a, waves, s) : launch_rows_t<true, I8, 8, 3>(p, a, waves, s);
+      return CHATTS_E_SHAPE;
   }
 }
 int launch_rows(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s) {

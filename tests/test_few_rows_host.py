@@ -67,3 +67,36 @@ def test_results_leave_the_sums_that_are_read_alone(lib, over):
     chain = _lib.NormChain(row_ss={"c": OUT + 64, "c_hi": OUT - 16 * 256 * 4 + 16, "c_lo": OUT + (1 << 24)}[over], row_ss_parts=256, row_eps=1e-6)
     assert int(lib.chatts_linear_chain(C.byref(a), C.byref(chain), None)) == _lib.E_SHAPE
     assert b"overlap" in lib.chatts_last_error()
+
+
+# both sides of every line: us of the split with its epilogue / of the few-rows kernel beside the shape
+@pytest.mark.parametrize("form,m,n,k,takes", [
+    ("bf16", 8, 4096, 4096, True),         # 10.7 / 9.6
+    ("bf16", 3, 4096, 12288, True),        # 147 KB of X: 19.9 / 19.2
+    ("bf16", 8, 4096, 12288, False),       # 393 KB: 20.1 / 23.5
+    ("bf16", 6, 5120, 5120, True),         # 13.0 / 12.5
+    ("bf16", 6, 5120, 13824, False),       # 25.2 / 26.3
+    ("bf16", 8, 8192, 8192, True),         # four ranges, 256 KB: 32.9 / 31.2
+    ("bf16", 7, 8192, 10240, False),       # 28.8 / 31.9
+    ("bf16", 2, 4096, 16384, False),       # rows 32 KB apart: 33.3 / 37.6
+    ("bf16", 8, 7168, 5120, True),         # the split has more workgroups than CUs: 20.6 / 15.7
+    ("bf16", 8, 2048, 6144, True),         # sixteen ranges: 13.2 / 10.7
+    ("fp8", 8, 4096, 4096, True),          # 8.3 / 7.6
+    ("fp8", 3, 4096, 12288, False),
+    ("fp8", 4, 4096, 12288, False),        # 13.1 / 13.8
+    ("fp8", 8, 4096, 12288, False),        # 13.2 / 17.7
+    ("fp8", 4, 6144, 4096, True),          # 9.4 / 8.4
+    ("fp8", 4, 6144, 10240, False),        # five ranges, 164 KB
+    ("fp8", 2, 5120, 13824, False),        # six ranges, a third of the fragments empty: 15.6 / 17.2
+    ("fp8", 2, 5120, 2048, True),          # four ranges: 31 % less here
+    ("int8", 4, 7168, 11264, True),
+    ("int8", 8, 4096, 4096, True),         # 8.7 / 7.7
+    ("int8", 8, 4096, 12288, False),       # 14.0 / 17.9
+])
+def test_the_faster_of_the_two(lib, form, m, n, k, takes):
+    a = args(m=m, n=n, k=k, lda=k, ldw=k, ldc=n, ld_planes=k, a_lo=A_HI + m * k * 2)
+    if form != "bf16":
+        a.w8, a.w8_scale, a.ldw8, a.w8_format = 0x7e0000000000, 0x7d0000000000, k, _lib.W8_INT8 if form == "int8" else _lib.W8_FP8
+    assert (few_rows(lib, a) > 1) == takes
+    a.post_norm_w, a.post_hi, a.post_lo, a.ld_post = 0x60000000, OUT + (1 << 24), OUT + (2 << 24), n
+    assert int(lib.chatts_linear_post_ss_parts(C.byref(a))) == 256      # (either of the two hands a norm on)
