@@ -259,6 +259,7 @@ static bool planes_path(const ChattsDecoder* d, int m, int k, bool fp8 = false) 
 // factor 1 / rms to this one (batched steps)
 static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream, ChattsNormChain* chain = nullptr) {
   if (planes_path(d, la->m, la->k, la->w8 != nullptr)) {
+    CHATTS_REQUIRE(chain || !d->ss_parts, CHATTS_E_BADARG, "decoder: a norm that was handed on without its factor has no projection to take it");
     la->a = nullptr; la->a_hi = d->b.planes_hi; la->a_lo = d->b.planes_lo; la->ld_planes = la->k;
     if (d->normed && d->ss_parts && chain) {
       la->a_hi = d->b.planes2_hi; la->a_lo = d->b.planes2_lo;
