@@ -581,10 +581,10 @@ __device__ __forceinline__ void f16q_put4(const F16qPlanes& o, int row, int col,
   }
 }
 
-// RMSNorm with the row written as f16q planes (rmsnorm_kernel<true>'s arithmetic; one workgroup per row)
-__global__ __launch_bounds__(256) void rmsnorm_f16q_kernel(const float* __restrict__ x, const float* __restrict__ w, int hidden, float eps, F16qPlanes o) {
+// RMSNorm with the row written as f16q planes (rmsnorm_kernel<true>'s arithmetic; one workgroup per row; rows of x are ldx apart, a multiple of 4)
+__global__ __launch_bounds__(256) void rmsnorm_f16q_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, int hidden, float eps, F16qPlanes o) {
   __shared__ float red[4];
-  const float* xr = x + (size_t)blockIdx.x * hidden;
+  const float* xr = x + (size_t)blockIdx.x * ldx;
   float ss = 0.f;
   for (int k = threadIdx.x * 4; k < hidden; k += 1024) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(xr + k);
@@ -769,17 +769,21 @@ extern "C" int chatts_tile_e4m3(const uint8_t* src, int rows, int k, int ld, uin
   return CHATTS_OK;
 }
 
-extern "C" int chatts_rmsnorm_f16q(const float* x, const float* w, chatts_f16* hi, uint8_t* lo8, uint8_t* scale, int ld_planes, int ld_scale, int t,
-                                   int hidden, float eps, int tiled, chatts_stream_t stream) {
+static int rmsnorm_f16q_rows(const float* x, int ldx, const float* w, chatts_f16* hi, uint8_t* lo8, uint8_t* scale, int ld_planes, int ld_scale, int t, int hidden, float eps,
+                             int tiled, chatts_stream_t stream) {
   CHATTS_REQUIRE(!tiled || ld_planes == hidden, CHATTS_E_SHAPE, "rmsnorm_f16q: tiled planes need ld_planes == hidden");
   CHATTS_REQUIRE(t >= 0 && hidden > 0 && hidden % kF16qBlock == 0, CHATTS_E_SHAPE, "rmsnorm_f16q: t=%d hidden=%d (a multiple of 128)", t, hidden);
   if (t == 0) return CHATTS_OK;
   CHATTS_REQUIRE(x && w && hi && lo8 && scale, CHATTS_E_BADARG, "rmsnorm_f16q: null pointer");
   CHATTS_REQUIRE(ld_planes >= hidden && ld_planes % 4 == 0 && ld_scale >= hidden / kF16qBlock, CHATTS_E_SHAPE, "rmsnorm_f16q: leading dimensions");
   F16qPlanes o{reinterpret_cast<_Float16*>(hi), lo8, scale, ld_planes, ld_scale, tiled};
-  hipLaunchKernelGGL(rmsnorm_f16q_kernel, dim3(t), dim3(256), 0, as_stream(stream), x, w, hidden, eps, o);
+  hipLaunchKernelGGL(rmsnorm_f16q_kernel, dim3(t), dim3(256), 0, as_stream(stream), x, ldx, w, hidden, eps, o);
   CHATTS_CHECK_LAUNCH("rmsnorm_f16q");
   return CHATTS_OK;
+}
+extern "C" int chatts_rmsnorm_f16q(const float* x, const float* w, chatts_f16* hi, uint8_t* lo8, uint8_t* scale, int ld_planes, int ld_scale, int t,
+                                   int hidden, float eps, int tiled, chatts_stream_t stream) {
+  return rmsnorm_f16q_rows(x, hidden, w, hi, lo8, scale, ld_planes, ld_scale, t, hidden, eps, tiled, stream);
 }
 
 extern "C" size_t chatts_linear_f16q_workspace(int m, int n, int k) {
@@ -842,6 +846,6 @@ extern "C" int chatts_linear_f16q(const ChattsLinearF16qArgs* a, chatts_stream_t
   CHATTS_CHECK_LAUNCH("gemm_f16q");
   if (sk > 1) return f16q_splitk_epilogue(a, sk, as_stream(stream));
   if (a->post_norm_w)
-    return chatts_rmsnorm_f16q(a->c, a->post_norm_w, a->post_hi, a->post_lo8, a->post_scale, a->ld_post, a->ld_pscale, a->m, a->n, a->post_norm_eps, a->planes_tiled, stream);
+    return rmsnorm_f16q_rows(a->c, a->ldc, a->post_norm_w, a->post_hi, a->post_lo8, a->post_scale, a->ld_post, a->ld_pscale, a->m, a->n, a->post_norm_eps, a->planes_tiled, stream);
   return CHATTS_OK;
 }

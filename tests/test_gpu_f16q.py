@@ -270,3 +270,31 @@ def test_linear_f16q_on_tiled_operands_is_bitwise_the_row_major_result(lib, epi,
         pad = lambda t: torch.cat([t, torch.zeros((m16 - m, t.shape[1]), dtype=t.dtype, device=DEV)]) if m16 > m else t
         assert torch.equal(_tile16(pad(ph0)).view(torch.int16), ph1.view(-1).view(torch.int16))
         assert torch.equal(_tile8_rows16(pl0, m)[0], pl1.view(-1)) and torch.equal(ps0, ps1)
+
+
+@pytest.mark.parametrize("gap", [64, 4])
+@pytest.mark.parametrize("m,n,k", [(17, 512, 128), (100, 1024, 2048)])      # K in one piece and split
+def test_norm_planes_where_rows_of_c_lie_further_apart(m, n, k, gap):
+    lib = _lib.load()
+    g = torch.Generator(device=DEV).manual_seed(m)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, w, nw, resid = r(m, k), (r(n, k) * k ** -0.5).bfloat16(), 1 + 0.1 * r(n), r(m, n)
+    half, byte = (lambda *s: torch.zeros(s, dtype=torch.float16, device=DEV)), (lambda *s: torch.zeros(s, dtype=torch.uint8, device=DEV))
+    hi, lo, sc = half(m, k), byte(m, k), byte(m, k // 128)
+    w16, w8, w8e = half(n, k), byte(n, k), byte(n)
+    _lib.check(lib.chatts_split_f16q(x.data_ptr(), m, k, k, hi.data_ptr(), lo.data_ptr(), sc.data_ptr(), k, k // 128, 0, st()))
+    _lib.check(lib.chatts_weights_f16q(w.data_ptr(), n, k, k, w16.data_ptr(), w8.data_ptr(), w8e.data_ptr(), k, st()))
+    ws = byte(max(int(lib.chatts_linear_f16q_workspace(m, n, k)), 16))
+    got = []
+    for ldc in (n, n + gap):
+        c, add = torch.full((2, m, ldc), 1e6, device=DEV)
+        add[:, :n] = resid
+        ph, pl, ps = half(m, n), byte(m, n), byte(m, n // 128)
+        a = _lib.LinearF16qArgs(a_hi=hi.data_ptr(), a_lo8=lo.data_ptr(), a_scale=sc.data_ptr(), ld_a=k, ld_scale=k // 128, w16=w16.data_ptr(), w8=w8.data_ptr(), w8_exp=w8e.data_ptr(),
+                                ldw=k, resid=add.data_ptr(), c=c.data_ptr(), m=m, n=n, k=k, ldc=ldc, epilogue=_lib.EPI_RESID, workspace=ws.data_ptr(), workspace_bytes=ws.numel())
+        a.post_norm_w, a.post_norm_eps, a.post_hi, a.post_lo8, a.post_scale, a.ld_post, a.ld_pscale = nw.data_ptr(), 1e-6, ph.data_ptr(), pl.data_ptr(), ps.data_ptr(), n, n // 128
+        _lib.check(lib.chatts_linear_f16q(a, st()))
+        torch.cuda.synchronize()
+        assert bool((c[:, n:] == 1e6).all())
+        got.append((c[:, :n].clone(), ph, pl, ps))
+    assert all(torch.equal(p, q) for p, q in zip(*got))
