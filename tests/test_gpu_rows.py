@@ -1,4 +1,4 @@
-"""Projections of 2 .. 8 rows by the few-rows kernel (csrc/gemm_rows.hip) against float64 on the stored weights, and bit for bit against the weight-streaming
+"""Projections of 2 .. 8 rows (csrc/gemm_rows.hip, or the split where that is faster) against float64 on the stored weights, and bit for bit against the weight-streaming
 kernel that runs 16 rows: columns that deal unevenly over the CUs, K ranges of unequal length, every weight format and epilogue, and an RMSNorm between two
 projections."""
 import ctypes as C
@@ -70,7 +70,8 @@ def reference(epi, z, resid):
     return {_lib.EPI_NONE: z, _lib.EPI_GELU: torch.nn.functional.gelu(z), _lib.EPI_RELU2: z.clamp(min=0) ** 2, _lib.EPI_RESID: resid.double() + z}[epi]
 
 
-# 4 .. 64 columns a workgroup, 1 .. 8 pieces, columns that leave some workgroups a group more, fewer groups than CUs, 2 .. 16 waves
+# columns that leave some workgroups a group more, fewer groups than CUs, 2 .. 16 waves; shapes on either side of the line to the split (test_every_size_of_a_workgroup
+# has those that the few-rows kernel takes, and says so)
 @pytest.mark.parametrize("form", ["bf16", "fp8", "int8"])
 @pytest.mark.parametrize("m,n,k", [(2, 64, 1024), (8, 5120, 5120), (5, 4096, 1024), (7, 7168, 2048), (8, 5120, 13824), (7, 6160, 1152), (3, 10256, 640), (8, 16384, 512),
                                    (5, 14352, 512), (6, 2048, 4096), (4, 8192, 2176)])
@@ -147,3 +148,43 @@ def test_a_result_in_the_place_of_its_own_input(lib, form, m, as_planes):
     assert lo.data_ptr() == hi.data_ptr() + m * k * 2
     out = hi.double() + lo.double() if as_planes else torch.as_strided(hi, (m, 2 * n), (2 * n, 1)).view(torch.float32)
     assert rel(out, want) < 1e-5
+
+
+# 8-row pieces of W a workgroup (1 .. 8; bf16 up to 6), K ranges of it; 8-bit with fewer ranges than fragments, so that a wave only helps to finish
+@pytest.mark.parametrize("form,m,n,k,pieces,ranges", [
+    ("bf16", 8, 1040, 4096, 1, 16), ("bf16", 2, 2048, 2048, 1, 8), ("bf16", 6, 4112, 4096, 3, 8), ("bf16", 8, 4096, 4096, 2, 8), ("bf16", 8, 5120, 4096, 3, 6), ("bf16", 5, 7184, 2048, 4, 4),
+    ("bf16", 3, 9232, 1536, 5, 4), ("bf16", 8, 10240, 2048, 5, 3), ("bf16", 7, 11280, 1024, 6, 3), ("bf16", 4, 12288, 2048, 6, 3),
+    *((form, m, n, k, p, r) for form in ("fp8", "int8") for m, n, k, p, r in [(3, 1040, 2048, 1, 4), (8, 4096, 4096, 2, 8), (4, 4112, 2048, 3, 4), (2, 8192, 2048, 4, 4), (4, 10240, 4096, 5, 3), (3, 9232, 1536, 5, 3),
+                                                                         (4, 11280, 1024, 6, 2), (2, 13328, 2048, 7, 2), (4, 14336, 1280, 7, 2), (4, 16384, 1152, 8, 2), (3, 15376, 4096, 8, 2)])])
+@pytest.mark.parametrize("epi", [_lib.EPI_NONE, _lib.EPI_RESID])
+def test_every_size_of_a_workgroup(lib, form, m, n, k, pieces, ranges, epi):
+    x, w, bias, resid, q, scale = problem(16, n, k, form, n + k)
+    hi, lo = planes(lib, x)
+    want = x.double() @ w.double().T + bias.double() + (resid.double() if epi == _lib.EPI_RESID else 0)
+    out, all16 = (torch.full((r, n), float("nan"), device=DEV) for r in (m, 16))
+    more = dict(bias=bias.data_ptr(), ldc=n, epilogue=epi, resid=resid.data_ptr())
+    a = args(m, n, k, hi, lo, w, q, scale, form, out, **more)
+    assert (-(-(n // 4) // 256) * 4 + 7) // 8 == pieces and int(lib.chatts_linear_few_rows(C.byref(a), None)) == ranges
+    run(lib, a, m, n, k)
+    assert rel(out, want[:m]) < 1e-5                      # (x to 2^-17, sums in 32 bits: 3e-6 measured)
+    run(lib, args(16, n, k, hi, lo, w, q, scale, form, all16, **more), 16, n, k)
+    assert torch.equal(out, all16[:m])
+
+
+# one fragment of gates and two, the last workgroups with a group less
+@pytest.mark.parametrize("form,m,n,k,ranges", [("bf16", 8, 6144, 2048, 5), ("bf16", 4, 96, 512, 2), ("bf16", 5, 8192, 1024, 4), ("bf16", 3, 5152, 1024, 4),
+                                               *((form, m, n, k, r) for form in ("fp8", "int8") for m, n, k, r in [(4, 96, 1024, 2), (2, 8192, 2048, 4), (4, 12288, 1024, 2), (3, 8224, 2048, 3), (4, 16384, 1024, 2)])])
+@pytest.mark.parametrize("epi", sorted(GLU))
+def test_gated_as_with_sixteen_rows(lib, form, m, n, k, ranges, epi):
+    x, w, bias, _, q, scale = problem(16, n, k, form, n + k)
+    hi, lo = planes(lib, x)
+    got = []
+    for rows in (m, 16):
+        ph, pl = torch.full((2, rows, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+        a = args(rows, n, k, hi, lo, w, q, scale, form, None, bias=bias.data_ptr(), ldc=n // 2, c_hi=ph.data_ptr(), c_lo=pl.data_ptr(), ld_cplanes=n // 2, epilogue=epi, glu_limit=1.5, glu_alpha=1.7)
+        assert int(lib.chatts_linear_few_rows(C.byref(a), None)) == (ranges if rows == m else 0)
+        run(lib, a, rows, n, k)
+        got.append((ph[:m], pl[:m]))
+    want = reference(epi, x.double() @ w.double().T + bias.double(), None)
+    assert rel(got[0][0].double() + got[0][1].double(), want[:m]) < 1e-5
+    assert all(torch.equal(a, b) for a, b in zip(*got))
