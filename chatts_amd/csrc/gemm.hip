@@ -288,7 +288,9 @@ __device__ __forceinline__ void wait_stages(int later) {
 // wave (LDS reads -> fp8 widening -> MFMAs) is what paces a workgroup when it is alone on its CU (a deeper ring changes nothing,
 // profiles/r3_stream_sweep_fp8.txt), and two waves per SIMD overlap their chains.  Every output column still sees its K-steps in
 // the same order with the same operands: bit-identical to NW = 4.
-template <int NSTAGE, bool W8, int MB, int NW = 4, bool I8 = false>
+// SS: the rows' factors 1 / rms come from p.row_ss.  An instance of its own, because the loads in front and the factors behind cost the other calls 1 % (bf16) to 2 - 3 %
+// (int8: 5120 x 13824, 16 rows 18.1 -> 17.6 us).
+template <int NSTAGE, bool W8, int MB, int NW = 4, bool I8 = false, bool SS = false>
 __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, const uint16_t* __restrict__ a_hi,
                                                               const uint16_t* __restrict__ a_lo, int ldp) {
   if (gridDim.y > 1) {      // (uniform) one of several products of the same shape
@@ -297,6 +299,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
     a_lo += blockIdx.y * p.a_stride;
     p.c += blockIdx.y * p.c_stride;
   }
+  static_assert(!SS || MB == 1, "row factors are for M <= 16");
   static_assert(!W8 || MB == 1, "the fp8 weight stream is a batched-decode format (M <= 16)");
   static_assert(NW == 4 || (NW == 8 && (W8 || MB % 2 == 0)), "8 waves: fp8 W (one A piece per wave), or bf16 W with an even block count");
   // wave grid inside the 16 MB x 128 tile: WM x WN.  4 waves: 1 x 4 (32 columns each).  8 waves, fp8 W (M <= 16): 1 x 8 (16 columns).
@@ -367,7 +370,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[b][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   f32x4 rs_part[16 / NW];
-  if constexpr (MB == 1) row_rstd_load(p, wave, NW, lane, rs_part);
+  if constexpr (SS) row_rstd_load(p, wave, NW, lane, rs_part);
 #pragma unroll
   for (int s = 0; s < NSTAGE - 1; ++s)
     if (s < nk) issue(s);
@@ -412,18 +415,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(GemmParams p, cons
       }
     }
   }
-  if constexpr (MB == 1) {
-    if (p.row_ss) {                              // (uniform; the factors take the ring's place: 80 KB of LDS a workgroup let two share a CU)
-      float* rstd_s = reinterpret_cast<float*>(smem);
-      __syncthreads();
-      row_rstd_store(p, wave, NW, lane, rs_part, rstd_s);
-      __syncthreads();
+  if constexpr (SS) {                            // (the factors take the ring's place: 80 KB of LDS a workgroup let two share a CU)
+    float* rstd_s = reinterpret_cast<float*>(smem);
+    __syncthreads();
+    row_rstd_store(p, wave, NW, lane, rs_part, rstd_s);
+    __syncthreads();
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float f = rstd_s[(lane >> 4) * 4 + r];
+    for (int r = 0; r < 4; ++r) {
+      const float f = rstd_s[(lane >> 4) * 4 + r];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[0][j][r] *= f;
-      }
+      for (int j = 0; j < FN; ++j) acc[0][j][r] *= f;
     }
   }
   if constexpr (FN == 1) {
@@ -955,19 +956,25 @@ static int pick_stream_sk(int m, int n, int k, bool w8) {
   return sk;
 }
 
-template <int NSTAGE, bool W8, int MB = 1, int NW = 4, bool I8 = false>
-static int launch_stream_t(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s) {
+template <int NSTAGE, bool W8, int MB, int NW, bool I8, bool SS>
+static int launch_stream_ss(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s) {
   constexpr int LDS = NSTAGE * stream_stage(W8, MB);
   static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_stream_kernel<NSTAGE, W8, MB, NW, I8>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_stream_kernel<NSTAGE, W8, MB, NW, I8, SS>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_stream: cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(e));
     configured = true;
   }
   dim3 grid((a->n + kStreamBN - 1) / kStreamBN, a->batch > 1 ? a->batch : 1, sk), block(64 * NW);
-  hipLaunchKernelGGL((gemm_stream_kernel<NSTAGE, W8, MB, NW, I8>), grid, block, LDS, s, p, a->a_hi, a->a_lo, a->ld_planes);
+  hipLaunchKernelGGL((gemm_stream_kernel<NSTAGE, W8, MB, NW, I8, SS>), grid, block, LDS, s, p, a->a_hi, a->a_lo, a->ld_planes);
   return CHATTS_OK;
+}
+template <int NSTAGE, bool W8, int MB = 1, int NW = 4, bool I8 = false>
+static int launch_stream_t(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s) {
+  if constexpr (MB == 1)
+    if (p.row_ss) return launch_stream_ss<NSTAGE, W8, MB, NW, I8, true>(p, a, sk, s);
+  return launch_stream_ss<NSTAGE, W8, MB, NW, I8, false>(p, a, sk, s);
 }
 
 // can the weight-streaming kernel run all members of ChattsLinearArgs.batch at once (and the plain split-K epilogue finish them)?
