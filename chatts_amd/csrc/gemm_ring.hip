@@ -292,11 +292,12 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 
 // ---- host side ------------------------------------------------------------------------------------------------------------------
 // (T, sk) per shape: a cost model in cycles of the slowest workgroup - rounds x (K-steps x step + a per-unit constant) + the split-K epilogue launch.  Fitted to
-// 4500 measurements of every (T, sk) for 14 projections (K 2048 .. 13824, N 1536 .. 27648) at 100 .. 1300 rows: a 64-deep step of a tile with f fragments
+// 4500 measurements of (T, sk), T up to five above the fewest, for 14 projections (K 2048 .. 13824, N 1536 .. 27648) at 100 .. 1300 rows: a 64-deep step of a tile with f fragments
 // takes 253 f + 1069 cycles (the 16 f MFMAs per SIMD and the (32 f + 256) x 128 bytes of LDS-DMA overlap only partly), a unit 4800 of prologue and stores, a
 // split-K epilogue 5 us (8 from five slabs on, more where its threads cannot ask for all slabs at once) and its slab traffic at ~4.5 to 5 TB/s, less
-// where the slabs outgrow 64 MB.  Over these shapes its pick is 0.8 % slower than the best pair in the mean; the constants before (235 f + 900, 9000 a unit, a
-// row-walking epilogue from five slabs on) gave 1.4 % and up to 17 %: 5120 x 13824 at 223 rows (3, 4) 80.3 us, now (2, 6) 72.5; 4096 x 4096 at 900 rows 80.8 / 71.4.
+// where the slabs outgrow 64 MB.  Over these its pick is 0.8 % slower than the best pair in the mean, the constants before (235 f + 900, 9000 a unit, a
+// row-walking epilogue from five slabs on) gave 1.4 %.  Over 480 cells of 24 projections at 129 .. 2048 rows with any T it is 2.5 % (at most 23: 8192 x 2048, 129 rows, where (3, 2)
+// beats (2, 4)), before 3.3 % (33); where the two picks differ by more than 3 %, this one is faster in 58 cells and slower in 20.  5120 x 13824 at 223 rows (3, 4) 80.3 us, now (2, 6) 72.5; 4096 x 4096 at 900 rows 80.8 / 71.4.
 // Panels of 192 rows are the second width: a step costs 215 f + 1080 there, dearer per column, but where panels of 256 leave CUs without a unit it fills them:
 // 24576 x 4096 gated, 223 rows: 96 panels x 2 tiles on 192 CUs 94.5 us, 128 x 2 on 256 CUs 90.3; 6144 x 4096 at 223 rows 36.4 / 34.2, 5120 x 5120 at 150 rows
 // 36.9 / 34.4, 6144 x 2048 at 380 rows 31.5 / 26.6; 27648 x 5120 (108 panels; 144 would need two rounds) stays at 256: 125.7 / 162.
@@ -312,10 +313,14 @@ void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int forc
   for (int nf = 4; nf >= 3; --nf) {
     if (force_nf && nf != force_nf) continue;
     const int P = (n + 64 * nf - 1) / (64 * nf);
+    const double frag = nf == 4 ? 253.0 : 215.0, tile = nf == 4 ? 1069.0 : 1080.0;
     for (int T = tmin; T <= tmax; ++T) {
       const int fmax = (F + T - 1) / T;
-      const double step = nf == 4 ? 253.0 * fmax + 1069.0 : 215.0 * fmax + 1080.0;
-      if ((double)T * P * nk * step > best * slots) break;      // (the work itself, evenly spread: more tiles only add to it)
+      const double step = frag * fmax + tile;
+      // the work itself, evenly spread over the CUs.  Its fragments and a constant a tile: more tiles only add to that.  With the fragments that are not there it rises and
+      // falls (128 fragments: 31 tiles of 5, 32 tiles of 4)
+      if ((frag * F + tile * T) * P * nk > best * slots) break;
+      if ((double)T * P * nk * step > best * slots) continue;
       for (int sk = 1; sk <= 16; ++sk) {
         if (sk > 1 && nk / sk < 4) break;
         const long long units = (long long)T * P * sk;
@@ -326,6 +331,8 @@ void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int forc
           const double slabs = (double)m * n * 4.0;
           t += (sk <= 4 ? 10200.0 : sk <= 8 ? 17600.0 : 30000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1840.0 : sk <= 4 ? 2200.0 : 2480.0);
         }
+        // a split that is no more than 0.6 % nearer counts as equal: slabs are the part that the model knows least (6144 x 4096, 700 rows: (5, 2) 68.3 us, (9, 1) 62.7)
+        if (sk > 1) t *= 1.006;
         if (t < best) { best = t; bt = T; bs = sk; bf = nf; }
       }
     }

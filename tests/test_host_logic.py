@@ -193,6 +193,13 @@ def test_decode_gemv_kernel_choice_is_pinned_by_shape():
 
 
 
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 4096), (900, 2048, 2048), (512, 2048, 4096)])
+def test_prefill_tiles_are_searched_to_the_end(m, n, k):
+    """2048 rows are 128 fragments: 31 tiles take five fragments each and more work than 16 tiles with K in two; 32 tiles take four and beat both (63.1 us against 68.0).  The search used to
+    stop at 31.  A split that is as near as makes no difference loses to K in one piece, which needs no scratch."""
+    assert (int(_lib.load().chatts_linear_workspace(m, n, k)) == 0) == (m > 512)
+
+
 def test_tuning_options_table_set_get_unset_and_the_environment_mirror(monkeypatch):
     """chatts_set_option / _unset_option / _get_option / _option_name (include/chatts_amd.h): the table is host code - every name the
     header documents exists, unknown names are refused with a message, a leading CHATTS_ is ignored, unset(NULL) clears everything, and
