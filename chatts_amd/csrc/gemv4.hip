@@ -256,9 +256,10 @@ int launch_gemv4(const ChattsLinearArgs* a, hipStream_t s, bool* done) {
   p.parts_inv = parts > 1 ? (unsigned)((0x100000000ull + parts - 1) / parts) : 0u;      // (units of a workgroup stay below 65536)
   const size_t lds = q4_lds(a->k, (quads + grid - 1) / grid);
   // Short rows of few codes stay with gemv4_ldsx_kernel: laying x out as operands and the reduction over the waves cost 4.3 us before any code is read, its batches
-  // 3 us (us there / here: 1024 x 512 3.0 / 4.3, 4096 x 1024 3.8 / 4.4, 4096 x 2048 4.6 / 5.0, 8192 x 1024 4.55 / 4.8; but 16384 x 1024 6.5 / 5.6,
-  // 9728 x 896 6.4 / 5.3, and from 4096 codes a row on at any n: 1024 x 4096 5.8 / 5.1, 256 x 4096 5.2 / 5.0).
-  const bool small = a->k <= 2048 && (size_t)a->n * a->k <= (size_t)1 << 23;
+  // 3 us and a step for every 1024 codes a row.  us there / here: 1024 x 512 3.0 / 4.3, 4096 x 1024 3.8 / 4.4, 8192 x 1024 4.55 / 4.8, 6144 x 2048 5.1 / 5.9, 1536 x 2560 4.7 / 5.2,
+  // 4096 x 2560 5.2 / 5.45; but 7168 x 1536 1 to 8 % less here, 9728 x 896 6.4 / 5.3, 16384 x 1024 6.5 / 5.6, 3072 x 2560 with the norm 7 % less, and from 3073 codes a row on
+  // at any n (1024 x 4096 5.8 / 5.1, 256 x 4096 within 3 %).  Left over: 7168 x 2048 (9 % without the norm), 10240 x 1024 (12 %).
+  const bool small = (a->k <= 2048 && (a->n <= 6144 || (size_t)a->n * a->k <= (size_t)1 << 23)) || (a->k <= 3072 && a->n <= (a->norm_w ? 2048 : 4096));
   *done = !small && a->w4_group >= 32 && a->n % 16 == 0 && a->k % 32 == 0 && a->k <= kQ4Turns * kQ4Threads * 8 && a->ldw4 % 16 == 0 && ((uintptr_t)a->w4 % 16) == 0 && ((uintptr_t)a->a % 16) == 0 &&
           ((uintptr_t)a->norm_w % 16) == 0 && (size_t)a->n * a->ldw4 < kQ4Far && (size_t)a->n * p.ng * 8 < kQ4Far && ((uintptr_t)a->w4_sz % 8) == 0 && lds <= 156 * 1024 &&
           (a->epilogue == CHATTS_EPI_NONE || a->epilogue == CHATTS_EPI_RESID || a->epilogue == CHATTS_EPI_SWIGLU);

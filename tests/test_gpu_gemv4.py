@@ -32,7 +32,8 @@ def run(x, w4, sz, deq, group, epi, bias=None, resid=None, norm=None):
 
 # the smallest of K, of N, of both; K that ends inside a unit; a row of units for some workgroups only; the largest K; both sides of the line to the old kernel
 SHAPES = [(16, 2560, 128), (16, 2080, 32), (1040, 2112, 64), (5120, 5120, 128), (7168, 5120, 128), (96, 13824, 128), (13200, 640, 64), (98304, 96, 32), (4096, 12288, 64),
-          (320, 16384, 128), (4096, 2048, 1024), (4112, 2048, 1024), (32, 4096, 256), (48, 96, 32), (1040, 1024, 32)]
+          (320, 16384, 128), (4096, 2048, 1024), (4112, 2048, 1024), (32, 4096, 256), (48, 96, 32), (1040, 1024, 32),
+          (16, 3584, 128), (16, 3104, 32), (1040, 3136, 64), (6144, 2048, 1024), (6160, 2048, 1024), (4096, 2560, 64), (4112, 2560, 64), (2064, 3072, 32)]
 
 
 @pytest.mark.parametrize("n,k,group", SHAPES)
@@ -69,7 +70,7 @@ def test_sums(n, k, group, norm, epi):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("k", [2592, 2560, 5088])
+@pytest.mark.parametrize("k", [2592, 2560, 5088, 3616, 3584])
 def test_rows_do_not_read_each_other(k):
     x, (w4, sz), deq, *_ = problem(128, k, 32, k)
     clean = run(x, w4, sz, deq, 32, _lib.EPI_NONE)
@@ -79,7 +80,7 @@ def test_rows_do_not_read_each_other(k):
 
 
 @pytest.mark.parametrize("at", [0, 1])                # the first columns of a wider matrix, and the last ones: the last row ends where the memory ends
-@pytest.mark.parametrize("k,group", [(2592, 32), (4096 + 64, 64), (5088, 32), (5120, 128)])
+@pytest.mark.parametrize("k,group", [(2592, 32), (3104, 32), (4096 + 64, 64), (5088, 32), (5120, 128)])
 def test_columns_of_a_wider_matrix(at, k, group):
     n = 96
     x, (w4, sz), deq, *_ = problem(n, k, group, k)
