@@ -41,6 +41,7 @@ struct ChattsDecoder {
   bool x_in_xn = false;     // batched step: o_proj left the residual stream in b.xn (ping-pong, see layer_part_batched); down_proj brings it back
   bool normed = false;      // planes 0 already hold RMSNorm(x) for the projection that comes next (written by the previous
                             // projection's fused epilogue): norm_into only binds them
+  bool normed_tiled = false;      // ... in the prefill kernel's blocks
   int ss_parts = 0;         // > 0, with normed: ... planes 1 hold norm_w * x without the factor 1 / rms; each row's sum of squares is that many parts in
                             // b.attn: a step of 2 .. 16 sequences behind a projection that hands its norm on (request_post_ss)
   bool sampling = false;    // token selection of the decode steps: greedy argmax, or the sampler with `sa`
@@ -257,11 +258,12 @@ static bool planes_path(const ChattsDecoder* d, int m, int k, bool fp8 = false) 
   return m >= 96 && !fp8;
 }
 
-// x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.  chain: where the projection before may have left the
-// factor 1 / rms to this one (batched steps)
-// planes of a prefill chunk of m rows and width k in the prefill kernel's blocks?  (its producers and consumers ask alike)
+// planes of a prefill chunk of m rows and width k in the prefill kernel's blocks?  Asked once for each set of planes, by whoever writes them: PLANE_TILES may change beside a running call
 static bool tiles_path(const ChattsDecoder* d, int m, int k) { return planes_path(d, m, k) && planes_tiled_for(m, k); }
-static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream, ChattsNormChain* chain = nullptr, bool tiled = false) {
+// x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.  chain: where the projection before may have left the
+// factor 1 / rms to this one (batched steps).  tiled: (a prefill chunk) the form of the planes that la gets
+static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream, ChattsNormChain* chain = nullptr, bool* tiled = nullptr) {
+  if (tiled) *tiled = false;
   if (planes_path(d, la->m, la->k, la->w8 != nullptr)) {
     CHATTS_REQUIRE(chain || !d->ss_parts, CHATTS_E_BADARG, "decoder: a norm that was handed on without its factor has no projection to take it");
     la->a = nullptr; la->a_hi = d->b.planes_hi; la->a_lo = d->b.planes_lo; la->ld_planes = la->k;
@@ -271,8 +273,14 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
       d->normed = false; d->ss_parts = 0;
       return CHATTS_OK;
     }
-    if (d->normed) { d->normed = false; return CHATTS_OK; }
-    if (tiled) return launch_rmsnorm_planes(d->b.x, la->k, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, la->m & ~15, as_stream(stream));
+    if (d->normed) {
+      CHATTS_REQUIRE(tiled || !d->normed_tiled, CHATTS_E_BADARG, "decoder: planes in tiles are the prefill kernel's");
+      if (tiled) *tiled = d->normed_tiled;
+      d->normed = false;
+      return CHATTS_OK;
+    }
+    if (tiled) *tiled = tiles_path(d, la->m, la->k);
+    if (tiled && *tiled) return launch_rmsnorm_planes(d->b.x, la->k, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, la->m & ~15, as_stream(stream));
     return chatts_rmsnorm_planes(d->b.x, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, stream);
   }
   d->normed = false; d->ss_parts = 0;
@@ -307,7 +315,9 @@ static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const floa
   la->post_norm_w = next_norm_w; la->post_norm_eps = d->cfg.rms_eps;
   la->post_hi = d->b.planes_hi; la->post_lo = d->b.planes_lo; la->ld_post = la->n;
   d->normed = true;
+  d->normed_tiled = tiles_path(d, la->m, la->n);
 }
+static PlaneTiles after(const ChattsDecoder* d, const ChattsLinearArgs& la, bool a_tiled) { return {a_tiled, false, la.post_norm_w && d->normed_tiled}; }      // (of a projection behind request_post_norm)
 
 extern "C" int chatts_decoder_set_sampling(ChattsDecoder* d, const ChattsSamplingArgs* sa) {
   CHATTS_REQUIRE(d, CHATTS_E_BADARG, "decoder_set_sampling: null decoder");
@@ -546,7 +556,8 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   const ChattsLayerWeights& lw = d->layers[layer];
   const bool tp = c.tp_world > 1;
   const int H = c.hidden;
-  const bool tile_h = t > 1 && tiles_path(d, t, H), tile_act = t > 1 && tiles_path(d, t, c.inter), tile_attn = t > 1 && tiles_path(d, t, c.n_q * kHeadDim);
+  const bool tile_act = t > 1 && tiles_path(d, t, c.inter), tile_attn = t > 1 && tiles_path(d, t, c.n_q * kHeadDim);
+  bool tile_h = false;
   int rc;
   ChattsLinearArgs la;
   if (part == 0) {
@@ -561,7 +572,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
       la.w8 = lw.qkv8; la.w8_scale = lw.qkv8_scale; la.ldw8 = H; la.w8_format = d->cfg.w8_format;
       la.w4 = lw.qkv4; la.w4_sz = lw.qkv4_sz; la.ldw4 = H / 2; la.w4_group = lw.w4_group;
     } else {
-      if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, tile_h)) != 0) return rc;
+      if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
     }
     ChattsKvCache kc = layer_cache(d, layer, d->cur_seq);
     bool rope_done = false;
@@ -620,7 +631,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
     } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
     else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
     request_post_norm(d, &la, lw.post_norm, false);
-    return linear_tiled(&la, stream, {tile_attn, false, tile_h && la.post_norm_w});
+    return linear_tiled(&la, stream, after(d, la, tile_attn));
   }
   // part 1: RMSNorm -> gate_up + SwiGLU -> down (+ residual / partial)
   la = ChattsLinearArgs{};
@@ -632,7 +643,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
     la.w8 = lw.gate_up8; la.w8_scale = lw.gate_up8_scale; la.ldw8 = H; la.w8_format = d->cfg.w8_format;
     la.w4 = lw.gate_up4; la.w4_sz = lw.gate_up4_sz; la.ldw4 = H / 2; la.w4_group = lw.w4_group;
   } else {
-    if ((rc = norm_into(d, lw.post_norm, &la, stream, nullptr, tile_h)) != 0) return rc;
+    if ((rc = norm_into(d, lw.post_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
   }
   const bool act_planes = t > 1 && planes_path(d, t, c.inter);   // SwiGLU output goes straight into down_proj's operand format
   if (act_planes) { la.c = nullptr; la.c_hi = d->b.planes2_hi; la.c_lo = d->b.planes2_lo; la.ld_cplanes = c.inter; }
@@ -653,7 +664,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
   else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
   request_post_norm(d, &la, layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : nullptr, false);
-  return linear_tiled(&la, stream, {tile_act, false, tile_h && la.post_norm_w});
+  return linear_tiled(&la, stream, after(d, la, tile_act));
 }
 
 extern "C" int chatts_decoder_layer_part_add(ChattsDecoder* d, int add_delta, int layer, int part, int t, int pos0,
@@ -855,8 +866,8 @@ static int layer_last_row(ChattsDecoder* d, int layer, int t, int pos0, chatts_s
   la.w = lw.qkv; la.w_tiled = lw.qkv_t; la.bias = lw.qkv_bias; la.c = d->b.qkv; la.m = t; la.n = qkv_n; la.k = H;
   la.lda = H; la.ldw = H; la.ldc = qkv_n; la.epilogue = CHATTS_EPI_NONE;
   la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
-  const bool tile_h = tiles_path(d, t, H);
-  if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, tile_h)) != 0) return rc;
+  bool tile_h;
+  if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
   if ((rc = linear_tiled(&la, stream, {tile_h, false, false})) != 0) return rc;
   ChattsKvCache kc = layer_cache(d, layer, d->cur_seq);
   if ((rc = chatts_rope_kv_write(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0,
@@ -934,7 +945,8 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
   const ChattsDecoderConfig& c = d->cfg;
   const ChattsLayerWeights& lw = d->layers[layer];
   const int H = c.hidden, qkv_n = (c.n_q + 2 * c.n_kv) * kHeadDim, na = c.n_q * kHeadDim;
-  const bool tile_h = t > 1 && tiles_path(d, t, H), tile_attn = t > 1 && tiles_path(d, t, na);
+  const bool tile_attn = t > 1 && tiles_path(d, t, na);
+  bool tile_h;
   int rc;
   d->normed_q = false;      // (f16q mode: this half runs the default kernels and is about to overwrite planes 0 - the next MLP half recomputes its norm)
   const bool f8 = d->prefill_fp8 && t >= 16;          // speed mode: qkv and o_proj as fp8 x fp8 GEMMs (layer_part_fp8's arithmetic)
@@ -951,7 +963,7 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
     la.w = lw.qkv; la.w_tiled = lw.qkv_t; la.bias = lw.qkv_bias; la.c = d->b.qkv; la.m = t; la.n = qkv_n; la.k = H;
     la.lda = H; la.ldw = H; la.ldc = qkv_n; la.epilogue = CHATTS_EPI_NONE;
     la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
-    if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, tile_h)) != 0) return rc;
+    if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
     if ((rc = linear_tiled(&la, stream, {tile_h, false, false})) != 0) return rc;
   }
   for (int i = 0; i < n_segs; ++i) {
@@ -983,7 +995,7 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
   }
   la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID;
   request_post_norm(d, &la, lw.post_norm, false);
-  return linear_tiled(&la, stream, {tile_attn, false, tile_h && la.post_norm_w});
+  return linear_tiled(&la, stream, after(d, la, tile_attn));
 }
 
 extern "C" int chatts_decoder_prefill_packed(ChattsDecoder* d, const ChattsPrefillSegment* segs, int n_segs, chatts_stream_t stream) {

@@ -1,5 +1,7 @@
 """Planes between the projections of a prefill chunk and of the encoder in the prefill kernel's blocks (PLANE_TILES, on from 129 rows): the same bits as row-major planes, for chunks
 that end with a whole block of 16 rows, with one more row and with one row less, split and unsplit projections, packed prompts, and every kernel that writes such planes."""
+import threading
+
 import pytest
 import torch
 
@@ -92,3 +94,29 @@ def test_the_encoder(name, patches, fused):
     with _lib.options(TS_L0_FUSED=int(fused)):
         on, off = both(lambda: e(x.view(3, -1, 1), valid_lengths=lengths)[0].clone())
     assert on.shape[0] >= patches and torch.isfinite(on).all() and torch.equal(on, off)
+
+
+def test_a_switch_thrown_beside_running_prompts(model):
+    """PLANE_TILES changed by another thread while the layers are being enqueued: every projection reads its planes in the form in which they were written"""
+    ids, stop = prompt(300, 7), threading.Event()
+    lib = _lib.load()
+
+    def run():
+        return model.generate_one(ids, None, None, max_new_tokens=1, return_logits=True)[1].clone()
+
+    want = run()
+
+    def throw():
+        while not stop.is_set():
+            for v in (0, 1) * 50:
+                lib.chatts_set_option(b"PLANE_TILES", v)
+
+    t = threading.Thread(target=throw)
+    t.start()
+    try:
+        got = [run() for _ in range(40)]
+    finally:
+        stop.set()
+        t.join()
+        lib.chatts_unset_option(b"PLANE_TILES")
+    assert all(torch.equal(g, want) for g in got)
