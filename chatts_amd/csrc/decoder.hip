@@ -258,7 +258,8 @@ static bool planes_path(const ChattsDecoder* d, int m, int k, bool fp8 = false) 
   return m >= 96 && !fp8;
 }
 
-// planes of a prefill chunk of m rows and width k in the prefill kernel's blocks?  Asked once for each set of planes, by whoever writes them: PLANE_TILES may change beside a running call
+// planes of a prefill chunk of m rows and width k in the prefill kernel's blocks?  Asked once for each set of planes, by whoever writes them: PLANE_TILES may change beside a running call.
+// A projection writes them so only if it runs that kernel: its own operand comes as planes and nothing else (a width of half a K-step more than whole ones does not)
 static bool tiles_path(const ChattsDecoder* d, int m, int k) { return planes_path(d, m, k) && planes_tiled_for(m, k); }
 // x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.  chain: where the projection before may have left the
 // factor 1 / rms to this one (batched steps).  tiled: (a prefill chunk) the form of the planes that la gets
@@ -315,7 +316,7 @@ static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const floa
   la->post_norm_w = next_norm_w; la->post_norm_eps = d->cfg.rms_eps;
   la->post_hi = d->b.planes_hi; la->post_lo = d->b.planes_lo; la->ld_post = la->n;
   d->normed = true;
-  d->normed_tiled = tiles_path(d, la->m, la->n);
+  d->normed_tiled = !la->a && tiles_path(d, la->m, la->n);
 }
 static PlaneTiles after(const ChattsDecoder* d, const ChattsLinearArgs& la, bool a_tiled) { return {a_tiled, false, la.post_norm_w && d->normed_tiled}; }      // (of a projection behind request_post_norm)
 
@@ -556,7 +557,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   const ChattsLayerWeights& lw = d->layers[layer];
   const bool tp = c.tp_world > 1;
   const int H = c.hidden;
-  const bool tile_act = t > 1 && tiles_path(d, t, c.inter), tile_attn = t > 1 && tiles_path(d, t, c.n_q * kHeadDim);
+  const bool tile_attn = t > 1 && tiles_path(d, t, c.n_q * kHeadDim);
   bool tile_h = false;
   int rc;
   ChattsLinearArgs la;
@@ -645,7 +646,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   } else {
     if ((rc = norm_into(d, lw.post_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
   }
-  const bool act_planes = t > 1 && planes_path(d, t, c.inter);   // SwiGLU output goes straight into down_proj's operand format
+  const bool act_planes = t > 1 && planes_path(d, t, c.inter), tile_act = act_planes && !la.a && tiles_path(d, t, c.inter);   // SwiGLU output goes straight into down_proj's operand format
   if (act_planes) { la.c = nullptr; la.c_hi = d->b.planes2_hi; la.c_lo = d->b.planes2_lo; la.ld_cplanes = c.inter; }
   if ((rc = linear_tiled(&la, stream, {tile_h, tile_act, false})) != 0) return rc;
   la = ChattsLinearArgs{};

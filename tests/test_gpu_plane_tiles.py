@@ -120,3 +120,14 @@ def test_a_switch_thrown_beside_running_prompts(model):
         t.join()
         lib.chatts_unset_option(b"PLANE_TILES")
     assert all(torch.equal(g, want) for g in got)
+
+
+# widths that are whole K-steps of the prefill kernel and widths that are half a step more: hidden, feed-forward, both
+@pytest.mark.parametrize("hidden,inter", [(288, 512), (256, 544), (288, 544), (256, 512)])
+@pytest.mark.parametrize("n", [128, 129, 150])
+def test_widths_that_other_kernels_take(hidden, inter, n):
+    cfg = preset("chatts-8b", num_hidden_layers=3, hidden_size=hidden, intermediate_size=inter, vocab_size=4096, ts_token_start_index=4000, eos_token_id=[4003, 4002], pad_token_id=4002)
+    m = ChatTSForCausalLM.from_synthetic(cfg, seed=5, max_ctx=256, max_prefill_tokens=256, max_batch=1, enable_prefix_caching=False)
+    ids = prompt(n, n)
+    on, off = both(lambda: m.generate_one(ids, None, None, max_new_tokens=1, return_logits=True)[1].clone())
+    assert torch.isfinite(on).all() and torch.equal(on, off)
