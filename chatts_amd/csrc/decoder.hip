@@ -18,6 +18,7 @@ size_t gemm_workspace_batch(int m, int n, int k, int batch);
 int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain, PlaneTiles tiles);
 int gemm_post_ss_parts(const ChattsLinearArgs* a);
 int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
+bool gemm_takes_cols(const ChattsLinearArgs* a);
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w,
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
@@ -91,6 +92,7 @@ extern "C" int chatts_linear_post_ss_parts(const ChattsLinearArgs* a) {
 extern "C" int chatts_linear_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* ch) {
   return a && a->w && a->m >= 2 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && !a->exact_f32 ? gemm_few_rows(a, ch) : 0;
 }
+extern "C" int chatts_linear_cols(const ChattsLinearArgs* a) { return a && a->w && a->m >= 2 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && !a->exact_f32 && gemm_takes_cols(a); }
 extern "C" size_t chatts_linear_workspace(int m, int n, int k) { return gemm_workspace(m, n, k); }
 extern "C" size_t chatts_linear_workspace_batch(int m, int n, int k, int batch) {
   const size_t one = gemm_workspace(m, n, k), all = gemm_workspace_batch(m, n, k, batch);

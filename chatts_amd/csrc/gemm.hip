@@ -1027,6 +1027,7 @@ static int gemm_takes_rows(const ChattsLinearArgs* a) {
   return sk > 1 && use_rows(a, sk) ? sk : 0;
 }
 // the same for a call of chatts_linear or chatts_linear_chain: a whole norm behind the product stays with the split, whose epilogue writes it (a launch of its own here)
+bool gemm_takes_cols(const ChattsLinearArgs* a) { return use_stream(a) && use_cols(a); }
 int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain) {
   return a->post_norm_w && !(chain && chain->post_ss) ? 0 : gemm_takes_rows(a);
 }
@@ -1121,7 +1122,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   p.row_ss = ch.row_ss; p.row_ss_parts = ch.row_ss_parts; p.row_eps = ch.row_eps;
   p.post_ss = nullptr;
   CHATTS_REQUIRE(!ch.row_ss || (stream && a->m <= 16 && batch == 1), CHATTS_E_SHAPE, "linear: row_ss is for 2 <= M <= 16 on planes (M=%d K=%d take another kernel)", a->m, a->k);
-  if (stream && use_cols(a)) {                  // wide ones: K whole, whatever sk says
+  if (stream && gemm_takes_cols(a)) {           // wide ones: K whole, whatever sk says
     p.c = a->c;
     CHATTS_REQUIRE(!ch.post_ss, CHATTS_E_SHAPE, "linear: post_ss is written where K is split over few rows (M=%d N=%d K=%d is not)", a->m, a->n, a->k);
     if (const int rc = launch_cols(p, a, s)) return rc;

@@ -278,6 +278,23 @@ static int cols_panels(int n, int epilogue) {
   const int cap = kColsMaxFN * (epi_is_glu(epilogue) ? 2 : 4);
   return (cols_most(n, epilogue) + cap - 1) / cap;
 }
+static int cols_fn(int n, int epilogue) {              // 4, 6 or 8 (fragments without rows cost next to nothing)
+  const int panels = cols_panels(n, epilogue), rows = (cols_most(n, epilogue) + panels - 1) / panels * 4, fn = (rows + 15) / 16 * (epi_is_glu(epilogue) ? 2 : 1);
+  return fn <= 4 ? 4 : (fn <= 6 ? 6 : 8);
+}
+// dynamic LDS: the rings, behind them (or, for a single panel, in their place) the waves' sums, and the columns' scales and biases.  rstd_s is static beside it
+constexpr int kColsLds = 159 * 1024;
+static int cols_place(const ChattsLinearArgs* a, bool m8, ColsGeom& g) {
+  const bool w8 = a->w8 != nullptr;
+  const int fn = cols_fn(a->n, a->epilogue), nw = cols_waves(w8, fn), most = cols_most(a->n, a->epilogue) * (epi_is_glu(a->epilogue) ? 8 : 4) * (int)sizeof(float);
+  int at = nw * cols_ring(w8, m8, fn) * 1024;
+  g.sums_at = 0;
+  if (g.panels > 1) { g.sums_at = at; at += nw * fn * 1024; }
+  g.scale_at = at;
+  if (w8) at += most;
+  g.bias_at = at;
+  return a->bias ? at + most : at;
+}
 
 bool use_cols(const ChattsLinearArgs* a) {
   const int opt = opt_get(OPT_GEMM_COLS, 1);           // 0: never, 2: wherever it can
@@ -290,6 +307,8 @@ bool use_cols(const ChattsLinearArgs* a) {
   if (!(a->m >= 2 && a->m <= 16 && a->batch <= 1 && a->n % 16 == 0 && (!glu || a->n % 32 == 0) && !a->planes_tiled && wbytes < (size_t)kColsFar &&
         (size_t)a->m * a->ld_planes * 2 < (size_t)kColsFar && cols_most(a->n, a->epilogue) * (glu ? 8 : 4) <= kColsTurns * 256))
     return false;
+  ColsGeom g{0, 0, cols_panels(a->n, a->epilogue), 0, 0, 0};
+  if (cols_place(a, false, g) > kColsLds) return false;      // (as for 16 rows: the number of rows decides nothing)
   if (a->ldc % 4 != 0 || !al(a->c, 16) || !al(a->resid, 16) || (a->c_hi && (a->ld_cplanes % 4 != 0 || !al(a->c_hi, 8) || !al(a->c_lo, 8)))) return false;
   return opt == 2 || cols_pay(a);
 }
@@ -298,20 +317,16 @@ template <bool W8, bool I8, bool GLU, int FN, bool M8>
 static int launch_cols_t(const GemmParams& p, const ChattsLinearArgs* a, hipStream_t s) {
   static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_cols_kernel<W8, I8, GLU, FN, M8>), hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
-    CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_cols: cannot reserve 159 KB of LDS: %s", hipGetErrorString(e));
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_cols_kernel<W8, I8, GLU, FN, M8>), hipFuncAttributeMaxDynamicSharedMemorySize, kColsLds);
+    CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_cols: cannot reserve %d KB of LDS: %s", kColsLds / 1024, hipGetErrorString(e));
     configured = true;
   }
   constexpr int NW = cols_waves(W8, FN);
-  constexpr size_t ring = (size_t)NW * cols_ring(W8, M8, FN) * 1024, sums = (size_t)NW * FN * 1024, columns = (size_t)kColsTurns * 256 * sizeof(float);
-  static_assert(sums <= ring && ring + (FN > 4 ? sums : 0) + 2 * columns <= 160 * 1024, "sums of a single panel take the rings' place, those of several lie behind them");
+  constexpr int ring = NW * cols_ring(W8, M8, FN) * 1024, sums = NW * FN * 1024;
+  static_assert(sums <= ring && ring + (FN > 4 ? sums : 0) <= kColsLds && kColsLds + 16 * sizeof(float) <= 160 * 1024, "the sums of a single panel take the rings' place, those of several (of five fragments and more) lie behind them");
   const int groups = a->n / (GLU ? 8 : 4), grid = cols_grid(a->n, a->epilogue);
   ColsGeom g{groups / grid, groups % grid, cols_panels(a->n, a->epilogue), 0, 0, 0};
-  size_t at = ring;
-  if (g.panels > 1) { g.sums_at = (int)at; at += sums; }
-  const size_t most = (size_t)cols_most(a->n, a->epilogue) * (GLU ? 8 : 4) * sizeof(float);
-  g.scale_at = (int)at; if (W8) at += most;
-  g.bias_at = (int)at; if (a->bias) at += most;
+  const int at = cols_place(a, M8, g);
   hipLaunchKernelGGL((gemm_cols_kernel<W8, I8, GLU, FN, M8>), dim3(grid), dim3(64 * NW), at, s, p, a->a_hi, a->a_lo, a->ld_planes, g);
   CHATTS_CHECK_LAUNCH("gemm_cols");
   return CHATTS_OK;
@@ -319,9 +334,9 @@ static int launch_cols_t(const GemmParams& p, const ChattsLinearArgs* a, hipStre
 template <bool W8, bool I8, bool M8>
 static int launch_cols_w(const GemmParams& p, const ChattsLinearArgs* a, hipStream_t s) {
   const bool glu = epi_is_glu(a->epilogue);
-  const int panels = cols_panels(a->n, a->epilogue), rows = (cols_most(a->n, a->epilogue) + panels - 1) / panels * 4, fn = (rows + 15) / 16 * (glu ? 2 : 1);      // (4, 6 or 8: fragments without rows cost next to nothing)
-  if (glu) return fn <= 4 ? launch_cols_t<W8, I8, true, 4, M8>(p, a, s) : (fn <= 6 ? launch_cols_t<W8, I8, true, 6, M8>(p, a, s) : launch_cols_t<W8, I8, true, 8, M8>(p, a, s));
-  return fn <= 4 ? launch_cols_t<W8, I8, false, 4, M8>(p, a, s) : (fn <= 6 ? launch_cols_t<W8, I8, false, 6, M8>(p, a, s) : launch_cols_t<W8, I8, false, 8, M8>(p, a, s));
+  const int fn = cols_fn(a->n, a->epilogue);
+  if (glu) return fn == 4 ? launch_cols_t<W8, I8, true, 4, M8>(p, a, s) : (fn == 6 ? launch_cols_t<W8, I8, true, 6, M8>(p, a, s) : launch_cols_t<W8, I8, true, 8, M8>(p, a, s));
+  return fn == 4 ? launch_cols_t<W8, I8, false, 4, M8>(p, a, s) : (fn == 6 ? launch_cols_t<W8, I8, false, 6, M8>(p, a, s) : launch_cols_t<W8, I8, false, 8, M8>(p, a, s));
 }
 int launch_cols(const GemmParams& p, const ChattsLinearArgs* a, hipStream_t s) {
   const bool m8 = a->m <= 8;

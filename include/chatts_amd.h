@@ -273,6 +273,8 @@ int chatts_linear_post_ss_parts(const ChattsLinearArgs* a);
 /* Host-only query: K ranges if this call (chain may be NULL) runs on the few-rows kernel, which holds whole columns and has no second launch; 0 = another kernel
  * runs.  Lets a test pin which shapes take which kernel. */
 int chatts_linear_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
+/* Host-only query: 1 if this call runs on the kernel of wide projections of few rows, which splits K over the waves of a workgroup and nowhere else. */
+int chatts_linear_cols(const ChattsLinearArgs* a);
 size_t chatts_linear_workspace(int m, int n, int k);
 size_t chatts_linear_workspace_batch(int m, int n, int k, int batch);
 /* Host-only query (no device work): how many waves share a row group of the M == 1 bf16 GEMV for this shape on the current device

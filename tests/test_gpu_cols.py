@@ -100,3 +100,15 @@ def test_strides_and_calls_that_stay_out(lib):
     odd = torch.full((m, n + 1), float("nan"), device=DEV)
     run(lib, args(m, n, k, hi, lo, w, None, None, "bf16", odd, bias=bias.data_ptr(), ldc=n + 1, epilogue=_lib.EPI_NONE), m, n, k)
     assert rel(odd[:, :n], want) < 1e-5
+
+
+@pytest.mark.parametrize("form,n", [("fp8", 229376), ("fp8", 229392), ("int8", 262144)])
+def test_the_widest(lib, form, n):
+    """scales and biases of as many columns a workgroup as its LDS holds; of one group more, and of the most: the kernel that runs there without a limit"""
+    m, k = 16, 256
+    x, w, bias, _, q, scale = problem(m, n, k, form, n)
+    hi, lo = planes(lib, x)
+    out = torch.full((m, n), float("nan"), device=DEV)
+    with _lib.options(GEMM_COLS=2):
+        run(lib, args(m, n, k, hi, lo, w, q, scale, form, out, bias=bias.data_ptr(), ldc=n, epilogue=_lib.EPI_NONE), m, n, k)
+    assert rel(out, x.double() @ w.double().T + bias.double()) < 1e-5
