@@ -558,8 +558,8 @@ class ChatTSForCausalLM(SlotModel):
         return n + head + T["final_norm"].numel() * 4
 
     def tiled_weight_bytes_local(self):
-        """Bytes of the prefill kernel's tiled weight copies on this rank (resident beside the tensors weight_bytes_local() counts)."""
-        return sum(t.numel() * t.element_size() for tl in self._tiled for t in tl.values())
+        """Bytes of the prefill kernel's tiled weight copies on this rank, the encoder's among them (resident beside the tensors weight_bytes_local() counts and the encoder's)."""
+        return sum(t.numel() * t.element_size() for tl in self._tiled for t in tl.values()) + self.ts_encoder.tiled_weight_bytes()
 
     def f16q_weight_bytes_local(self):
         """Bytes of the f16q weight copies (precision='f16q' only)"""

@@ -47,7 +47,8 @@ class TimeSeriesEmbedding:
         self._w8 = None
         self.position_embedding = None               # f32 [max_seq+1, emb]
         self.weights = [None] * self.num_layers      # bf16 [H, Kpad_l]
-        self._tiled = [None] * self.num_layers       # the same in the prefill kernel's blocks (layers after the first)
+        self._tiled = [None] * self.num_layers       # the same in the prefill kernel's blocks (layers after the first) ...
+        self._tiled_of = [None] * self.num_layers    # ... and what they were made from: (tensor, its version)
         self.biases = [None] * self.num_layers       # f32 [H]
 
     # ---- weights ---------------------------------------------------------------------------------
@@ -101,13 +102,28 @@ class TimeSeriesEmbedding:
                 self._tile(l)
 
     def _tile(self, l):
-        """a second copy of a hidden layer's weights in the order in which the prefill kernel's loader reads them (chatts_tile_bf16)"""
+        """A second copy of a hidden layer's weights in the order in which the prefill kernel's loader reads them (chatts_tile_bf16).  It follows the first one: forward() makes it again where
+        weights[l] is another tensor or has been written in place since (the tensor's version says so; writes past it, through .data or by a kernel on the pointer, are followed by
+        load_tensor).  A tensor without a version (made under inference_mode) gets none: its layer reads row-major."""
         w = self.weights[l]
         if l == 0 or not w.is_cuda or w.shape[1] % 64:
             return
+        self._tsw = None
+        if w.is_inference():
+            self._tiled[l] = self._tiled_of[l] = None
+            return
         lib = _lib.load()
-        self._tiled[l] = torch.empty(int(lib.chatts_tile_bf16_elems(*w.shape)), dtype=torch.bfloat16, device=w.device)
+        n = int(lib.chatts_tile_bf16_elems(*w.shape))
+        if self._tiled[l] is None or self._tiled[l].numel() != n:
+            self._tiled[l] = torch.empty(n, dtype=torch.bfloat16, device=w.device)
         _lib.check(lib.chatts_tile_bf16(_lib.ptr(w), *w.shape, w.shape[1], _lib.ptr(self._tiled[l]), _lib.stream_ptr()))
+        self._tiled_of[l] = (w, w._version)
+
+    def _follow_weights(self):
+        for l in range(1, self.num_layers):
+            w, of = self.weights[l], self._tiled_of[l]
+            if of is not None and (of[0] is not w or of[1] != w._version):
+                self._tile(l)
 
     def set_precision(self, precision):
         """"bf16x2" (default, parity grade: float32 activations as bf16 hi + lo planes) or "fp8" - the SPEED mode of
@@ -171,6 +187,10 @@ class TimeSeriesEmbedding:
         n = sum(w.numel() * 2 for w in self.weights) + sum(b.numel() * 4 for b in self.biases)
         return n
 
+    def tiled_weight_bytes(self):
+        """Bytes of the second copies (resident beside what weight_bytes() counts)."""
+        return sum(t.numel() * 2 for t in self._tiled if t is not None)
+
     # ---- forward -----------------------------------------------------------------------------------
     def get_patch_cnt(self, x):
         """chatts_vllm.py:198-207 on the device: [N, 2*Lmax, 1] -> (valid_len int32 [N], patch_cnt int64 [N])."""
@@ -230,6 +250,7 @@ class TimeSeriesEmbedding:
                               h1=torch.empty((P, H), dtype=torch.float32, device=dev),
                               ws=torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev), ws_bytes=ws_bytes)
             self._buf_key = key
+        self._follow_weights()
         if getattr(self, "_tsw", None) is None:
             if self.num_layers > 8:
                 raise ValueError("ts num_layers > 8 is not supported")

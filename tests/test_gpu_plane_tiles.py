@@ -131,3 +131,45 @@ def test_widths_that_other_kernels_take(hidden, inter, n):
     ids = prompt(n, n)
     on, off = both(lambda: m.generate_one(ids, None, None, max_new_tokens=1, return_logits=True)[1].clone())
     assert torch.isfinite(on).all() and torch.equal(on, off)
+
+
+@pytest.mark.parametrize("change", ["in place", "by a view", "another tensor", "without a version"])
+def test_the_encoder_follows_its_weights(change):
+    """weights changed after they were loaded act on calls of any size: the copy that calls of 129 rows and more read follows"""
+    from chatts_amd.ts_encoder import TimeSeriesEmbedding
+    ts = dict(preset("chatts-8b").ts, hidden_size=256)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    k = [ts["patch_size"] * (1 + ts["embedding_dim"])] + [256] * (ts["num_layers"] - 1)
+    draw = lambda: [(torch.randn((256, n), generator=g, device="cuda") * n ** -0.5).bfloat16() for n in k]
+    pos, bias, first, then = torch.randn((ts["max_sequence_length"] + 1, ts["embedding_dim"]), generator=g, device="cuda"), torch.randn(256, generator=g, device="cuda"), draw(), draw()
+
+    def encoder(weights):
+        e = TimeSeriesEmbedding(ts, device="cuda")
+        e.load_tensor("position_embedding.weight", pos)
+        for l, w in enumerate(weights):
+            e.load_tensor(f"mlp.{2 * l}.weight", w)
+            e.load_tensor(f"mlp.{2 * l}.bias", bias)
+        return e
+
+    def call(e, patches):
+        x = torch.zeros((1, patches * ts["patch_size"], 2), device="cuda")
+        x[0, :, 0], x[0, :, 1] = torch.sin(torch.arange(x.shape[1], device="cuda") * 0.1), 1.0
+        return e(x.view(1, -1, 1), valid_lengths=[x.shape[1]])[0].clone()
+
+    e, want = encoder(first), encoder([first[0]] + then[1:])
+    before = call(e, 300)
+    assert torch.equal(before, call(encoder(first), 300))
+    for l in range(1, len(k)):
+        if change == "in place":
+            with torch.no_grad():
+                e.weights[l].copy_(then[l])
+        elif change == "by a view":
+            e.weights[l].view(-1)[:] = then[l].view(-1)
+        elif change == "another tensor":
+            e.weights[l] = then[l].clone()
+        else:
+            with torch.inference_mode():
+                e.weights[l] = then[l].clone()
+    for patches in (300, 128, 129):
+        assert torch.equal(call(e, patches), call(want, patches))
+    assert not torch.equal(before, call(e, 300))
