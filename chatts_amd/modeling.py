@@ -95,6 +95,21 @@ def rope_tables(cfg, max_pos, device):
     return fr.cos().contiguous().to(device), fr.sin().contiguous().to(device)
 
 
+def batched_slots(max_batch, nq, nkv, n_splits):
+    """16-key slots per sequence of the batched decode attention, at most: its kernel uses fewer for a short context.  A slot is a wave per kv head (two for groups of more than six
+    heads), and a tile more in the longest of them is 1.2 us for all.  The number may not depend on how many sequences run, because a row's bits would; so it is what both ends bear: 1024
+    waves where every place is taken (more repeat the prologue and lengthen the merge), but for the few sequences of a server that is not full no fewer than 32 slots, up to 1792 waves
+    (seven a CU).  Both launches in a graph over rotating caches, us, 1024 waves and 12 slots / this rule, 40 heads on 8 kv heads:
+      8 places (16 / 28 slots), one taken, context 223 / 801 / 1800 / 4000   8.2 / 8.3   13.0 / 10.6   19.8 / 15.4   33.4 / 22.1;   all taken   10.3 / 11.1   17.4 / 18.0   26.7 / 27.3   46.7 / 49.6
+     16 places (12 / 14 slots)                                               9.9 / 8.3   14.9 / 13.4   23.7 / 21.7   41.8 / 36.8;               12.7 / 12.4   24.1 / 23.6   43.1 / 43.4   85.7 / 85.9
+      5 places (25 / 32 slots)                                               8.3 / 8.4   11.9 / 10.4   15.3 / 13.8   24.7 / 20.3;                9.7 / 10.5   14.8 / 14.7   19.9 / 20.2   32.9 / 34.2
+    5 heads on one kv head (a shard), 8 places (16 / 64)                     7.8 / 8.0   12.7 /  8.5   19.2 / 10.6   32.2 / 13.5;                8.1 /  8.6   13.2 /  9.7   19.6 / 11.7   33.4 / 15.8
+    Dearest: 1.1 us where every place holds about a hundred keys (8.6 / 9.8).  Groups of more than six keep 1024 waves' slots, eight at least: more cost 15 .. 30 % where all are taken."""
+    by_waves = 1024 // (nkv * max_batch)
+    least = 8 if nq // nkv > 6 else min(32, max(12, 224 // max_batch))
+    return max(1, min(n_splits, max(least, by_waves)))
+
+
 class ChatTSForCausalLM(SlotModel):
     packed_modules_mapping = packed_modules_mapping
 
@@ -820,16 +835,9 @@ class ChatTSForCausalLM(SlotModel):
         self._cur_slot = int(slot)
 
     def _n_splits_batched(self):
-        """16-key slots per sequence of the batched decode attention, at most: its kernel uses fewer for a short context.  A slot is a wave
-        per kv head; with the waves that the card holds at once already there, more of them only repeat the prologue and lengthen the merge
-        (both launches at context 800 / 1800, 40 heads: 16 sequences 12 / 16 / 24 slots 23.9 / 24.2 / 28.0 and 42.2 / 43.1 / 47.5 us,
-        8 sequences 18.1 / 18.0 / 18.1 and 28.1 / 27.1 / 26.9; 32 heads, 5 sequences 16 / 24 / 48 slots 13.9 / 14.0 / 15.8)."""
         import os
         forced = int(os.environ.get("CHATTS_BATCH_NSPLITS", "0") or 0)          # tuning only
-        if forced > 0:
-            return max(1, min(self.n_splits, forced))
-        least = 12 if self.plan.nq // self.plan.nkv <= 6 else 8                  # (larger groups: two waves a slot)
-        return max(1, min(self.n_splits, max(least, 128 // self.max_batch)))
+        return max(1, min(self.n_splits, forced)) if forced > 0 else batched_slots(self.max_batch, self.plan.nq, self.plan.nkv, self.n_splits)
 
     def _batched_step_eager(self):
         B = self.buf
