@@ -1021,19 +1021,20 @@ static int stream_ranges(const ChattsLinearArgs* a) {
   const int kps = k_per_split(a->k, pick_stream_sk(a->m, a->n, a->k, a->w8 != nullptr), stream_bk(a->w8 != nullptr));
   return (a->k + kps - 1) / kps;
 }
-static int gemm_takes_rows(const ChattsLinearArgs* a) {
+static int gemm_takes_rows(const ChattsLinearArgs* a, bool hands_on) {
   if (a->m > 8 || a->batch > 1 || opt_get(OPT_GEMM_SK, 0) != 0 || !use_stream(a) || use_cols(a)) return 0;
   const int sk = stream_ranges(a);
-  return sk > 1 && use_rows(a, sk) ? sk : 0;
+  return sk > 1 && use_rows(a, sk, hands_on) ? sk : 0;
 }
-// the same for a call of chatts_linear or chatts_linear_chain: a whole norm behind the product stays with the split, whose epilogue writes it (a launch of its own here)
 bool gemm_takes_cols(const ChattsLinearArgs* a) { return use_stream(a) && use_cols(a); }
+// the same for a call of chatts_linear or chatts_linear_chain: a whole norm behind the product stays with the split, whose epilogue writes it (a launch of its own here)
 int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain) {
-  return a->post_norm_w && !(chain && chain->post_ss) ? 0 : gemm_takes_rows(a);
+  const bool hands_on = chain && chain->post_ss;
+  return a->post_norm_w && !hands_on ? 0 : gemm_takes_rows(a, hands_on);
 }
 // parts of post_ss that launch_gemm would write for these arguments (post_norm_w and planes are there), 0: it would not
 int gemm_post_ss_parts(const ChattsLinearArgs* a) {
-  if (gemm_takes_rows(a)) return rows_grid(a->n, a->epilogue);
+  if (gemm_takes_rows(a, true)) return rows_grid(a->n, a->epilogue);
   if (use_cols(a) || a->m > 16 || a->batch > 1 || !use_stream(a) || a->ldc % 4 || ((uintptr_t)a->c % 16) || ((uintptr_t)a->resid % 16) || ((uintptr_t)a->bias % 16) ||
       (a->w8 && ((uintptr_t)a->w8_scale % 16)) || ((uintptr_t)a->workspace % 16)) return 0;
   const int sk = stream_ranges(a);

@@ -147,7 +147,7 @@ __device__ __forceinline__ void row_rstd_store(const GemmParams& p, int wave, in
 }
 
 // gemm_rows.hip: few rows, whole K per workgroup
-bool use_rows(const ChattsLinearArgs* a, int sk);      // sk: K ranges of gemm_stream_kernel
+bool use_rows(const ChattsLinearArgs* a, int sk, bool hands_on);      // sk: K ranges of gemm_stream_kernel; hands_on: post_ss is asked for
 int rows_grid(int n, int epilogue);      // workgroups = parts of post_ss
 int launch_rows(const GemmParams& p, const ChattsLinearArgs* a, int sk, hipStream_t s);
 // gemm_cols.hip: wide projections of few rows, K whole

@@ -253,23 +253,30 @@ static int rows_ahead(bool w8, int np, int waves) { return waves > 8 ? 3 : (w8 ?
 //     13 % less, 6144 x 10240 15 % more.  Its waves spend their time widening W: five to seven waves load the four SIMDs unevenly;
 //   * and 8-bit not at all with five to seven ranges where more than a third of the fragments is rows that are not there: fp8 5120 x 13824, 2 rows 15.6 / 17.2;
 //   * rows of W 32 KB apart: 4096 x 16384 bf16, 2 rows 33.3 / 37.6;
-//   * X up to 192 KB with more than eight ranges: 2048 x 6144, 2 / 4 rows 8.9 / 7.8, 8.9 / 8.3, but 8 rows 9.0 / 10.6; 2048 x 8192, 4 rows 10.3 / 10.5, 8 rows 10.4 / 13.0; 2048 x 3072,
-//     8 rows 7.4 / 7.3; 1024 x 4096, 2 / 8 rows 6.5 / 6.8, 6.8 / 8.4;
+//   * with more than eight ranges (bf16, up to 2048 columns: more than eight sums to add and eight rows of W or fewer a workgroup), against the epilogue that asks for sixteen slabs at once:
+//     72 KB up to twelve ranges (512 x 2304, 8 rows 6.2 / 5.8; 1024 x 3072, 6 / 8 rows 6.4 / 6.4, 6.4 / 7.1); with thirteen and fourteen 36 KB, 72 from 6 million weights on (1024 x 3584, 2 / 4
+//     rows 6.3 / 6.3, 6.5 / 6.8; 2048 x 3584, 5 / 7 rows 7.3 / 7.1, 7.5 / 7.8); with more 96 KB from 8 million on (2048 x 6144, 4 / 8 rows 8.9 / 8.5, 9.1 / 10.7; 2048 x 4096, 4 / 8 rows 7.7 / 7.7,
+//     7.9 / 8.7) and not below (1024 x 4096, 2 / 8 rows 6.3 / 6.8, 6.6 / 8.4).
+//     A norm is handed on from here only (that epilogue does not): 192 KB where one is, against a launch more;
 //   * always where the split has more workgroups than CUs: 7168 x 5120 20.6 / 15.7.
 // Beyond the line it would still win up to 14 % at K = 8192 with 5 to 8 rows and up to 11 % at 5120 or 6144 columns with K of 9216 to 12288; within it, it loses up to 3 %
 // at a few (5120 x 5120, 8 rows; fp8 4096 x 10240, 3 rows: 5 %).
-static bool rows_pay(const ChattsLinearArgs* a, int sk, int np) {
+static bool rows_pay(const ChattsLinearArgs* a, int sk, int np, bool hands_on) {
   const int groups = a->n / (epi_is_glu(a->epilogue) ? 8 : 4), grid = rows_grid(a->n, a->epilogue), wrows = (groups + grid - 1) / grid * (epi_is_glu(a->epilogue) ? 8 : 4);
   const bool w8 = a->w8 != nullptr, fp8 = w8 && a->w8_format != CHATTS_W8_INT8;
   if ((a->n + 127) / 128 * sk > device_cus()) return true;
-  if (sk > 8) return (size_t)a->m * a->k * 4 <= 192 * 1024;
+  if (sk > 8) {
+    const size_t weights = (size_t)a->n * a->k;
+    const int most = hands_on ? 192 : sk <= 12 ? 72 : (sk <= 14 ? (weights >= 6000000 ? 72 : 36) : (weights >= 8000000 ? 96 : 0));
+    return (size_t)a->m * a->k * 4 <= (size_t)most * 1024;
+  }
   if (sk > 4 && (w8 ? (size_t)a->ldw8 : 2 * (size_t)a->ldw) >= 32768) return false;
   if (sk > 4 && sk < 8 && w8 && 16 * ((np + 1) / 2) * 2 > 3 * wrows) return false;
   const int kb = sk <= 4 ? 256 : (!fp8 ? 168 : (sk == 8 ? 128 : 72));
   return (size_t)a->m * a->k * 4 <= (size_t)kb * 1024;
 }
 
-bool use_rows(const ChattsLinearArgs* a, int sk) {
+bool use_rows(const ChattsLinearArgs* a, int sk, bool hands_on) {
   // a workgroup stores its result while others still read A (the split's epilogue is a launch behind them)
   for (int i = 0; i < 3; ++i)
     if (meets_planes(a, result_range(a, i))) return false;
@@ -278,7 +285,7 @@ bool use_rows(const ChattsLinearArgs* a, int sk) {
   const size_t wbytes = w8 ? (size_t)a->n * a->ldw8 : (size_t)a->n * a->ldw * 2;
   const int np = rows_pieces(a->n, a->epilogue), waves = rows_waves(np, sk);
   const ptrdiff_t apart = reinterpret_cast<const char*>(a->a_lo) - reinterpret_cast<const char*>(a->a_hi);
-  return a->m >= 2 && a->m <= 8 && a->n % 16 == 0 && rows_pay(a, sk, np) && !a->planes_tiled && np <= (w8 ? 2 * kRowsMaxFN : 6) && waves <= (np == 1 && !w8 ? 16 : 8) && (!w8 || a->m <= 4 || waves == 8) &&
+  return a->m >= 2 && a->m <= 8 && a->n % 16 == 0 && rows_pay(a, sk, np, hands_on) && !a->planes_tiled && np <= (w8 ? 2 * kRowsMaxFN : 6) && waves <= (np == 1 && !w8 ? 16 : 8) && (!w8 || a->m <= 4 || waves == 8) &&
          rows_lds(np, rows_ahead(w8, np, waves), waves) <= 156 * 1024 && wbytes < kRowsFar && (size_t)(apart < 0 ? -apart : apart) + (size_t)a->m * a->ld_planes * 2 < kRowsNoToken && a->ldc % 4 == 0 &&
          al(a->c) && al(a->resid) && al(a->bias) && al(a->w8_scale) &&
          (!a->c_hi || (a->ld_cplanes % 4 == 0 && ((uintptr_t)a->c_hi % 8) == 0 && ((uintptr_t)a->c_lo % 8) == 0));

@@ -80,7 +80,18 @@ def test_results_leave_the_sums_that_are_read_alone(lib, over):
     ("bf16", 7, 8192, 10240, False),       # 28.8 / 31.9
     ("bf16", 2, 4096, 16384, False),       # rows 32 KB apart: 33.3 / 37.6
     ("bf16", 8, 7168, 5120, True),         # the split has more workgroups than CUs: 20.6 / 15.7
-    ("bf16", 8, 2048, 6144, True),         # sixteen ranges: 13.2 / 10.7
+    ("bf16", 8, 2048, 6144, False),        # sixteen ranges (the epilogue asks for all their slabs at once): 9.1 / 10.7
+    ("bf16", 4, 2048, 6144, True),         # 8.9 / 8.5
+    ("bf16", 8, 2048, 4096, False),        # 7.9 / 8.7
+    ("bf16", 4, 2048, 4096, True),         # 7.7 / 7.7
+    ("bf16", 2, 1024, 4096, False),        # under 8 million weights: 6.3 / 6.8
+    ("bf16", 5, 2048, 3584, True),         # fourteen ranges: 7.3 / 7.1
+    ("bf16", 6, 2048, 3584, False),        # 7.4 / 7.4
+    ("bf16", 2, 1024, 3584, True),         # 6.3 / 6.3
+    ("bf16", 4, 1024, 3584, False),        # 6.5 / 6.8
+    ("bf16", 6, 1024, 3072, True),         # twelve: 6.4 / 6.4
+    ("bf16", 8, 1024, 3072, False),        # 6.4 / 7.1
+    ("bf16", 8, 1024, 2304, True),         # nine: 6.3 / 6.0
     ("fp8", 8, 4096, 4096, True),          # 8.3 / 7.6
     ("fp8", 3, 4096, 12288, False),
     ("fp8", 4, 4096, 12288, False),        # 13.1 / 13.8
@@ -99,4 +110,12 @@ def test_the_faster_of_the_two(lib, form, m, n, k, takes):
         a.w8, a.w8_scale, a.ldw8, a.w8_format = 0x7e0000000000, 0x7d0000000000, k, _lib.W8_INT8 if form == "int8" else _lib.W8_FP8
     assert (few_rows(lib, a) > 1) == takes
     a.post_norm_w, a.post_hi, a.post_lo, a.ld_post = 0x60000000, OUT + (1 << 24), OUT + (2 << 24), n
-    assert int(lib.chatts_linear_post_ss_parts(C.byref(a))) == 256      # (either of the two hands a norm on)
+    assert int(lib.chatts_linear_post_ss_parts(C.byref(a))) == 256      # (either of the two hands a norm on; with more than eight ranges the few-rows kernel alone)
+
+
+@pytest.mark.parametrize("m,k,takes", [(8, 6144, True), (7, 8192, False)])
+def test_a_norm_handed_on_from_more_than_eight_ranges(lib, m, k, takes):
+    """up to 192 KB of X, and from this kernel only: what the host promises is what the launch does"""
+    a = args(m=m, n=2048, k=k, lda=k, ldw=k, ldc=2048, ld_planes=k, a_lo=A_HI + m * k * 2, post_norm_w=0x60000000, post_hi=OUT + (1 << 24), post_lo=OUT + (2 << 24), ld_post=2048)
+    assert (int(lib.chatts_linear_post_ss_parts(C.byref(a))) == 256) == takes
+    assert (few_rows(lib, a, _lib.NormChain(post_ss=0x70000000)) > 1) == takes and few_rows(lib, a) == 0
