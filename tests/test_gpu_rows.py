@@ -152,7 +152,7 @@ def test_a_result_in_the_place_of_its_own_input(lib, form, m, as_planes):
 
 # 8-row pieces of W a workgroup (1 .. 8; bf16 up to 6), K ranges of it; 8-bit with fewer ranges than fragments, so that a wave only helps to finish
 @pytest.mark.parametrize("form,m,n,k,pieces,ranges", [
-    ("bf16", 8, 1040, 4096, 1, 16), ("bf16", 2, 2048, 2048, 1, 8), ("bf16", 6, 4112, 4096, 3, 8), ("bf16", 8, 4096, 4096, 2, 8), ("bf16", 8, 5120, 4096, 3, 6), ("bf16", 5, 7184, 2048, 4, 4),
+    ("bf16", 4, 1968, 4096, 1, 16), ("bf16", 8, 1040, 2304, 1, 9), ("bf16", 2, 2048, 2048, 1, 8), ("bf16", 6, 4112, 4096, 3, 8), ("bf16", 8, 4096, 4096, 2, 8), ("bf16", 8, 5120, 4096, 3, 6), ("bf16", 5, 7184, 2048, 4, 4),
     ("bf16", 3, 9232, 1536, 5, 4), ("bf16", 8, 10240, 2048, 5, 3), ("bf16", 7, 11280, 1024, 6, 3), ("bf16", 4, 12288, 2048, 6, 3),
     *((form, m, n, k, p, r) for form in ("fp8", "int8") for m, n, k, p, r in [(3, 1040, 2048, 1, 4), (8, 4096, 4096, 2, 8), (4, 4112, 2048, 3, 4), (2, 8192, 2048, 4, 4), (4, 10240, 4096, 5, 3), (3, 9232, 1536, 5, 3),
                                                                          (4, 11280, 1024, 6, 2), (2, 13328, 2048, 7, 2), (4, 14336, 1280, 7, 2), (4, 16384, 1152, 8, 2), (3, 15376, 4096, 8, 2)])])
