@@ -58,7 +58,10 @@ __device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const R
 
 // SINGLE: the "bf16" speed mode - the lo plane is neither staged nor multiplied (activations rounded to bf16: NOT parity grade)
 // NF: column fragments of a compute wave - a panel is 64 NF rows of W
-template <bool SINGLE, bool GROUPED = false, int NF = 4>
+// TILES: planes of A or of the result whose whole blocks lie in tiles and whose last rows do not (a_tiled, c_tiled).  An instance of its own: the choice a piece cost row-major planes up
+// to 4 % (us with it / without, W in tiles: 300 rows 4096 x 4096 35.5 / 34.2, 12288 x 4096 gated 70.3 / 69.4; 700 rows 6144 x 4096 77.3 / 76.0; 129 rows 5120 x 5120 33.4 / 32.6; 2048 rows
+// 12288 x 4096 gated 313.6 / 312.3).
+template <bool SINGLE, bool GROUPED = false, int NF = 4, bool TILES = false>
 __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, const uint16_t* __restrict__ a_hi,
                                                                  const uint16_t* __restrict__ a_lo, int ldp, RingGeom g, RingGroup gr) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -70,7 +73,6 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
   // at the same K offset - each K-slice of a panel is fetched into that L2 once for all of them
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   if constexpr (GROUPED) {
-    p.c_tiled = 0;
     g.T = *gr.count;
     g.units = g.T * g.P;
   }
@@ -94,12 +96,12 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     const int prow = lane >> 2, gchunk = (lane & 3) ^ ((lane >> 5) << 1);
     // tiled operands (chatts_tile_bf16): piece (16-row block b, half-stage t) is the 1 KB at ((b * K / 32) + t) * 1 KB, already in LDS
     // order - whole cache lines per request instead of 16 half lines (profiles/r6_feed_probe.txt)
-    const bool wtiled = p.wt != nullptr;
-    const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64;
+    const bool wtiled = p.wt != nullptr, alltiled = p.planes_tiled != 0;
+    const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64, astep = alltiled ? 1024 : 64;
     // three fragments do not hold whole (gate, up) pairs of 16 columns: there a gated product's W block is 8 gates and their 8 up rows
     const bool mixed = NF == 3 && p.direct && epi_is_glu(p.epilogue);
     const char* src[NF + 5];
-    int dst[NF + 5], ashift[5];      // (a shift a piece: a product there cost plain row-major planes 1 %)
+    int dst[NF + 5], ashift[TILES ? 5 : 1];
     int np = 0, nh_cur = 0, hh = 0, ucur = u0;
     auto setup = [&](int u) {
       int matrix = 0, places = 0;
@@ -131,8 +133,8 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
         const int q = L + 4 * h;
         if (q < na) {
           const int plane = q >= r.f, frag = plane ? q - r.f : q;
-          const bool atiled = !GROUPED && (p.planes_tiled || r.m0 + frag * 16 < p.a_tiled);      // (a_tiled: a last block that is not whole stays row-major; lists never lie in tiles)
-          ashift[h] = atiled ? 10 : 6;
+          const bool atiled = TILES ? alltiled || r.m0 + frag * 16 < p.a_tiled : alltiled;
+          if constexpr (TILES) ashift[h] = atiled ? 10 : 6;
           if (atiled) {
             src[NF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + ((size_t)((r.m0 >> 4) + frag) * nkt + (r.kbeg >> 5)) * 512) + lane * 16;
           } else {
@@ -154,10 +156,10 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     auto issue = [&]() -> int {                                // request the next half-stage (if any); -> its piece count
       if (ucur >= uend) return 0;
       char* base = smem + (gi & (kRingSlots - 1)) * kRingHalf;
-      const size_t koffw = (size_t)hh * wstep;
+      const size_t koffw = (size_t)hh * wstep, koffa = (size_t)hh * astep;
 #pragma unroll
       for (int h = 0; h < NF + 5; ++h)
-        if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < NF ? koffw : (size_t)((unsigned)hh << ashift[h < NF ? 0 : h - NF]))), (lptr_t)(base + dst[h]), 16, 0, 0);
+        if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < NF ? koffw : (TILES ? (size_t)((unsigned)hh << ashift[h < NF ? 0 : h - NF]) : koffa))), (lptr_t)(base + dst[h]), 16, 0, 0);
       const int n = np;
       ++gi;
       if (++hh == nh_cur) {
@@ -267,28 +269,28 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 
     const int tok0 = r.m0 + rowblk * 16, fb0 = r.panel * BN + wn * 16 * NF;
     const bool planes = p.c_hi != nullptr;
-    if (!p.direct) ring_store<kStRaw, false>(p, acc, fml, tok0, fb0, lane, r.split);
+    if (!p.direct) ring_store<kStRaw, false, TILES>(p, acc, fml, tok0, fb0, lane, r.split);
     else if (p.epilogue == CHATTS_EPI_SWIGLU) {
-      if (planes) ring_store<kStSwiglu, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStSwiglu, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStSwiglu, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStSwiglu, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else if (p.epilogue == CHATTS_EPI_RESID) {
-      if (planes) ring_store<kStResid, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStResid, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStResid, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStResid, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else if (p.epilogue == CHATTS_EPI_GELU) {
-      if (planes) ring_store<kStGelu, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStGelu, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStGelu, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStGelu, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else if (p.epilogue == CHATTS_EPI_CLAMPGLU) {
-      if (planes) ring_store<kStClampGlu, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStClampGlu, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStClampGlu, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStClampGlu, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else if (p.epilogue == CHATTS_EPI_GEGLU) {
-      if (planes) ring_store<kStGeglu, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStGeglu, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStGeglu, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStGeglu, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else if (p.epilogue == CHATTS_EPI_RELU2) {
-      if (planes) ring_store<kStRelu2, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStRelu2, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStRelu2, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStRelu2, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     } else {
-      if (planes) ring_store<kStNone, true>(p, acc, fml, tok0, fb0, lane, 0);
-      else ring_store<kStNone, false>(p, acc, fml, tok0, fb0, lane, 0);
+      if (planes) ring_store<kStNone, true, TILES>(p, acc, fml, tok0, fb0, lane, 0);
+      else ring_store<kStNone, false, TILES>(p, acc, fml, tok0, fb0, lane, 0);
     }
   }
 }
@@ -350,17 +352,21 @@ void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int forc
   g.wpx = wpx;
 }
 
-template <bool SINGLE, int NF>
-static int launch_ring_t(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, hipStream_t s) {
+template <bool SINGLE, int NF, bool TILES>
+static int launch_ring_n(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, hipStream_t s) {
   static bool configured = false;     // > 64 KB of dynamic LDS must be opted into once
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<SINGLE, false, NF>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<SINGLE, false, NF, TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                              kRingLds);
     CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "gemm_ring: cannot reserve %d bytes of LDS: %s", kRingLds, hipGetErrorString(e));
     configured = true;
   }
-  hipLaunchKernelGGL((gemm_ring_kernel<SINGLE, false, NF>), dim3(8 * g.wpx), dim3(kRingThreads), kRingLds, s, p, a_hi, a_lo, ldp, g, RingGroup{});
+  hipLaunchKernelGGL((gemm_ring_kernel<SINGLE, false, NF, TILES>), dim3(8 * g.wpx), dim3(kRingThreads), kRingLds, s, p, a_hi, a_lo, ldp, g, RingGroup{});
   return CHATTS_OK;
+}
+template <bool SINGLE, int NF>
+static int launch_ring_t(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, hipStream_t s) {
+  return p.a_tiled || p.c_tiled ? launch_ring_n<SINGLE, NF, true>(p, a_hi, a_lo, ldp, g, s) : launch_ring_n<SINGLE, NF, false>(p, a_hi, a_lo, ldp, g, s);
 }
 int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGroup& gr, int most_tiles, hipStream_t s) {
   static_assert(kRingTile == kRingMaxF * 16, "a tile's places");

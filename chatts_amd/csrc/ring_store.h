@@ -40,7 +40,8 @@ __device__ __forceinline__ RingUnit ring_unit(const GemmParams& p, const RingGeo
 // The epilogue of one wave: acc[i][j] = D[feature = fb .. fb + 3][token] of fragment pair (i, j), fb = fb0 + j * 16 + (lane >> 4) * 4,
 // token = m0 + rowbase + i * 16 + (lane & 15).  MODE / PLANES are compile-time: no branches, all loads of a row block in flight at once.
 // Three column fragments and a gated epilogue: a fragment is 8 gates (lanes 0 - 31) and their 8 up rows (lanes 32 - 63), fragment j the units fb0 / 2 + 8 j ..
-template <int MODE, bool PLANES, int NF>
+// TILES: planes of the result as plane_at has them (c_tiled); without, the loads and stores of row-major callers bear none of it.
+template <int MODE, bool PLANES, bool TILES = false, int NF>
 __device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&acc)[5][NF], int fml, int tok0, int fb0, int lane, int split) {
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
   const int tl = lane & 15, fq = (lane >> 4) * 4;
@@ -54,7 +55,7 @@ __device__ __forceinline__ void ring_store(const GemmParams& p, const f32x4 (&ac
         hv[r] = h;
         lv[r] = (__bf16)(v[r] - (float)h);
       }
-      const size_t at = plane_at(tok, col, p.ldcp, p.c_tiled);
+      const size_t at = TILES ? plane_at(tok, col, p.ldcp, p.c_tiled) : (size_t)tok * p.ldcp + col;
       *reinterpret_cast<bf16x4_t*>(p.c_hi + at) = hv;
       *reinterpret_cast<bf16x4_t*>(p.c_lo + at) = lv;
     } else {
