@@ -305,7 +305,8 @@ SIGNATURES = {
     "chatts_linear_chain": (c_int, [c_void_p, c_void_p, c_void_p]),
     "chatts_linear_post_ss_parts": (c_int, [c_void_p]),
     "chatts_linear_few_rows": (c_int, [c_void_p, c_void_p]),
-    "chatts_linear_cols": (c_int, [c_void_p]),
+    "chatts_linear_cols": (c_int, [C.POINTER(LinearArgs)]),
+    "chatts_gemv_ring": (c_int, [C.POINTER(LinearArgs)]),
     "chatts_gemv_ksplit": (c_int, [c_int, c_int, c_int, c_int]),
     "chatts_linear": (c_int, [C.POINTER(LinearArgs), c_void_p]),
     "chatts_quantize_rows_fp8": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_void_p]),

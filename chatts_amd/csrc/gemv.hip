@@ -607,6 +607,17 @@ int gemv_pick_ksplit(int tasks, int nchunks, bool norm, double w_bytes, int cus)
 int launch_gemv4(const ChattsLinearArgs* a, hipStream_t s, bool* done);      // gemv4.hip
 bool gemv_ring_takes(const ChattsLinearArgs* a);                             // gemv_ring.hip
 int launch_gemv_ring(const GemvParams& p, const ChattsLinearArgs* a, hipStream_t s);
+// waves that share a row group of a bf16 call (1: whole rows)
+static int gemv_ksplit(const ChattsLinearArgs* a) {
+  const int nchunks = (a->k + 511) / 512;
+  if (a->tp_reduce || a->w8 || a->w4 || opt_get(OPT_GEMV_ROWS, 2) == 4 || opt_get(OPT_GEMV_UNR, 2) == 4 || nchunks < 4) return 1;
+  const int batch = a->batch > 1 ? a->batch : 1, units = epi_is_glu(a->epilogue) ? a->n / 2 : a->n, upt = epi_is_glu(a->epilogue) ? 1 : 2;
+  const int ks = opt_get(OPT_GEMV_KS, gemv_pick_ksplit((units + upt - 1) / upt * batch, nchunks, a->norm_w != nullptr, (double)a->n * a->k * 2.0 * batch, device_cus()));
+  return ks > 16 ? 16 : (ks > 1 ? ks : 1);
+}
+bool gemv_on_ring(const ChattsLinearArgs* a) {
+  return gemv_ring_takes(a) && (a->w8 || (opt_get(OPT_GEMV_ROWS, 2) != 4 && opt_get(OPT_GEMV_UNR, 2) != 4 && gemv_ksplit(a) == 1));
+}
 int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
   GemvParams p;
   p.tp = TpParams{}; p.spread = 0;
@@ -688,7 +699,7 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
   }
   p.glu_limit = a->glu_limit; p.glu_alpha = a->glu_alpha;
   p.x_stride = a->a_stride; p.w_stride = a->w_stride; p.out_stride = a->c_stride;
-  if (a->w8 && gemv_ring_takes(a)) return launch_gemv_ring(p, a, s);
+  if (gemv_on_ring(a)) return launch_gemv_ring(p, a, s);
   if (a->w8 != nullptr) {                       // 8-bit weights: rows x chunks of 1024 elements in flight per lane (GEMV8_ROWS x GEMV8_UNR)
     const int nchunks8 = (a->k + 1023) / 1024;
     const size_t lds8 = (size_t)nchunks8 * 1024 * 4 + 64 * 4;
@@ -728,10 +739,8 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
   // row is long enough to split.  Every TP = 1 shape of the supported models has >= 10 waves per CU and keeps the whole-K kernel.
   p.ks = 1;
   const int batch = a->batch > 1 ? a->batch : 1;
-  if (!a->tp_reduce && rows == 2 && unr == 2 && nchunks >= 4) {
-    int ks = gemv_pick_ksplit(p.tasks * batch, nchunks, norm, (double)a->n * a->k * 2.0 * batch, cus);
-    ks = opt_get(OPT_GEMV_KS, ks);
-    if (ks > 16) ks = 16;
+  {
+    const int ks = gemv_ksplit(a);
     if (ks > 1) {
       int groups = 16 / ks;
       if (groups < 1) groups = 1;
@@ -771,7 +780,6 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
       return CHATTS_OK;
     }
   }
-  if (rows == 2 && unr == 2 && gemv_ring_takes(a)) return launch_gemv_ring(p, a, s);
   p.spread = gemv_spread((size_t)a->ldw * 2, nchunks);
   if (a->tp_reduce) p.tp = tp_issue(a->tp_reduce, false);
   if (rows == 4 && unr == 2) launch_ldsx<4, 2>(p, epilogue, norm, dim3(blocks, batch), threads, lds_launch, s);
@@ -783,6 +791,8 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s) {
 }
 
 }  // namespace chatts
+
+extern "C" int chatts_gemv_ring(const ChattsLinearArgs* a) { return a && a->m == 1 && a->n > 0 && a->k > 0 && a->epilogue != CHATTS_EPI_GELU && chatts::gemv_on_ring(a); }
 
 // host-only query (no device touched): the K-split factor the bf16 decode GEMV picks for a shape on this device - see gemv_pick_ksplit
 extern "C" int chatts_gemv_ksplit(int n, int k, int epilogue, int has_norm) {

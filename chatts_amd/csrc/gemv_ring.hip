@@ -5,7 +5,7 @@
 // ONE sequence of units, a 1 KB chunk of each of the task's rows, that runs through a ring of D units in registers: the loads of the next D - 1 units are always under way,
 // over the end of a task, too, and the first ones since before x was staged.  Requests past a row's end or the last task lie outside the row's buffer: they return zeros.
 // Lane j keeps the j-th task's sums, and the epilogues of up to 64 tasks run side by side behind them: a residual asked for between two units would wait for the whole ring.
-// Each row is summed in gemv_ldsx_kernel's order: the same bits.
+// Each row is summed in gemv_ldsx_kernel's order: the same bits, but where a norm is fused: its sum of squares runs over the workgroup's threads, and the two have other numbers of waves.
 #include "common.h"
 #include "gemv_common.h"
 
@@ -194,7 +194,9 @@ static size_t ring_lds(const ChattsLinearArgs* a) {
 }
 
 // Rows of more than 2048 k: shorter ones are one or two of gemv_ldsx_kernel's batches, and the ring's code costs more than it hides (us there / here: 8192 x 2048 bf16 7.6 / 8.1, fp8
-// 5.4 / 6.2; 4096 x 1024 fp8 3.4 / 3.9).  Six tasks a CU: with fewer the K split has more under way.  8-bit weights from 32 MB on (6144 x 4096 int8 7.5 / 7.9, 5120 x 5120 7.7 / 8.0).
+// 5.4 / 6.2; 4096 x 1024 fp8 3.4 / 3.9).  Six tasks a CU: with fewer the K split has more under way.  8-bit weights of more than 32 MB (6144 x 4096 int8 7.5 / 7.9, 5120 x 5120 7.7 / 8.0,
+// 8192 x 4096 8.7 / 8.9), and with 9 to 12 tasks a CU, whose waves suit neither one walk nor two, from 44 MB on (fp8 5120 x 8192 10.1 / 10.4, 6144 x 7168 10.8 /
+// 11.2, 5120 x 10240 11.6 / 11.4).
 // Vocabularies in bf16 (hundreds of tasks a CU) keep two workgroups a CU of that kernel: 152064 x 5120 232 / 235, 151936 x 4096 192 / 192.
 // The exchange over ranks stays there, too: its pushes stand between the loads.
 bool gemv_ring_takes(const ChattsLinearArgs* a) {
@@ -202,22 +204,37 @@ bool gemv_ring_takes(const ChattsLinearArgs* a) {
   if (opt == 0 || a->w4 || a->tp_reduce || ring_lds(a) > 64 * 1024 || a->n % 2 != 0) return false;
   const int tasks = a->n / 2, batch = a->batch > 1 ? a->batch : 1;
   const size_t per_cu = (size_t)tasks * batch / device_cus();
-  return opt == 2 || (a->k > 2048 && per_cu >= 6 && (a->w8 ? (size_t)a->n * a->k >= (size_t)32 << 20 : per_cu < 128));
+  const size_t bytes = (size_t)a->n * a->k, each = (tasks + device_cus() - 1) / device_cus();
+  return opt == 2 || (a->k > 2048 && per_cu >= 6 && (a->w8 ? bytes > (size_t)32 << 20 && (each < 9 || each > 12 || bytes >= (size_t)44 << 20) : per_cu < 128));
 }
 
-// One workgroup per CU, whose waves keep 10 KB each under way: eight of them, or as many as the CU has tasks where that is 5 .. 10 (o and down projections: one task a wave; with eight,
-// two of them would walk K twice: 5120 x 5120 12.6 / 11.1 us, 5120 x 13824 27.8 / 24.0).  More only stretch the prologue (7168 x 5120 12 / 8 waves 17.1 / 14.2, fp8 10.4 / 9.0), but
-// for hundreds of tasks a CU (152064 x 5120 fp8 8 / 12 waves 122.4 / 117.7) and 8-bit rows that are one task for 9 or 10 of them (5120 x 13824 fp8 10 / 12 14.75 / 14.2).  Four rows a task instead of two: the same within 2 %.
+// Waves of a workgroup, one of which a CU has; each keeps 10 KB under way.  Eight of them, or as many as let all walk the same number of tasks where a CU has few: a wave that walks one more
+// holds the launch up.  More only stretch the prologue, which long rows bear (7168 x 5120, 14 tasks a CU, 12 / 8 waves 17.1 / 14.2 us, fp8 10.4 / 9.0).  As a part of gemv_ldsx_kernel's time,
+// 8 waves / the choice:
+//   5 .. 8 tasks: one a wave.
+//   9 or 10: 12 for K from 8192 on (4608 x 12288 1.22 / 0.96, fp8 5120 x 12288 1.13 / 0.96, 5120 x 8192 1.13 / 0.96), 5 with two each below 4608 (4608 x 4096 1.12 / 0.98, 5120 x 4096 1.09 /
+//     1.00), one a wave between (5120 x 5120 1.12 / 1.00);
+//   11 or 12: 12 from 5120 on (6144 x 5120 1.00 / 0.95, x 12288 1.04 / 0.96, gated 1.05 / 0.96, fp8 1.01 / 0.93), 6 with two each below (6144 x 4096 0.97 / 0.95);
+//   17 .. 20: 10 with two each in bf16, and in 8 bits from 8192 on (9216 x 4096 1.01 / 0.94, x 12288 1.08 / 0.99, fp8 1.02 / 0.96; but fp8 10240 x 4096 0.90 / 0.94);
+//   hundreds (vocabularies in 8 bits): 12 (152064 x 5120 fp8 122.4 / 117.7 us).
+// Over 870 shapes of 3072 to 27648 rows and K 2560 to 12288 in the three formats, the calls that come here take 0.935 of gemv_ldsx_kernel's time in the mean.  What still loses, 1 .. 3 %: 14336
+// and 18432 rows with K of 8192 and more, 27648 x 12288 gated in bf16.  Four rows a task instead of two: the same within 2 %.
+static int ring_waves(const ChattsLinearArgs* a) {
+  const int cus = device_cus(), tasks = a->n / 2, each = (tasks + cus - 1) / cus;
+  if (tasks / cus >= 128) return 12;
+  if (each >= 5 && each <= 8) return tasks % cus == 0 ? each : 8;
+  if (each == 9 || each == 10) return a->k >= 8192 ? 12 : (a->k < 4608 ? 5 : each);
+  if (each == 11 || each == 12) return a->k >= 5120 ? 12 : 6;
+  if (each >= 17 && each <= 20 && (!a->w8 || a->k >= 8192)) return 10;
+  return 8;
+}
 // Measured in a graph over rotating weights, gemv_ldsx_kernel / here, us: bf16 24576 x 4096 gated 34.3 / 33.4, 4096 x 12288 19.8 / 18.5, 6144 x 4096 10.8 / 10.5, 4096 x 4096 8.2 / 7.9,
 // 7168 x 5120 14.9 / 14.3, 5120 x 13824 25.4 / 24.2, 12288 x 3072 14.7 / 13.9; fp8 24576 x 4096 gated 21.1 / 18.6, 27648 x 5120 gated 26.7 / 24.9, 4096 x 12288 12.2 / 11.0, 7168 x 5120
 // 9.7 / 9.0, 152064 x 5120 127 / 122; int8 24576 x 4096 gated 22.0 / 19.0, 4096 x 12288 12.5 / 11.2.
 int launch_gemv_ring(const GemvParams& from, const ChattsLinearArgs* a, hipStream_t s) {
   GemvParams p = from;
-  const int cus = device_cus(), per_cu = a->n / 2 / cus;
-  int nw = 8;
-  if (per_cu >= 128) nw = 12;
-  else if (a->n / 2 % cus == 0 && per_cu >= 5 && per_cu <= 10) nw = a->w8 && per_cu > 8 ? 12 : per_cu;
-  nw = opt_get(OPT_GEMV_NW, nw);
+  const int cus = device_cus();
+  int nw = opt_get(OPT_GEMV_NW, ring_waves(a));
   if (nw < 1 || nw > 16) nw = 8;
   p.tasks = a->n / 2;                                     // two rows, gated: a gate and its up row
   p.spread = gemv_spread(a->w8 ? (size_t)a->ldw8 : (size_t)a->ldw * 2, (a->k + (a->w8 ? 1023 : 511)) / (a->w8 ? 1024 : 512));

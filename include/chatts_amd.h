@@ -281,6 +281,8 @@ size_t chatts_linear_workspace_batch(int m, int n, int k, int batch);
  * (1 = the whole-K kernel every TP = 1 projection of the supported models runs; > 1 = the K-split form of shard-sized column-parallel
  * projections, which sums a row in another order).  Lets a host-side test pin which shapes take which kernel. */
 int chatts_gemv_ksplit(int n, int k, int epilogue, int has_norm);
+/* Host-only query: 1 if this M == 1 call runs on the kernel whose waves stream through a ring of loads. */
+int chatts_gemv_ring(const ChattsLinearArgs* a);
 /* hi = bf16(x) (RNE), lo = bf16(x - hi): the operand split of the bf16x2 GEMM, done once per activation matrix. */
 int chatts_split_bf16x2(const float* x, int m, int k, int ldx, chatts_bf16* hi, chatts_bf16* lo, int ld_planes,
                         chatts_stream_t stream);
@@ -290,11 +292,13 @@ int chatts_split_bf16x2(const float* x, int m, int k, int ldx, chatts_bf16* hi, 
  * block of a ragged row count) repeat the last row.  dst holds chatts_tile_bf16_elems(rows, k) = ceil(rows / 16) * 16 * k elements. */
 size_t chatts_tile_bf16_elems(int rows, int k);
 int chatts_tile_bf16(const chatts_bf16* src, int rows, int k, int ld, chatts_bf16* dst, chatts_stream_t stream);
-/* Dispatch: M == 1       -> weight-streaming GEMV (gemv_ldsx_kernel: exact f32 VALU products, x staged in LDS, HBM-bound);
- *           2 <= M <= 16 -> with pre-split planes: gemm_stream_kernel (W and the A planes staged by whole-line LDS-DMA through a
- *                           4-deep ring, split-K over workgroups); with float32 A: the register-staged gemm_bf16x2_kernel;
- *           larger M     -> gemm_dma_kernel (LDS-DMA, loader + compute waves) on pre-split planes for M >= 96 and K % 64 == 0,
- *                           otherwise gemm_bf16x2_kernel (register-staged LDS tiles);
+/* Dispatch: M == 1       -> weight-streaming GEMV (exact f32 VALU products, x staged in LDS, HBM-bound): gemv_ring_kernel for long rows
+ *                           (chatts_gemv_ring), gemv4_kernel for 4-bit codes, else gemv_ldsx_kernel and its K-split form;
+ *           2 <= M <= 16 -> with pre-split planes: gemm_cols_kernel (chatts_linear_cols), gemm_rows_kernel (chatts_linear_few_rows) or
+ *                           gemm_stream_kernel (W and the A planes staged by whole-line LDS-DMA through a ring, split-K over
+ *                           workgroups); with float32 A: the register-staged gemm_bf16x2_kernel;
+ *           larger M     -> on pre-split planes with K % 64 == 0 gemm_stream_kernel in several row blocks up to 128 rows, gemm_ring_kernel
+ *                           (LDS-DMA, loader + compute waves) for M >= 96 or without a float32 A; otherwise gemm_bf16x2_kernel;
  *           all MFMA paths: v_mfma_f32_16x16x32_bf16 with the bf16x2 split of A. */
 int chatts_linear(const ChattsLinearArgs* args, chatts_stream_t stream);
 

@@ -79,3 +79,19 @@ def test_several_products_in_a_launch():
         torch.cuda.synchronize()
         outs.append(out)
     assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
+# waves that the rule picks: 5, 9, 12 (two tasks some, one the others), 6, 12, 10, 8 with a ragged last walk
+@pytest.mark.parametrize("fmt,n,k", [("bf16", 5120, 4096), ("bf16", 4608, 5120), ("bf16", 4608, 8192), ("fp8", 5120, 10240), ("bf16", 6000, 4096), ("int8", 6144, 8192), ("bf16", 9216, 2560), ("fp8", 10240, 8192),
+                                     ("int8", 11264, 4096)])
+def test_the_shipped_geometry(fmt, n, k):
+    """the waves of the launch as it is chosen, a norm among them, against float64"""
+    lib = _lib.load()
+    x, norm, ops = operands(n, k, k, fmt, n + k)
+    x *= 3.0
+    w = ops["w"].double() if fmt == "bf16" else (ops["w8"].view(torch.float8_e4m3fn if fmt == "fp8" else torch.int8).double() * ops["w8_scale"].double()[:, None])
+    bias = torch.randn(n, device=DEV)
+    for nm in (None, norm):
+        z = w @ (x.double() if nm is None else x.double() * torch.rsqrt((x.double() ** 2).mean() + 1e-6) * norm.double()) + bias.double()
+        out = call(lib, x, nm, ops, n, k, _lib.EPI_NONE, fmt, bias, None)
+        assert float((out.double() - z).norm() / z.norm()) < 1e-6      # (products exact, sums of at most 10240 terms and the norm in 32 bits)
