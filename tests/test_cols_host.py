@@ -28,3 +28,35 @@ def takes(lib, form, m, n, k, epi=_lib.EPI_NONE, **kw):
 @pytest.mark.parametrize("m", [2, 8, 9, 16])
 def test_what_a_workgroup_holds(lib, form, n, k, bias, want, m):
     assert takes(lib, form, m, n, k, bias=0x30000000 if bias else None) == want
+
+
+# both sides of the line, which the matrix draws alone: us of the other two / of this one beside the shape
+@pytest.mark.parametrize("form,n,k,epi,want", [
+    ("bf16", 24576, 4096, _lib.EPI_SWIGLU, 1),            # 5 rows 39 / 32.5, 16 rows 40.7 / 33.0
+    ("bf16", 18432, 4096, _lib.EPI_NONE, 1),              # 44 / 26
+    ("bf16", 12288, 4096, _lib.EPI_NONE, 1),
+    ("bf16", 12288, 2048, _lib.EPI_NONE, 0),              # 2 rows 10.9 / 11.5
+    ("bf16", 12304, 2048, _lib.EPI_NONE, 1),
+    ("bf16", 32000, 2048, _lib.EPI_NONE, 1),              # 31 / 23.7
+    ("bf16", 12272, 8192, _lib.EPI_NONE, 0),              # 10240 columns 0.83 .. 1.2 times as fast, 8192 0.6 .. 1.0
+    ("fp8", 24576, 4096, _lib.EPI_SWIGLU, 1),             # 25.8 / 20.9
+    ("fp8", 16384, 4096, _lib.EPI_NONE, 0),               # short K at the lower end: the widest instances of the other two
+    ("fp8", 16400, 4096, _lib.EPI_NONE, 1),
+    ("fp8", 16384, 8192, _lib.EPI_NONE, 1),               # 37 / 28
+    ("fp8", 12288, 4224, _lib.EPI_NONE, 1),
+    ("int8", 12288, 4096, _lib.EPI_NONE, 0),
+    ("int8", 152064, 5120, _lib.EPI_NONE, 1),
+])
+def test_the_faster_side(lib, form, n, k, epi, want):
+    for m in (2, 5, 8, 9, 16):
+        assert takes(lib, form, m, n, k, epi) == want, m
+
+
+@pytest.mark.parametrize("why,kw", [("17 rows", dict(m=17)), ("a result that does not start on 16 bytes", dict(c=OUT + 4)), ("a result at an odd stride", dict(ldc=24577)), ("a result over A", dict(c=A + 64)),
+                                    ("planes of a result over A", dict(c=None, c_hi=A, c_lo=OUT, ld_cplanes=24576)), ("planes at an odd stride", dict(c=None, c_hi=OUT, c_lo=OUT + (1 << 24), ld_cplanes=24578)),
+                                    ("a K that ends inside a line", dict(k=4096 + 32, ld_planes=4096 + 32, ldw=4096 + 32)), ("no planes", dict(a_hi=None, a_lo=None, a=A)), ("tiles", dict(planes_tiled=1)),
+                                    ("several products", dict(batch=2))])
+def test_calls_that_stay_out(lib, why, kw):
+    assert takes(lib, "bf16", 5, 24576, 4096) == 1
+    kw = dict(kw)
+    assert takes(lib, "bf16", kw.pop("m", 5), 24576, kw.pop("k", 4096), **kw) == 0
