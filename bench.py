@@ -125,9 +125,11 @@ def median(xs):
 
 
 def roofline_gate_up(model, reps=2, m=1):
-    """Dominant kernel: gemv_kernel<.., SWIGLU, NORM> on gate_up (2*I_local x H bf16 per launch).  Launch it once
+    """Dominant kernel: the projection with SwiGLU (and, for one row, RMSNorm) on gate_up (2*I_local x H bf16 per launch).  Launch it once
     per layer over every layer's own weights (13.6 GB at TP=1: no cache reuse) between two HIP events recorded on
     the launching stream; achieved = algorithmic bytes per launch / average launch duration."""
+    import ctypes
+
     import torch
     from chatts_amd import _lib
     lib, cfg, plan = model.lib, model.config, model.plan
@@ -144,24 +146,20 @@ def roofline_gate_up(model, reps=2, m=1):
         wsb = max(int(lib.chatts_linear_workspace(m, n, H)), 16)
         ws = torch.empty(wsb, dtype=torch.uint8, device=model.device)
 
+    fmt = _lib.W8_INT8 if model.weight_format == "int8" else _lib.W8_FP8
+
+    def args(lw):
+        common = dict(w=lw["gate_up"].data_ptr(), m=m, n=n, k=H, lda=H, ldw=H, ldc=plan.inter, epilogue=_lib.EPI_SWIGLU, w8=_lib.ptr(lw.get("gate_up8")),
+                      w8_scale=_lib.ptr(lw.get("gate_up8_scale")), ldw8=H, w8_format=fmt)
+        if m == 1:
+            return _lib.LinearArgs(a=x.data_ptr(), c=out.data_ptr(), norm_w=lw["post_norm"].data_ptr(), norm_eps=cfg.rms_norm_eps, w4=_lib.ptr(lw.get("gate_up4")),
+                                   w4_sz=_lib.ptr(lw.get("gate_up4_sz")), ldw4=H // 2, w4_group=model.int4_group, **common)
+        return _lib.LinearArgs(workspace=ws.data_ptr(), workspace_bytes=wsb, a_hi=hi.data_ptr(), a_lo=lo.data_ptr(), ld_planes=H, c_hi=chi.data_ptr(), c_lo=clo.data_ptr(),
+                               ld_cplanes=plan.inter, **common)
+
     def sweep():
         for lw in model.layers:
-            if m == 1:
-                la = _lib.LinearArgs(a=x.data_ptr(), w=lw["gate_up"].data_ptr(), bias=None, resid=None, c=out.data_ptr(),
-                                     norm_w=lw["post_norm"].data_ptr(), norm_eps=cfg.rms_norm_eps, m=1, n=n, k=H, lda=H,
-                                     ldw=H, ldc=plan.inter, epilogue=_lib.EPI_SWIGLU, workspace=None, workspace_bytes=0,
-                                     w8=_lib.ptr(lw.get("gate_up8")), w8_scale=_lib.ptr(lw.get("gate_up8_scale")), ldw8=H,
-                                     w4=_lib.ptr(lw.get("gate_up4")), w4_sz=_lib.ptr(lw.get("gate_up4_sz")), ldw4=H // 2,
-                                     w4_group=model.int4_group,
-                                     w8_format=_lib.W8_INT8 if model.weight_format == "int8" else _lib.W8_FP8)
-            else:
-                la = _lib.LinearArgs(a=None, w=lw["gate_up"].data_ptr(), bias=None, resid=None, c=None, norm_w=None, norm_eps=0.0,
-                                     m=m, n=n, k=H, lda=H, ldw=H, ldc=plan.inter, epilogue=_lib.EPI_SWIGLU, workspace=ws.data_ptr(),
-                                     workspace_bytes=wsb, w8=_lib.ptr(lw.get("gate_up8")), w8_scale=_lib.ptr(lw.get("gate_up8_scale")),
-                                     ldw8=H, a_hi=hi.data_ptr(), a_lo=lo.data_ptr(), ld_planes=H, c_hi=chi.data_ptr(),
-                                     c_lo=clo.data_ptr(), ld_cplanes=plan.inter,
-                                     w8_format=_lib.W8_INT8 if model.weight_format == "int8" else _lib.W8_FP8)
-            _lib.check(lib.chatts_linear(la, stream.cuda_stream))
+            _lib.check(lib.chatts_linear(args(lw), stream.cuda_stream))
 
     sweep()
     torch.cuda.synchronize()
@@ -179,12 +177,15 @@ def roofline_gate_up(model, reps=2, m=1):
     bytes_per_launch = n * H * (1 if fp8 else 2) + (n * 4 if fp8 else 0) + m * (H * 4 + H * 4 + plan.inter * 4)
     if int4:
         bytes_per_launch = n * H // 2 + n * (H // model.int4_group) * 8 + H * 4 + H * 4 + plan.inter * 4
+    first = args(model.layers[0])
+    weights = "int8" if fp8 and fmt == _lib.W8_INT8 else "fp8" if fp8 else "bf16"
     if m > 1:
-        return dict(kernel=f"gemm_stream_kernel<4,{'fp8' if fp8 else 'bf16'}> (gate_up_proj + SwiGLU, M = {m} sequences, bf16 planes in/out)",
-                    launches=launches, avg_us=avg_s * 1e6, bytes_per_launch=bytes_per_launch, gbs=bytes_per_launch / avg_s / 1e9)
-    return dict(kernel=("gemv4_ldsx_kernel" if int4 else "gemv8_ldsx_kernel" if fp8 else "gemv_ldsx_kernel") +
-                "<2,2,SWIGLU,NORM> (gate_up_proj + fused RMSNorm + SwiGLU)", launches=launches,
-                avg_us=avg_s * 1e6, bytes_per_launch=bytes_per_launch, gbs=bytes_per_launch / avg_s / 1e9)
+        name = "gemm_cols_kernel" if lib.chatts_linear_cols(first) else "gemm_rows_kernel" if lib.chatts_linear_few_rows(ctypes.byref(first), None) else "gemm_stream_kernel"
+        what = f"gate_up_proj + SwiGLU, {weights}, M = {m} sequences, bf16 planes in/out"
+    else:
+        name = "gemv4_kernel" if int4 else "gemv_ring_kernel" if lib.chatts_gemv_ring(first) else "gemv8_ldsx_kernel" if fp8 else "gemv_ldsx_kernel"
+        what = f"gate_up_proj + fused RMSNorm + SwiGLU, {'int4' if int4 else weights}"
+    return dict(kernel=f"{name} ({what})", launches=launches, avg_us=avg_s * 1e6, bytes_per_launch=bytes_per_launch, gbs=bytes_per_launch / avg_s / 1e9)
 
 
 def prefill_mfma_gate_up(model, T, reps=1):

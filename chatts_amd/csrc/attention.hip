@@ -26,7 +26,8 @@ namespace chatts {
 namespace chatts {
 
 // ---------------------------------------------------------------------------------------------------
-// decode: grid (n_kv, n_slots), 64 threads.  Slot s walks tiles s, s + n_slots, ... of 16 keys.
+// decode: grid (n_kv, n_splits, sequences), 64 threads; TWO: (n_kv, 2 n_splits, sequences).  Slot s of the S that a context uses (attn_slots, at most n_splits) walks tiles s, s + S, ...
+// of 16 keys; the others leave.
 // ---------------------------------------------------------------------------------------------------
 // TWO: groups of 7 and 8 heads, whose sums do not fit the registers of two waves per SIMD: two waves a slot, four heads and the rest, next to each other on one XCD (a row of the
 // cache comes from memory once).  One wave per SIMD with all heads was 1.1 .. 1.4 times slower from 12 sequences on, spilling 10 registers 1.1 .. 1.3 times nearly everywhere.

@@ -1,4 +1,4 @@
-// gemv_common.h - the arithmetic of the batch-1 weight-streaming GEMV, shared by gemv.hip and decode_mega.hip so that both
+// gemv_common.h - the arithmetic of the batch-1 weight-streaming GEMV, shared by gemv.hip and gemv_ring.hip so that both
 // accumulate a row in exactly the same order (bit-identical results).
 #pragma once
 #include "common.h"

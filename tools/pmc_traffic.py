@@ -7,7 +7,7 @@
     python tools/pmc_traffic.py ts /tmp/fst/.../p_results.db "<command>" profiles/r4_ts_encoder_pmc_fetch_size.txt
 
 Every entry records a digest of the kernel sources it was measured on (code_digest below); bench.py prints `traffic: null` when
-the digest of the checked-out sources differs - a counter leg must describe the code it is quoted for (VERDICT r3, weak #10).
+the digest of the checked-out sources differs - a counter leg must describe the code it is quoted for.
 gfx950: FETCH_SIZE counts 64 B per 128-B request of a wide coalesced stream -> bytes = KiB x 1024 x 2 (MI355X_MICROARCH.md, HBM)."""
 import hashlib
 import json
@@ -17,7 +17,7 @@ import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 OUT = os.environ.get("PMC_TRAFFIC_OUT") or os.path.join(ROOT, "profiles", "pmc_traffic.json")      # (a GPU-box job writes under gpurun_out/)
-GEMV_FILES = ["chatts_amd/csrc/gemv.hip", "chatts_amd/csrc/gemv_common.h", "chatts_amd/csrc/tp_common.h", "chatts_amd/csrc/common.h"]
+GEMV_FILES = ["chatts_amd/csrc/gemv.hip", "chatts_amd/csrc/gemv_ring.hip", "chatts_amd/csrc/gemv_common.h", "chatts_amd/csrc/tp_common.h", "chatts_amd/csrc/common.h"]
 TS_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_ring.hip", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/ts_frontend.hip",
             "chatts_amd/csrc/common.h"]
 BATCHED_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/attention.hip", "chatts_amd/csrc/attn_decode.h",
@@ -57,12 +57,12 @@ def save(d):
 
 
 def headline(db, cmd, src):
-    rows = [r for r in counter_rows(db) if "gemv_ldsx_kernel<2, 2, 3, true>" in r[0]]
+    rows = [r for r in counter_rows(db) if "gemv_ring_kernel<3, true" in r[0] or "gemv_ldsx_kernel<2, 2, 3, true>" in r[0]]
     name, grid, wg, n, kib, us = max(rows, key=lambda r: r[4])            # gate_up: the SwiGLU GEMV with the most bytes
     inter = 13824
     d = load()
     d.update({"source": f"{src} ({cmd}, MI355X, round 6)", "code_digest": code_digest(GEMV_FILES), "code_files": GEMV_FILES,
-              "kernel": f"gemv_ldsx_kernel<2,2,SWIGLU,NORM> (gate_up_proj, grid {grid} = {grid // wg} workgroups x {wg} threads)",
+              "kernel": f"{'gemv_ring_kernel' if 'gemv_ring' in name else 'gemv_ldsx_kernel'}<SWIGLU,NORM> (gate_up_proj, grid {grid} = {grid // wg} workgroups x {wg} threads)",
               "launches_counted": n, "fetch_size_kib_per_launch": round(kib, 1), "gfx950_fetch_correction": 2.0,
               "write_bytes_per_launch": inter * 4, "hbm_bytes_per_launch": int(kib * 1024 * 2 + inter * 4), "avg_us_under_pmc": round(us, 2)})
     save(d)
