@@ -48,7 +48,7 @@ class TimeSeriesEmbedding:
         self.position_embedding = None               # f32 [max_seq+1, emb]
         self.weights = [None] * self.num_layers      # bf16 [H, Kpad_l]
         self._tiled = [None] * self.num_layers       # the same in the prefill kernel's blocks (layers after the first) ...
-        self._tiled_of = [None] * self.num_layers    # ... and what they were made from: (tensor, its version)
+        self._tiled_of = []                          # ... and what they were made from: (layer, tensor, its version)
         self.biases = [None] * self.num_layers       # f32 [H]
 
     # ---- weights ---------------------------------------------------------------------------------
@@ -109,21 +109,21 @@ class TimeSeriesEmbedding:
         if l == 0 or not w.is_cuda or w.shape[1] % 64:
             return
         self._tsw = None
+        self._tiled_of = [t for t in self._tiled_of if t[0] != l]
         if w.is_inference():
-            self._tiled[l] = self._tiled_of[l] = None
+            self._tiled[l] = None
             return
         lib = _lib.load()
         n = int(lib.chatts_tile_bf16_elems(*w.shape))
         if self._tiled[l] is None or self._tiled[l].numel() != n:
             self._tiled[l] = torch.empty(n, dtype=torch.bfloat16, device=w.device)
         _lib.check(lib.chatts_tile_bf16(_lib.ptr(w), *w.shape, w.shape[1], _lib.ptr(self._tiled[l]), _lib.stream_ptr()))
-        self._tiled_of[l] = (w, w._version)
+        self._tiled_of.append((l, w, w._version))
 
     def _follow_weights(self):
-        for l in range(1, self.num_layers):
-            w, of = self.weights[l], self._tiled_of[l]
-            if of is not None and (of[0] is not w or of[1] != w._version):
-                self._tile(l)
+        for l, w, version in self._tiled_of:
+            if self.weights[l] is not w or w._version != version:
+                self._tile(l)                        # (puts a list of its own in the place of the one that is walked)
 
     def set_precision(self, precision):
         """"bf16x2" (default, parity grade: float32 activations as bf16 hi + lo planes) or "fp8" - the SPEED mode of
