@@ -98,16 +98,17 @@ def rope_tables(cfg, max_pos, device):
 def batched_slots(max_batch, nq, nkv, n_splits):
     """16-key slots per sequence of the batched decode attention, at most: its kernel uses fewer for a short context.  A slot is a wave per kv head (two for groups of more than six
     heads), and a tile more in the longest of them is 1.2 us for all.  The number may not depend on how many sequences run, because a row's bits would; so it is what both ends bear: 1024
-    waves where every place is taken (more repeat the prologue and lengthen the merge), but for the few sequences of a server that is not full no fewer than 32 slots, up to 1792 waves
-    (seven a CU).  Both launches in a graph over rotating caches, us, 1024 waves and 12 slots / this rule, 40 heads on 8 kv heads:
+    waves where every place is taken (more repeat the prologue and lengthen the merge), but where those give fewer than 32 slots, for the few sequences of a server that is not full, 36
+    of them up to 1792 waves (seven a CU).  Both launches in a graph over rotating caches, us, 1024 waves and 12 slots / this rule, 40 heads on 8 kv heads:
       8 places (16 / 28 slots), one taken, context 223 / 801 / 1800 / 4000   8.2 / 8.3   13.0 / 10.6   19.8 / 15.4   33.4 / 22.1;   all taken   10.3 / 11.1   17.4 / 18.0   26.7 / 27.3   46.7 / 49.6
      16 places (12 / 14 slots)                                               9.9 / 8.3   14.9 / 13.4   23.7 / 21.7   41.8 / 36.8;               12.7 / 12.4   24.1 / 23.6   43.1 / 43.4   85.7 / 85.9
-      5 places (25 / 32 slots)                                               8.3 / 8.4   11.9 / 10.4   15.3 / 13.8   24.7 / 20.3;                9.7 / 10.5   14.8 / 14.7   19.9 / 20.2   32.9 / 34.2
+      5 places (25 / 36 slots)                                               8.2 / 8.4   11.6 / 10.5   15.1 / 13.8   24.7 / 19.5;                9.7 /  9.8   14.6 / 14.4   19.8 / 20.3   32.9 / 34.8
     5 heads on one kv head (a shard), 8 places (16 / 64)                     7.8 / 8.0   12.7 /  8.5   19.2 / 10.6   32.2 / 13.5;                8.1 /  8.6   13.2 /  9.7   19.6 / 11.7   33.4 / 15.8
-    Dearest: 1.1 us where every place holds about a hundred keys (8.6 / 9.8).  Groups of more than six keep 1024 waves' slots, eight at least: more cost 15 .. 30 % where all are taken."""
+    Dearest: 1.6 us with 8 places that hold 400 keys each (12.4 / 14.1).  Not 16 or 32: the heads' partials then lie 8 or 16 KB apart, on the same channels (5 places of 100 keys, 32 slots 9.6 us, 36 8.6; 14 of 60, 16 slots 10.4, 15 8.9).
+    Groups of more than six keep 1024 waves' slots, eight at least: more cost 15 .. 30 % where all are taken."""
     by_waves = 1024 // (nkv * max_batch)
-    least = 8 if nq // nkv > 6 else min(32, max(12, 224 // max_batch))
-    return max(1, min(n_splits, max(least, by_waves)))
+    least = 8 if nq // nkv > 6 else min(36, max(12, 224 // max_batch))
+    return max(1, min(n_splits, by_waves if by_waves >= 32 else max(least - (least % 16 == 0), by_waves)))
 
 
 class ChatTSForCausalLM(SlotModel):
