@@ -109,14 +109,14 @@ class TimeSeriesEmbedding:
         if l == 0 or not w.is_cuda or w.shape[1] % 64:
             return
         self._tsw = None
+        written = any(at == l and of is w for at, of, _ in self._tiled_of)      # in place: its copy is, too (another tensor's copy gets memory of its own, for calls on other streams read the old one)
         self._tiled_of = [t for t in self._tiled_of if t[0] != l]
         if w.is_inference():
             self._tiled[l] = None
             return
         lib = _lib.load()
-        n = int(lib.chatts_tile_bf16_elems(*w.shape))
-        if self._tiled[l] is None or self._tiled[l].numel() != n:
-            self._tiled[l] = torch.empty(n, dtype=torch.bfloat16, device=w.device)
+        if not written:
+            self._tiled[l] = torch.empty(int(lib.chatts_tile_bf16_elems(*w.shape)), dtype=torch.bfloat16, device=w.device)
         _lib.check(lib.chatts_tile_bf16(_lib.ptr(w), *w.shape, w.shape[1], _lib.ptr(self._tiled[l]), _lib.stream_ptr()))
         self._tiled_of.append((l, w, w._version))
 
