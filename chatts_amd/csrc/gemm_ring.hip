@@ -296,16 +296,15 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 }
 
 // ---- host side ------------------------------------------------------------------------------------------------------------------
-// (T, sk) per shape: a cost model in cycles of the slowest workgroup - rounds x (K-steps x step + a per-unit constant) + the split-K epilogue launch.  Fitted to
-// 4500 measurements of (T, sk), T up to five above the fewest, for 14 projections (K 2048 .. 13824, N 1536 .. 27648) at 100 .. 1300 rows: a 64-deep step of a tile with f fragments
-// takes 253 f + 1069 cycles (the 16 f MFMAs per SIMD and the (32 f + 256) x 128 bytes of LDS-DMA overlap only partly), a unit 4800 of prologue and stores, a
-// split-K epilogue 5 us (8 from five slabs on, more where its threads cannot ask for all slabs at once) and its slab traffic at ~4.5 to 5 TB/s, less
-// where the slabs outgrow 64 MB.  Over these its pick is 0.8 % slower than the best pair in the mean, the constants before (235 f + 900, 9000 a unit, a
-// row-walking epilogue from five slabs on) gave 1.4 %.  Over 480 cells of 24 projections at 129 .. 2048 rows with any T it is 2.5 % (at most 23: 8192 x 2048, 129 rows, where (3, 2)
-// beats (2, 4)), before 3.3 % (33); where the two picks differ by more than 3 %, this one is faster in 58 cells and slower in 20.  5120 x 13824 at 223 rows (3, 4) 80.3 us, now (2, 6) 72.5; 4096 x 4096 at 900 rows 80.8 / 71.4.
-// Panels of 192 rows are the second width: a step costs 215 f + 1080 there, dearer per column, but where panels of 256 leave CUs without a unit it fills them:
-// 24576 x 4096 gated, 223 rows: 96 panels x 2 tiles on 192 CUs 94.5 us, 128 x 2 on 256 CUs 90.3; 6144 x 4096 at 223 rows 36.4 / 34.2, 5120 x 5120 at 150 rows
-// 36.9 / 34.4, 6144 x 2048 at 380 rows 31.5 / 26.6; 27648 x 5120 (108 panels; 144 would need two rounds) stays at 256: 125.7 / 162.
+// (T, sk, panel) per shape: a cost model in cycles of the slowest workgroup - its K-steps, a constant per unit, the split-K epilogue launch.  Fitted to what its pick costs against the best
+// of 16000 measurements, planes and W in tiles: 13 projections (K 2048 .. 13824, N 2048 .. 27648; epilogues none, GELU, gated, residual with the norm behind it) at 40 .. 2048 rows.  A 64-deep
+// step of a tile with f fragments takes 260 f + 1045 cycles in panels of 256 rows, 214 f + 965 in panels of 192 (the 4 f NF MFMAs per SIMD and the (32 f + 64 NF) x 128 bytes of LDS-DMA
+// overlap only partly); of several units a workgroup meets the longest tile once and the mean one else; a unit costs 4900 of prologue and stores, a split 5 us of epilogue (7 from five slabs on,
+// 16 from nine on, which the row-wise norm cannot hold in registers) and its slab traffic at ~4 to 5 TB/s, less where the slabs outgrow 64 MB.  Over these its pick is 1.0 % slower than the best
+// triple in the mean (1.1 up to 144 rows, 0.4 above 900; at most 10: 7168 x 5120, 80 rows); the constants before, fitted to row-major planes, the longest tile for every unit: 2.0 (3.6, 0.8; 46).
+// us before / now: 5120 x 13824, 80 rows 57.8 / 41.9; 6144 x 4096, 384 rows 49.1 / 44.0; 4096 x 4096 GELU, 1036 rows 74.4 / 68.0; 7168 x 5120, 600 rows 86.7 / 81.1; 27648 x 5120 gated, 2048
+// rows (13 tiles / 14: six rounds both) 883 / 830.  What lies on the wrong side by more than 1 %: 24576 x 4096 gated, 600 rows 191.8 / 197.9.
+// Panels of 192 rows are dearer per column, but fill CUs that panels of 256 leave without a unit: 24576 x 4096 gated, 223 rows: 96 panels x 2 tiles on 192 CUs 94.6 us, 128 x 2 on 256 CUs 80.0.
 void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int force_nf, RingGeom& g) {
   const int F = (m + 15) / 16, nk = k / 64;
   g.F = F;
@@ -318,26 +317,24 @@ void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int forc
   for (int nf = 4; nf >= 3; --nf) {
     if (force_nf && nf != force_nf) continue;
     const int P = (n + 64 * nf - 1) / (64 * nf);
-    const double frag = nf == 4 ? 253.0 : 215.0, tile = nf == 4 ? 1069.0 : 1080.0;
+    const double frag = nf == 4 ? 260.0 : 214.0, tile = nf == 4 ? 1045.0 : 965.0;
     for (int T = tmin; T <= tmax; ++T) {
       const int fmax = (F + T - 1) / T;
-      const double step = frag * fmax + tile;
-      // the work itself, evenly spread over the CUs.  Its fragments and a constant a tile: more tiles only add to that.  With the fragments that are not there it rises and
-      // falls (128 fragments: 31 tiles of 5, 32 tiles of 4)
-      if ((frag * F + tile * T) * P * nk > best * slots) break;
-      if ((double)T * P * nk * step > best * slots) continue;
+      const double most = frag * fmax + tile, mean = frag * F / T + tile;
+      // the work itself, evenly spread over the CUs: its fragments and a constant a tile, so more tiles only add to it
+      if (mean * T * P * nk > best * slots) break;
       for (int sk = 1; sk <= 16; ++sk) {
         if (sk > 1 && nk / sk < 4) break;
         const long long units = (long long)T * P * sk;
         const long long rounds = (units + slots - 1) / slots;
         const int steps = (nk + sk - 1) / sk;
-        double t = (double)rounds * (steps * step + 4800.0);
+        double t = steps * (most + (double)(rounds - 1) * mean) + rounds * 4900.0;
         if (sk > 1) {
           const double slabs = (double)m * n * 4.0;
-          t += (sk <= 4 ? 10200.0 : sk <= 8 ? 17600.0 : 30000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1840.0 : sk <= 4 ? 2200.0 : 2480.0);
+          t += (sk <= 4 ? 10300.0 : sk <= 8 ? 14200.0 : 34000.0) + (sk + 2) * slabs / (sk * slabs > 64e6 ? 1365.0 : sk <= 4 ? 2200.0 : 1770.0);
         }
-        // a split that is no more than 0.6 % nearer counts as equal: slabs are the part that the model knows least (6144 x 4096, 700 rows: (5, 2) 68.3 us, (9, 1) 62.7)
-        if (sk > 1) t *= 1.006;
+        // a split that is no more than 0.7 % nearer counts as equal: slabs are the part that the model knows least
+        if (sk > 1) t *= 1.007;
         if (t < best) { best = t; bt = T; bs = sk; bf = nf; }
       }
     }
