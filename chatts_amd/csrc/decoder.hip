@@ -43,6 +43,7 @@ struct ChattsDecoder {
   bool normed = false;      // planes 0 already hold RMSNorm(x) for the projection that comes next (written by the previous
                             // projection's fused epilogue): norm_into only binds them
   bool normed_tiled = false;      // ... in the prefill kernel's blocks
+  bool mid_planes = false;  // chunks of 17 .. 95 rows on planes: no bias of a layer is one that the plane path refuses and the float32 path takes (not 16-byte aligned)
   int ss_parts = 0;         // > 0, with normed: ... planes 1 hold norm_w * x without the factor 1 / rms; each row's sum of squares is that many parts in
                             // b.attn: a step of 2 .. 16 sequences behind a projection that hands its norm on (request_post_ss)
   bool sampling = false;    // token selection of the decode steps: greedy argmax, or the sampler with `sa`
@@ -225,6 +226,8 @@ extern "C" ChattsDecoder* chatts_decoder_create(const ChattsDecoderConfig* c, co
   d->layers.assign(w->layers, w->layers + c->n_layers);
   d->w.layers = d->layers.data();
   d->b = *b;
+  d->mid_planes = true;
+  for (const ChattsLayerWeights& l : d->layers) d->mid_planes = d->mid_planes && (uintptr_t)l.qkv_bias % 16 == 0;
   return d;
 }
 
@@ -252,17 +255,16 @@ static ChattsKvCache layer_cache(const ChattsDecoder* d, int layer, int seq) {
   return c;
 }
 
-// Projections whose A operand is a pair of bf16 hi / lo planes: prefill chunks of >= 96 rows (LDS-DMA GEMM) and batched
-// decode with 2..16 sequences on bf16 weights (weight-streaming kernel).
+// Projections whose A operand is a pair of bf16 hi / lo planes: prefill chunks (of 17 .. 95 rows: kMidPlanesK) and batched decode with 2..16 sequences on bf16 weights.
 static bool planes_path(const ChattsDecoder* d, int m, int k, bool fp8 = false) {
   if (!(d->b.planes_hi && d->b.planes_lo && d->b.planes2_hi && d->b.planes2_lo) || k % 64 != 0) return false;
   if (m >= 2 && m <= 16) return !fp8 || k % 128 == 0;      // (the fp8 stream's K-step is one 128-byte line = 128 values)
-  return m >= 96 && !fp8;
+  return (m >= 96 || (d->mid_planes && m > 16 && k >= kMidPlanesK)) && !fp8;
 }
 
-// planes of a prefill chunk of m rows and width k in the prefill kernel's blocks?  Asked once for each set of planes, by whoever writes them: PLANE_TILES may change beside a running call.
+// planes of a prefill chunk of m rows and width k, for a projection to n, in the prefill kernel's blocks?  Asked once for each set of planes, by whoever writes them: PLANE_TILES may change beside a running call.
 // A projection writes them so only if it runs that kernel: its own operand comes as planes and nothing else (a width of half a K-step more than whole ones does not)
-static bool tiles_path(const ChattsDecoder* d, int m, int k) { return planes_path(d, m, k) && planes_tiled_for(m, k); }
+static bool tiles_path(const ChattsDecoder* d, int m, int n, int k) { return planes_path(d, m, k) && planes_tiled_for(m, n, k); }
 // x -> RMSNorm -> la's input: planes written by the norm kernel itself (plane path) or float32 xn.  chain: where the projection before may have left the
 // factor 1 / rms to this one (batched steps).  tiled: (a prefill chunk) the form of the planes that la gets
 static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la, chatts_stream_t stream, ChattsNormChain* chain = nullptr, bool* tiled = nullptr) {
@@ -282,7 +284,7 @@ static int norm_into(ChattsDecoder* d, const float* norm_w, ChattsLinearArgs* la
       d->normed = false;
       return CHATTS_OK;
     }
-    if (tiled) *tiled = tiles_path(d, la->m, la->k);
+    if (tiled) *tiled = tiles_path(d, la->m, la->n, la->k);
     if (tiled && *tiled) return launch_rmsnorm_planes(d->b.x, la->k, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, la->m & ~15, as_stream(stream));
     return chatts_rmsnorm_planes(d->b.x, norm_w, d->b.planes_hi, d->b.planes_lo, la->k, la->m, la->k, d->cfg.rms_eps, stream);
   }
@@ -307,18 +309,18 @@ static bool request_post_ss(ChattsDecoder* d, ChattsLinearArgs* la, ChattsNormCh
   d->normed = true; d->ss_parts = parts;
   return true;
 }
-// The residual-updating projection also produces the NEXT projection's operand: RMSNorm(x) with `next_norm_w` as planes 0, when that projection will take the
-// plane path for the same M.
-static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const float* next_norm_w, bool next_fp8) {
+// The residual-updating projection also produces the NEXT projection's operand: RMSNorm(x) with `next_norm_w` as planes 0, when that projection (to next_n; 0: of a batched step, whose
+// planes are never tiled) will take the plane path for the same M.
+static void request_post_norm(ChattsDecoder* d, ChattsLinearArgs* la, const float* next_norm_w, int next_n, bool next_fp8) {
   if (!d->chain || d->cfg.tp_world > 1 || !next_norm_w || la->epilogue != CHATTS_EPI_RESID) return;
   // the fused epilogue runs one workgroup per row - fine for a prefill chunk; at batched-decode M it needs several workgroups per row,
   // which re-read resid while others write c: only when the caller gave it a c that does not alias resid (layer_part_batched)
-  if (la->m < 64 && !(la->m <= 16 && la->c != la->resid && gemm_post_norm_small_m())) return;
+  if (la->m < 17 && !(la->m <= 16 && la->c != la->resid && gemm_post_norm_small_m())) return;
   if (!planes_path(d, la->m, la->n, next_fp8)) return;
   la->post_norm_w = next_norm_w; la->post_norm_eps = d->cfg.rms_eps;
   la->post_hi = d->b.planes_hi; la->post_lo = d->b.planes_lo; la->ld_post = la->n;
   d->normed = true;
-  d->normed_tiled = !la->a && tiles_path(d, la->m, la->n);
+  d->normed_tiled = next_n && !la->a && tiles_path(d, la->m, next_n, la->n);
 }
 static PlaneTiles after(const ChattsDecoder* d, const ChattsLinearArgs& la, bool a_tiled) { return {a_tiled, false, la.post_norm_w && d->normed_tiled}; }      // (of a projection behind request_post_norm)
 
@@ -559,7 +561,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   const ChattsLayerWeights& lw = d->layers[layer];
   const bool tp = c.tp_world > 1;
   const int H = c.hidden;
-  const bool tile_attn = t > 1 && tiles_path(d, t, c.n_q * kHeadDim);
+  const bool tile_attn = t > 1 && tiles_path(d, t, H, c.n_q * kHeadDim);
   bool tile_h = false;
   int rc;
   ChattsLinearArgs la;
@@ -633,7 +635,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
       d->tp_fused = true;
     } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
     else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
-    request_post_norm(d, &la, lw.post_norm, false);
+    request_post_norm(d, &la, lw.post_norm, 2 * c.inter, false);
     return linear_tiled(&la, stream, after(d, la, tile_attn));
   }
   // part 1: RMSNorm -> gate_up + SwiGLU -> down (+ residual / partial)
@@ -648,7 +650,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   } else {
     if ((rc = norm_into(d, lw.post_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
   }
-  const bool act_planes = t > 1 && planes_path(d, t, c.inter), tile_act = act_planes && !la.a && tiles_path(d, t, c.inter);   // SwiGLU output goes straight into down_proj's operand format
+  const bool act_planes = t > 1 && planes_path(d, t, c.inter), tile_act = act_planes && !la.a && tiles_path(d, t, 2 * c.inter, H) && tiles_path(d, t, H, c.inter);   // SwiGLU output goes straight into down_proj's operand format
   if (act_planes) { la.c = nullptr; la.c_hi = d->b.planes2_hi; la.c_lo = d->b.planes2_lo; la.ld_cplanes = c.inter; }
   if ((rc = linear_tiled(&la, stream, {tile_h, tile_act, false})) != 0) return rc;
   la = ChattsLinearArgs{};
@@ -666,7 +668,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
     d->tp_fused = true;
   } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
   else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
-  request_post_norm(d, &la, layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : nullptr, false);
+  request_post_norm(d, &la, layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : nullptr, (c.n_q + 2 * c.n_kv) * kHeadDim, false);
   return linear_tiled(&la, stream, after(d, la, tile_act));
 }
 
@@ -732,7 +734,7 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
       la.c = d->b.xn;
       d->x_in_xn = true;
     }
-    request_post_norm(d, &la, lw.post_norm, lw.gate_up8 != nullptr);
+    request_post_norm(d, &la, lw.post_norm, 0, lw.gate_up8 != nullptr);
     if (d->x_in_xn && !la.post_norm_w) { la.c = d->b.x; d->x_in_xn = false; }      // not fused after all: the norm launch reads x
     return chatts_linear(&la, stream);
   }
@@ -760,7 +762,7 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
   const float* next_norm = layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : d->w.final_norm;
   const bool next_fp8 = (layer + 1 < c.n_layers ? d->layers[layer + 1].qkv8 : d->w.lm_head8) != nullptr;
   chain = ChattsNormChain{};
-  if (!request_post_ss(d, &la, &chain, next_norm, next_fp8)) request_post_norm(d, &la, next_norm, next_fp8);
+  if (!request_post_ss(d, &la, &chain, next_norm, next_fp8)) request_post_norm(d, &la, next_norm, 0, next_fp8);
   return chatts_linear_chain(&la, &chain, stream);
 }
 
@@ -948,7 +950,7 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
   const ChattsDecoderConfig& c = d->cfg;
   const ChattsLayerWeights& lw = d->layers[layer];
   const int H = c.hidden, qkv_n = (c.n_q + 2 * c.n_kv) * kHeadDim, na = c.n_q * kHeadDim;
-  const bool tile_attn = t > 1 && tiles_path(d, t, na);
+  const bool tile_attn = t > 1 && tiles_path(d, t, H, na);
   bool tile_h;
   int rc;
   d->normed_q = false;      // (f16q mode: this half runs the default kernels and is about to overwrite planes 0 - the next MLP half recomputes its norm)
@@ -997,7 +999,7 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
     la.a_hi = d->b.planes_hi; la.a_lo = d->b.planes_lo; la.ld_planes = na;
   }
   la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID;
-  request_post_norm(d, &la, lw.post_norm, false);
+  request_post_norm(d, &la, lw.post_norm, 2 * c.inter, false);
   return linear_tiled(&la, stream, after(d, la, tile_attn));
 }
 

@@ -957,6 +957,8 @@ static bool stream_multiblock(int m, int n, int k, bool w8) {
   return m > 16 && m <= max_m && m <= 128 && !w8 && k % 64 == 0 && k >= 1024 &&
          2 * 8 * (((n + kRingPanel - 1) / kRingPanel + 7) / 8) <= device_cus();
 }
+// (not at 64 rows and less: the product that reads them may be chunked otherwise by then, and 16-row blocks are few)
+bool planes_tiled_for(int m, int n, int k) { return m > 64 && k % 64 == 0 && !stream_multiblock(m, n, k, false) && opt_get(OPT_PLANE_TILES, 1) != 0; }
 static bool use_stream(const ChattsLinearArgs* a) {
   if (!(a->a_hi && a->a_lo) || opt_get(OPT_GEMM_STREAM, 1) == 0) return false;
   if (a->m >= 2 && a->m <= 16) return a->k % stream_bk(a->w8 != nullptr) == 0;
@@ -1071,7 +1073,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     a_copy.w8 = nullptr; a_copy.w8_scale = nullptr;
     a = &a_copy;
   }
-  const bool stream = use_stream(a) && !(tiles.a || tiles.c || tiles.post);
+  const bool stream = use_stream(a) && !(tiles.a || tiles.c || tiles.ring);
   const bool ring = !stream && use_ring(a);
   const int batch = a->batch > 1 ? a->batch : 1;      // > 1: gemm_batched_stream(a) holds
   RingGeom rg{};
@@ -1103,8 +1105,10 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   p.w8 = a->w8; p.w8_scale = a->w8_scale; p.ldw8 = a->ldw8; p.w8_format = a->w8_format;
   p.c_hi = a->c_hi; p.c_lo = a->c_lo; p.ldcp = a->ld_cplanes;
   p.wt = ring ? a->w_tiled : nullptr; p.planes_tiled = a->planes_tiled;
-  CHATTS_REQUIRE(!(tiles.a || tiles.c || tiles.post) || (ring && batch == 1 && (!tiles.a || a->ld_planes == a->k) && (!tiles.c || a->ld_cplanes % 32 == 0) && (!tiles.post || a->ld_post % 32 == 0)),
+  CHATTS_REQUIRE(!(tiles.a || tiles.c) || (ring && batch == 1 && (!tiles.a || a->ld_planes == a->k) && (!tiles.c || a->ld_cplanes % 32 == 0)),
                  CHATTS_E_SHAPE, "linear: planes in tiles are the prefill kernel's (M=%d N=%d K=%d)", a->m, a->n, a->k);
+  // (the norm behind a weight stream may write them too: it runs in the split's epilogue or in a launch of its own)
+  CHATTS_REQUIRE(!tiles.post || ((ring || stream) && batch == 1 && a->m > 16 && a->ld_post % 32 == 0), CHATTS_E_SHAPE, "linear: a norm's planes in tiles follow the plane path, M > 16 (M=%d N=%d K=%d)", a->m, a->n, a->k);
   const int whole = a->m & ~15, ctile = tiles.c ? whole : 0, ptile = tiles.post ? whole : 0;
   p.a_tiled = tiles.a ? whole : 0; p.c_tiled = ctile;
   p.glu_limit = a->glu_limit; p.glu_alpha = a->glu_alpha;

@@ -96,8 +96,13 @@ __device__ __forceinline__ float glu_value(int epilogue, float g, float u, float
 // 83.2 / 81.8; 1473 rows 7168 x 5120 211 / 185, 4096 x 12288 242 / 229.  The same products in the same order: the same bits.
 struct PlaneTiles {
   bool a, c, post;
+  bool ring = false;      // the prefill kernel whatever the form of the planes
 };
-inline bool planes_tiled_for(int m, int k) { return m > 128 && k % 64 == 0 && opt_get(OPT_PLANE_TILES, 1) != 0; }      // (up to 128 rows the weight stream may run)
+// 17 .. 95 rows on planes from this K on (up to 64 rows, and up to 128 where N is 8192 at most, the weight stream runs; else the prefill kernel): the register-staged kernel, which takes
+// float32, needs 1.2 to 1.6 times as long.  us with the epilogue, float32 / planes: 17 rows 6144 x 4096 19.7 / 13.9, 24576 x 4096 gated 51.5 / 42.4, 4096 x 12288 34.2 / 21.7, 2048 x 2048
+// 11.2 / 8.0; 48 rows 7168 x 5120 30.2 / 22.6, 27648 x 5120 gated 85.9 / 64.1; 80 rows 5120 x 13824 57.0 / 44.1, 8192 x 2048 23.7 / 20.5.  Shorter K is not the weight stream's.
+constexpr int kMidPlanesK = 1024;
+bool planes_tiled_for(int m, int n, int k);      // (gemm.hip: of the A of an m x n x k product)
 int linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles);      // chatts_linear on such planes (decoder.hip)
 
 constexpr int kRingPanel = 256;      // W rows per panel of the prefill kernel

@@ -15,11 +15,12 @@
 //   -> depth_norm (x += mult y; norm2(x)) -> router -> experts, beside a shared one: gate_up -> down
 //   -> depth_norm (x += mult (y + experts); average over depth; the next layer's norm1)
 // Operands between the launches travel in the format the next projection's kernel takes for this row count: bf16 hi / lo planes
-// (2 .. 16 rows: weight-streaming kernel; >= 96 rows: the prefill kernel) or float32.
+// (2 .. 16 rows: weight-streaming kernel; >= 96 rows: the prefill kernel; between them one of the two where K is long enough: kMidPlanesK) or float32.
 #include <new>
 #include <vector>
 
 #include "common.h"
+#include "gemm_common.h"
 
 namespace chatts {
 
@@ -45,7 +46,7 @@ struct ChattsMixDecoder {
   std::vector<ChattsMixRun> runs;
 };
 
-static bool mix_planes(const ChattsMixConfig& c, int m, int k) { return !c.exact && k % 64 == 0 && ((m >= 2 && m <= 16) || m >= 96); }
+static bool mix_planes(const ChattsMixConfig& c, int m, int k) { return !c.exact && k % 64 == 0 && (m >= 96 || (m >= 2 && (m <= 16 || k >= kMidPlanesK))); }
 
 static int mix_equal_blocks(const ChattsMixLayer& l, int i) {      // how many operand blocks from i on have the size of block i
   const int rows = l.mix_row[i + 1] - l.mix_row[i];
