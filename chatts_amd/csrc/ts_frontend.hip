@@ -463,9 +463,11 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
   // the splits of exactly the float32 numbers the float32 path would hold, so both paths give the same result.
   const int P = total_patches, H = w->hidden;
   const bool planes = P > 1 && w->in_features_pad % 64 == 0 && H % 64 == 0 && opt_get(OPT_TS_F32_PATH, 0) == 0;
-  const bool tile = planes && planes_tiled_for(P, H);      // activations between the layers in the prefill kernel's blocks
+  // The prefill kernel from 65 rows on, where the weights lie in its blocks (us a layer, weight stream / prefill kernel: 66 rows 5120 x 5120 25.1 / 20.8, 4096 x 4096 20.1 / 18.6; 96 rows
+  // 28.3 / 23.8, 22.3 / 19.8; 128 rows 29.2 / 27.2, 23.5 / 23.9); without, up to 128 rows the weight stream.  Activations between its layers in blocks, too.
+  const bool mid = planes && w_tiled && P > 64 && P <= 128;
+  const bool tile = planes && (mid ? opt_get(OPT_PLANE_TILES, 1) != 0 : planes_tiled_for(P, H, H));
   // The weights in blocks likewise, where the caller has them so: a 1 KB piece of the loader is 1 KB of memory.  1036 rows of 5120 x 5120, us a layer: 88.6 -> 82.4.
-  // (Not below: at 128 rows the weight stream reads them in the other order.)
   auto hi_of = [&](float* buf) { return reinterpret_cast<chatts_bf16*>(buf); };
   auto lo_of = [&](float* buf, int k) { return reinterpret_cast<chatts_bf16*>(buf) + (size_t)P * k; };
   if (planes) { pa.out = nullptr; pa.out_hi = hi_of(feat); pa.out_lo = lo_of(feat, w->in_features_pad); }
@@ -525,7 +527,7 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
     la.w = w->w[l]; la.bias = w->b[l]; la.m = P; la.n = H; la.k = k;
     la.lda = k; la.ldw = k; la.ldc = H; la.epilogue = last ? CHATTS_EPI_NONE : CHATTS_EPI_GELU;
     la.workspace = workspace; la.workspace_bytes = workspace_bytes;
-    if (tile && w_tiled && l > 0) la.w_tiled = w_tiled[l];
+    if ((tile || mid) && w_tiled && l > 0) la.w_tiled = w_tiled[l];
     if (planes) {
       la.a_hi = hi_of(cur); la.a_lo = lo_of(cur, k); la.ld_planes = k;
       if (last) la.c = dst;
@@ -533,7 +535,7 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
     } else {
       la.a = cur; la.c = dst;
     }
-    if ((rc = linear_tiled(&la, stream, {tile && l > 0, tile && !last, false})) != 0) return rc;
+    if ((rc = linear_tiled(&la, stream, {tile && l > 0, tile && !last, false, mid && l > 0})) != 0) return rc;
     cur = dst;
     k = H;
   }
