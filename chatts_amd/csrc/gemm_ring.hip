@@ -39,15 +39,19 @@ constexpr int kRingLds = kRingSlots * kRingHalf;             // 144 KB
 constexpr int kRingThreads = 768, kRingCompute = 8, kRingLoaders = 4;
 
 
-// GROUPED (launch_ring_group): unit = (W panel, tile of a list), the tiles' number is only known on the device
-__device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const RingGroup& gr, int T, int u, int& matrix, int& places) {
+// GROUPED (launch_ring_group): unit = (W panel, tile of a list), the tiles' number is only known on the device.  All panels of two tiles (an expert's, mostly) come one after the other: the
+// panels on an XCD then read the same rows of A at the same time, which are 1.2 GB of half lines a layer out of L2 or from behind it, and those of 16 experts do not fit beside the weights
+// that stream.  us for both products of 32 experts, 4 a token, 4096 x 1536, panel by panel over all tiles / so: 400 tokens 303 / 290, 700 353 / 330, 1024 420 / 392, 2048 650 / 608; one
+// tile instead of two 289, 333, 395, 618, four 298, 338, 402, 613.
+constexpr int kRingGroupTiles = 2;
+__device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const RingGroup& gr, int T, int P, int u, int& matrix, int& places) {
   RingUnit r;
-  const int mt = u % T;
-  const int32_t* t = gr.tiles + (size_t)mt * 4;
+  const int first = u / (kRingGroupTiles * P) * kRingGroupTiles, at = u - first * P, n = T - first < kRingGroupTiles ? T - first : kRingGroupTiles;
+  const int32_t* t = gr.tiles + (size_t)(first + at % n) * 4;
   matrix = t[0];
   r.m0 = t[1];
   places = t[2];
-  r.panel = u / T;
+  r.panel = at / n;
   r.split = 0;
   r.f = (places + 15) >> 4;
   r.f0 = (r.f + 1) >> 1;
@@ -77,7 +81,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     g.units = g.T * g.P;
   }
   auto unit = [&](int u, int& matrix, int& places) __attribute__((always_inline)) {
-    if constexpr (GROUPED) return ring_group_unit(p, gr, g.T, u, matrix, places);
+    if constexpr (GROUPED) return ring_group_unit(p, gr, g.T, g.P, u, matrix, places);
     else return ring_unit(p, g, u);
   };
   const int share = g.units >> 3, rem = g.units & 7;
