@@ -300,6 +300,8 @@ SIGNATURES = {
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "chatts_ts_encode_tiled": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, C.POINTER(TsWeights), C.POINTER(c_void_p), c_void_p,
                                  c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "chatts_ts_encode_known": (c_int, [c_void_p, C.POINTER(C.c_int32), c_int, c_int, c_void_p, c_void_p, c_void_p, C.POINTER(TsWeights), C.POINTER(c_void_p), c_void_p, c_void_p,
+                                 c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "chatts_linear_workspace": (c_size_t, [c_int, c_int, c_int]),
     "chatts_linear_workspace_batch": (c_size_t, [c_int, c_int, c_int, c_int]),
     "chatts_linear_chain": (c_int, [c_void_p, c_void_p, c_void_p]),

@@ -235,9 +235,18 @@ __device__ __forceinline__ void ts_feature8(const ChattsPatchifyArgs& a, unsigne
 
 constexpr int kL0Waves = 4, kL0Cols = 32;      // waves (16 rows each) of a workgroup, columns of a step
 
+// Lengths that the host knows, for the first layer itself: no launch before it writes them and no wave waits for them (2.3 us of device and 4 of host time a call).  Up to kL0Known series;
+// places behind the last one hold offsets that no row reaches.
+constexpr int kL0Known = 64;
+struct TsKnown {
+  int32_t off[kL0Known], len[kL0Known];
+  int32_t n;               // 0: row_off and valid_len on the device
+  int64_t* patch_cnt;      // counts from the masks, by workgroups of their own (the last of grid.y), or NULL
+};
+
 template <int KSTEPS, int MODE>      // K-steps of 32 (feature count rounded up) and the feature mode: compiled in, so that every load is in flight at once
 __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatchifyArgs a, unsigned emb8_inv, const uint16_t* w0, int ldw, const float* b0, int hidden, int steps_each,
-                                                                     uint16_t* out_hi, uint16_t* out_lo, int ld_out, int tiled) {
+                                                                     uint16_t* out_hi, uint16_t* out_lo, int ld_out, int tiled, TsKnown known) {
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
   // W0 of a step: 32 rows of 4 KSTEPS 16-byte chunks, twice.  Chunk c of a K-step of row r lies at place c ^ (r >> turn): eight rows' chunks then meet
   // different banks whatever KSTEPS makes of the row's length
@@ -245,6 +254,10 @@ __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatch
   __shared__ __attribute__((aligned(1024))) char smem[2][PIECES * 1024];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r0 = ((int)blockIdx.y * kL0Waves + wave) * 16;
+  if ((int)blockIdx.y * kL0Waves * 16 >= a.total_patches) {    // (a whole workgroup)
+    for (int i = (int)blockIdx.x * kL0Waves + wave; i < known.n; i += (int)gridDim.x * kL0Waves) ts_count_series(a.series, i, a.lmax, a.patch_size, lane, nullptr, known.patch_cnt);
+    return;
+  }
   const bool mine = r0 < a.total_patches;                      // (else a wave that only fetches W0)
   const int frow = lane & 15, kc = lane >> 4;                  // this lane's row of a 16-row block, and its 8 K-values of a 32-deep step
   int n0 = (int)blockIdx.x * steps_each * kL0Cols;
@@ -259,16 +272,27 @@ __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatch
       __builtin_amdgcn_global_load_lds((gptr_t)(w0 + (size_t)row * ldw + ((x & ~3) | ((x & 3) ^ ((r >> TURN) & 3))) * 8), (lptr_t)(smem[b] + piece * 1024), 16, 0, 0);
     }
   };
-  // the patch row this lane feeds, clamped to the last real row (stores are masked).  Its series: up to 63 series - lane i holds
+  // the patch row this lane feeds, clamped to the last real row (stores are masked).  Its series: of lengths by value, the last that begins at or before the row (scalar
+  // loads, 16 series at a time); up to 63 series - lane i holds
   // row_off[i] / valid_len[i] (ONE round trip), the search is a wave-uniform walk over lanes and two ds_bpermute; more series - the
   // binary search of ts_patchify_kernel (log2 N dependent round trips)
   const int nser = a.n_series;
-  const int my_off = a.row_off[lane <= nser ? lane : nser];
-  const int my_vl = a.valid_len[lane < nser ? lane : nser - 1];
   int p = r0 + frow;
   if (p > a.total_patches - 1) p = a.total_patches - 1;
   int sidx = 0, off = 0, vl = 0;
-  if (nser <= 63) {
+  if (known.n) {
+    for (int i0 = 0; i0 < known.n; i0 += 16)
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int o = known.off[i0 + u], l = known.len[i0 + u];
+        const bool at = o <= p;
+        sidx = at ? i0 + u : sidx;
+        off = at ? o : off;
+        vl = at ? l : vl;
+      }
+  } else if (nser <= 63) {
+    const int my_off = a.row_off[lane <= nser ? lane : nser];
+    const int my_vl = a.valid_len[lane < nser ? lane : nser - 1];
     for (int i = 1; i < nser; ++i) sidx += __builtin_amdgcn_readlane(my_off, i) <= p ? 1 : 0;
     off = __shfl(my_off, sidx, 64);
     vl = __shfl(my_vl, sidx, 64);
@@ -443,9 +467,10 @@ extern "C" int chatts_ts_patchify(const ChattsPatchifyArgs* a, chatts_stream_t s
 
 // Whole encoder in one call (the C-ABI SURVEY.md section 8b proposes for a3 + a4): patchify, then the MLP
 // (Linear + exact-erf GELU) x (n-1) + Linear, ping-ponging between two caller-owned [P, H] buffers.
-extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_off, const int32_t* valid_len, int n_series, int lmax,
-                                int max_valid_len, int total_patches, const ChattsTsWeights* w, const chatts_bf16* const* w_tiled, float* feat, float* h0,
-                                float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream) {
+// lengths: the same on the host, or NULL.  Then row_off and valid_len are written by chatts_ts_lengths where the first layer does not take them as arguments, and patch_cnt by one of the two.
+static int ts_encode(const float* series, const int32_t* lengths, int32_t* row_off, int32_t* valid_len, int64_t* patch_cnt, int n_series, int lmax,
+                     int max_valid_len, int total_patches, const ChattsTsWeights* w, const chatts_bf16* const* w_tiled, float* feat, float* h0,
+                     float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream) {
   CHATTS_REQUIRE(w != nullptr && w->num_layers >= 1 && w->num_layers <= 8, CHATTS_E_BADARG, "ts_encode: bad weights");
   if (total_patches == 0) return CHATTS_OK;
   StageRange stage("chatts.ts_encode");
@@ -480,8 +505,21 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
   const int feat_n = w->mode == 1 ? w->patch_size * (1 + w->emb_dim) : (w->mode == 2 ? 2 * w->patch_size : w->patch_size);
   const int ksteps = (feat_n + 31) / 32;
   const bool l0_shape = w->mode == 1 ? (w->patch_size % 8 == 0 && w->emb_dim % 8 == 0 && ksteps <= 10) : (w->patch_size % 8 == 0 && ksteps <= 2);
-  if (planes && w->num_layers >= 2 && H % 16 == 0 && ksteps >= 1 && l0_shape && ksteps * 32 <= w->in_features_pad && h0 &&
-      ((uintptr_t)w->w[0] % 16) == 0 && ((uintptr_t)w->b[0] % 16) == 0 && ((uintptr_t)w->pos_table % 16) == 0 && opt_get(OPT_TS_L0_FUSED, 1) != 0) {
+  const bool fused = planes && w->num_layers >= 2 && H % 16 == 0 && ksteps >= 1 && l0_shape && ksteps * 32 <= w->in_features_pad && h0 &&
+      ((uintptr_t)w->w[0] % 16) == 0 && ((uintptr_t)w->b[0] % 16) == 0 && ((uintptr_t)w->pos_table % 16) == 0 && opt_get(OPT_TS_L0_FUSED, 1) != 0;
+  TsKnown known{};
+  if (lengths) {
+    if (fused && n_series <= kL0Known && series) {
+      known.n = n_series; known.patch_cnt = patch_cnt;
+      for (int i = 0, at = 0; i < kL0Known; ++i) {
+        known.off[i] = i < n_series ? at : 0x7fffffff;
+        if (i < n_series) { known.len[i] = lengths[i]; at += (lengths[i] + w->patch_size - 1) / w->patch_size; }
+      }
+    } else if ((rc = chatts_ts_lengths(lengths, n_series, w->patch_size, valid_len, row_off, series, lmax, patch_cnt, stream)) != 0) {
+      return rc;
+    }
+  }
+  if (fused) {
     CHATTS_REQUIRE(pa.series && pa.row_off && pa.valid_len && (w->mode != 1 || (pa.pos_table && w->emb_dim > 0 && w->max_seq_len > 0)), CHATTS_E_BADARG,
                    "ts_encode: null series / offsets / position table");
     // four row blocks a workgroup; the columns in as many parts as three workgroups per CU ask for
@@ -490,10 +528,10 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
     parts = parts < 1 ? 1 : (parts > steps ? steps : parts);
     const int steps_each = (steps + parts - 1) / parts, emb8 = w->mode == 1 ? w->emb_dim / 8 : 1;
     const unsigned emb8_inv = emb8 > 1 ? (unsigned)((0x100000000ull + emb8 - 1) / emb8) : 0u;      // (exact for the at most 40 groups of a row)
-    const dim3 grid((steps + steps_each - 1) / steps_each, groups), block(64 * kL0Waves);
+    const dim3 grid((steps + steps_each - 1) / steps_each, groups + (known.n && known.patch_cnt ? 1 : 0)), block(64 * kL0Waves);
     uint16_t* oh = hi_of(h0);
     uint16_t* ol = lo_of(h0, H);
-#define CHATTS_TS_L0(KS, MD) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD>), grid, block, 0, as_stream(stream), pa, emb8_inv, w->w[0], w->in_features_pad, w->b[0], H, steps_each, oh, ol, H, tile ? P & ~15 : 0)
+#define CHATTS_TS_L0(KS, MD) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD>), grid, block, 0, as_stream(stream), pa, emb8_inv, w->w[0], w->in_features_pad, w->b[0], H, steps_each, oh, ol, H, tile ? P & ~15 : 0, known)
     if (w->mode == 1) {
       switch (ksteps) {
         case 1: CHATTS_TS_L0(1, 1); break;
@@ -540,6 +578,24 @@ extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_of
     k = H;
   }
   return CHATTS_OK;
+}
+extern "C" int chatts_ts_encode_tiled(const float* series, const int32_t* row_off, const int32_t* valid_len, int n_series, int lmax,
+                                int max_valid_len, int total_patches, const ChattsTsWeights* w, const chatts_bf16* const* w_tiled, float* feat, float* h0,
+                                float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream) {
+  return ts_encode(series, nullptr, const_cast<int32_t*>(row_off), const_cast<int32_t*>(valid_len), nullptr, n_series, lmax, max_valid_len, total_patches, w, w_tiled, feat, h0, h1, out,
+                   workspace, workspace_bytes, stream);
+}
+extern "C" int chatts_ts_encode_known(const float* series, const int32_t* lengths, int n_series, int lmax, int32_t* valid_len, int32_t* row_off, int64_t* patch_cnt, const ChattsTsWeights* w,
+                                      const chatts_bf16* const* w_tiled, float* feat, float* h0, float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream) {
+  CHATTS_REQUIRE(w && lengths && valid_len && row_off && n_series >= 0 && lmax >= 0 && w->patch_size > 0, CHATTS_E_BADARG, "ts_encode_known: bad arguments");
+  int total = 0, longest = 0;
+  for (int i = 0; i < n_series; ++i) {
+    CHATTS_REQUIRE(lengths[i] >= 0 && lengths[i] <= lmax, CHATTS_E_BADARG, "ts_encode_known: series %d of %d steps in rows of %d", i, lengths[i], lmax);
+    total += (lengths[i] + w->patch_size - 1) / w->patch_size;
+    if (lengths[i] > longest) longest = lengths[i];
+  }
+  if (total == 0) return chatts_ts_lengths(lengths, n_series, w->patch_size, valid_len, row_off, series, lmax, patch_cnt, stream);
+  return ts_encode(series, lengths, row_off, valid_len, patch_cnt, n_series, lmax, longest, total, w, w_tiled, feat, h0, h1, out, workspace, workspace_bytes, stream);
 }
 extern "C" int chatts_ts_encode(const float* series, const int32_t* row_off, const int32_t* valid_len, int n_series, int lmax, int max_valid_len, int total_patches, const ChattsTsWeights* w,
                                 float* feat, float* h0, float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream) {

@@ -236,11 +236,14 @@ class TimeSeriesEmbedding:
         if any(v > self.max_sequence_length for v in vl_host) and self.mode == 1:
             raise IndexError("index out of range in self")     # nn.Embedding lookup, chatts_vllm.py:165
         P = sum((v + ps - 1) // ps for v in vl_host)
-        if host_given:                               # offsets and lengths go to the device as kernel arguments; the counts from the masks are formed in the same launch
-            _lib.check(lib.chatts_ts_lengths((_lib.C.c_int32 * n)(*vl_host), n, ps, _lib.ptr(vl_dev), _lib.ptr(row_off_dev), _lib.ptr(x), lmax, _lib.ptr(pc_dev), _lib.stream_ptr()))
+        known = (_lib.C.c_int32 * n)(*vl_host) if host_given else None
+        if host_given and (P == 0 or self.precision == "fp8"):
+            _lib.check(lib.chatts_ts_lengths(known, n, ps, _lib.ptr(vl_dev), _lib.ptr(row_off_dev), _lib.ptr(x), lmax, _lib.ptr(pc_dev), _lib.stream_ptr()))
+            known = None
         if P == 0:
             return torch.empty((0, self.hidden_size), dtype=torch.float32, device=dev), pc_dev
-        # one C call: patchify + the whole MLP (chatts_ts_encode_tiled); buffers are cached per patch count
+        # one C call: patchify + the whole MLP (chatts_ts_encode_known, which takes lengths from the host and forms the counts from the masks beside the first layer, or
+        # chatts_ts_encode_tiled); buffers are cached per patch count
         key = (P, dev)
         if getattr(self, "_buf_key", None) != key:
             H = self.hidden_size
@@ -265,6 +268,7 @@ class TimeSeriesEmbedding:
         B = self._bufs
         out = torch.empty((P, self.hidden_size), dtype=torch.float32, device=dev)
         self._last = (x, row_off_dev, vl_dev, n, lmax, max(vl_host) if vl_host else 0, P, out)
+        self._last_known = (known, pc_dev)
         self.replay_last()
         return out, pc_dev
 
@@ -276,6 +280,11 @@ class TimeSeriesEmbedding:
             return self._replay_fp8()
         lib, B = _lib.load(), self._bufs
         x, row_off_dev, vl_dev, n, lmax, maxvl, P, out = self._last
+        known, pc_dev = self._last_known
+        if known is not None:
+            _lib.check(lib.chatts_ts_encode_known(_lib.ptr(x), known, n, lmax, _lib.ptr(vl_dev), _lib.ptr(row_off_dev), _lib.ptr(pc_dev), C.byref(self._tsw), self._tsw_tiled,
+                                                  _lib.ptr(B["feat"]), _lib.ptr(B["h0"]), _lib.ptr(B["h1"]), _lib.ptr(out), _lib.ptr(B["ws"]), B["ws_bytes"], _lib.stream_ptr()))
+            return out
         _lib.check(lib.chatts_ts_encode_tiled(_lib.ptr(x), _lib.ptr(row_off_dev), _lib.ptr(vl_dev), n, lmax, maxvl, P,
                                               C.byref(self._tsw), self._tsw_tiled, _lib.ptr(B["feat"]), _lib.ptr(B["h0"]), _lib.ptr(B["h1"]),
                                               _lib.ptr(out), _lib.ptr(B["ws"]), B["ws_bytes"], _lib.stream_ptr()))

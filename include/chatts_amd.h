@@ -157,6 +157,10 @@ int chatts_ts_encode(const float* series, const int32_t* row_off, const int32_t*
 int chatts_ts_encode_tiled(const float* series, const int32_t* row_off, const int32_t* valid_len, int n_series, int lmax,
                            int max_valid_len, int total_patches, const ChattsTsWeights* weights, const chatts_bf16* const* w_tiled, float* feat, float* h0,
                            float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream);
+/* ... of lengths that the host knows (host array): chatts_ts_lengths and chatts_ts_encode_tiled in one call, and for up to 64 series in one launch less.  valid_len [n_series] and
+ * row_off [n_series + 1] are scratch on the device; patch_cnt [n_series], the counts from the masks, may be NULL.  out and the scratch hold sum(ceil(length / patch_size)) rows. */
+int chatts_ts_encode_known(const float* series, const int32_t* lengths, int n_series, int lmax, int32_t* valid_len, int32_t* row_off, int64_t* patch_cnt, const ChattsTsWeights* weights,
+                           const chatts_bf16* const* w_tiled, float* feat, float* h0, float* h1, float* out, void* workspace, size_t workspace_bytes, chatts_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Linear layers:  C[M,N] = epilogue(A[M,K] . W[N,K]^T)   A,C float32, W bfloat16 row-major [N,K]
