@@ -161,6 +161,17 @@ int launch_cols(const GemmParams& p, const ChattsLinearArgs* a, hipStream_t s);
 // chatts_rmsnorm_planes on rows that lie ldx apart (elementwise.hip)
 int launch_rmsnorm_planes(const float* x, int ldx, const float* w, uint16_t* hi, uint16_t* lo, int ld_planes, int t, int hidden, float eps, int tiled, hipStream_t s);
 
+// moe.hip: a feed-forward of the experts' kind beside them, for all rows, in their launches (up to 16 rows): up as gate_up of an expert, f = its activations [rows, ff], y [rows, width_p]
+struct MoeBeside {
+  const chatts_bf16 *up, *up_t, *down, *down_t;
+  int ff;
+  chatts_bf16 *f_hi, *f_lo;
+  float* y;
+  float limit, alpha;      // CHATTS_EXPERT_CLAMPGLU
+};
+bool moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh);
+int moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, chatts_stream_t stream);
+
 typedef const __attribute__((address_space(1))) void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
 

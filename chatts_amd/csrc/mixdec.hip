@@ -409,6 +409,16 @@ static ChattsMoeArgs mix_moe_args(const ChattsMixDecoder* d, const ChattsMixLaye
   return a;
 }
 
+// the feed-forward beside the experts, as their launches take it (the experts' kind of activation; into y)
+static MoeBeside mix_beside(const ChattsMixDecoder* d, const ChattsMixLayer& l, int kind) {
+  MoeBeside b{};
+  if (!l.up || l.moe.act_kind != kind) return b;
+  b.up = l.up; b.up_t = l.up_t; b.down = l.down; b.down_t = l.down_t; b.ff = l.ff;
+  b.f_hi = d->b.b_hi; b.f_lo = d->b.b_lo; b.y = d->b.y;
+  b.limit = l.glu_limit; b.alpha = l.glu_alpha;
+  return b;
+}
+
 // x += what the experts of `moe` owe it; then the norms of `next` (or its joined input)
 static int mix_pair_norm(const ChattsMixDecoder* d, int t, const ChattsMixLayer* moe, const float* w1, const float* w2, const ChattsOperand& out1, const ChattsOperand& out2,
                          bool join, const ChattsMixLayer* shift, float* prev, chatts_stream_t s) {
@@ -534,17 +544,20 @@ static int mix_post_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, c
     X = stream_operand(d, t, moe);
     if ((rc = mix_post_norm(d, t, d->b.y, nullptr, l.norm1, X, s)) != 0) return rc;
     if (l.ff_kind == CHATTS_FF_NONE) continue;
-    if (l.up) {
-      const ChattsOperand F = operand(d, true, t, l.ff);
-      if ((rc = mix_linear(d, linear_form(X), l.up, l.up_t, t, moe ? l.ff : 2 * l.ff, wp, moe ? CHATTS_EPI_RELU2 : CHATTS_EPI_GEGLU, F, s)) != 0) return rc;
-      if ((rc = mix_linear(d, F, l.down, l.down_t, t, wp, l.ff, CHATTS_EPI_NONE, Y, s)) != 0) return rc;
-    }
+    bool beside = false;
     if (moe) {
       StageRange stage("chatts.mix.experts");
       if ((rc = mix_linear(d, linear_form(X), l.router, l.router_t, t, l.router_n, wp, CHATTS_EPI_NONE, f32_out(d->b.moe_logits, l.router_n), s)) != 0) return rc;
       const ChattsMoeArgs m = mix_moe_args(d, l, t, X);
       if ((rc = chatts_moe_route(&m, s)) != 0) return rc;
-      if ((rc = chatts_moe_experts(&m, s)) != 0) return rc;
+      const MoeBeside sh = mix_beside(d, l, CHATTS_EXPERT_RELU2);
+      beside = moe_takes_beside(&m, sh);
+      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, s)) != 0) return rc;
+    }
+    if (l.up && !beside) {
+      const ChattsOperand F = operand(d, true, t, l.ff);
+      if ((rc = mix_linear(d, linear_form(X), l.up, l.up_t, t, moe ? l.ff : 2 * l.ff, wp, moe ? CHATTS_EPI_RELU2 : CHATTS_EPI_GEGLU, F, s)) != 0) return rc;
+      if ((rc = mix_linear(d, F, l.down, l.down_t, t, wp, l.ff, CHATTS_EPI_NONE, Y, s)) != 0) return rc;
     }
     X = stream_operand(d, t, false);
     if ((rc = mix_post_norm(d, t, l.up ? d->b.y : nullptr, moe ? &l : nullptr, l.norm2, X, s)) != 0) return rc;
@@ -646,14 +659,17 @@ static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, co
     }
     const ChattsOperand N = second_norm(d, l, t);
     if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s)) != 0) return rc;
+    bool beside = false;
     if (moe) {
       StageRange stage("chatts.mix.experts");
       if ((rc = mix_linear(d, linear_form(N), l.router, l.router_t, t, l.router_n, wp, CHATTS_EPI_NONE, f32_out(d->b.moe_logits, l.router_n), s)) != 0) return rc;
       const ChattsMoeArgs m = mix_moe_args(d, l, t, N);
       if ((rc = chatts_moe_route(&m, s)) != 0) return rc;
-      if ((rc = chatts_moe_experts(&m, s)) != 0) return rc;
+      const MoeBeside sh = mix_beside(d, l, CHATTS_EXPERT_CLAMPGLU);
+      beside = moe_takes_beside(&m, sh);
+      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, s)) != 0) return rc;
     }
-    if (l.up) {
+    if (l.up && !beside) {
       const ChattsOperand F = operand(d, true, t, l.ff);
       if ((rc = mix_linear(d, linear_form(N), l.up, l.up_t, t, 2 * l.ff, wp, CHATTS_EPI_CLAMPGLU, F, s, l.glu_limit, l.glu_alpha)) != 0) return rc;
       if ((rc = mix_linear(d, F, l.down, l.down_t, t, wp, l.ff, CHATTS_EPI_NONE, Y, s)) != 0) return rc;

@@ -327,24 +327,36 @@ __device__ __forceinline__ void moe_relu2_4(const ChattsOperand& o, size_t row, 
   store_operand4(o, row, col, v);
 }
 
-// ---- up to 16 rows: grid (blocks of 16 RF weight rows, tiles), NW waves split K; D = W . A^T: a lane holds 4 consecutive outputs of one token.
-// pairs (RF = 2): the two 16-row halves of a block are gate and up rows of the same outputs ----
+// ---- up to 16 rows: a workgroup has 16 RF weight rows of a tile, NW waves split K; D = W . A^T: a lane holds 4 consecutive outputs of one token.
+// pairs (RF = 2): the two 16-row halves of a block are gate and up rows of the same outputs.
+// The first sh_blocks workgroups stream the feed-forward beside the experts for all rows, nx ones a tile follow: as products of their own it took two launches for its weights and two for
+// their splits' sums (21 us a layer of 16 rows, 2048 x 3072 beside 32 experts of 768; here 7) ----
 // TILED: weights from the chatts_tile_bf16 copy: a fragment's 64 pieces are 1 KB of consecutive memory
 template <int STEP, bool TILED, int NW, int RF>
-__global__ __launch_bounds__(64 * NW) void moe_stream_kernel(ChattsMoeArgs p) {
+__global__ __launch_bounds__(64 * NW) void moe_stream_kernel(ChattsMoeArgs p, MoeBeside sh, int sh_blocks, int nx) {
   __shared__ f32x4 red[NW][RF][64];
   static_assert(!moe_pairs(STEP) || RF == 2, "a pair of fragments");
   constexpr bool IN = STEP != kDown;
-  const int32_t* tile = p.tiles + (size_t)blockIdx.y * 4;
-  const int e = tile[0];
-  if (e < 0) return;
-  const int place0 = tile[1], count = tile[2], lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fg = lane >> 4;
-  const int K = IN ? p.width_p : p.ff_p, N = IN ? moe_in_rows(p) : p.width_p, n0 = blockIdx.x * 16 * RF;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fg = lane >> 4;
+  int e = 0, place0 = 0, count = p.n_rows, n0 = (int)blockIdx.x * 16 * RF;
+  const bool beside = (int)blockIdx.x < sh_blocks;
+  if (beside) {      // (from here on an expert of its own, whose list is the rows)
+    p.gate_up = sh.up; p.gate_up_t = sh.up_t; p.down = sh.down; p.down_t = sh.down_t; p.ff_p = sh.ff;
+    p.act.hi = sh.f_hi; p.act.lo = sh.f_lo; p.act.ld = sh.ff; p.y = sh.y; p.glu_limit = sh.limit; p.glu_alpha = sh.alpha;
+  } else {
+    const int at = (int)blockIdx.x - sh_blocks;
+    const int32_t* tile = p.tiles + (size_t)(at / nx) * 4;
+    n0 = at % nx * 16 * RF;
+    e = tile[0];
+    if (e < 0) return;
+    place0 = tile[1]; count = tile[2];
+  }
+  const int K = IN ? p.width_p : p.ff_p, N = IN ? moe_in_rows(p) : p.width_p;
   const uint16_t* w = TILED ? (IN ? p.gate_up_t : p.down_t) + ((size_t)e * N + n0) * K + (fr * 4 + (fg ^ ((fr >> 3) << 1))) * 8
                             : (IN ? p.gate_up : p.down) + ((size_t)e * N + n0 + fr) * K + fg * 8;
   constexpr int kStep = TILED ? 16 : 1;      // elements of w per K-value
   const int pl = place0 + (fr < count ? fr : 0);
-  const size_t arow = IN ? (size_t)(p.order[pl] / p.top) * p.h.ld : (size_t)pl * p.act.ld;
+  const size_t arow = IN ? (size_t)(beside ? pl : p.order[pl] / p.top) * p.h.ld : (size_t)pl * p.act.ld;
   const uint16_t* ah = (IN ? p.h.hi : p.act.hi) + arow + fg * 8;
   const uint16_t* al = (IN ? p.h.lo : p.act.lo) + arow + fg * 8;
   f32x4 acc[RF];
@@ -592,17 +604,18 @@ static int moe_tile_bound(int rows, int top, int experts, int bm) {      // sum 
 }
 
 template <int STEP, int RF>
-static void launch_moe_stream_as(const ChattsMoeArgs* a, int n, int tiles, hipStream_t s) {
+static void launch_moe_stream_as(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {
   constexpr int NW = moe_pairs(STEP) ? 4 : 16;
-  const dim3 g(n / (16 * RF), tiles), b(64 * NW);
-  if (STEP == kDown ? a->down_t : a->gate_up_t) hipLaunchKernelGGL((moe_stream_kernel<STEP, true, NW, RF>), g, b, 0, s, *a);
-  else hipLaunchKernelGGL((moe_stream_kernel<STEP, false, NW, RF>), g, b, 0, s, *a);
+  const int sh_n = !sh.up ? 0 : STEP == kDown ? a->width_p : moe_pairs(STEP) ? 2 * sh.ff : sh.ff, sh_blocks = sh_n / (16 * RF), nx = n / (16 * RF);
+  const dim3 g(sh_blocks + nx * tiles), b(64 * NW);
+  if (STEP == kDown ? a->down_t : a->gate_up_t) hipLaunchKernelGGL((moe_stream_kernel<STEP, true, NW, RF>), g, b, 0, s, *a, sh, sh_blocks, nx);
+  else hipLaunchKernelGGL((moe_stream_kernel<STEP, false, NW, RF>), g, b, 0, s, *a, sh, sh_blocks, nx);
 }
 template <int STEP>
-static void launch_moe_stream(const ChattsMoeArgs* a, int n, int tiles, hipStream_t s) {      // few workgroups: smaller ones, so that the CUs get as much each
+static void launch_moe_stream(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {      // few workgroups: smaller ones, so that the CUs get as much each
   if constexpr (!moe_pairs(STEP))
-    if (n / 32 * tiles < 2 * device_cus()) return launch_moe_stream_as<STEP, 1>(a, n, tiles, s);
-  launch_moe_stream_as<STEP, 2>(a, n, tiles, s);
+    if (n / 32 * tiles < 2 * device_cus()) return launch_moe_stream_as<STEP, 1>(a, sh, n, tiles, s);
+  launch_moe_stream_as<STEP, 2>(a, sh, n, tiles, s);
 }
 
 template <int STEP, int BM, int WM, int WN>
@@ -644,10 +657,15 @@ extern "C" int chatts_moe_route(const ChattsMoeArgs* a, chatts_stream_t stream) 
   return CHATTS_OK;
 }
 
-extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream) {
+bool chatts::moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh) {
+  return moe_small(a) && sh.up && sh.down && sh.f_hi && sh.f_lo && sh.y && sh.ff % 64 == 0 && a->width_p % 64 == 0 && !sh.up_t == !a->gate_up_t && !sh.down_t == !a->down_t;
+}
+extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream) { return moe_experts(a, MoeBeside{}, stream); }
+int chatts::moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, chatts_stream_t stream) {
   if (const int rc = check_moe(a, "moe_experts")) return rc;
   CHATTS_REQUIRE(a->gate_up && a->down && a->y && (a->exact ? a->h.f32 && a->act.f32 : a->h.hi && a->h.lo && a->act.hi && a->act.lo) && a->h.ld >= a->width_p &&
                      a->act.ld >= a->ff_p && a->h.ld % 8 == 0 && a->act.ld % 8 == 0, CHATTS_E_BADARG, "moe_experts: operands");
+  CHATTS_REQUIRE(!sh.up || moe_takes_beside(a, sh), CHATTS_E_SHAPE, "moe_experts: a feed-forward of %d beside experts of %d rows", sh.ff, a->n_rows);
   if (a->n_rows == 0) return CHATTS_OK;
   hipStream_t s = as_stream(stream);
   const int bm = moe_bm(a), tiles = moe_tile_bound(a->n_rows, a->top, a->experts, bm), in_rows = moe_in_rows(*a);
@@ -661,10 +679,10 @@ extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream
     return CHATTS_OK;
   }
   if (moe_small(a)) {
-    if (relu2) launch_moe_stream<kRelu2>(a, in_rows, tiles, s);
-    else if (clamped) launch_moe_stream<kClamped>(a, in_rows, tiles, s);
-    else launch_moe_stream<kGated>(a, in_rows, tiles, s);
-    launch_moe_stream<kDown>(a, a->width_p, tiles, s);
+    if (relu2) launch_moe_stream<kRelu2>(a, sh, in_rows, tiles, s);
+    else if (clamped) launch_moe_stream<kClamped>(a, sh, in_rows, tiles, s);
+    else launch_moe_stream<kGated>(a, sh, in_rows, tiles, s);
+    launch_moe_stream<kDown>(a, sh, a->width_p, tiles, s);
     CHATTS_CHECK_LAUNCH("moe_stream");
     return CHATTS_OK;
   }
