@@ -1,16 +1,42 @@
 // depth.hip - the residual stream of layers with norms before their sublayers only: a sublayer's share (its output, the experts' weighted sum) enters x
 // with a factor, the streams of all earlier layers are averaged, and the next norm's operand leaves in the same launch, a workgroup per row.
 // Also the cap of the logits.
-#include "common.h"
+#include "gemm_common.h"
+#include "moe_route.h"
 
 namespace chatts {
 
+// The router behind the norm: logits of NR x 16 outputs and the row's choice.  w: [16 NR][ldx], row-major (step 1) or chatts_tile_bf16's copy of it (step 16: a K-step is 1 KB further)
+struct DepthChoose {
+  const uint16_t* w;
+  int step;
+  ChattsMoeArgs moe;
+};
+
 // a thread keeps its columns in registers.  NT: threads (more of them for a few rows: then every load of a row is in flight at once)
-template <int NT, int NV>
-__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p) {
+// NR > 0 (few rows): the same launch multiplies the row by the router, as the planes that it writes, and chooses its experts.  A projection, its split's epilogue and a workgroup that chose
+// for all rows and made lists of them were three launches: 12.5 us a layer of 32 experts at 16 rows of 2048, now 1.  The router's first K-steps are requested before the row is there.
+template <int NT, int NV, int NR = 0>
+__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch) {
   __shared__ float red[NT / 64];
+  constexpr int NW = NT / 64, NX = NV * NT * 4;
+  __shared__ __attribute__((aligned(16))) uint16_t xh[NR ? NX : 1], xl[NR ? NX : 1];
+  __shared__ __attribute__((aligned(16))) float part[NR ? NW : 1][NR ? NR * 16 : 1];
   const size_t row = blockIdx.x;
   const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4, steps = p.ldx >> 5;
+  const uint16_t* rw = NR ? ch.w + (ch.step == 1 ? (size_t)fr * p.ldx + fg * 8 : (size_t)(fr * 4 + (fg ^ ((fr >> 3) << 1))) * 8) : nullptr;
+  constexpr int RU = 4;      // K-steps of a wave requested at once: wave, wave + NW, ..
+  bf16x8_t wf[NR ? RU : 1][NR ? NR : 1];
+  auto request = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int s = s0 + u * NW < steps ? s0 + u * NW : wave < steps ? wave : 0;
+#pragma unroll
+      for (int f = 0; f < NR; ++f) wf[u][f] = *reinterpret_cast<const bf16x8_t*>(rw + (size_t)f * 16 * p.ldx + (size_t)s * 32 * ch.step);
+    }
+  };
+  if constexpr (NR > 0) request(wave);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   constexpr int U = NV <= 2 ? 4 : 2;      // rows requested at once
   f32x4 x[NV], add[NV];
@@ -108,6 +134,42 @@ __global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = c + k < p.width ? x[i][k] * inv * w[i][k] : 0.f;
     store_operand4(p.out, row, c, v);
+    if constexpr (NR > 0) {
+      ChattsOperand own{};
+      own.hi = xh; own.lo = xl;
+      store_operand4(own, 0, c, v);
+    }
+  }
+  if constexpr (NR > 0) {
+    __syncthreads();
+    f32x4 acc[NR];
+#pragma unroll
+    for (int f = 0; f < NR; ++f) acc[f] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int s0 = wave; s0 < steps; s0 += RU * NW) {
+      if (s0 != wave) request(s0);
+#pragma unroll
+      for (int u = 0; u < RU; ++u) {
+        const int s = s0 + u * NW;
+        if (s >= steps) break;      // (uniform)
+        const bf16x8_t h = *reinterpret_cast<const bf16x8_t*>(xh + s * 32 + fg * 8), l = *reinterpret_cast<const bf16x8_t*>(xl + s * 32 + fg * 8);      // (the row in every column)
+#pragma unroll
+        for (int f = 0; f < NR; ++f) {
+          acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][f], l, acc[f], 0, 0, 0);
+          acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][f], h, acc[f], 0, 0, 0);
+        }
+      }
+    }
+    if (fr == 0)
+#pragma unroll
+      for (int f = 0; f < NR; ++f) *reinterpret_cast<f32x4*>(&part[wave][f * 16 + fg * 4]) = acc[f];
+    __syncthreads();
+    if (wave) return;
+    float z = 0.f;
+    if (lane < NR * 16)
+#pragma unroll
+      for (int i = 0; i < NW; ++i) z += part[i][lane];
+    const int id = moe_route_row64(ch.moe, (int)row, lane, z);
+    if (lane < ch.moe.top) ch.moe.place[row * ch.moe.top + lane] = id >= 0 ? (int)row * ch.moe.top + lane : -1;
   }
 }
 
@@ -128,7 +190,7 @@ __global__ __launch_bounds__(256) void soft_cap_kernel(float* __restrict__ x, in
 
 using namespace chatts;
 
-extern "C" int chatts_depth_norm(const ChattsDepthNormArgs* a, chatts_stream_t stream) {
+static int check_depth_norm(const ChattsDepthNormArgs* a) {
   CHATTS_REQUIRE(a && a->x && a->t >= 0 && a->width > 0, CHATTS_E_BADARG, "depth_norm: bad arguments");
   CHATTS_REQUIRE(a->ldx >= a->width && a->ldx % 4 == 0 && a->ldx <= 16384, CHATTS_E_SHAPE, "depth_norm: a width of %d in rows of %d (at most 16384)", a->width, a->ldx);
   CHATTS_REQUIRE(!a->ey || (a->place && a->weight && a->top > 0), CHATTS_E_BADARG, "depth_norm: experts");
@@ -137,17 +199,36 @@ extern "C" int chatts_depth_norm(const ChattsDepthNormArgs* a, chatts_stream_t s
   CHATTS_REQUIRE(!a->w || ((a->out.f32 || a->out.hi) && a->out.ld >= a->ldx && a->out.ld % 4 == 0), CHATTS_E_SHAPE, "depth_norm: operand rows of %d", a->out.ld);
   CHATTS_REQUIRE((((uintptr_t)a->x | (uintptr_t)a->y | (uintptr_t)a->ey | (uintptr_t)a->w | (uintptr_t)a->streams | (uintptr_t)a->out.f32) % 16) == 0 &&
                      (((uintptr_t)a->out.hi | (uintptr_t)a->out.lo) % 8) == 0, CHATTS_E_SHAPE, "depth_norm: pointers must be aligned (16 bytes, planes 8)");
+  return CHATTS_OK;
+}
+extern "C" int chatts_depth_norm(const ChattsDepthNormArgs* a, chatts_stream_t stream) {
+  if (const int rc = check_depth_norm(a)) return rc;
   if (a->t == 0) return CHATTS_OK;
+  const DepthChoose none{};
   const dim3 g(a->t);
   hipStream_t s = as_stream(stream);
-  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a);
-  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a);
-  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a);
-  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a);
-  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a);
-  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a);
-  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a);
+  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a, none);
+  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a, none);
+  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a, none);
+  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a, none);
+  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a, none);
+  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a, none);
+  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a, none);
   CHATTS_CHECK_LAUNCH("depth_norm");
+  return CHATTS_OK;
+}
+
+// ... and the choice of experts for rows that moe_takes_choice: ids, weight, place (a pair's own) and kept
+bool chatts::depth_norm_can_choose(int ldx) { return ldx % 64 == 0 && ldx <= 4096; }
+int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, chatts_stream_t stream) {
+  if (const int rc = check_depth_norm(a)) return rc;
+  CHATTS_REQUIRE(moe && router && a->w && a->out.hi && a->out.lo && depth_norm_can_choose(a->ldx) && moe_takes_choice(moe) && moe->n_rows == a->t && moe->ids && moe->place && moe->weight &&
+                     moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);
+  if (a->t == 0) return CHATTS_OK;
+  const DepthChoose ch{router_t ? router_t : router, router_t ? 16 : 1, *moe};
+  if (moe->experts + moe->identity <= 32) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch);
+  else hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 4>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch);
+  CHATTS_CHECK_LAUNCH("depth_norm_choose");
   return CHATTS_OK;
 }
 

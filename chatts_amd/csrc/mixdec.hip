@@ -552,7 +552,7 @@ static int mix_post_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, c
       if ((rc = chatts_moe_route(&m, s)) != 0) return rc;
       const MoeBeside sh = mix_beside(d, l, CHATTS_EXPERT_RELU2);
       beside = moe_takes_beside(&m, sh);
-      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, s)) != 0) return rc;
+      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, false, s)) != 0) return rc;
     }
     if (l.up && !beside) {
       const ChattsOperand F = operand(d, true, t, l.ff);
@@ -616,14 +616,15 @@ static int mix_one(const ChattsMixDecoder* d, const ChattsMixLayer& l, int kind,
 }
 
 // x += mult (y + what the experts of `moe` owe it), averaged over depth after the run number `stream` of a layer with such weights; then the next norm
+// choose: the experts for whose router the norm is (depth_norm_choose)
 static int mix_depth_norm(const ChattsMixDecoder* d, int t, const float* y, const ChattsMixLayer* moe, const float* depth, int stream, const float* w, const ChattsOperand& out,
-                          chatts_stream_t s) {
+                          chatts_stream_t s, const ChattsMoeArgs* choose = nullptr, const ChattsMixLayer* router = nullptr) {
   ChattsDepthNormArgs a{};
   a.x = d->b.x; a.t = t; a.width = d->c.width; a.ldx = d->c.width_p; a.mult = d->c.mult; a.eps = d->c.eps; a.y = y;
   if (moe) { a.ey = d->b.moe_y; a.place = d->b.moe_place; a.weight = d->b.moe_weight; a.top = moe->moe.top; }
   a.depth = depth; a.streams = d->b.streams; a.stream_stride = d->b.stream_stride; a.n_streams = stream + 1; a.keep = depth && stream + 1 < d->c.n_runs;
   a.w = w; a.out = out;
-  return chatts_depth_norm(&a, s);
+  return choose ? depth_norm_choose(&a, choose, router->router, router->router_t, s) : chatts_depth_norm(&a, s);
 }
 
 static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, const ChattsSpan* spans, int n_spans, bool single, chatts_stream_t s) {
@@ -658,16 +659,21 @@ static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, co
       continue;
     }
     const ChattsOperand N = second_norm(d, l, t);
-    if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s)) != 0) return rc;
     bool beside = false;
     if (moe) {
-      StageRange stage("chatts.mix.experts");
-      if ((rc = mix_linear(d, linear_form(N), l.router, l.router_t, t, l.router_n, wp, CHATTS_EPI_NONE, f32_out(d->b.moe_logits, l.router_n), s)) != 0) return rc;
       const ChattsMoeArgs m = mix_moe_args(d, l, t, N);
-      if ((rc = chatts_moe_route(&m, s)) != 0) return rc;
+      const bool choose = moe_takes_choice(&m) && depth_norm_can_choose(wp);
+      if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s, choose ? &m : nullptr, &l)) != 0) return rc;
+      StageRange stage("chatts.mix.experts");
+      if (!choose) {
+        if ((rc = mix_linear(d, linear_form(N), l.router, l.router_t, t, l.router_n, wp, CHATTS_EPI_NONE, f32_out(d->b.moe_logits, l.router_n), s)) != 0) return rc;
+        if ((rc = chatts_moe_route(&m, s)) != 0) return rc;
+      }
       const MoeBeside sh = mix_beside(d, l, CHATTS_EXPERT_CLAMPGLU);
       beside = moe_takes_beside(&m, sh);
-      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, s)) != 0) return rc;
+      if ((rc = moe_experts(&m, beside ? sh : MoeBeside{}, choose, s)) != 0) return rc;
+    } else if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s)) != 0) {
+      return rc;
     }
     if (l.up && !beside) {
       const ChattsOperand F = operand(d, true, t, l.ff);

@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "moe_route.h"
 
 namespace chatts {
 
@@ -35,62 +36,10 @@ __device__ __forceinline__ int wave_scan_i(int x) {                // sum over t
   return x;
 }
 
-// what is chosen for a row: lane j has choice j
-struct MoeChoice {
-  int own, id;              // output, expert (-1: an identity output, or none)
-  float mine;               // its score or logit
-  float total, kept;        // sums over the choices: scores, those of identity outputs
-};
-__device__ __forceinline__ int moe_route_end(const ChattsMoeArgs& p, int row, int lane, bool parked, MoeChoice c) {
-  if (p.choose == CHATTS_CHOOSE_LOGITS) {      // softmax over the chosen logits
-    const float mx = wave_max(c.mine);
-    c.mine = lane < p.top ? expf(c.mine - mx) : 0.f;
-    c.total = wave_sum(c.mine);
-    c.kept = wave_sum(c.own >= p.experts ? c.mine : 0.f);
-  }
-  const float inv = p.choose == CHATTS_CHOOSE_SCORES ? p.weight_scale : 1.0f / (c.total + 1e-20f);
-  const int id = parked ? -1 : c.id;
-  if (lane < p.top) {
-    p.ids[(size_t)row * p.top + lane] = id;
-    p.weight[(size_t)row * p.top + lane] = c.mine * inv;
-    p.place[(size_t)row * p.top + lane] = -1;
-  }
-  if (lane == 0) p.kept[row] = parked ? 0.f : c.kept * inv;
-  return id;
-}
-
-// Up to 64 outputs without choice groups: a lane an output, nothing goes through LDS.  The same values as below.  Returns the expert of choice `lane`.
-__device__ __forceinline__ int moe_route_row64(const ChattsMoeArgs& p, int row, int lane) {
-  const int N = p.experts + p.identity;
-  const bool in = lane < N, logits = p.choose == CHATTS_CHOOSE_LOGITS;
-  const int at = in ? lane : 0;
-  const float z = p.logits[(size_t)row * p.ld_logits + at], cor = p.correction ? p.correction[at] : 0.f;
-  const bool parked = p.rows[row].pos < 0;
-  float sc = z;
-  if (!logits) {
-    const float mx = wave_max(in ? z : -INFINITY);
-    const float e = in ? expf(z - mx) : 0.f;
-    sc = e / wave_sum(e);
-  }
-  const float c0 = sc + cor;
-  float ch = in && c0 > -INFINITY ? c0 : -INFINITY;      // (NaN is never chosen)
-  MoeChoice c{-1, -1, logits ? -INFINITY : 0.f, 0.f, 0.f};
-  for (int j = 0; j < p.top; ++j) {
-    const float m = wave_max(ch);
-    if (m == -INFINITY) break;                           // (nothing left)
-    const int b = (int)__builtin_ctzll(__ballot(ch == m));
-    const float s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), b));
-    if (lane == b) ch = -INFINITY;
-    c.total += s;
-    if (b >= p.experts) c.kept += s;
-    if (lane == j) { c.own = b; c.id = b < p.experts ? b : -1; c.mine = s; }
-  }
-  return moe_route_end(p, row, lane, parked, c);
-}
-
 // scratch: 2 N + groups floats of LDS owned by this wave
 __device__ __forceinline__ int moe_route_row(const ChattsMoeArgs& p, int row, int lane, float* sc) {
-  if (p.experts + p.identity <= 64 && p.keep >= p.groups) return moe_route_row64(p, row, lane);
+  if (p.experts + p.identity <= 64 && p.keep >= p.groups)
+    return moe_route_row64(p, row, lane, p.logits[(size_t)row * p.ld_logits + (lane < p.experts + p.identity ? lane : 0)]);
   const int N = p.experts + p.identity, per = N / p.groups;
   float* ch = sc + N;
   float* gr = ch + N;
@@ -338,25 +287,36 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(ChattsMoeArgs p, Mo
   static_assert(!moe_pairs(STEP) || RF == 2, "a pair of fragments");
   constexpr bool IN = STEP != kDown;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, fg = lane >> 4;
-  int e = 0, place0 = 0, count = p.n_rows, n0 = (int)blockIdx.x * 16 * RF;
+  int e = 0, place0 = 0, count = p.n_rows, pair = 0, n0 = (int)blockIdx.x * 16 * RF;
   const bool beside = (int)blockIdx.x < sh_blocks;
   if (beside) {      // (from here on an expert of its own, whose list is the rows)
     p.gate_up = sh.up; p.gate_up_t = sh.up_t; p.down = sh.down; p.down_t = sh.down_t; p.ff_p = sh.ff;
     p.act.hi = sh.f_hi; p.act.lo = sh.f_lo; p.act.ld = sh.ff; p.y = sh.y; p.glu_limit = sh.limit; p.glu_alpha = sh.alpha;
   } else {
     const int at = (int)blockIdx.x - sh_blocks;
-    const int32_t* tile = p.tiles + (size_t)(at / nx) * 4;
     n0 = at % nx * 16 * RF;
-    e = tile[0];
-    if (e < 0) return;
-    place0 = tile[1]; count = tile[2];
+    if (!p.tiles) {      // an expert a tile, its places the pairs that chose it (at most 64 pairs): the j-th of them goes to lane j, the others behind
+      e = at / nx;
+      const int n = p.n_rows * p.top;
+      const bool hit = p.ids[lane < n ? lane : 0] == e && lane < n;
+      const unsigned long long mask = __ballot(hit), below = (1ull << lane) - 1;
+      count = __popcll(mask);
+      if (count == 0) return;
+      pair = __builtin_amdgcn_ds_permute(4 * (hit ? __popcll(mask & below) : count + __popcll(~mask & below)), lane);
+    } else {
+      const int32_t* tile = p.tiles + (size_t)(at / nx) * 4;
+      e = tile[0];
+      if (e < 0) return;
+      place0 = tile[1]; count = tile[2];
+    }
   }
   const int K = IN ? p.width_p : p.ff_p, N = IN ? moe_in_rows(p) : p.width_p;
   const uint16_t* w = TILED ? (IN ? p.gate_up_t : p.down_t) + ((size_t)e * N + n0) * K + (fr * 4 + (fg ^ ((fr >> 3) << 1))) * 8
                             : (IN ? p.gate_up : p.down) + ((size_t)e * N + n0 + fr) * K + fg * 8;
   constexpr int kStep = TILED ? 16 : 1;      // elements of w per K-value
-  const int pl = place0 + (fr < count ? fr : 0);
-  const size_t arow = IN ? (size_t)(beside ? pl : p.order[pl] / p.top) * p.h.ld : (size_t)pl * p.act.ld;
+  const bool direct = !beside && !p.tiles;
+  const int own = fr < count ? fr : 0, pl = direct ? __shfl(pair, own, 64) : place0 + own;
+  const size_t arow = IN ? (size_t)(beside ? pl : (direct ? pl : p.order[pl]) / p.top) * p.h.ld : (size_t)pl * p.act.ld;
   const uint16_t* ah = (IN ? p.h.hi : p.act.hi) + arow + fg * 8;
   const uint16_t* al = (IN ? p.h.lo : p.act.lo) + arow + fg * 8;
   f32x4 acc[RF];
@@ -404,14 +364,14 @@ __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(ChattsMoeArgs p, Mo
     }
   if (fr >= count) return;
   if (STEP == kRelu2) {
-    moe_relu2_4(p.act, place0 + fr, n0 + wave * 16 + fg * 4, s[0]);
+    moe_relu2_4(p.act, pl, n0 + wave * 16 + fg * 4, s[0]);
   } else if (moe_pairs(STEP)) {
     float v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = moe_unit<STEP>(p, s[0][r], s[1][r]);
-    store_operand4(p.act, place0 + fr, (n0 >> 1) + fg * 4, v);
+    store_operand4(p.act, pl, (n0 >> 1) + fg * 4, v);
   } else {
-    *reinterpret_cast<f32x4*>(p.y + (size_t)(place0 + fr) * p.width_p + n0 + wave * 16 + fg * 4) = s[0];
+    *reinterpret_cast<f32x4*>(p.y + (size_t)pl * p.width_p + n0 + wave * 16 + fg * 4) = s[0];
   }
 }
 
@@ -603,19 +563,25 @@ static int moe_tile_bound(int rows, int top, int experts, int bm) {      // sum 
   return (int)(pairs / bm + lists);
 }
 
-template <int STEP, int RF>
+template <int STEP, int RF, int NW>
 static void launch_moe_stream_as(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {
-  constexpr int NW = moe_pairs(STEP) ? 4 : 16;
   const int sh_n = !sh.up ? 0 : STEP == kDown ? a->width_p : moe_pairs(STEP) ? 2 * sh.ff : sh.ff, sh_blocks = sh_n / (16 * RF), nx = n / (16 * RF);
   const dim3 g(sh_blocks + nx * tiles), b(64 * NW);
   if (STEP == kDown ? a->down_t : a->gate_up_t) hipLaunchKernelGGL((moe_stream_kernel<STEP, true, NW, RF>), g, b, 0, s, *a, sh, sh_blocks, nx);
   else hipLaunchKernelGGL((moe_stream_kernel<STEP, false, NW, RF>), g, b, 0, s, *a, sh, sh_blocks, nx);
 }
+// Few workgroups: smaller ones, so that the CUs get as much each, and more waves in each.  Waves of a workgroup, a step of Muvetar 2048 wide, us (gated / down): 16 sequences 4 / 16 931,
+// 8 / 16 898, 8 / 8 892, 4 / 4 977, 16 / 16 949; 2 sequences 8 / 16 629, 8 / 8 647; 4096 wide, 16 sequences 4 / 16 2240, 8 / 8 2177, one 8 / 16 1125, 8 / 8 1150.
 template <int STEP>
-static void launch_moe_stream(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {      // few workgroups: smaller ones, so that the CUs get as much each
-  if constexpr (!moe_pairs(STEP))
-    if (n / 32 * tiles < 2 * device_cus()) return launch_moe_stream_as<STEP, 1>(a, sh, n, tiles, s);
-  launch_moe_stream_as<STEP, 2>(a, sh, n, tiles, s);
+static void launch_moe_stream(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {
+  if constexpr (moe_pairs(STEP)) {
+    launch_moe_stream_as<STEP, 2, 8>(a, sh, n, tiles, s);
+  } else {
+    const int pairs = a->n_rows * a->top, lists = pairs < a->experts ? pairs : a->experts, wgs = n / 32 * lists;
+    if (wgs < 2 * device_cus()) launch_moe_stream_as<STEP, 1, 16>(a, sh, n, tiles, s);
+    else if (wgs < 4 * device_cus()) launch_moe_stream_as<STEP, 2, 16>(a, sh, n, tiles, s);
+    else launch_moe_stream_as<STEP, 2, 8>(a, sh, n, tiles, s);
+  }
 }
 
 template <int STEP, int BM, int WM, int WN>
@@ -660,15 +626,21 @@ extern "C" int chatts_moe_route(const ChattsMoeArgs* a, chatts_stream_t stream) 
 bool chatts::moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh) {
   return moe_small(a) && sh.up && sh.down && sh.f_hi && sh.f_lo && sh.y && sh.ff % 64 == 0 && a->width_p % 64 == 0 && !sh.up_t == !a->gate_up_t && !sh.down_t == !a->down_t;
 }
-extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream) { return moe_experts(a, MoeBeside{}, stream); }
-int chatts::moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, chatts_stream_t stream) {
+bool chatts::moe_takes_choice(const ChattsMoeArgs* a) {
+  return moe_small(a) && a->n_rows * a->top <= 64 && a->experts + a->identity <= 64 && a->keep >= a->groups;
+}
+extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream) { return moe_experts(a, MoeBeside{}, false, stream); }
+int chatts::moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, bool direct, chatts_stream_t stream) {
   if (const int rc = check_moe(a, "moe_experts")) return rc;
   CHATTS_REQUIRE(a->gate_up && a->down && a->y && (a->exact ? a->h.f32 && a->act.f32 : a->h.hi && a->h.lo && a->act.hi && a->act.lo) && a->h.ld >= a->width_p &&
                      a->act.ld >= a->ff_p && a->h.ld % 8 == 0 && a->act.ld % 8 == 0, CHATTS_E_BADARG, "moe_experts: operands");
   CHATTS_REQUIRE(!sh.up || moe_takes_beside(a, sh), CHATTS_E_SHAPE, "moe_experts: a feed-forward of %d beside experts of %d rows", sh.ff, a->n_rows);
   if (a->n_rows == 0) return CHATTS_OK;
   hipStream_t s = as_stream(stream);
-  const int bm = moe_bm(a), tiles = moe_tile_bound(a->n_rows, a->top, a->experts, bm), in_rows = moe_in_rows(*a);
+  CHATTS_REQUIRE(!direct || moe_takes_choice(a), CHATTS_E_SHAPE, "moe_experts: choices without lists are for few rows (%d rows, %d of %d experts)", a->n_rows, a->top, a->experts);
+  ChattsMoeArgs without = *a;
+  if (direct) { without.tiles = nullptr; a = &without; }
+  const int bm = moe_bm(a), tiles = direct ? a->experts : moe_tile_bound(a->n_rows, a->top, a->experts, bm), in_rows = moe_in_rows(*a);
   const bool relu2 = a->act_kind == CHATTS_EXPERT_RELU2, clamped = a->act_kind == CHATTS_EXPERT_CLAMPGLU;
   if (a->exact) {
     if (relu2) hipLaunchKernelGGL(moe_gemm_f32_kernel<kRelu2>, dim3(tiles, in_rows / 64), dim3(256), 0, s, *a);
