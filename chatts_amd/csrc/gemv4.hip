@@ -9,10 +9,10 @@
 //   * products on the matrix pipe: a wave's unit is FOUR rows ("quad") x 512 k, one 16-byte load per lane = 256 consecutive bytes of each row.  The 16
 //     rows of an MFMA operand are 4 rows x 4 parts of K; x comes as columns (part, hi / lo), and the wanted sums are the blocks where the parts
 //     agree: nothing is wasted on rows that are not there, and a wave ends up with 8 vectors of 4 rows instead of a 64-lane reduction;
-//   * the quads of a workgroup (one per CU, N / 4 / 256 of them) x the parts of K are dealt evenly over 8 waves, loads five units ahead and the first
+//   * the quads of a workgroup (one per CU, N / 4 / 256 of them) x the parts of K are dealt evenly over 8 waves, loads two units ahead and the first
 //     ones before x is staged; requests past the end of a wave's share carry an offset outside the buffer: they return nothing.
-// Measured back to back in a graph, there -> here: qkv 7168 x 5120 10.8 -> 8.7 us, o 5120 x 5120 8.7 -> 7.75, gate_up 27648 x 5120 27.9 -> 20.4 (75 MB with scales:
-// 3.7 TB/s; v_fma_mix and v_cvt_pk issue at half rate, so the conversion alone is 13 us of it), down 5120 x 13824 17.0 -> 11.7.  16 waves instead of 8: 1 us
+// Measured back to back in a graph, there -> here: qkv 7168 x 5120 10.8 -> 8.4 us, o 5120 x 5120 8.7 -> 7.4, gate_up 27648 x 5120 27.9 -> 19.9 (75 MB with scales:
+// 3.8 TB/s; v_fma_mix and v_cvt_pk issue at half rate, so the conversion alone is 13 us of it), down 5120 x 13824 17.0 -> 12.2.  16 waves instead of 8: 1 us
 // more everywhere (the prologue is serial per SIMD); scales staged in LDS: 1 to 2 us more.
 // x = hi + lo bf16 (2^-17), products exact, float32 sums: the accuracy of the kernel it replaces.
 #include <type_traits>
@@ -39,7 +39,9 @@ struct Gemv4Params {
   unsigned parts_inv;              // ceil(2^32 / parts of K), 0 where there is one: a quotient without a division
 };
 
-constexpr int kQ4Waves = 8, kQ4Threads = 64 * kQ4Waves, kQ4Turns = 4, kQ4Bufs = 6, kQ4Ahead = kQ4Bufs - 1, kQ4Early = 2;
+// Units of the ring: more of them only cost code and registers.  us with 8 / 6 / 4 / 3 / 2: 7168 x 5120 9.9 / 9.1 / 9.0 / 8.4 / 9.3, 5120 x 5120 8.5 / 8.2 / 7.4 / 7.4 / 7.7, 27648 x 5120 gated
+// 21.5 / 20.3 / 20.2 / 19.9 / 22.4, 5120 x 13824 13.9 / 12.6 / 12.6 / 12.2 / 13.7, 24576 x 4096 gated 17.0 / 16.4 / 15.3 / 15.2 / 16.4, 4096 x 12288 11.5 / 10.3 / 9.9 / 10.0 / 10.8.
+constexpr int kQ4Waves = 8, kQ4Threads = 64 * kQ4Waves, kQ4Turns = 4, kQ4Bufs = 3, kQ4Ahead = kQ4Bufs - 1, kQ4Early = 1;
 constexpr int kQ4Piece = 512 + 32;      // bytes of an operand: (k group) x (part, hi / lo) x 16; the 32 keep the writes of x apart
 constexpr unsigned kQ4Far = 0x7ffffff0u;
 __host__ __device__ constexpr int q4_parts(int k) { return (k + 511) >> 9; }
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
     if (++rs == S) { rs = 0; ++rq; }
   };
   // x: eight k a thread and turn, times the norm's weights, split, written as operands.  It is requested before the weights (loads return in order: x comes from
-  // L2, weights from HBM), and only two units of those before it is there: more would stand in front of the x that later waves ask for.
+  // L2, weights from HBM), and only one unit of those before it is there: more would stand in front of the x that later waves ask for.
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, K * 4, 0x00020000);      // (past K: zeros)
   const __amdgpu_buffer_rsrc_t nr = __builtin_amdgcn_make_buffer_rsrc((void*)(NORM ? p.norm_w : p.x), 0, K * 4, 0x00020000);
   f32x4 xv[kQ4Turns][2], gw[kQ4Turns][2];

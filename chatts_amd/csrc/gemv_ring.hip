@@ -1,6 +1,6 @@
 // gemv_ring.hip - batch-1 projections of long rows: y[N] = epilogue(W[N,K] . norm(x)), W bf16, fp8 (OCP e4m3fn) or int8 with a power-of-two scale per row.
 //
-// What bounds it: W is read once from HBM, 6.5 TB/s where enough of it is under way (64 KB a CU and more) from the launch's start to its end.  gemv_ldsx_kernel (gemv.hip) asks for 2 rows x
+// What bounds it: W is read once from HBM, 6.5 TB/s where enough of it is under way (32 KB a CU) from the launch's start to its end.  gemv_ldsx_kernel (gemv.hip) asks for 2 rows x
 // 2 chunks, waits for all of them and computes: 8 waves have 32 KB a CU under way, then nothing, and nothing at all while x is staged.  Here a wave's tasks (two rows each) are
 // ONE sequence of units, a 1 KB chunk of each of the task's rows, that runs through a ring of D units in registers: the loads of the next D - 1 units are always under way,
 // over the end of a task, too, and the first ones since before x was staged.  Requests past a row's end or the last task lie outside the row's buffer: they return zeros.
@@ -36,7 +36,10 @@ __device__ __forceinline__ void gemv_finish(const GemvParams& p, int task, float
   }
 }
 
-constexpr int kRingRows = 2, kRingUnits = 6;    // rows of a task; units of the ring (8 of them: the same)
+// Rows of a task; units of the ring, two of them under way beside the one that is computed.  More cost code and registers and hide nothing; us with 8 / 6 / 4 / 3 / 2 units: bf16 7168 x 5120
+// 14.1 / 13.7 / 13.1 / 13.0 / 13.5, 27648 x 5120 gated 45.3 / 44.9 / 44.7 / 43.9 / 44.5, 4096 x 4096 8.5 / 8.5 / 7.9 / 7.8 / 7.8, 24576 x 4096 gated 32.5 / 32.2 / 32.2 / 31.4 / 31.8, 4096 x 12288
+// 18.6 / 18.2 / 18.2 / 18.2 / 18.2; fp8 27648 x 5120 gated 25.4 / 24.9 / 24.2 / 23.5 / 23.9, 5120 x 13824 15.2 / 14.7 / 13.9 / 14.2 / 14.3, 24576 x 4096 gated 18.9 / 18.3 / 17.8 / 17.4 / 17.9.
+constexpr int kRingRows = 2, kRingUnits = 3;
 constexpr int kGemvTurns = 4;                   // pieces of x that a thread holds while the first weights are requested
 template <int EPI, bool NORM, int FMT>
 __global__ __launch_bounds__(1024) void gemv_ring_kernel(GemvParams p) {
@@ -208,7 +211,7 @@ bool gemv_ring_takes(const ChattsLinearArgs* a) {
   return opt == 2 || (a->k > 2048 && per_cu >= 6 && (a->w8 ? bytes > (size_t)32 << 20 && (each < 9 || each > 12 || bytes >= (size_t)44 << 20) : per_cu < 128));
 }
 
-// Waves of a workgroup, one of which a CU has; each keeps 10 KB under way.  Eight of them, or as many as let all walk the same number of tasks where a CU has few: a wave that walks one more
+// Waves of a workgroup, one of which a CU has; each keeps 4 KB under way.  Eight of them, or as many as let all walk the same number of tasks where a CU has few: a wave that walks one more
 // holds the launch up.  More only stretch the prologue, which long rows bear (7168 x 5120, 14 tasks a CU, 12 / 8 waves 17.1 / 14.2 us, fp8 10.4 / 9.0).  As a part of gemv_ldsx_kernel's time,
 // 8 waves / the choice:
 //   5 .. 8 tasks: one a wave.
@@ -228,9 +231,9 @@ static int ring_waves(const ChattsLinearArgs* a) {
   if (each >= 17 && each <= 20 && (!a->w8 || a->k >= 8192)) return 10;
   return 8;
 }
-// Measured in a graph over rotating weights, gemv_ldsx_kernel / here, us: bf16 24576 x 4096 gated 34.3 / 33.4, 4096 x 12288 19.8 / 18.5, 6144 x 4096 10.8 / 10.5, 4096 x 4096 8.2 / 7.9,
-// 7168 x 5120 14.9 / 14.3, 5120 x 13824 25.4 / 24.2, 12288 x 3072 14.7 / 13.9; fp8 24576 x 4096 gated 21.1 / 18.6, 27648 x 5120 gated 26.7 / 24.9, 4096 x 12288 12.2 / 11.0, 7168 x 5120
-// 9.7 / 9.0, 152064 x 5120 127 / 122; int8 24576 x 4096 gated 22.0 / 19.0, 4096 x 12288 12.5 / 11.2.
+// Measured in a graph over rotating weights, gemv_ldsx_kernel / here, us: bf16 24576 x 4096 gated 34.3 / 31.4, 4096 x 12288 19.8 / 18.2, 6144 x 4096 10.8 / 10.2, 4096 x 4096 8.2 / 7.8,
+// 7168 x 5120 14.9 / 13.0, 5120 x 13824 25.4 / 24.4, 12288 x 3072 14.7 / 13.9; fp8 24576 x 4096 gated 21.1 / 17.4, 27648 x 5120 gated 26.7 / 23.5, 4096 x 12288 12.2 / 11.4, 7168 x 5120
+// 9.7 / 8.3, 152064 x 5120 127 / 122; int8 24576 x 4096 gated 22.0 / 19.0, 4096 x 12288 12.5 / 11.2.
 int launch_gemv_ring(const GemvParams& from, const ChattsLinearArgs* a, hipStream_t s) {
   GemvParams p = from;
   const int cus = device_cus();
