@@ -670,67 +670,82 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_bf16x3_kernel(AttnParams 
 //     A and B agree: slot 8 g + j of lane group g means key 4 g + j (j < 4) or 16 + 4 g + (j - 4), and kv_planes_kernel writes the
 //     V^T rows in that slot order, so the A fragment is still one 16-byte LDS read;
 //   * O^T in the C layout gives a lane 4 consecutive head dims of its query: alpha applies as is, the output is 16-byte stores.
-// Staging is 8 16-byte copies per thread.  Same three-pass bf16 split products as the kernel above; the sums run in another order, so
+// Same three-pass bf16 split products as the kernel above; the sums run in another order, so
 // the two agree to rounding (tests: both against the float64 reference).  Needs the host to know pos0 (plane count) and a free
 // workspace; otherwise the kernel above runs.
-// Plane layout, per (kv head, 32-key tile) 32 KB: K_hi [32 keys][128], K_lo, V^T_hi [128 dims][32 slots], V^T_lo; rows past the last
-// key repeat it (finite values behind the causal mask).
+// Plane layout, per (kv head, 32-key tile) 32 KB: K_hi [32 keys][128], K_lo, V^T_hi [128 dims][32 slots], V^T_lo, every row's 16-byte chunks where LDS wants them (chunk c of key k at
+// c ^ (k & 15), chunk c of dim d at c ^ ((d >> 2) & 2)), so that a tile goes to LDS as it lies, by DMA; rows past the last key repeat it (finite values behind the causal mask).
 // ---------------------------------------------------------------------------------------------------
+// Bound by the round trip to the cache for a few hundred keys, by bytes for thousands.  A thread writes whole chunks and the lanes of a wave write next to each other; 8 bytes of V^T every
+// 64 took 5.1 / 8 / 18 us for 223 / 806 / 2048 keys of 8 heads, this 3.7 / 5.8 / 16.6 (with 16-byte loads of V the same).
 __global__ __launch_bounds__(256) void kv_planes_kernel(AttnParams p, int n_keys, uint16_t* planes) {
   constexpr int KT = 32;
   const int tid = threadIdx.x, kt = blockIdx.x, hk = blockIdx.y;
   const KvLayout kvl{p.table, p.n_kv, p.max_ctx, p.log_block};
   const size_t toff = kv_tile_off(kvl, hk, kt * KT);
-  uint16_t* dst = planes + ((size_t)hk * gridDim.x + kt) * (4 * KT * kHeadDim);
+  char* dst = reinterpret_cast<char*>(planes) + ((size_t)hk * gridDim.x + kt) * (8 * KT * kHeadDim);
   const int last = n_keys - 1 - kt * KT;                    // last valid row inside this tile (>= 0)
+  f32x4 kv[2][2];
+  float vv[2][8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {                             // K: thread = (key, 4 dims), rows stay rows
-    const int idx = tid + i * 256;
-    const int key = idx >> 5, c4 = idx & 31;
-    const int kr = key <= last ? key : last;
-    const f32x4 v = *reinterpret_cast<const f32x4*>(p.kc + toff + (size_t)kr * kHeadDim + c4 * 4);
-    const float x[4] = {v.x, v.y, v.z, v.w};
-    abf16x4_t h, l;
+  for (int i = 0; i < 2; ++i) {                             // K: thread = (key, chunk of 8 dims), rows stay rows
+    const int key = (tid >> 4) + i * 16, kr = key <= last ? key : last;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const __bf16 hh = (__bf16)x[e];
-      h[e] = hh;
-      l[e] = (__bf16)(x[e] - (float)hh);
-    }
-    *reinterpret_cast<abf16x4_t*>(dst + key * kHeadDim + c4 * 4) = h;
-    *reinterpret_cast<abf16x4_t*>(dst + KT * kHeadDim + key * kHeadDim + c4 * 4) = l;
+    for (int h = 0; h < 2; ++h) kv[i][h] = *reinterpret_cast<const f32x4*>(p.kc + toff + (size_t)kr * kHeadDim + (tid & 15) * 8 + h * 4);
   }
-  // V transposed: thread = (head dim, 16 keys kg*16 ..); a wave reads 64 consecutive dims of one key (256 contiguous bytes) per load.
-  // Keys kg*16 + 4 g + j (j = 0..3) go to slots 8 g + 4 kg + j.
-  const int d = tid & 127, kg = tid >> 7;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    abf16x4_t h, l;
+  for (int i = 0; i < 2; ++i) {                             // V transposed: thread = (head dim, chunk g of 8 slots); slot 8 g + j is key 4 g + j or (from j = 4 on) 12 + 4 g + j
+    const int d = (tid >> 2) + i * 64, g = tid & 3;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int key = kg * 16 + 4 * g + j;
-      const int vr = key <= last ? key : last;
-      const float x = p.vc[toff + (size_t)vr * kHeadDim + d];
-      const __bf16 hh = (__bf16)x;
-      h[j] = hh;
-      l[j] = (__bf16)(x - (float)hh);
+    for (int j = 0; j < 8; ++j) {
+      const int key = 4 * g + j + (j < 4 ? 0 : 12), vr = key <= last ? key : last;
+      vv[i][j] = p.vc[toff + (size_t)vr * kHeadDim + d];
     }
-    *reinterpret_cast<abf16x4_t*>(dst + 2 * KT * kHeadDim + d * KT + 8 * g + 4 * kg) = h;
-    *reinterpret_cast<abf16x4_t*>(dst + 3 * KT * kHeadDim + d * KT + 8 * g + 4 * kg) = l;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int key = (tid >> 4) + i * 16, d = (tid >> 2) + i * 64;
+    const float x[8] = {kv[i][0].x, kv[i][0].y, kv[i][0].z, kv[i][0].w, kv[i][1].x, kv[i][1].y, kv[i][1].z, kv[i][1].w};
+    abf16x8_t h, l;
+    split8(x, h, l);
+    char* to = dst + key * 256 + (((tid & 15) ^ (key & 15)) << 4);
+    *reinterpret_cast<abf16x8_t*>(to) = h;
+    *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
+    split8(vv[i], h, l);
+    to = dst + 16384 + d * 64 + (((tid & 3) ^ ((d >> 2) & 2)) << 4);
+    *reinterpret_cast<abf16x8_t*>(to) = h;
+    *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
   }
 }
 
-__global__ __launch_bounds__(256, 2) void attn_prefill_planes_kernel(AttnParams p) {
-  // LDS rows WITHOUT padding, 16-byte chunks XOR-swizzled for ds_read_b128's lane groups ({0-3, 12-15, 20-27}, {4-11, 16-19, 28-31}, ...:
-  // every group holds each qi once, with g = g0 for eight of them and g0 + 1 for the other eight): K chunk c of key k sits at
-  // c ^ (k & 15), V^T chunk c of dim d at c ^ ((d >> 2) & 2) - each group then covers all 64 banks exactly once (272- / 80-byte padded
-  // rows, right for 16 consecutive lanes, gave every group a 2-way conflict: 44 % of the LDS cycles).
-  constexpr int KT = 32, KROW = 256, VROW = 64;
-  __shared__ __attribute__((aligned(16))) char k_hi[KT * KROW];
-  __shared__ __attribute__((aligned(16))) char k_lo[KT * KROW];
-  __shared__ __attribute__((aligned(16))) char vt_hi[kHeadDim * VROW];
-  __shared__ __attribute__((aligned(16))) char vt_lo[kHeadDim * VROW];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+typedef __attribute__((address_space(3))) void* lptr_t;
+
+// the maximum over lanes 16 (32) apart
+__device__ __forceinline__ float swap_max16(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float swap_max32(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// QW waves of QB x 16 queries each, KP parts of the keys: wave (part, w) takes tiles part, part + KP, ... for its queries, and the parts' sums meet in LDS at the end.
+// What bounds it, by size: for some hundred rows the chain of a wave's tiles, each ~1 us of LDS reads, products and softmax one after the other (parts shorten the chain; fewer queries a
+// workgroup spread the work where CUs would be idle); above that LDS: 16 queries read every tile whole, 32 KB of LDS reads for 48 products (QB = 2: for 96); from some thousand rows on the
+// matrix pipe at the rate its power allows.  So: all of K's fragments are asked for at once, V's before the softmax, products run in four chains, tiles come by DMA, one ahead (three
+// ahead gained nothing), with one barrier a tile.  With tiles through registers, reads four at a time and 16 queries x one part only, us with kv_planes_kernel (before / now),
+// 32 heads: 64 rows 10.1 / 8.1, 223 17.6 / 13.2, 512 32.6 / 24.3, 806 49.0 / 34.8, 2048 145.9 / 122, 64 rows behind 700 keys 42 / 25.6; 40 heads: 806 50 / 41, 2048 174.7 / 142.
+// LDS rows have no padding, their 16-byte chunks are XOR-swizzled for ds_read_b128's lane groups ({0-3, 12-15, 20-27}, {4-11, 16-19, 28-31}, ...: every group holds each qi once, with
+// g = g0 for eight of them and g0 + 1 for the other eight): each group covers all 64 banks exactly once.
+template <int QW, int QB, int KP>
+__global__ __launch_bounds__(64 * QW * KP, 2) void attn_prefill_planes_kernel(AttnParams p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int KT = 32, TILE = 8 * KT * kHeadDim, PIECES = TILE / 1024 / QW;
+  extern __shared__ __attribute__((aligned(1024))) char tiles_s[];      // [part][2][K_hi, K_lo, V^T_hi, V^T_lo]
+  const int lane = threadIdx.x & 63;
+  const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x / (64 * QW)), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64 % QW);
+  char* mine = tiles_s + part * (2 * TILE);
   const int G = p.n_q / p.n_kv;
   // XCD-aware order.  Workgroups go to the 8 XCDs round robin by linear index, each XCD has its own 4 MB L2, and every workgroup
   // streams its kv head's planes (0.8 MB at 798 keys; 233 MB of tile reads per launch in total).  With (query tile, query head) as
@@ -752,162 +767,258 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_planes_kernel(AttnParams 
   const int heads = p.n_q + 2 * p.n_kv;
   const int T = p.t, pos0 = p.pos0;
   const int qt = p.units - 1 - xi;                          // heaviest query tiles (most key tiles) first, over ALL heads
-  const int q0 = qt * 64;
+  const int q0 = qt * (16 * QB * QW), qw = q0 + wave * (16 * QB);      // first query of the workgroup, of this wave
   const int qi = lane & 15, g = lane >> 4;                  // this lane's query (of the wave's 16) and its group of 8 K-values / 4 C rows
   const float scale2 = 0.08838834764831845f * 1.4426950408889634f;   // d^-1/2 * log2(e): the softmax runs on exp2
 
-  abf16x8_t q_hi[4], q_lo[4];                                // B fragments of Q^T: query qi, dims ks*32 + g*8 .. +7
-  {
-    int qrow = q0 + wave * 16 + qi;
+  const int last_q = q0 + 16 * QB * QW - 1 < T - 1 ? q0 + 16 * QB * QW - 1 : T - 1;
+  const int nkt = (pos0 + last_q) / KT + 1;                 // tiles up to the last key any row of this workgroup may see
+  f32x4 q_in[QB][8];
+#pragma unroll
+  for (int b = 0; b < QB; ++b) {
+    int qrow = qw + b * 16 + qi;
     if (qrow > T - 1) qrow = T - 1;                         // padded rows compute garbage that is never stored
     const float* qp = p.qkv + ((size_t)qrow * heads + hq) * kHeadDim + g * 8;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(qp + ks * 32), b = *reinterpret_cast<const f32x4*>(qp + ks * 32 + 4);
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      split8(x, q_hi[ks], q_lo[ks]);
-    }
+    for (int ks = 0; ks < 8; ++ks) q_in[b][ks] = *reinterpret_cast<const f32x4*>(qp + (ks >> 1) * 32 + (ks & 1) * 4);
   }
-  const int qpos = pos0 + q0 + wave * 16 + qi;
-  float m_run = -INFINITY, l_part = 0.f;                    // l_part: this lane's 8 slots only; the four groups meet after the loop
-  f32x4 o_acc[8];                                           // O^T: head dims db*16 + 4 g + r of query qi
+  // a tile of this part, on its way to its place in LDS; past the last one a request returns zeros
+  const char* src0 = reinterpret_cast<const char*>(p.kv_planes) + (size_t)hk * p.kv_plane_tiles * TILE;
+  auto request = [&](int kt, int at) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(src0 + (size_t)kt * TILE), 0, kt < nkt ? TILE : 0, 0x00020000);
 #pragma unroll
-  for (int db = 0; db < 8; ++db) o_acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const int last_q = q0 + 63 < T - 1 ? q0 + 63 : T - 1;
-  const int nkt = (pos0 + last_q) / KT + 1;                 // tiles up to the last key any row of this workgroup may see
-  // 512 16-byte chunks per 8 KB plane: thread takes chunks tid and tid + 256.  K chunk j: key j >> 4, column j & 15; V^T chunk j: dim
-  // j >> 2, column j & 3.  Loads run TWO tiles ahead in two register sets: a tile's matrix work (~1.4k cycles) does not cover an L2
-  // round trip.
-  f32x4 kreg[2][4], vreg[2][4];
-  const uint16_t* src0 = p.kv_planes + (size_t)hk * p.kv_plane_tiles * (4 * KT * kHeadDim) + tid * 8;
-  auto load_tile = [&](int kt, f32x4 (&kr)[4], f32x4 (&vr)[4]) {
-    if (kt >= nkt) return;
-    const uint16_t* src = src0 + (size_t)kt * (4 * KT * kHeadDim);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      kr[i] = *reinterpret_cast<const f32x4*>(src + i * 2048);
-      kr[2 + i] = *reinterpret_cast<const f32x4*>(src + KT * kHeadDim + i * 2048);
-      vr[i] = *reinterpret_cast<const f32x4*>(src + 2 * KT * kHeadDim + i * 2048);
-      vr[2 + i] = *reinterpret_cast<const f32x4*>(src + 3 * KT * kHeadDim + i * 2048);
-    }
+    for (int i = 0; i < PIECES; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lptr_t)(mine + at * TILE + (wave * PIECES + i) * 1024), 16, (wave * PIECES + i) * 1024 + lane * 16, 0, 0, 0);
   };
-  auto store_tile = [&](int kt, const f32x4 (&kr)[4], const f32x4 (&vr)[4]) {
-    if (kt >= nkt) return;
+  __builtin_amdgcn_sched_barrier(0);
+  request(part, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  abf16x8_t q_hi[QB][4], q_lo[QB][4];                        // B fragments of Q^T: query qi, dims ks*32 + g*8 .. +7
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int j = tid + i * 256;
-      const int ko = (j >> 4) * KROW + (((j & 15) ^ ((j >> 4) & 15)) << 4);
-      const int vo = (j >> 2) * VROW + (((j & 3) ^ ((j >> 4) & 2)) << 4);         // (d >> 2) & 2 with d = j >> 2
-      *reinterpret_cast<f32x4*>(k_hi + ko) = kr[i];
-      *reinterpret_cast<f32x4*>(k_lo + ko) = kr[2 + i];
-      *reinterpret_cast<f32x4*>(vt_hi + vo) = vr[i];
-      *reinterpret_cast<f32x4*>(vt_lo + vo) = vr[2 + i];
-    }
-  };
-  auto tile = [&](int kt) {
-    const int k0 = kt * KT;
-    if (kt >= nkt || k0 > pos0 + q0 + wave * 16 + 15) return;      // no tile / every score of this wave masked: wave-uniform skip
-
-    f32x4 s_acc[2];                                         // S^T: keys k0 + nb*16 + 4 g + r, query qi
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) s_acc[nb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < QB; ++b)
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
+      const f32x4 v0 = q_in[b][2 * ks], v1 = q_in[b][2 * ks + 1];
+      const float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+      split8(x, q_hi[b][ks], q_lo[b][ks]);
+    }
+  const int qpos = pos0 + qw + qi;
+  float m_run[QB], l_part[QB];                              // l_part: this lane's 8 slots only; the four groups meet after the loop
+  f32x4 o_acc[QB][8];                                       // O^T: head dims db*16 + 4 g + r of query qi
+#pragma unroll
+  for (int b = 0; b < QB; ++b) {
+    m_run[b] = -INFINITY;
+    l_part[b] = 0.f;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) o_acc[b][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+
+  auto tile = [&](int kt, int at) __attribute__((always_inline)) {
+    const int k0 = kt * KT;
+    if (kt >= nkt || k0 > pos0 + qw + 16 * QB - 1) return;      // no tile / every score of this wave masked: wave-uniform skip
+    const char* base = mine + at * TILE;
+    abf16x8_t fh[8], fl[8];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
-        const int off = (nb * 16 + qi) * KROW + (((ks * 4 + g) ^ qi) << 4);
-        const abf16x8_t ah = *reinterpret_cast<const abf16x8_t*>(k_hi + off);
-        const abf16x8_t al = *reinterpret_cast<const abf16x8_t*>(k_lo + off);
-        s_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, q_lo[ks], s_acc[nb], 0, 0, 0);
-        s_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, q_hi[ks], s_acc[nb], 0, 0, 0);
-        s_acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, q_hi[ks], s_acc[nb], 0, 0, 0);
+        const char* from = base + (nb * 16 + qi) * 256 + (((ks * 4 + g) ^ qi) << 4);
+        fh[ks * 2 + nb] = *reinterpret_cast<const abf16x8_t*>(from);
+        fl[ks * 2 + nb] = *reinterpret_cast<const abf16x8_t*>(from + 8192);
       }
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int NC = QB > 1 ? 1 : 2;                      // S^T: keys k0 + nb*16 + 4 g + r, query qi; in four chains of products
+    f32x4 s_acc[QB][2][NC];
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) s_acc[b][nb][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb) {
+            f32x4& to = s_acc[b][nb][t == 1 ? NC - 1 : 0];
+            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t == 2 ? fl[ks * 2 + nb] : fh[ks * 2 + nb], t == 0 ? q_lo[b][ks] : q_hi[b][ks], to, 0, 0, 0);
+          }
     }
-    const bool diag = k0 + KT - 1 > pos0 + q0 + wave * 16;  // wave-uniform: only such a tile holds keys some query of this wave cannot see
-    float e[8];
-    float mx = -INFINITY;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int db = 0; db < 8; ++db) {                        // head dims db*16 .. db*16+15: A fragment = 8 slots of dim db*16 + qi; under way while the softmax runs
+      const char* from = base + 16384 + (db * 16 + qi) * 64 + ((g ^ ((qi >> 2) & 2)) << 4);
+      fh[db] = *reinterpret_cast<const abf16x8_t*>(from);
+      fl[db] = *reinterpret_cast<const abf16x8_t*>(from + 8192);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const bool diag = k0 + KT - 1 > pos0 + qw;  // wave-uniform: only such a tile holds keys some query of this wave cannot see
+    abf16x8_t p_hi[QB], p_lo[QB];                            // B fragments of P^T: slots 8 g .. 8 g + 7 of query qi
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float sc = s_acc[nb][r] * scale2;
-        if (diag && k0 + nb * 16 + 4 * g + r > qpos) sc = -INFINITY;   // causal mask
-        e[nb * 4 + r] = sc;
-        mx = fmaxf(mx, sc);
+    for (int b = 0; b < QB; ++b) {
+      float e[8];
+      float mx = -INFINITY;
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float sc = s_acc[b][nb][0][r];
+          if (NC > 1) sc += s_acc[b][nb][NC - 1][r];
+          sc *= scale2;
+          if (diag && k0 + nb * 16 + 4 * g + r > qpos + b * 16) sc = -INFINITY;   // causal mask
+          e[nb * 4 + r] = sc;
+          mx = fmaxf(mx, sc);
+        }
       }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float m_new = fmaxf(m_run, mx);
-    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_ref);
-    m_run = m_new;
-    float ps = 0.f;
+      mx = swap_max16(mx);
+      mx = swap_max32(mx);
+      const float m_new = fmaxf(m_run[b], mx);
+      const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m_run[b] - m_ref);
+      m_run[b] = m_new;
+      float ps = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      e[j] = __builtin_amdgcn_exp2f(e[j] - m_ref);
-      ps += e[j];
-    }
-    l_part = l_part * alpha + ps;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {    // some running maximum of this wave moved
-#pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        o_acc[db].x *= alpha; o_acc[db].y *= alpha; o_acc[db].z *= alpha; o_acc[db].w *= alpha;
+      for (int j = 0; j < 8; ++j) {
+        e[j] = __builtin_amdgcn_exp2f(e[j] - m_ref);
+        ps += e[j];
       }
-    }
-    abf16x8_t p_hi, p_lo;                                    // B fragment of P^T: slots 8 g .. 8 g + 7 of query qi
-    split8(e, p_hi, p_lo);
+      l_part[b] = l_part[b] * alpha + ps;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {    // some running maximum of this wave moved
 #pragma unroll
-    for (int db = 0; db < 8; ++db) {                        // head dims db*16 .. db*16+15: A fragment = 8 slots of dim db*16 + qi
-      const int off = (db * 16 + qi) * VROW + ((g ^ ((qi >> 2) & 2)) << 4);
-      const abf16x8_t vh = *reinterpret_cast<const abf16x8_t*>(vt_hi + off);
-      const abf16x8_t vl = *reinterpret_cast<const abf16x8_t*>(vt_lo + off);
-      o_acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, p_lo, o_acc[db], 0, 0, 0);
-      o_acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vl, p_hi, o_acc[db], 0, 0, 0);
-      o_acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, p_hi, o_acc[db], 0, 0, 0);
+        for (int db = 0; db < 8; ++db) {
+          o_acc[b][db].x *= alpha; o_acc[b][db].y *= alpha; o_acc[b][db].z *= alpha; o_acc[b][db].w *= alpha;
+        }
+      }
+      split8(e, p_hi[b], p_lo[b]);
+    }
+    constexpr int ND = 4 / QB;                               // (four chains here, too)
+#pragma unroll
+    for (int d0 = 0; d0 < 8; d0 += ND) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int db = d0; db < d0 + ND; ++db)
+#pragma unroll
+          for (int b = 0; b < QB; ++b)
+            o_acc[b][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t == 1 ? fl[db] : fh[db], t == 0 ? p_lo[b] : p_hi[b], o_acc[b][db], 0, 0, 0);
     }
   };
-  load_tile(0, kreg[0], vreg[0]);
-  load_tile(1, kreg[1], vreg[1]);
-  for (int kt = 0; kt < nkt; kt += 2) {
-    __syncthreads();                                        // the previous tile has been consumed by every wave
-    store_tile(kt, kreg[0], vreg[0]);
-    __syncthreads();
-    load_tile(kt + 2, kreg[0], vreg[0]);
-    tile(kt);
-    if (kt + 1 >= nkt) break;
-    __syncthreads();
-    store_tile(kt + 1, kreg[1], vreg[1]);
-    __syncthreads();
-    load_tile(kt + 3, kreg[1], vreg[1]);
-    tile(kt + 1);
+  for (int k0 = 0, at = 0; k0 < nkt; k0 += KP, at ^= 1) {     // (the same for all parts: they meet at the barriers)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                            // all of this tile has landed, and the tile before it has been consumed by every wave
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    request(k0 + part + KP, at ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    tile(k0 + part, at);
   }
-  float l = l_part + __shfl_xor(l_part, 16);
-  l += __shfl_xor(l, 32);
-  const int qrow = q0 + wave * 16 + qi;
-  if (qrow >= T) return;
-  const float inv = 1.0f / l;
-  const size_t oi = ((size_t)qrow * p.n_q + hq) * kHeadDim + 4 * g;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (no request outlives its LDS)
+  if constexpr (KP > 1) {                                    // part 0 has seen key 0: its maximum is that of a score unless there is none
+    f32x4* sums = reinterpret_cast<f32x4*>(tiles_s);         // [part - 1][wave][block][o 0 .. 7, (m, l)][lane]
+    __syncthreads();
+    if (part > 0) {
 #pragma unroll
-  for (int db = 0; db < 8; ++db) {
-#pragma clang fp contract(off)   // lo = split of the ROUNDED product, as chatts_split_bf16x2 of the float32 output would give
-    const float v[4] = {o_acc[db].x * inv, o_acc[db].y * inv, o_acc[db].z * inv, o_acc[db].w * inv};
-    if (p.out_hi) {
-      abf16x4_t h, lo;
+      for (int b = 0; b < QB; ++b) {
+        f32x4* to = sums + (((part - 1) * QW + wave) * QB + b) * (9 * 64) + lane;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const __bf16 hh = (__bf16)v[j];
-        h[j] = hh;
-        lo[j] = (__bf16)(v[j] - (float)hh);
+        for (int db = 0; db < 8; ++db) to[db * 64] = o_acc[b][db];
+        to[8 * 64] = (f32x4){m_run[b], l_part[b], 0.f, 0.f};
       }
-      const size_t at = plane_at(qrow, hq * kHeadDim + 4 * g + db * 16, p.n_q * kHeadDim, p.out_tiled);
-      *reinterpret_cast<abf16x4_t*>(p.out_hi + at) = h;
-      *reinterpret_cast<abf16x4_t*>(p.out_lo + at) = lo;
-    } else {
-      *reinterpret_cast<f32x4*>(p.out + oi + db * 16) = (f32x4){v[0], v[1], v[2], v[3]};
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int j = 0; j < KP - 1; ++j)
+#pragma unroll
+      for (int b = 0; b < QB; ++b) {
+        const f32x4* from = sums + ((j * QW + wave) * QB + b) * (9 * 64) + lane;
+        const f32x4 ml = from[8 * 64];
+        const float m_new = fmaxf(m_run[b], ml.x), m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float wa = __builtin_amdgcn_exp2f(m_run[b] - m_ref), wb = __builtin_amdgcn_exp2f(ml.x - m_ref);
+        m_run[b] = m_new;
+        l_part[b] = l_part[b] * wa + ml.y * wb;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) {
+          const f32x4 o = from[db * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o_acc[b][db][e] = o_acc[b][db][e] * wa + o[e] * wb;
+        }
+      }
+  }
+#pragma unroll
+  for (int b = 0; b < QB; ++b) {
+    float l = l_part[b] + __shfl_xor(l_part[b], 16);
+    l += __shfl_xor(l, 32);
+    const int qrow = qw + b * 16 + qi;
+    if (qrow >= T) continue;
+    const float inv = 1.0f / l;
+    const size_t oi = ((size_t)qrow * p.n_q + hq) * kHeadDim + 4 * g;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+#pragma clang fp contract(off)   // lo = split of the ROUNDED product, as chatts_split_bf16x2 of the float32 output would give
+      const float v[4] = {o_acc[b][db].x * inv, o_acc[b][db].y * inv, o_acc[b][db].z * inv, o_acc[b][db].w * inv};
+      if (p.out_hi) {
+        abf16x4_t h, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const __bf16 hh = (__bf16)v[j];
+          h[j] = hh;
+          lo[j] = (__bf16)(v[j] - (float)hh);
+        }
+        const size_t at_o = plane_at(qrow, hq * kHeadDim + 4 * g + db * 16, p.n_q * kHeadDim, p.out_tiled);
+        *reinterpret_cast<abf16x4_t*>(p.out_hi + at_o) = h;
+        *reinterpret_cast<abf16x4_t*>(p.out_lo + at_o) = lo;
+      } else {
+        *reinterpret_cast<f32x4*>(p.out + oi + db * 16) = (f32x4){v[0], v[1], v[2], v[3]};
+      }
     }
   }
+#endif
+}
+
+// The form, by how the workgroups fill the CUs.  Two waves of queries, two parts of the keys: while there is a CU for every workgroup.  Four waves and two parts: as long as all tiles
+// together would take the CUs no longer than the heaviest workgroup takes by itself (the causal mask leaves the others less).  Then one part, two workgroups a CU, 16 or 32 queries a wave: the smaller
+// estimate of the larger of all tiles spread over the CUs, the heaviest workgroup's, and, where there are more workgroups than places, two that follow each other in one place (us a tile: 0.75
+// spread, 1.05 alone for 16 queries, 1.3 and 1.9 for 32).  us of the four forms: 223 rows of 32 heads 13.2 / 14.1 / 14.7 / 20.2, 512 25.2 / 24.3 / 27.2 / 37.5, 806 48.7 / 34.8 / 40.4 / 55,
+// 1400 110 / 78 / 69 / 94, 4000 - / - / 415 / 383; 40 heads: 650 45 / 33.9 / 34.4 / 45.7, 806 60 / 44.2 / 41.4 / 57, 2048 260 / 166 / 150 / 143, 2048 behind 2048 - / - / 410 / 429,
+// 2600 behind 2048 - / - / 576 / 513.
+enum { PLANES_2X2, PLANES_4X2, PLANES_4X1, PLANES_4X1_32 };
+static int prefill_planes_form(int t, int pos0, int n_q, int cus) {
+  // tiles of the workgroups of the i-th heaviest tile of q queries
+  auto tiles = [&](int q, int i) { return (pos0 + (i == 0 ? t : ((t + q - 1) / q - i) * q) + 31) / 32; };
+  auto all = [&](int q) {
+    double sum = 0;
+    for (int i = 0; i < (t + q - 1) / q; ++i) sum += tiles(q, i);
+    return sum * n_q;
+  };
+  auto estimate = [&](int q, double spread, double alone) {
+    const double a = all(q) / cus * spread, b = tiles(q, 0) * alone;
+    const int first = 2 * cus / n_q;
+    const double c = (t + q - 1) / q > first ? 2 * tiles(q, first) * 2 * spread : 0;
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
+  };
+  if (n_q * ((t + 31) / 32) <= cus) return PLANES_2X2;
+  if (all(64) <= (double)cus * tiles(64, 0)) return PLANES_4X2;
+  return estimate(128, 1.3, 1.9) < estimate(64, 0.75, 1.05) ? PLANES_4X1_32 : PLANES_4X1;
+}
+
+template <int QW, int QB, int KP>
+static int launch_prefill_planes(AttnParams& p, hipStream_t s) {
+  constexpr int lds = KP * 2 * 4 * 32 * kHeadDim * (int)sizeof(uint16_t);
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_planes_kernel<QW, QB, KP>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    CHATTS_REQUIRE(e == hipSuccess, CHATTS_E_LAUNCH, "attention: cannot reserve %d KB of LDS: %s", lds / 1024, hipGetErrorString(e));
+    configured = true;
+  }
+  const int G = p.n_q / p.n_kv;
+  p.units = (p.t + 16 * QB * QW - 1) / (16 * QB * QW);
+  const int grid = p.xcd_share ? 8 * ((G * p.units + p.xcd_share - 1) / p.xcd_share) : p.n_q * p.units;
+  hipLaunchKernelGGL((attn_prefill_planes_kernel<QW, QB, KP>), dim3(grid), dim3(64 * QW * KP), lds, s, p);
+  return CHATTS_OK;
 }
 
 // merge the split partials of attn_rows_kernel (splits that saw no tile hold m = -inf, l = 0)
@@ -1053,16 +1164,19 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
                         ((uintptr_t)workspace % 16) == 0;
     if (planes) {
       uint16_t* pl = static_cast<uint16_t*>(workspace);
-      const int nqt = (t + 63) / 64;
       hipLaunchKernelGGL(kv_planes_kernel, dim3(tiles, n_kv), dim3(256), 0, as_stream(stream), p, n_keys, pl);
       CHATTS_CHECK_LAUNCH("kv_planes");
       p.kv_planes = pl; p.kv_plane_tiles = tiles;
       const bool xcd_on = opt_get(OPT_ATTN_XCD, 1) != 0;
-      p.units = nqt;
       p.xcd_share = xcd_on && n_kv <= 8 && 8 % n_kv == 0 ? 8 / n_kv : 0;
-      const int G = n_q / n_kv;
-      const int grid = p.xcd_share ? 8 * ((G * p.units + p.xcd_share - 1) / p.xcd_share) : n_q * p.units;
-      hipLaunchKernelGGL(attn_prefill_planes_kernel, dim3(grid), dim3(256), 0, as_stream(stream), p);
+      int rc;
+      switch (prefill_planes_form(t, pos0, n_q, device_cus())) {
+        case PLANES_2X2: rc = launch_prefill_planes<2, 1, 2>(p, as_stream(stream)); break;
+        case PLANES_4X2: rc = launch_prefill_planes<4, 1, 2>(p, as_stream(stream)); break;
+        case PLANES_4X1: rc = launch_prefill_planes<4, 1, 1>(p, as_stream(stream)); break;
+        default: rc = launch_prefill_planes<4, 2, 1>(p, as_stream(stream));
+      }
+      if (rc) return rc;
     } else if (bf16x3) hipLaunchKernelGGL(attn_prefill_bf16x3_kernel, dim3((t + 63) / 64, n_q, n_splits), dim3(256), 0, as_stream(stream), p);
     else hipLaunchKernelGGL(attn_prefill_mfma_kernel<32>, dim3((t + 63) / 64, n_q, n_splits), dim3(256), 0, as_stream(stream), p);
     CHATTS_CHECK_LAUNCH("attn_prefill_mfma");

@@ -39,7 +39,7 @@ struct AttnParams {
   int out_tiled;       // prefill: so many rows of out_hi / out_lo in tiles (plane_at)
   int kv_round;        // experiment knob, see kv_round_f (0 = off)
   // prefill (bf16x3 kernel), optional: this sequence's K / V rows 0 .. kv_plane_keys-1 already split into bf16 hi / lo planes by
-  // kv_planes_kernel, per (kv head, 32-key tile) 32 KB: K_hi [32][128], K_lo, V^T_hi [128][32], V^T_lo.  NULL: split while staging
+  // kv_planes_kernel (its layout is described there).  NULL: split while staging
   const uint16_t* kv_planes;
   int kv_plane_tiles;  // tiles per kv head
   // attn_prefill_planes_kernel's 1-D grid: query tiles per head and, when n_kv divides 8, the number of XCDs that share one kv head

@@ -1,0 +1,58 @@
+"""The forms of the prefill attention on K / V planes: 32 or 64 queries and two parts of the keys, 64 or 128 queries and one part, chosen by how the workgroups fill the CUs."""
+import ctypes as C
+
+import pytest
+import torch
+
+from chatts_amd import _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _lib.load()
+
+
+def _reference(q, k, v, pos0):
+    """float64, one head at a time"""
+    T, nq, _ = q.shape
+    n, group = pos0 + T, nq // k.shape[0]
+    hidden = torch.arange(n, device=DEV)[None, :] > (pos0 + torch.arange(T, device=DEV))[:, None]
+    out = torch.empty((T, nq, 128), dtype=torch.float64, device=DEV)
+    for h in range(nq):
+        s = (q[:, h].double() @ k[h // group, :n].double().T.contiguous()) * 128 ** -0.5
+        s.masked_fill_(hidden, float("-inf"))
+        out[:, h] = torch.softmax(s, -1) @ v[h // group, :n].double()
+    return out
+
+
+# on 256 CUs: two waves of queries and two parts; four and two; four and one; four of 32 queries.  First and last tiles whole, one row, one row short; parts with one tile more than the other and without any
+@pytest.mark.parametrize("nq,nkv,T,pos0", [
+    (10, 2, 64, 0), (10, 2, 65, 0), (32, 8, 95, 0), (32, 8, 256, 0), (8, 8, 97, 31), (5, 1, 129, 700), (28, 4, 64, 1),
+    (32, 8, 257, 0), (40, 8, 200, 33), (40, 8, 511, 0), (12, 12, 705, 2),
+    (40, 8, 806, 0), (40, 8, 769, 100), (64, 8, 575, 31), (24, 3, 1409, 0),
+    (40, 8, 2049, 0), (64, 8, 1407, 0), (32, 8, 1472, 2047)])
+def test_every_form(lib, nq, nkv, T, pos0):
+    """Against float64.  A product of split operands is off by 2^-18 of each factor and the dropped lo x lo: 4e-6 of a score's scale (rms), and P and V bring 2e-6 each, so 5e-6 of the
+    output's norm; four times that is allowed."""
+    ctx = pos0 + T + 5
+    g = torch.Generator(device=DEV).manual_seed(T + pos0 + nq)
+    qkv = torch.randn((T, (nq + 2 * nkv) * 128), generator=g, device=DEV)
+    k = torch.randn((nkv, ctx, 128), generator=g, device=DEV)
+    v = torch.randn((nkv, ctx, 128), generator=g, device=DEV)
+    k[:, 40] *= 4.0                          # a key of the second tile that outweighs the others: the parts' maxima differ
+    want = _reference(qkv.view(T, nq + 2 * nkv, 128)[:, :nq], k, v, pos0)
+    k[:, pos0 + T:] = float("nan")           # rows past the context are not read
+    v[:, pos0 + T:] = float("nan")
+    qkv[T // 2, 128:256] = float("nan")      # a query without a score: only its own row
+    cache = _lib.KvCache(k=k.data_ptr(), v=v.data_ptr(), max_ctx=ctx)
+    ws = torch.empty(((pos0 + T + 31) // 32) * nkv * 32768, dtype=torch.uint8, device=DEV)
+    out = torch.zeros((T, nq * 128), device=DEV)
+    _lib.check(lib.chatts_attention(qkv.data_ptr(), T, nq, nkv, pos0, None, C.byref(cache), out.data_ptr(), 1, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    got = out.view(T, nq, 128).double()
+    assert got[T // 2, 1].isnan().all()
+    got[T // 2, 1] = want[T // 2, 1]
+    assert ((got - want).norm() / want.norm()).item() < 2e-5
+    assert (got - want).abs().max().item() < 2e-5 * want.abs().max().item()
