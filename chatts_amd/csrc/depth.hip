@@ -17,7 +17,7 @@ struct DepthChoose {
 // NR > 0 (few rows): the same launch multiplies the row by the router, as the planes that it writes, and chooses its experts.  A projection, its split's epilogue and a workgroup that chose
 // for all rows and made lists of them were three launches: 12.5 us a layer of 32 experts at 16 rows of 2048, now 1.  The router's first K-steps are requested before the row is there.
 template <int NT, int NV, int NR = 0>
-__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch) {
+__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch, int tiled) {
   __shared__ float red[NT / 64];
   constexpr int NW = NT / 64, NX = NV * NT * 4;
   __shared__ __attribute__((aligned(16))) uint16_t xh[NR ? NX : 1], xl[NR ? NX : 1];
@@ -133,7 +133,14 @@ __global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, D
     float v[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = c + k < p.width ? x[i][k] * inv * w[i][k] : 0.f;
-    store_operand4(p.out, row, c, v);
+    if (NR == 0 && tiled) {      // (rows from `tiled` on: plane_at has them where row-major has)
+      ChattsOperand at{};
+      const size_t place = plane_at((int)row, c, p.ldx, tiled);
+      at.hi = p.out.hi + place; at.lo = p.out.lo + place;
+      store_operand4(at, 0, 0, v);
+    } else {
+      store_operand4(p.out, row, c, v);
+    }
     if constexpr (NR > 0) {
       ChattsOperand own{};
       own.hi = xh; own.lo = xl;
@@ -201,19 +208,22 @@ static int check_depth_norm(const ChattsDepthNormArgs* a) {
                      (((uintptr_t)a->out.hi | (uintptr_t)a->out.lo) % 8) == 0, CHATTS_E_SHAPE, "depth_norm: pointers must be aligned (16 bytes, planes 8)");
   return CHATTS_OK;
 }
-extern "C" int chatts_depth_norm(const ChattsDepthNormArgs* a, chatts_stream_t stream) {
+extern "C" int chatts_depth_norm(const ChattsDepthNormArgs* a, chatts_stream_t stream) { return depth_norm(a, false, stream); }
+int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t stream) {
   if (const int rc = check_depth_norm(a)) return rc;
+  CHATTS_REQUIRE(!tiles || (a->w && a->out.hi && a->out.lo && !a->out.f32 && a->out.ld == a->ldx && a->ldx % 32 == 0), CHATTS_E_SHAPE, "depth_norm: planes in tiles of %d columns", a->ldx);
   if (a->t == 0) return CHATTS_OK;
+  const int tiled = tiles ? a->t & ~15 : 0;
   const DepthChoose none{};
   const dim3 g(a->t);
   hipStream_t s = as_stream(stream);
-  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a, none);
-  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a, none);
-  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a, none);
-  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a, none);
-  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a, none);
-  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a, none);
-  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a, none);
+  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a, none, tiled);
+  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a, none, tiled);
+  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a, none, tiled);
+  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a, none, tiled);
+  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a, none, tiled);
+  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a, none, tiled);
+  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a, none, tiled);
   CHATTS_CHECK_LAUNCH("depth_norm");
   return CHATTS_OK;
 }
@@ -226,8 +236,8 @@ int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs*
                      moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);
   if (a->t == 0) return CHATTS_OK;
   const DepthChoose ch{router_t ? router_t : router, router_t ? 16 : 1, *moe};
-  if (moe->experts + moe->identity <= 32) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch);
-  else hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 4>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch);
+  if (moe->experts + moe->identity <= 32) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
+  else hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 4>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
   CHATTS_CHECK_LAUNCH("depth_norm_choose");
   return CHATTS_OK;
 }
