@@ -678,30 +678,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_bf16x3_kernel(AttnParams 
 // ---------------------------------------------------------------------------------------------------
 // Bound by the round trip to the cache for a few hundred keys, by bytes for thousands.  A thread writes whole chunks and the lanes of a wave write next to each other; 8 bytes of V^T every
 // 64 took 5.1 / 8 / 18 us for 223 / 806 / 2048 keys of 8 heads, this 3.7 / 5.8 / 16.6 (with 16-byte loads of V the same).
-__global__ __launch_bounds__(256) void kv_planes_kernel(AttnParams p, int n_keys, uint16_t* planes) {
-  constexpr int KT = 32;
-  const int tid = threadIdx.x, kt = blockIdx.x, hk = blockIdx.y;
-  const KvLayout kvl{p.table, p.n_kv, p.max_ctx, p.log_block};
-  const size_t toff = kv_tile_off(kvl, hk, kt * KT);
-  char* dst = reinterpret_cast<char*>(planes) + ((size_t)hk * gridDim.x + kt) * (8 * KT * kHeadDim);
-  const int last = n_keys - 1 - kt * KT;                    // last valid row inside this tile (>= 0)
+// a tile's planes from key4(key, d): K at dims d .. d + 3, and value(key, d): V
+template <typename K4, typename V1>
+__device__ __forceinline__ void store_kv_planes(char* dst, int tid, K4 key4, V1 value) {
   f32x4 kv[2][2];
   float vv[2][8];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {                             // K: thread = (key, chunk of 8 dims), rows stay rows
-    const int key = (tid >> 4) + i * 16, kr = key <= last ? key : last;
+  for (int i = 0; i < 2; ++i)                               // K: thread = (key, chunk of 8 dims), rows stay rows
 #pragma unroll
-    for (int h = 0; h < 2; ++h) kv[i][h] = *reinterpret_cast<const f32x4*>(p.kc + toff + (size_t)kr * kHeadDim + (tid & 15) * 8 + h * 4);
-  }
+    for (int h = 0; h < 2; ++h) kv[i][h] = key4((tid >> 4) + i * 16, (tid & 15) * 8 + h * 4);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {                             // V transposed: thread = (head dim, chunk g of 8 slots); slot 8 g + j is key 4 g + j or (from j = 4 on) 12 + 4 g + j
-    const int d = (tid >> 2) + i * 64, g = tid & 3;
+  for (int i = 0; i < 2; ++i)                               // V transposed: thread = (head dim, chunk g of 8 slots); slot 8 g + j of chunk g is key 4 g + j or (from j = 4 on) 12 + 4 g + j
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int key = 4 * g + j + (j < 4 ? 0 : 12), vr = key <= last ? key : last;
-      vv[i][j] = p.vc[toff + (size_t)vr * kHeadDim + d];
-    }
-  }
+    for (int j = 0; j < 8; ++j) vv[i][j] = value(4 * (tid & 3) + j + (j < 4 ? 0 : 12), (tid >> 2) + i * 64);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int key = (tid >> 4) + i * 16, d = (tid >> 2) + i * 64;
@@ -716,6 +705,62 @@ __global__ __launch_bounds__(256) void kv_planes_kernel(AttnParams p, int n_keys
     *reinterpret_cast<abf16x8_t*>(to) = h;
     *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
   }
+}
+
+__global__ __launch_bounds__(256) void kv_planes_kernel(AttnParams p, int n_keys, uint16_t* planes) {
+  constexpr int KT = 32;
+  const int tid = threadIdx.x, kt = blockIdx.x, hk = blockIdx.y;
+  const KvLayout kvl{p.table, p.n_kv, p.max_ctx, p.log_block};
+  const size_t toff = kv_tile_off(kvl, hk, kt * KT);
+  char* dst = reinterpret_cast<char*>(planes) + ((size_t)hk * gridDim.x + kt) * (8 * KT * kHeadDim);
+  const int last = n_keys - 1 - kt * KT;                    // last valid row inside this tile (>= 0)
+  store_kv_planes(dst, tid, [&](int key, int d) { return *reinterpret_cast<const f32x4*>(p.kc + toff + (size_t)(key <= last ? key : last) * kHeadDim + d); },
+                  [&](int key, int d) { return p.vc[toff + (size_t)(key <= last ? key : last) * kHeadDim + d]; });
+}
+
+// The same from qkv rows that no launch has rotated yet: the chunk's K and V rows go through rope_kv_kernel's work (a wave a row, the same bits) into the cache and, from LDS, into the planes;
+// rows before the chunk come from the cache.  The queries are left to attn_prefill_planes_kernel.  Where the qkv projection has no split whose epilogue does it, rope_kv_kernel read and wrote all
+// heads and kv_planes_kernel read the cache back: 12.6 + 6.3 us for 798 rows of 40 + 16 heads, 28 + 10 for 2048; here 9 and 12, and the attention 1 more for the queries.  Prompts, ms: 14B of 798 rows
+// 36.9 / 36.7, of 2300 105.5 / 104.8, 8B of 1000 24.1 / 23.9.
+__global__ __launch_bounds__(256) void rope_kv_planes_kernel(const float* __restrict__ qkv, RopeFuse r, int n_keys, uint16_t* __restrict__ planes) {
+  constexpr int KT = 32, LD = kHeadDim + 4;
+  __shared__ __attribute__((aligned(16))) float k_s[KT * LD];
+  __shared__ __attribute__((aligned(16))) float v_s[KT * LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kt = blockIdx.x, hk = blockIdx.y;
+  const int heads = r.n_q + 2 * r.n_kv, last = n_keys - 1 - kt * KT;
+  const size_t toff = kv_tile_off(r.kvl, hk, kt * KT);
+  float k[8][2], v[8][2], c[8], s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int key = wave * 8 + i, kr = key <= last ? key : last, pos = kt * KT + kr, tok = pos - r.pos0;      // (rows past the last key repeat it)
+    const float* kp = tok >= 0 ? qkv + ((size_t)tok * heads + r.n_q + hk) * kHeadDim : r.kc + toff + (size_t)kr * kHeadDim;
+    const float* vp = tok >= 0 ? qkv + ((size_t)tok * heads + r.n_q + r.n_kv + hk) * kHeadDim : r.vc + toff + (size_t)kr * kHeadDim;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) { k[i][h] = kp[lane + 64 * h]; v[i][h] = vp[lane + 64 * h]; }
+    c[i] = r.cos_tab[(size_t)pos * 64 + lane];
+    s[i] = r.sin_tab[(size_t)pos * 64 + lane];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int key = wave * 8 + i, kr = key <= last ? key : last;
+    if (kt * KT + kr >= r.pos0) {                           // (uniform)
+      norm_rope(k[i][0], k[i][1], r.k_norm_w, r.eps, c[i], s[i], lane);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        k[i][h] = kv_round_f(k[i][h], r.kv_round);
+        v[i][h] = kv_round_f(v[i][h], r.kv_round);
+        if (key <= last) {
+          r.kc[toff + (size_t)kr * kHeadDim + lane + 64 * h] = k[i][h];
+          r.vc[toff + (size_t)kr * kHeadDim + lane + 64 * h] = v[i][h];
+        }
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) { k_s[key * LD + lane + 64 * h] = k[i][h]; v_s[key * LD + lane + 64 * h] = v[i][h]; }
+  }
+  __syncthreads();
+  store_kv_planes(reinterpret_cast<char*>(planes) + ((size_t)hk * gridDim.x + kt) * (8 * KT * kHeadDim), tid, [&](int key, int d) { return *reinterpret_cast<const f32x4*>(k_s + key * LD + d); },
+                  [&](int key, int d) { return v_s[key * LD + d]; });
 }
 
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -782,6 +827,23 @@ __global__ __launch_bounds__(64 * QW * KP, 2) void attn_prefill_planes_kernel(At
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) q_in[b][ks] = *reinterpret_cast<const f32x4*>(qp + (ks >> 1) * 32 + (ks & 1) * 4);
   }
+  f32x4 turn[QB][8], weight[8];                             // cosines and sines, the norm's weights: only for rows that rope_kv_planes_kernel left as they were
+  if (p.cos_tab) {
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      int qrow = qw + b * 16 + qi;
+      if (qrow > T - 1) qrow = T - 1;
+      const size_t at = (size_t)(pos0 + qrow) * 64 + g * 8;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        turn[b][ks] = *reinterpret_cast<const f32x4*>(p.cos_tab + at + (ks >> 1) * 32 + (ks & 1) * 4);
+        turn[b][4 + ks] = *reinterpret_cast<const f32x4*>(p.sin_tab + at + (ks >> 1) * 32 + (ks & 1) * 4);
+      }
+    }
+    if (p.q_norm_w)
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) weight[ks] = *reinterpret_cast<const f32x4*>(p.q_norm_w + g * 8 + (ks >> 1) * 32 + (ks & 1) * 4);
+  }
   // a tile of this part, on its way to its place in LDS; past the last one a request returns zeros
   const char* src0 = reinterpret_cast<const char*>(p.kv_planes) + (size_t)hk * p.kv_plane_tiles * TILE;
   auto request = [&](int kt, int at) __attribute__((always_inline)) {
@@ -793,6 +855,34 @@ __global__ __launch_bounds__(64 * QW * KP, 2) void attn_prefill_planes_kernel(At
   __builtin_amdgcn_sched_barrier(0);
   request(part, 0);
   __builtin_amdgcn_sched_barrier(0);
+  if (p.cos_tab) {                                          // norm and rotation of 128 dims: 32 in each of four lanes, d and d + 64 in one
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      if (p.q_norm_w) {
+        float ss = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ss += q_in[b][ks][e] * q_in[b][ks][e];
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        const float rstd = rsqrtf(ss / (float)kHeadDim + p.eps);
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q_in[b][ks][e] = weight[ks][e] * (q_in[b][ks][e] * rstd);
+      }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = q_in[b][ks][e], y = q_in[b][ks + 4][e], c = turn[b][ks][e], sn = turn[b][4 + ks][e];
+          q_in[b][ks][e] = x * c - y * sn;
+          q_in[b][ks + 4][e] = y * c + x * sn;
+        }
+    }
+  }
   abf16x8_t q_hi[QB][4], q_lo[QB][4];                        // B fragments of Q^T: query qi, dims ks*32 + g*8 .. +7
 #pragma unroll
   for (int b = 0; b < QB; ++b)
@@ -1119,7 +1209,27 @@ static int bind_cache(AttnParams& p, const ChattsKvCache* cache) {
 
 namespace chatts {
 int attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev, const ChattsKvCache* cache, float* out,
-                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0);
+                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr);
+
+// The attention on K / V planes: the positions known here, keys in one split, the caller's workspace free and large enough for the planes
+static size_t prefill_plane_bytes(int n_keys, int n_kv) { return (size_t)((n_keys + 31) / 32) * n_kv * 4 * 32 * kHeadDim * sizeof(uint16_t); }
+static bool prefill_on_planes(int t, int n_kv, int pos0, const int32_t* pos0_dev, bool out_planes, int n_splits, const void* workspace, size_t workspace_bytes) {
+  return opt_get(OPT_ATTN_BF16X3, 1) != 0 && opt_get(OPT_ATTN_PLANES, 1) != 0 && (opt_get(OPT_ATTN_ROWS, 0) == 0 || out_planes) && !pos0_dev && n_splits == 1 && t >= 64 && workspace &&
+         workspace_bytes >= prefill_plane_bytes(pos0 + t, n_kv) && ((uintptr_t)workspace % 16) == 0;
+}
+// chatts_rope_kv_write and chatts_attention, in one launch fewer and without the queries' way through memory where the planes' writer can do the keys' and values' part
+int rope_attention_impl(float* qkv, int t, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w, float norm_eps, const float* cos_tab, const float* sin_tab, int pos0,
+                        const int32_t* pos0_dev, const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes,
+                        chatts_stream_t stream, int out_tiled) {
+  if (t > 0 && opt_get(OPT_ROPE_FUSE, 1) != 0 && prefill_on_planes(t, n_kv, pos0, pos0_dev, out_hi != nullptr, n_splits, workspace, workspace_bytes) &&
+      (((uintptr_t)cos_tab | (uintptr_t)sin_tab | (uintptr_t)q_norm_w) % 16) == 0) {
+    RopeFuse r;
+    if (const int rc = rope_fuse_prepare(t, n_q, n_kv, q_norm_w, k_norm_w, norm_eps, cos_tab, sin_tab, pos0, nullptr, cache, &r)) return rc;
+    return attention_impl(qkv, t, n_q, n_kv, pos0, nullptr, cache, out, out_hi, out_lo, n_splits, workspace, workspace_bytes, stream, out_tiled, &r);
+  }
+  if (const int rc = chatts_rope_kv_write(qkv, t, n_q, n_kv, q_norm_w, k_norm_w, norm_eps, cos_tab, sin_tab, pos0, pos0_dev, cache, stream)) return rc;
+  return attention_impl(qkv, t, n_q, n_kv, pos0, pos0_dev, cache, out, out_hi, out_lo, n_splits, workspace, workspace_bytes, stream, out_tiled);
+}
 }  // namespace chatts
 
 extern "C" int chatts_attention(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev,
@@ -1133,7 +1243,7 @@ extern "C" int chatts_attention(const float* qkv, int t, int n_q, int n_kv, int 
 // Planes are written by the MFMA kernel / its combine only (t >= 16, n_splits <= 4): the caller checks that.
 int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev,
                            const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits,
-                           void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled) {
+                           void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled, const RopeFuse* rope) {
   CHATTS_REQUIRE(t >= 0 && n_q > 0 && n_kv > 0 && n_splits >= 1 && n_splits <= kMaxSlots, CHATTS_E_BADARG,
                  "attention: bad sizes");
   if (t == 0) return CHATTS_OK;
@@ -1157,14 +1267,15 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
     // (64-key tiles were measured too: 155 us vs 148 us at T = 798 - the per-tile work is not what is slow)
     const int bf16x3 = opt_get(OPT_ATTN_BF16X3, 1);      // 0: the float32-MFMA kernel
     // K / V split into bf16 planes once (kv_planes_kernel) when the caller's workspace is free (one key split) and holds them
-    const bool planes_on = opt_get(OPT_ATTN_PLANES, 1) != 0;
     const int n_keys = pos0 + t, tiles = (n_keys + 31) / 32;
-    const size_t plane_bytes = (size_t)tiles * n_kv * 4 * 32 * kHeadDim * sizeof(uint16_t);
-    const bool planes = bf16x3 && planes_on && !pos0_dev && n_splits == 1 && t >= 64 && workspace && workspace_bytes >= plane_bytes &&
-                        ((uintptr_t)workspace % 16) == 0;
-    if (planes) {
+    if (prefill_on_planes(t, n_kv, pos0, pos0_dev, out_hi != nullptr, n_splits, workspace, workspace_bytes)) {
       uint16_t* pl = static_cast<uint16_t*>(workspace);
-      hipLaunchKernelGGL(kv_planes_kernel, dim3(tiles, n_kv), dim3(256), 0, as_stream(stream), p, n_keys, pl);
+      if (rope) {      // (rope_attention_impl: rows of qkv as the projection left them)
+        p.q_norm_w = rope->q_norm_w; p.cos_tab = rope->cos_tab; p.sin_tab = rope->sin_tab; p.eps = rope->eps;
+        hipLaunchKernelGGL(rope_kv_planes_kernel, dim3(tiles, n_kv), dim3(256), 0, as_stream(stream), qkv, *rope, n_keys, pl);
+      } else {
+        hipLaunchKernelGGL(kv_planes_kernel, dim3(tiles, n_kv), dim3(256), 0, as_stream(stream), p, n_keys, pl);
+      }
       CHATTS_CHECK_LAUNCH("kv_planes");
       p.kv_planes = pl; p.kv_plane_tiles = tiles;
       const bool xcd_on = opt_get(OPT_ATTN_XCD, 1) != 0;

@@ -23,8 +23,11 @@ int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int 
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
                                   int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream);
+int rope_attention_impl(float* qkv, int t, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w, float norm_eps, const float* cos_tab, const float* sin_tab, int pos0,
+                        const int32_t* pos0_dev, const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes,
+                        chatts_stream_t stream, int out_tiled = 0);
 int attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev, const ChattsKvCache* cache, float* out,
-                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0);
+                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr);
 int launch_split_bf16x2(const float* x, int m, int k, int ldx, uint16_t* hi, uint16_t* lo, int ldp, int tiled, hipStream_t s);
 size_t gemm_workspace(int m, int n, int k);
 }  // namespace chatts
@@ -480,10 +483,8 @@ static int layer_part_f16q(ChattsDecoder* d, int layer, int part, int t, int pos
     q.bias = lw.qkv_bias; q.c = d->b.qkv; q.ldc = qkv_n; q.epilogue = CHATTS_EPI_NONE;
     if ((rc = chatts_linear_f16q(&q, stream)) != 0) return rc;
     ChattsKvCache kc = layer_cache(d, layer, d->cur_seq);
-    if ((rc = chatts_rope_kv_write(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev,
-                                   &kc, stream)) != 0) return rc;
-    if ((rc = attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, nullptr, nullptr, 1, d->b.workspace,
-                             d->b.workspace_bytes, stream)) != 0) return rc;
+    if ((rc = rope_attention_impl(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev, &kc, d->b.attn, nullptr, nullptr, 1,
+                                  d->b.workspace, d->b.workspace_bytes, stream)) != 0) return rc;
     if ((rc = chatts_split_f16q(d->b.attn, t, na, na, A.hi, A.lo8, A.sc, na, na / 128, 1, stream)) != 0) return rc;
     base(q, A, na, lw.o16, lw.o_q8, lw.o_q8e, H);
     q.ldc = H;
@@ -523,10 +524,8 @@ static int layer_part_fp8(ChattsDecoder* d, int layer, int part, int t, int pos0
     f.m = t; f.n = qkv_n; f.k = H; f.lda8 = H; f.ldw8 = H; f.ldc = qkv_n; f.epilogue = CHATTS_EPI_NONE;
     if ((rc = chatts_linear_fp8(&f, stream)) != 0) return rc;
     ChattsKvCache kc = layer_cache(d, layer, d->cur_seq);
-    if ((rc = chatts_rope_kv_write(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev,
-                                   &kc, stream)) != 0) return rc;
-    if ((rc = attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, nullptr, nullptr, 1, d->b.workspace,
-                             d->b.workspace_bytes, stream)) != 0) return rc;
+    if ((rc = rope_attention_impl(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev, &kc, d->b.attn, nullptr, nullptr, 1,
+                                  d->b.workspace, d->b.workspace_bytes, stream)) != 0) return rc;
     if ((rc = chatts_quantize_rows_fp8(d->b.attn, t, na, na, nullptr, 0.f, b8, na, sb, stream)) != 0) return rc;
     f = ChattsLinearFp8Args{};
     f.a8 = b8; f.a_scale = sb; f.w8 = lw.o8; f.w_scale = lw.o8_scale; f.m = t; f.n = H; f.k = na; f.lda8 = na; f.ldw8 = na; f.ldc = H;
@@ -598,8 +597,6 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
         return rc;
       }
     } else {
-      if (!rope_done && (rc = chatts_rope_kv_write(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab,
-                                                   d->w.sin_tab, pos0, pos0_dev, &kc, stream)) != 0) return rc;
       // long chunks: split the keys over 2 workgroups per (query tile, head) - one sequence has too few waves otherwise
       const int env_ks = opt_get(OPT_ATTN_KSPLIT, 0);
       // (the bf16x3 kernel is fast enough per tile that the second key split + its combine launch no longer pay: 73.3 us
@@ -609,9 +606,12 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
       if (chatts_attn_workspace(t, c.n_q, ks) > d->b.workspace_bytes) ks = 1;
       // ... and, on the plane path, let the attention kernel (or its combine) write o_proj's operand format itself
       const bool out_planes = t >= 16 && planes_path(d, t, c.n_q * kHeadDim) && opt_get(OPT_ATTN_ROWS, 0) == 0;
-      if ((rc = attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, out_planes ? d->b.planes_hi : nullptr,
-                               out_planes ? d->b.planes_lo : nullptr, ks, d->b.workspace, d->b.workspace_bytes, stream, out_planes && tile_attn ? t & ~15 : 0)) != 0)
-        return rc;
+      uint16_t *out_hi = out_planes ? d->b.planes_hi : nullptr, *out_lo = out_planes ? d->b.planes_lo : nullptr;
+      const int out_tiled = out_planes && tile_attn ? t & ~15 : 0;
+      rc = rope_done ? attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, out_hi, out_lo, ks, d->b.workspace, d->b.workspace_bytes, stream, out_tiled)
+                     : rope_attention_impl(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev, &kc, d->b.attn, out_hi, out_lo, ks,
+                                           d->b.workspace, d->b.workspace_bytes, stream, out_tiled);
+      if (rc != 0) return rc;
       attn_out_planes = out_planes;
     }
     // o_proj (+ residual, or partial sum for the TP all-reduce)
@@ -975,11 +975,8 @@ static int layer_part0_packed(ChattsDecoder* d, int layer, int t, const ChattsPr
     const ChattsPrefillSegment& sg = segs[i];
     ChattsKvCache kc = layer_cache(d, layer, sg.slot);
     float* q = d->b.qkv + (size_t)sg.row0 * qkv_n;
-    if ((rc = chatts_rope_kv_write(q, sg.t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, sg.pos0,
-                                   nullptr, &kc, stream)) != 0) return rc;
-    const int ks = 1;
-    if ((rc = attention_impl(q, sg.t, c.n_q, c.n_kv, sg.pos0, nullptr, &kc, d->b.attn + (size_t)sg.row0 * na, nullptr, nullptr, ks,
-                             d->b.workspace, d->b.workspace_bytes, stream)) != 0) return rc;
+    if ((rc = rope_attention_impl(q, sg.t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, sg.pos0, nullptr, &kc, d->b.attn + (size_t)sg.row0 * na,
+                                  nullptr, nullptr, 1, d->b.workspace, d->b.workspace_bytes, stream)) != 0) return rc;
   }
   if (f8) {
     uint8_t* b8 = reinterpret_cast<uint8_t*>(d->b.planes_lo);

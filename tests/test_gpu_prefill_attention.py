@@ -5,6 +5,8 @@ import pytest
 import torch
 
 from chatts_amd import _lib
+from chatts_amd.config import preset
+from chatts_amd.modeling import ChatTSForCausalLM
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -56,3 +58,39 @@ def test_every_form(lib, nq, nkv, T, pos0):
     got[T // 2, 1] = want[T // 2, 1]
     assert ((got - want).norm() / want.norm()).item() < 2e-5
     assert (got - want).abs().max().item() < 2e-5 * want.abs().max().item()
+
+
+@pytest.fixture(scope="module", params=["chatts-8b", "chatts-14b"])
+def model(request):
+    cfg = preset(request.param, num_hidden_layers=2, vocab_size=4096, ts_token_start_index=4000, eos_token_id=[4003, 4002], pad_token_id=4002)
+    return ChatTSForCausalLM.from_synthetic(cfg, seed=3, max_ctx=1024, max_prefill_tokens=512, max_batch=2, enable_prefix_caching=False)
+
+
+# portions that end inside a tile, at its end and one row behind it, the first of a prompt and later ones, two prompts at once
+@pytest.mark.parametrize("portions", [[64], [65, 96], [77, 223], [300, 64, 97], [512, 31, 481]])
+def test_rotation_in_the_planes_writer(model, portions):
+    """ROPE_FUSE=0 rotates all heads in a launch of its own.  Keys and values are the same bits, and without a norm of the queries everything is.  That norm adds its squares in another order: a
+    last bit of a query, which its split (2^-18) does not always keep."""
+    ids = torch.randint(0, 4000, (sum(portions) + 70,), generator=torch.Generator().manual_seed(len(portions))).tolist()
+
+    def run():
+        at = 0
+        for i, n in enumerate(portions):
+            rows = [(0, ids[at:at + n], [n - 1])]
+            if i == 0:
+                rows.append((1, ids[:70], [69]))
+            got = model.step_tokens(rows)[0].clone()
+            at += n
+        model.release_slot(0)
+        model.release_slot(1)
+        return got
+
+    with _lib.options(GEMM_SK=1):            # (a split's epilogue does the same work)
+        fused = run()
+        with _lib.options(ROPE_FUSE=0):
+            apart = run()
+    assert torch.isfinite(fused).all()
+    if model.config.model_type == "qwen2":
+        assert torch.equal(fused, apart)
+    else:
+        assert ((fused - apart).norm() / apart.norm()).item() < 2e-5
