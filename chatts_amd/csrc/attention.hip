@@ -678,32 +678,40 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_bf16x3_kernel(AttnParams 
 // ---------------------------------------------------------------------------------------------------
 // Bound by the round trip to the cache for a few hundred keys, by bytes for thousands.  A thread writes whole chunks and the lanes of a wave write next to each other; 8 bytes of V^T every
 // 64 took 5.1 / 8 / 18 us for 223 / 806 / 2048 keys of 8 heads, this 3.7 / 5.8 / 16.6 (with 16-byte loads of V the same).
-// a tile's planes from key4(key, d): K at dims d .. d + 3, and value(key, d): V
+// one chunk of a tile's planes: 8 dims of a key; 8 slots of a head dim - slot 8 g + j of chunk g is key 4 g + j or (from j = 4 on) 12 + 4 g + j
+__device__ __forceinline__ int v_slot_key(int g, int j) { return 4 * g + j + (j < 4 ? 0 : 12); }
+__device__ __forceinline__ void store_k_chunk(char* dst, int key, int chunk, const float (&x)[8]) {
+  abf16x8_t h, l;
+  split8(x, h, l);
+  char* to = dst + key * 256 + ((chunk ^ (key & 15)) << 4);
+  *reinterpret_cast<abf16x8_t*>(to) = h;
+  *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
+}
+__device__ __forceinline__ void store_v_chunk(char* dst, int d, int g, const float (&x)[8]) {
+  abf16x8_t h, l;
+  split8(x, h, l);
+  char* to = dst + 16384 + d * 64 + ((g ^ ((d >> 2) & 2)) << 4);
+  *reinterpret_cast<abf16x8_t*>(to) = h;
+  *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
+}
+// a tile's planes from key4(key, d): K at dims d .. d + 3, and value(key, d): V.  Thread = (key, chunk) and (head dim, chunk), two of each
 template <typename K4, typename V1>
 __device__ __forceinline__ void store_kv_planes(char* dst, int tid, K4 key4, V1 value) {
   f32x4 kv[2][2];
   float vv[2][8];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)                               // K: thread = (key, chunk of 8 dims), rows stay rows
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int h = 0; h < 2; ++h) kv[i][h] = key4((tid >> 4) + i * 16, (tid & 15) * 8 + h * 4);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)                               // V transposed: thread = (head dim, chunk g of 8 slots); slot 8 g + j of chunk g is key 4 g + j or (from j = 4 on) 12 + 4 g + j
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) vv[i][j] = value(4 * (tid & 3) + j + (j < 4 ? 0 : 12), (tid >> 2) + i * 64);
+    for (int j = 0; j < 8; ++j) vv[i][j] = value(v_slot_key(tid & 3, j), (tid >> 2) + i * 64);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int key = (tid >> 4) + i * 16, d = (tid >> 2) + i * 64;
     const float x[8] = {kv[i][0].x, kv[i][0].y, kv[i][0].z, kv[i][0].w, kv[i][1].x, kv[i][1].y, kv[i][1].z, kv[i][1].w};
-    abf16x8_t h, l;
-    split8(x, h, l);
-    char* to = dst + key * 256 + (((tid & 15) ^ (key & 15)) << 4);
-    *reinterpret_cast<abf16x8_t*>(to) = h;
-    *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
-    split8(vv[i], h, l);
-    to = dst + 16384 + d * 64 + (((tid & 3) ^ ((d >> 2) & 2)) << 4);
-    *reinterpret_cast<abf16x8_t*>(to) = h;
-    *reinterpret_cast<abf16x8_t*>(to + 8192) = l;
+    store_k_chunk(dst, (tid >> 4) + i * 16, tid & 15, x);
+    store_v_chunk(dst, (tid >> 2) + i * 64, tid & 3, vv[i]);
   }
 }
 
@@ -761,6 +769,112 @@ __global__ __launch_bounds__(256) void rope_kv_planes_kernel(const float* __rest
   __syncthreads();
   store_kv_planes(reinterpret_cast<char*>(planes) + ((size_t)hk * gridDim.x + kt) * (8 * KT * kHeadDim), tid, [&](int key, int d) { return *reinterpret_cast<const f32x4*>(k_s + key * LD + d); },
                   [&](int key, int d) { return v_s[key * LD + d]; });
+}
+
+// x[i] += the slabs' values at at[i], slab after slab
+template <int N>
+__device__ __forceinline__ void sum_slabs(const float* __restrict__ slabs, int sk, size_t plane, const size_t (&at)[N], float (&x)[N]) {
+  int s = 0;
+  for (; s + 4 <= sk; s += 4) {
+    float t[4][N];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < N; ++i) t[u][i] = slabs[(s + u) * plane + at[i]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < N; ++i) x[i] += t[u][i];
+  }
+  for (; s < sk; ++s)
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] += slabs[s * plane + at[i]];
+}
+
+// ... and as a split's epilogue (splitk_epilogue_rope_kernel's work; the planes lie behind the slabs): four workgroups a tile and kv head, one for each half of K's keys (a rotation takes a whole
+// row) and of V's dims (a chunk takes 8 keys), the others a query head a wave.  One workgroup for a whole tile reads up to 400 KB of slabs by itself: 6 us.  Prompts, us, two launches / here: 8B of 223
+// rows 8363 / 8235, 14B of 430 19440 / 19330, 8B of 96 6100 / 6060, 14B of 66 the same.
+__global__ __launch_bounds__(256) void rope_epilogue_planes_kernel(const float* __restrict__ slabs, int sk, int m, int n, const float* __restrict__ bias, float* __restrict__ c, int ldc, RopeFuse r,
+                                                                   int tiles, uint16_t* __restrict__ planes) {
+  constexpr int KT = 32, LDK = kHeadDim + 4, LDV = kHeadDim / 2 + 4;
+  __shared__ __attribute__((aligned(16))) float rows_s[16 * LDK > KT * LDV ? 16 * LDK : KT * LDV];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), item = (int)blockIdx.x - tiles * r.n_kv * 4;
+  const size_t plane = (size_t)m * n;
+  if (item >= 0) {
+    const int gw = item * 4 + wave;
+    if (gw >= m * r.n_q) return;
+    const int tok = gw / r.n_q, h = gw - tok * r.n_q;
+    float x[2] = {0.f, 0.f};
+    const size_t from = (size_t)tok * n + h * kHeadDim + lane, at[2] = {from, from + 64};
+    sum_slabs(slabs, sk, plane, at, x);
+    if (bias) { x[0] += bias[h * kHeadDim + lane]; x[1] += bias[h * kHeadDim + lane + 64]; }
+    rope_kv_head(x[0], x[1], h, r.pos0 + tok, lane, c + (size_t)tok * ldc + h * kHeadDim, r);
+    return;
+  }
+  const int half = blockIdx.x & 1, is_v = (blockIdx.x >> 1) & 1, kt = (int)(blockIdx.x >> 2) % tiles, hk = (int)(blockIdx.x >> 2) / tiles, last = r.pos0 + m - 1 - kt * KT;
+  const int col = (r.n_q + hk + (is_v ? r.n_kv : 0)) * kHeadDim;      // the head's columns
+  const size_t toff = kv_tile_off(r.kvl, hk, kt * KT);
+  char* dst = reinterpret_cast<char*>(planes) + ((size_t)hk * tiles + kt) * (8 * KT * kHeadDim);
+  const bool any = kt * KT + (last < KT - 1 ? last : KT - 1) >= r.pos0;      // of the chunk's rows; those before them come from the cache, rows past the last key repeat it
+  float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  size_t at[8];
+  if (is_v) {                                               // 8 keys a wave, 64 dims
+    const int d = half * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int key = wave * 8 + i, kr = key <= last ? key : last, tok = kt * KT + kr - r.pos0;
+      at[i] = (size_t)(tok > 0 ? tok : 0) * n + col + d;
+    }
+    if (any) sum_slabs(slabs, sk, plane, at, x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int key = wave * 8 + i, kr = key <= last ? key : last;
+      float* row = r.vc + toff + (size_t)kr * kHeadDim + d;
+      if (kt * KT + kr >= r.pos0) {                         // (uniform)
+        if (bias) x[i] += bias[col + d];
+        x[i] = kv_round_f(x[i], r.kv_round);
+        if (key <= last) *row = x[i];
+      } else {
+        x[i] = *row;
+      }
+      rows_s[key * LDV + lane] = x[i];
+    }
+    __syncthreads();
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = rows_s[v_slot_key(tid & 3, j) * LDV + (tid >> 2)];
+    store_v_chunk(dst, half * 64 + (tid >> 2), tid & 3, o);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                             // four keys a wave
+    const int key = half * 16 + wave * 4 + i, kr = key <= last ? key : last, tok = kt * KT + kr - r.pos0;
+    at[2 * i] = (size_t)(tok > 0 ? tok : 0) * n + col + lane;
+    at[2 * i + 1] = at[2 * i] + 64;
+  }
+  if (any) sum_slabs(slabs, sk, plane, at, x);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k16 = wave * 4 + i, key = half * 16 + k16, kr = key <= last ? key : last, pos = kt * KT + kr;
+    float a = x[2 * i], b = x[2 * i + 1], *row = r.kc + toff + (size_t)kr * kHeadDim + lane;
+    if (pos >= r.pos0) {                                    // (uniform)
+      if (bias) { a += bias[col + lane]; b += bias[col + lane + 64]; }
+      norm_rope(a, b, r.k_norm_w, r.eps, r.cos_tab[(size_t)pos * 64 + lane], r.sin_tab[(size_t)pos * 64 + lane], lane);
+      a = kv_round_f(a, r.kv_round);
+      b = kv_round_f(b, r.kv_round);
+      if (key <= last) { row[0] = a; row[64] = b; }
+    } else {
+      a = row[0];
+      b = row[64];
+    }
+    rows_s[k16 * LDK + lane] = a;
+    rows_s[k16 * LDK + lane + 64] = b;
+  }
+  __syncthreads();
+  float o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = rows_s[(tid >> 4) * LDK + (tid & 15) * 8 + j];
+  store_k_chunk(dst, half * 16 + (tid >> 4), tid & 15, o);
 }
 
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -1209,13 +1323,19 @@ static int bind_cache(AttnParams& p, const ChattsKvCache* cache) {
 
 namespace chatts {
 int attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev, const ChattsKvCache* cache, float* out,
-                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr);
+                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr,
+                   const uint16_t* planes = nullptr);
 
 // The attention on K / V planes: the positions known here, keys in one split, the caller's workspace free and large enough for the planes
-static size_t prefill_plane_bytes(int n_keys, int n_kv) { return (size_t)((n_keys + 31) / 32) * n_kv * 4 * 32 * kHeadDim * sizeof(uint16_t); }
-static bool prefill_on_planes(int t, int n_kv, int pos0, const int32_t* pos0_dev, bool out_planes, int n_splits, const void* workspace, size_t workspace_bytes) {
+bool prefill_on_planes(int t, int n_kv, int pos0, const int32_t* pos0_dev, bool out_planes, int n_splits, const void* workspace, size_t workspace_bytes) {
   return opt_get(OPT_ATTN_BF16X3, 1) != 0 && opt_get(OPT_ATTN_PLANES, 1) != 0 && (opt_get(OPT_ATTN_ROWS, 0) == 0 || out_planes) && !pos0_dev && n_splits == 1 && t >= 64 && workspace &&
          workspace_bytes >= prefill_plane_bytes(pos0 + t, n_kv) && ((uintptr_t)workspace % 16) == 0;
+}
+int launch_rope_epilogue_planes(const float* slabs, int sk, int m, int n, const float* bias, float* c, int ldc, const RopeFuse& r, uint16_t* planes, hipStream_t s) {
+  const int tiles = (r.pos0 + m + 31) / 32;
+  hipLaunchKernelGGL(rope_epilogue_planes_kernel, dim3(tiles * r.n_kv * 4 + (m * r.n_q + 3) / 4), dim3(256), 0, s, slabs, sk, m, n, bias, c, ldc, r, tiles, planes);
+  CHATTS_CHECK_LAUNCH("rope_epilogue_planes");
+  return CHATTS_OK;
 }
 // chatts_rope_kv_write and chatts_attention, in one launch fewer and without the queries' way through memory where the planes' writer can do the keys' and values' part
 int rope_attention_impl(float* qkv, int t, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w, float norm_eps, const float* cos_tab, const float* sin_tab, int pos0,
@@ -1243,7 +1363,7 @@ extern "C" int chatts_attention(const float* qkv, int t, int n_q, int n_kv, int 
 // Planes are written by the MFMA kernel / its combine only (t >= 16, n_splits <= 4): the caller checks that.
 int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev,
                            const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits,
-                           void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled, const RopeFuse* rope) {
+                           void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled, const RopeFuse* rope, const uint16_t* planes) {
   CHATTS_REQUIRE(t >= 0 && n_q > 0 && n_kv > 0 && n_splits >= 1 && n_splits <= kMaxSlots, CHATTS_E_BADARG,
                  "attention: bad sizes");
   if (t == 0) return CHATTS_OK;
@@ -1270,7 +1390,9 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
     const int n_keys = pos0 + t, tiles = (n_keys + 31) / 32;
     if (prefill_on_planes(t, n_kv, pos0, pos0_dev, out_hi != nullptr, n_splits, workspace, workspace_bytes)) {
       uint16_t* pl = static_cast<uint16_t*>(workspace);
-      if (rope) {      // (rope_attention_impl: rows of qkv as the projection left them)
+      if (planes) {      // (launch_rope_epilogue_planes has written them)
+        pl = const_cast<uint16_t*>(planes);
+      } else if (rope) {      // (rope_attention_impl: rows of qkv as the projection left them)
         p.q_norm_w = rope->q_norm_w; p.cos_tab = rope->cos_tab; p.sin_tab = rope->sin_tab; p.eps = rope->eps;
         hipLaunchKernelGGL(rope_kv_planes_kernel, dim3(tiles, n_kv), dim3(256), 0, as_stream(stream), qkv, *rope, n_keys, pl);
       } else {

@@ -337,6 +337,16 @@ __device__ __forceinline__ void rope_kv_head(float a, float b, int h, int pos, i
     dst[lane + 64] = kv_round_f(ob, r.kv_round);
   }
 }
+// What became of a RopeFuse that went with a projection: in, whether the attention behind it reads K / V planes (prefill_on_planes); out, whether the rows are rotated and stored, and the planes,
+// where the split's epilogue wrote them, too (in the workspace, behind its slabs)
+struct RopeDone {
+  bool want_planes, rotated;
+  uint16_t* planes;
+};
+// (attention.hip)
+inline size_t prefill_plane_bytes(int n_keys, int n_kv) { return (size_t)((n_keys + 31) / 32) * n_kv * 4 * 32 * kHeadDim * sizeof(uint16_t); }
+bool prefill_on_planes(int t, int n_kv, int pos0, const int32_t* pos0_dev, bool out_planes, int n_splits, const void* workspace, size_t workspace_bytes);
+int launch_rope_epilogue_planes(const float* slabs, int sk, int m, int n, const float* bias, float* c, int ldc, const RopeFuse& r, uint16_t* planes, hipStream_t s);
 // host: validate the arguments of chatts_rope_kv_write and fill a RopeFuse (elementwise.hip)
 int rope_fuse_prepare(int t, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w, float norm_eps, const float* cos_tab,
                       const float* sin_tab, int pos0, const int32_t* pos0_dev, const ChattsKvCache* cache, RopeFuse* out);

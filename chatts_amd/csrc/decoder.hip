@@ -15,7 +15,7 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s);
 int launch_gemm_f32(const ChattsLinearArgs* a, hipStream_t s);
 bool gemm_batched_stream(const ChattsLinearArgs* a);
 size_t gemm_workspace_batch(int m, int n, int k, int batch);
-int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain, PlaneTiles tiles);
+int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles);
 int gemm_post_ss_parts(const ChattsLinearArgs* a);
 int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
 bool gemm_takes_cols(const ChattsLinearArgs* a);
@@ -27,7 +27,8 @@ int rope_attention_impl(float* qkv, int t, int n_q, int n_kv, const float* q_nor
                         const int32_t* pos0_dev, const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes,
                         chatts_stream_t stream, int out_tiled = 0);
 int attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0, const int32_t* pos0_dev, const ChattsKvCache* cache, float* out,
-                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr);
+                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, int out_tiled = 0, const RopeFuse* rope = nullptr,
+                   const uint16_t* planes = nullptr);
 int launch_split_bf16x2(const float* x, int m, int k, int ldx, uint16_t* hi, uint16_t* lo, int ldp, int tiled, hipStream_t s);
 size_t gemm_workspace(int m, int n, int k);
 }  // namespace chatts
@@ -62,7 +63,7 @@ struct ChattsDecoder {
 static int64_t embed_rows(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_rows : d->cfg.vocab_local; }
 static int64_t embed_offset(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_offset : d->cfg.vocab_offset; }
 
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain = nullptr, PlaneTiles tiles = {});
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain = nullptr, PlaneTiles tiles = {});
 extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream) {
   CHATTS_REQUIRE(a && ch, CHATTS_E_BADARG, "linear_chain: null args");
   CHATTS_REQUIRE(!ch->row_ss || (((uintptr_t)ch->row_ss % 16) == 0 && a->a_hi && a->a_lo && a->m >= 2 && a->m <= 16 && a->batch <= 1 && !a->exact_f32 && ch->row_ss_parts >= 1 &&
@@ -107,8 +108,8 @@ extern "C" int chatts_linear(const ChattsLinearArgs* a, chatts_stream_t stream) 
 int chatts::linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles) { return linear_impl(a, stream, nullptr, nullptr, nullptr, tiles); }
 
 // rope / rope_done: the qkv projection of a prefill chunk may carry rope_kv_kernel's work in its split-K epilogue (*rope_done says
-// whether it did; otherwise the caller launches chatts_rope_kv_write as before)
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
+// whether it did, and the planes of K and V with it; otherwise rope_attention_impl does both)
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
   CHATTS_REQUIRE(a != nullptr, CHATTS_E_BADARG, "linear: null args");
   CHATTS_REQUIRE(a->m >= 0 && a->n > 0 && a->k > 0, CHATTS_E_BADARG, "linear: bad sizes m=%d n=%d k=%d", a->m, a->n, a->k);
   if (a->m == 0) return CHATTS_OK;
@@ -579,12 +580,21 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
       if ((rc = norm_into(d, lw.input_norm, &la, stream, nullptr, &tile_h)) != 0) return rc;
     }
     ChattsKvCache kc = layer_cache(d, layer, d->cur_seq);
-    bool rope_done = false;
+    RopeDone rope_done{false, false, nullptr};
+    // long chunks: split the keys over 2 workgroups per (query tile, head) - one sequence has too few waves otherwise
+    // (the bf16x3 kernel is fast enough per tile that the second key split + its combine launch no longer pay: 73.3 us
+    // against 74.0 + 12 at T = 798; the float32-MFMA kernel, CHATTS_ATTN_BF16X3=0, still wants the split)
+    const int env_ks = opt_get(OPT_ATTN_KSPLIT, 0);
+    int ks = env_ks >= 1 && env_ks <= 4 ? env_ks : (t >= 256 && opt_get(OPT_ATTN_BF16X3, 1) == 0 ? 2 : 1);
+    if (chatts_attn_workspace(t, c.n_q, ks) > d->b.workspace_bytes) ks = 1;
+    // ... and, on the plane path, let the attention kernel (or its combine) write o_proj's operand format itself
+    const bool out_planes = t >= 16 && planes_path(d, t, c.n_q * kHeadDim) && opt_get(OPT_ATTN_ROWS, 0) == 0;
     const bool rope_fuse = opt_get(OPT_ROPE_FUSE, 1) != 0;
     if (t > 1 && rope_fuse) {   // prefill: the projection's split-K epilogue (when it has one) also rotates q / k and fills the cache
       RopeFuse rf;
       if ((rc = rope_fuse_prepare(t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev, &kc,
                                   &rf)) != 0) return rc;
+      rope_done.want_planes = prefill_on_planes(t, c.n_kv, pos0, pos0_dev, out_planes, ks, d->b.workspace, d->b.workspace_bytes);
       if ((rc = linear_impl(&la, stream, &rf, &rope_done, nullptr, {tile_h, false, false})) != 0) return rc;
     } else if ((rc = linear_tiled(&la, stream, {tile_h, false, false})) != 0) {
       return rc;
@@ -597,18 +607,10 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
         return rc;
       }
     } else {
-      // long chunks: split the keys over 2 workgroups per (query tile, head) - one sequence has too few waves otherwise
-      const int env_ks = opt_get(OPT_ATTN_KSPLIT, 0);
-      // (the bf16x3 kernel is fast enough per tile that the second key split + its combine launch no longer pay: 73.3 us
-      // against 74.0 + 12 at T = 798; the float32-MFMA kernel, CHATTS_ATTN_BF16X3=0, still wants the split)
-      const bool f32_attn = opt_get(OPT_ATTN_BF16X3, 1) == 0;
-      int ks = env_ks >= 1 && env_ks <= 4 ? env_ks : (t >= 256 && f32_attn ? 2 : 1);
-      if (chatts_attn_workspace(t, c.n_q, ks) > d->b.workspace_bytes) ks = 1;
-      // ... and, on the plane path, let the attention kernel (or its combine) write o_proj's operand format itself
-      const bool out_planes = t >= 16 && planes_path(d, t, c.n_q * kHeadDim) && opt_get(OPT_ATTN_ROWS, 0) == 0;
       uint16_t *out_hi = out_planes ? d->b.planes_hi : nullptr, *out_lo = out_planes ? d->b.planes_lo : nullptr;
       const int out_tiled = out_planes && tile_attn ? t & ~15 : 0;
-      rc = rope_done ? attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, out_hi, out_lo, ks, d->b.workspace, d->b.workspace_bytes, stream, out_tiled)
+      rc = rope_done.rotated ? attention_impl(d->b.qkv, t, c.n_q, c.n_kv, pos0, pos0_dev, &kc, d->b.attn, out_hi, out_lo, ks, d->b.workspace, d->b.workspace_bytes, stream, out_tiled,
+                                               nullptr, rope_done.planes)
                      : rope_attention_impl(d->b.qkv, t, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, pos0, pos0_dev, &kc, d->b.attn, out_hi, out_lo, ks,
                                            d->b.workspace, d->b.workspace_bytes, stream, out_tiled);
       if (rc != 0) return rc;

@@ -1064,7 +1064,7 @@ size_t gemm_workspace(int m, int n, int k) {
   return sk > 1 ? (size_t)sk * m * n * sizeof(float) : 0;
 }
 
-int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, bool* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
+int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
   int bm, sk;
   ChattsLinearArgs a_copy;
   const ChattsLinearArgs* a = a_in;
@@ -1242,11 +1242,16 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
   }
   if (sk > 1 && rope && rope_done && !post_norm && a->epilogue == CHATTS_EPI_NONE && !a->c_hi && !a->w8 &&
       a->n == (rope->n_q + 2 * rope->n_kv) * kHeadDim) {
+    rope_done->rotated = true;
+    const float* slabs = reinterpret_cast<const float*>(a->workspace);
+    const size_t planes_at = ((size_t)sk * a->m * a->n * sizeof(float) + 255) & ~(size_t)255;
+    if (rope_done->want_planes && ((uintptr_t)a->workspace % 16) == 0 && planes_at + prefill_plane_bytes(rope->pos0 + a->m, rope->n_kv) <= a->workspace_bytes) {
+      rope_done->planes = reinterpret_cast<uint16_t*>(static_cast<char*>(a->workspace) + planes_at);
+      return launch_rope_epilogue_planes(slabs, sk, a->m, a->n, a->bias, a->c, a->ldc, *rope, rope_done->planes, s);
+    }
     const int waves = a->m * (rope->n_q + 2 * rope->n_kv);
-    hipLaunchKernelGGL(splitk_epilogue_rope_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, reinterpret_cast<const float*>(a->workspace),
-                       sk, a->m, a->n, a->bias, a->c, a->ldc, *rope);
+    hipLaunchKernelGGL(splitk_epilogue_rope_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, slabs, sk, a->m, a->n, a->bias, a->c, a->ldc, *rope);
     CHATTS_CHECK_LAUNCH("splitk_epilogue_rope");
-    *rope_done = true;
     return CHATTS_OK;
   }
   const bool glu = epi_is_glu(a->epilogue);

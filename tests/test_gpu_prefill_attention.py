@@ -85,12 +85,21 @@ def test_rotation_in_the_planes_writer(model, portions):
         model.release_slot(1)
         return got
 
-    with _lib.options(GEMM_SK=1):            # (a split's epilogue does the same work)
-        fused = run()
-        with _lib.options(ROPE_FUSE=0):
-            apart = run()
+    same_bits(model, run, model.config.model_type == "qwen2")
+
+
+# a second chunk behind 512 rows: of 88, of 31 (too few for planes), of 481; split 1: the projection's own rows, 3: its split's epilogue, which rotates the queries, too
+@pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("n", [64, 65, 96, 127, 223, 512, 543, 600, 993])
+def test_rotation_behind_a_chunks_projection(model, n, split):
+    ids = torch.randint(0, 4000, (n,), generator=torch.Generator().manual_seed(n)).tolist()
+    with _lib.options(GEMM_SK=split):
+        same_bits(model, lambda: model.generate_one(ids, None, None, max_new_tokens=1, return_logits=True)[1].clone(), split > 1 or model.config.model_type == "qwen2")
+
+
+def same_bits(model, run, exactly):
+    fused = run()
+    with _lib.options(ROPE_FUSE=0):
+        apart = run()
     assert torch.isfinite(fused).all()
-    if model.config.model_type == "qwen2":
-        assert torch.equal(fused, apart)
-    else:
-        assert ((fused - apart).norm() / apart.norm()).item() < 2e-5
+    assert torch.equal(fused, apart) if exactly else ((fused - apart).norm() / apart.norm()).item() < 2e-5
