@@ -3,6 +3,8 @@
 // (NetManAIOps/ChatTS chatts/vllm/chatts_vllm.py:93-183): there, 2 .item() host syncs and ~10 tiny
 // torch ops per series; here one wave per series for the mask reduction and one wave per patch for
 // the feature row, no host sync.
+#include <type_traits>
+
 #include "common.h"
 #include "gemm_common.h"
 
@@ -240,22 +242,28 @@ constexpr int kL0Waves = 4, kL0Cols = 32;      // waves (16 rows each) of a work
 constexpr int kL0Known = 64;
 struct TsKnown {
   int32_t off[kL0Known], len[kL0Known];
-  int32_t n;               // 0: row_off and valid_len on the device
+  int32_t n;
   int64_t* patch_cnt;      // counts from the masks, by workgroups of their own (the last of grid.y), or NULL
 };
 
-template <int KSTEPS, int MODE>      // K-steps of 32 (feature count rounded up) and the feature mode: compiled in, so that every load is in flight at once
+struct TsOnDevice {        // row_off and valid_len (an instance of its own: one that takes either is 0.8 us of 28 slower for them)
+  static constexpr int32_t n = 0;
+};
+
+template <int KSTEPS, int MODE, typename LENGTHS>      // K-steps of 32 (feature count rounded up) and the feature mode: compiled in, so that every load is in flight at once
 __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatchifyArgs a, unsigned emb8_inv, const uint16_t* w0, int ldw, const float* b0, int hidden, int steps_each,
-                                                                     uint16_t* out_hi, uint16_t* out_lo, int ld_out, int tiled, TsKnown known) {
+                                                                     uint16_t* out_hi, uint16_t* out_lo, int ld_out, int tiled, LENGTHS known) {
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+  constexpr bool KNOWN = std::is_same<LENGTHS, TsKnown>::value;
   // W0 of a step: 32 rows of 4 KSTEPS 16-byte chunks, twice.  Chunk c of a K-step of row r lies at place c ^ (r >> turn): eight rows' chunks then meet
   // different banks whatever KSTEPS makes of the row's length
   constexpr int ROW = 4 * KSTEPS, PIECES = 2 * KSTEPS, TURN = KSTEPS % 2 ? 2 : (KSTEPS % 4 ? 1 : 0);
   __shared__ __attribute__((aligned(1024))) char smem[2][PIECES * 1024];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r0 = ((int)blockIdx.y * kL0Waves + wave) * 16;
-  if ((int)blockIdx.y * kL0Waves * 16 >= a.total_patches) {    // (a whole workgroup)
-    for (int i = (int)blockIdx.x * kL0Waves + wave; i < known.n; i += (int)gridDim.x * kL0Waves) ts_count_series(a.series, i, a.lmax, a.patch_size, lane, nullptr, known.patch_cnt);
+  if (KNOWN && (int)blockIdx.y * kL0Waves * 16 >= a.total_patches) {      // (a whole workgroup)
+    if constexpr (KNOWN)
+      for (int i = (int)blockIdx.x * kL0Waves + wave; i < known.n; i += (int)gridDim.x * kL0Waves) ts_count_series(a.series, i, a.lmax, a.patch_size, lane, nullptr, known.patch_cnt);
     return;
   }
   const bool mine = r0 < a.total_patches;                      // (else a wave that only fetches W0)
@@ -279,8 +287,10 @@ __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatch
   const int nser = a.n_series;
   int p = r0 + frow;
   if (p > a.total_patches - 1) p = a.total_patches - 1;
+  const int my_off = KNOWN ? 0 : a.row_off[lane <= nser ? lane : nser];      // (requested before the branch)
+  const int my_vl = KNOWN ? 0 : a.valid_len[lane < nser ? lane : nser - 1];
   int sidx = 0, off = 0, vl = 0;
-  if (known.n) {
+  if constexpr (KNOWN) {
     for (int i0 = 0; i0 < known.n; i0 += 16)
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
@@ -291,8 +301,6 @@ __global__ __launch_bounds__(64 * kL0Waves, 3) void ts_layer0_kernel(ChattsPatch
         vl = at ? l : vl;
       }
   } else if (nser <= 63) {
-    const int my_off = a.row_off[lane <= nser ? lane : nser];
-    const int my_vl = a.valid_len[lane < nser ? lane : nser - 1];
     for (int i = 1; i < nser; ++i) sidx += __builtin_amdgcn_readlane(my_off, i) <= p ? 1 : 0;
     off = __shfl(my_off, sidx, 64);
     vl = __shfl(my_vl, sidx, 64);
@@ -531,7 +539,8 @@ static int ts_encode(const float* series, const int32_t* lengths, int32_t* row_o
     const dim3 grid((steps + steps_each - 1) / steps_each, groups + (known.n && known.patch_cnt ? 1 : 0)), block(64 * kL0Waves);
     uint16_t* oh = hi_of(h0);
     uint16_t* ol = lo_of(h0, H);
-#define CHATTS_TS_L0(KS, MD) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD>), grid, block, 0, as_stream(stream), pa, emb8_inv, w->w[0], w->in_features_pad, w->b[0], H, steps_each, oh, ol, H, tile ? P & ~15 : 0, known)
+#define CHATTS_TS_L0_OF(KS, MD, L, known) hipLaunchKernelGGL((ts_layer0_kernel<KS, MD, L>), grid, block, 0, as_stream(stream), pa, emb8_inv, w->w[0], w->in_features_pad, w->b[0], H, steps_each, oh, ol, H, tile ? P & ~15 : 0, known)
+#define CHATTS_TS_L0(KS, MD) if (known.n) CHATTS_TS_L0_OF(KS, MD, TsKnown, known); else CHATTS_TS_L0_OF(KS, MD, TsOnDevice, TsOnDevice{})
     if (w->mode == 1) {
       switch (ksteps) {
         case 1: CHATTS_TS_L0(1, 1); break;
@@ -546,11 +555,12 @@ static int ts_encode(const float* series, const int32_t* lengths, int32_t* row_o
         default: CHATTS_TS_L0(10, 1); break;
       }
     } else if (w->mode == 2) {
-      if (ksteps == 1) CHATTS_TS_L0(1, 2); else CHATTS_TS_L0(2, 2);
+      if (ksteps == 1) { CHATTS_TS_L0(1, 2); } else { CHATTS_TS_L0(2, 2); }
     } else {
-      if (ksteps == 1) CHATTS_TS_L0(1, 0); else CHATTS_TS_L0(2, 0);
+      if (ksteps == 1) { CHATTS_TS_L0(1, 0); } else { CHATTS_TS_L0(2, 0); }
     }
 #undef CHATTS_TS_L0
+#undef CHATTS_TS_L0_OF
     CHATTS_CHECK_LAUNCH("ts_layer0");
     cur = h0;
     k = H;
