@@ -10,8 +10,8 @@
 // epilogue arithmetic (bias / GELU / residual / SwiGLU / fp8 row scale / plane output / split-K partials), and therefore produce
 // bit-identical results at equal split-K:
 //   gemm_bf16x2_kernel  register-staged, BM x 128 x 32 tiles, A split on the VALU while staging; any M, float32 A;
-//                       TS-encoder MLP, prefill chunks below 96 rows, generic callers
-//   gemm_ring_kernel    (gemm_ring.hip) prefill (M >= 96) on pre-split planes: persistent workgroups, balanced M-tiles x 256 columns,
+//                       callers with float32 A and rows for which planes do not pay (kMidPlanesK)
+//   gemm_ring_kernel    (gemm_ring.hip) prefill (M > 16) on pre-split planes: persistent workgroups, balanced M-tiles x 256 columns,
 //                       4 loader waves feeding a ring of four 32-deep half-stages by LDS-DMA, 8 compute waves
 //   gemm_stream_kernel  batched decode (2 <= M <= 16) on planes: 16 x 128 x 64 (128 for fp8 W), weight-streaming shape
 // The comments above each kernel say which measurement made it look the way it does.

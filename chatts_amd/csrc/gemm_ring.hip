@@ -1,4 +1,4 @@
-// gemm_ring.hip - the prefill projection (M >= 96 rows on pre-split bf16 hi / lo planes of A):  C = epilogue(A . W^T), bf16x2.
+// gemm_ring.hip - the prefill projection (M > 16 rows on pre-split bf16 hi / lo planes of A):  C = epilogue(A . W^T), bf16x2.
 // Round 5 rebuild of the LDS-DMA kernel (gemm_dma_kernel, round 1-4).  What the round-5 timeline probe of that kernel showed
 // (tools/gemm_probe.py, profiles/r5_gemm_probe_before.txt) and what this kernel does about it:
 //

@@ -167,7 +167,7 @@ class ChatTSForCausalLM(SlotModel):
         self.t_max = int(max(min(max_prefill_tokens, self.max_ctx), self.max_batch))
         # a second copy of the four projection matrices of every layer in the prefill kernel's tiled layout (chatts_tile_bf16: its LDS-DMA
         # pieces then read consecutive memory; bit-identical results, prefill projections -4 %, profiles/r6_tiled_check.txt).  None = when
-        # a prefill chunk can reach that kernel (>= 96 rows) and CHATTS_TILED_WEIGHTS != 0; costs the bf16 weight bytes once more.
+        # a prefill chunk can reach that kernel with more than a few rows (>= 96) and CHATTS_TILED_WEIGHTS != 0; costs the bf16 weight bytes once more.
         if prefill_tiled_weights is None:
             prefill_tiled_weights = self.t_max >= 96 and os.environ.get("CHATTS_TILED_WEIGHTS", "1") != "0" and self.precision != "f16q"
         self.prefill_tiled_weights = bool(prefill_tiled_weights)

@@ -239,7 +239,7 @@ typedef struct ChattsLinearArgs {
    * without the partial vector's round trip and without the stand-alone exchange launch.  n <= chatts_tp_max_elems(comm).  Every rank
    * must issue the same call (same N, same launch geometry) - like any collective. */
   ChattsTpComm* tp_reduce;
-  /* optional (prefill kernel only, i.e. planes given and M >= 96): the same bf16 matrix as `w` in the tiled layout of chatts_tile_bf16
+  /* optional (prefill kernel only, i.e. planes given and M >= 96 or no float32 A): the same bf16 matrix as `w` in the tiled layout of chatts_tile_bf16
    * (ldw == K).  The prefill kernel is bound by its operand feed, and an LDS-DMA piece of 16 rows x 64 bytes uses half of each of the 16
    * cache lines it touches (profiles/r6_feed_probe.txt: 18 B/clk/CU against 27-30 for 1 KB of consecutive memory).  Same products, same
    * order: bit-identical results.  planes_tiled != 0: a_hi / a_lo are in that layout as well (ld_planes ignored; every kernel other than
@@ -693,7 +693,7 @@ typedef struct ChattsDecoderBuffers {
   int t_max;
   int max_batch;      /* KV caches are [max_batch, n_layers, n_kv, max_ctx, 128]; 0 or 1 = single sequence */
   /* optional: two pairs of bf16 hi / lo planes, each plane [T_max, max(H, n_q*128, inter)] (ChattsLinearArgs.a_hi /
-   * a_lo / c_hi / c_lo).  When all four are set, prefill chunks of >= 96 rows run the LDS-DMA GEMM: the RMSNorms and
+   * a_lo / c_hi / c_lo).  When all four are set, prefill chunks of more than 16 rows run on planes (the LDS-DMA GEMM; weight streaming up to 64 or 128 rows): the RMSNorms and
    * the SwiGLU epilogue write planes directly (pair 0 = projection input, pair 1 = gate_up output).  Batched steps of 2 .. 16 sequences use both pairs in
    * turn: what a projection hands on lies in the pair that it does not read. */
   chatts_bf16* planes_hi;
