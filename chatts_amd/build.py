@@ -1,7 +1,6 @@
 """Build libchatts_amd.so (hand-written HIP for gfx950) in-tree with hipcc.
 
-The .so is git-ignored but travels to the GPU box with the gpurun snapshot.  hipcc cross-compiles
-without a GPU, so this also runs in the CPU-only build container (`__graft_entry__.build()`).
+The .so is git-ignored.  hipcc cross-compiles without a GPU, so this also runs where there is none (`__graft_entry__.build()`).
 """
 import hashlib
 import os
