@@ -868,6 +868,7 @@ __global__ __launch_bounds__(1024) void splitk_epilogue_ss_kernel(const float* w
 // The qkv projection's split-K epilogue that also does rope_kv_kernel's work (prefill): one wave per (token, head) sums the head's
 // 128 columns over the slabs in split order, adds the bias - splitk_epilogue_kernel's arithmetic - and hands the two values per lane
 // to rope_kv_head: q rotated into c, K / V rows into the cache.  One pass over the [T, 7168] rows less per layer.
+// (Where the attention reads K / V planes and the workspace has room for them behind the slabs, rope_epilogue_planes_kernel does it and writes them.)
 __global__ __launch_bounds__(256) void splitk_epilogue_rope_kernel(const float* __restrict__ ws, int sk, int m, int n,
                                                                   const float* __restrict__ bias, float* __restrict__ c, int ldc,
                                                                   RopeFuse r) {
