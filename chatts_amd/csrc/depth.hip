@@ -14,7 +14,7 @@ struct DepthChoose {
 };
 
 // a thread keeps its columns in registers.  NT: threads (more of them for a few rows: then every load of a row is in flight at once)
-// NR > 0 (few rows): the same launch multiplies the row by the router, as the planes that it writes, and chooses its experts.  A projection, its split's epilogue and a workgroup that chose
+// NR > 0 (2 to 16 rows): the same launch multiplies the row by the router, as the planes that it writes, and chooses its experts.  A projection, its split's epilogue and a workgroup that chose
 // for all rows and made lists of them were three launches: 12.5 us a layer of 32 experts at 16 rows of 2048, now 1.  The router's first K-steps are requested before the row is there.
 template <int NT, int NV, int NR = 0>
 __global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch, int tiled) {

@@ -161,7 +161,7 @@ int launch_cols(const GemmParams& p, const ChattsLinearArgs* a, hipStream_t s);
 // chatts_rmsnorm_planes on rows that lie ldx apart (elementwise.hip)
 int launch_rmsnorm_planes(const float* x, int ldx, const float* w, uint16_t* hi, uint16_t* lo, int ld_planes, int t, int hidden, float eps, int tiled, hipStream_t s);
 
-// moe.hip: a feed-forward of the experts' kind beside them, for all rows, in their launches (up to 16 rows): up as gate_up of an expert, f = its activations [rows, ff], y [rows, width_p]
+// moe.hip: a feed-forward of the experts' kind beside them, for all rows, in their launches (2 to 16 rows): up as gate_up of an expert, f = its activations [rows, ff], y [rows, width_p]
 struct MoeBeside {
   const chatts_bf16 *up, *up_t, *down, *down_t;
   int ff;
@@ -170,7 +170,7 @@ struct MoeBeside {
   float limit, alpha;      // CHATTS_EXPERT_CLAMPGLU
 };
 bool moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh);
-// direct: no lists.  A pair of a row and a choice is its own place (row * top + choice; order, offsets and tiles are not read), an expert's launch blocks find its pairs in ids.  For up
+// direct: no lists.  A pair of a row and a choice is its own place (row * top + choice; order, offsets and tiles are not read), an expert's launch blocks find its pairs in ids.  For 2 to 16 rows, up
 // to 64 pairs and outputs, no choice groups (moe_takes_choice); ids, weight, place and kept then come from the norm before the router (depth.hip)
 bool moe_takes_choice(const ChattsMoeArgs* a);
 int depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t stream);      // chatts_depth_norm; tiles: the operand's planes as plane_at has them, whole blocks of 16 rows in tiles

@@ -571,7 +571,7 @@ static void launch_moe_stream_as(const ChattsMoeArgs* a, const MoeBeside& sh, in
   else hipLaunchKernelGGL((moe_stream_kernel<STEP, false, NW, RF>), g, b, 0, s, *a, sh, sh_blocks, nx);
 }
 // Few workgroups: smaller ones, so that the CUs get as much each, and more waves in each.  Waves of a workgroup, a step of Muvetar 2048 wide, us (gated / down): 16 sequences 4 / 16 931,
-// 8 / 16 898, 8 / 8 892, 4 / 4 977, 16 / 16 949; 2 sequences 8 / 16 629, 8 / 8 647; 4096 wide, 16 sequences 4 / 16 2240, 8 / 8 2177, one 8 / 16 1125, 8 / 8 1150.
+// 8 / 16 898, 8 / 8 892, 4 / 4 977, 16 / 16 949; 2 sequences 8 / 16 629, 8 / 8 647; 4096 wide, 16 sequences 4 / 16 2240, 8 / 8 2177.
 template <int STEP>
 static void launch_moe_stream(const ChattsMoeArgs* a, const MoeBeside& sh, int n, int tiles, hipStream_t s) {
   if constexpr (moe_pairs(STEP)) {
@@ -623,11 +623,12 @@ extern "C" int chatts_moe_route(const ChattsMoeArgs* a, chatts_stream_t stream) 
   return CHATTS_OK;
 }
 
+// (one row goes through launches of its own in both: there the router and the feed-forward beside the experts take float32, and here they would take two bf16 parts of it)
 bool chatts::moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh) {
-  return moe_small(a) && sh.up && sh.down && sh.f_hi && sh.f_lo && sh.y && sh.ff % 64 == 0 && a->width_p % 64 == 0 && !sh.up_t == !a->gate_up_t && !sh.down_t == !a->down_t;
+  return moe_small(a) && a->n_rows > 1 && sh.up && sh.down && sh.f_hi && sh.f_lo && sh.y && sh.ff % 64 == 0 && a->width_p % 64 == 0 && !sh.up_t == !a->gate_up_t && !sh.down_t == !a->down_t;
 }
 bool chatts::moe_takes_choice(const ChattsMoeArgs* a) {
-  return moe_small(a) && a->n_rows * a->top <= 64 && a->experts + a->identity <= 64 && a->keep >= a->groups;
+  return moe_small(a) && a->n_rows > 1 && a->n_rows * a->top <= 64 && a->experts + a->identity <= 64 && a->keep >= a->groups;
 }
 extern "C" int chatts_moe_experts(const ChattsMoeArgs* a, chatts_stream_t stream) { return moe_experts(a, MoeBeside{}, false, stream); }
 int chatts::moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, bool direct, chatts_stream_t stream) {
