@@ -1383,12 +1383,14 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
     if (rc) return rc;
   }
   const bool force_rows = opt_get(OPT_ATTN_ROWS, 0) != 0;   // debugging aid: VALU kernel for every T
-  if (t >= 16 && n_splits <= 4 && (!force_rows || out_hi)) {
+  // rope / planes: prefill_on_planes has been asked, and nothing else can take these rows (not again: options may change beside a running call)
+  const bool on_planes = rope || planes;
+  if (t >= 16 && n_splits <= 4 && (!force_rows || out_hi || on_planes)) {
     // (64-key tiles were measured too: 155 us vs 148 us at T = 798 - the per-tile work is not what is slow)
     const int bf16x3 = opt_get(OPT_ATTN_BF16X3, 1);      // 0: the float32-MFMA kernel
     // K / V split into bf16 planes once (kv_planes_kernel) when the caller's workspace is free (one key split) and holds them
     const int n_keys = pos0 + t, tiles = (n_keys + 31) / 32;
-    if (prefill_on_planes(t, n_kv, pos0, pos0_dev, out_hi != nullptr, n_splits, workspace, workspace_bytes)) {
+    if (on_planes || prefill_on_planes(t, n_kv, pos0, pos0_dev, out_hi != nullptr, n_splits, workspace, workspace_bytes)) {
       uint16_t* pl = static_cast<uint16_t*>(workspace);
       if (planes) {      // (launch_rope_epilogue_planes has written them)
         pl = const_cast<uint16_t*>(planes);

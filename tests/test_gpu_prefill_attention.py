@@ -60,6 +60,41 @@ def test_every_form(lib, nq, nkv, T, pos0):
     assert (got - want).abs().max().item() < 2e-5 * want.abs().max().item()
 
 
+# rows that are not rotated yet, planes that a projection's epilogue has written: what chose them for this path stays chosen, also when an option changes beside the call
+@pytest.mark.parametrize("option,value", [("ATTN_PLANES", 0), ("ATTN_BF16X3", 0), ("ATTN_ROWS", 1)])
+@pytest.mark.parametrize("written", [False, True])
+def test_the_path_is_chosen_once(lib, option, value, written):
+    attend, prepare = (getattr(lib, n) for n in ("_ZN6chatts14attention_implEPKfiiiiPKiPK13ChattsKvCachePfPtS8_iPvmS9_iPKNS_8RopeFuseEPKt",
+                                                 "_ZN6chatts17rope_fuse_prepareEiiiPKfS1_fS1_S1_iPKiPK13ChattsKvCachePNS_8RopeFuseE"))
+    P, I, F, N = C.c_void_p, C.c_int, C.c_float, C.c_size_t
+    attend.argtypes, prepare.argtypes = [P, I, I, I, I, P, P, P, P, P, I, P, N, P, I, P, P], [I, I, I, P, P, F, P, P, I, P, P, P]
+    nq, nkv, T, pos0 = 8, 2, 96, 33
+    ctx = pos0 + T
+    g = torch.Generator(device=DEV).manual_seed(1)
+    raw, k0, v0 = (torch.randn(s, generator=g, device=DEV) for s in ((T, (nq + 2 * nkv) * 128), (nkv, ctx, 128), (nkv, ctx, 128)))
+    turn = torch.rand((ctx, 64), generator=g, device=DEV) * 6.0
+    cos, sin = turn.cos().contiguous(), turn.sin().contiguous()
+    ws = torch.zeros(((ctx + 31) // 32) * nkv * 32768, dtype=torch.uint8, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(**options):
+        qkv, k, v, out = raw.clone(), k0.clone(), v0.clone(), torch.zeros((T, nq * 128), device=DEV)
+        cache = _lib.KvCache(k=k.data_ptr(), v=v.data_ptr(), max_ctx=ctx)
+        rope = (C.c_char * 512)()
+        _lib.check(prepare(T, nq, nkv, None, None, 1e-6, cos.data_ptr(), sin.data_ptr(), pos0, None, C.byref(cache), rope))
+        if written:
+            _lib.check(lib.chatts_rope_kv_write(qkv.data_ptr(), T, nq, nkv, None, None, 1e-6, cos.data_ptr(), sin.data_ptr(), pos0, None, C.byref(cache), stream))
+            _lib.check(lib.chatts_attention(qkv.data_ptr(), T, nq, nkv, pos0, None, C.byref(cache), out.data_ptr(), 1, ws.data_ptr(), ws.numel(), stream))
+            out.zero_()
+        with _lib.options(**options):
+            _lib.check(attend(qkv.data_ptr(), T, nq, nkv, pos0, None, C.byref(cache), out.data_ptr(), None, None, 1, ws.data_ptr(), ws.numel(), stream, 0, None if written else rope,
+                              ws.data_ptr() if written else None))
+        return out, k, v
+
+    want, got = run(), run(**{option: value})
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and not torch.equal(want[1], k0) and want[0].abs().max() > 0.01
+
+
 @pytest.fixture(scope="module", params=["chatts-8b", "chatts-14b"])
 def model(request):
     cfg = preset(request.param, num_hidden_layers=2, vocab_size=4096, ts_token_start_index=4000, eos_token_id=[4003, 4002], pad_token_id=4002)
