@@ -229,14 +229,16 @@ int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t
 }
 
 // ... and the choice of experts for rows that moe_takes_choice: ids, weight, place (a pair's own) and kept
-bool chatts::depth_norm_can_choose(int ldx) { return ldx % 64 == 0 && ldx <= 4096; }
-int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, chatts_stream_t stream) {
+// (a router of router_rows x ldx, outputs of them in use: the kernel reads 32 rows or 64)
+static int router_blocks(int outputs) { return outputs <= 32 ? 2 : 4; }
+bool chatts::depth_norm_can_choose(int ldx, int router_rows, int outputs) { return ldx % 64 == 0 && ldx <= 4096 && outputs <= 64 && router_rows >= 16 * router_blocks(outputs); }
+int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream) {
   if (const int rc = check_depth_norm(a)) return rc;
-  CHATTS_REQUIRE(moe && router && a->w && a->out.hi && a->out.lo && depth_norm_can_choose(a->ldx) && moe_takes_choice(moe) && moe->n_rows == a->t && moe->ids && moe->place && moe->weight &&
-                     moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);
+  CHATTS_REQUIRE(moe && router && a->w && a->out.hi && a->out.lo && depth_norm_can_choose(a->ldx, router_rows, moe->experts + moe->identity) && moe_takes_choice(moe) &&
+                     moe->n_rows == a->t && moe->ids && moe->place && moe->weight && moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);
   if (a->t == 0) return CHATTS_OK;
   const DepthChoose ch{router_t ? router_t : router, router_t ? 16 : 1, *moe};
-  if (moe->experts + moe->identity <= 32) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
+  if (router_blocks(moe->experts + moe->identity) == 2) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
   else hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 4>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
   CHATTS_CHECK_LAUNCH("depth_norm_choose");
   return CHATTS_OK;

@@ -174,8 +174,8 @@ bool moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh);
 // to 64 pairs and outputs, no choice groups (moe_takes_choice); ids, weight, place and kept then come from the norm before the router (depth.hip)
 bool moe_takes_choice(const ChattsMoeArgs* a);
 int depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t stream);      // chatts_depth_norm; tiles: the operand's planes as plane_at has them, whole blocks of 16 rows in tiles
-bool depth_norm_can_choose(int ldx);
-int depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, chatts_stream_t stream);      // router: [64][ldx]
+bool depth_norm_can_choose(int ldx, int router_rows, int outputs);
+int depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream);
 int moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, bool direct, chatts_stream_t stream);
 
 typedef const __attribute__((address_space(1))) void* gptr_t;

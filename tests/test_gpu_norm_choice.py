@@ -32,3 +32,25 @@ def test_rows(width, experts, top):
         want = F.forward(cfg, sd, toks).double()
         assert float((got - want).norm() / want.norm()) < 2e-4, n
         m.release_slot(n % 2)
+
+
+class FewRouterRows(MuvetarForCausalLM):
+    """a C caller's router: as many rows as its outputs fill in blocks of 16"""
+
+    def _experts(self, L, m):
+        super()._experts(L, m)
+        L.router_n = -(-(len(m.experts) + m.identity) // 16) * 16
+
+
+# the norm's launch reads 32 rows of a router or 64: one that is shorter goes through launches of its own (its logits say so)
+@pytest.mark.parametrize("experts,own", [(9, True), (16, True), (17, False), (32, False), (33, True), (48, True), (49, False)])
+def test_a_router_of_few_rows(experts, own):
+    cfg, sd = model(128, experts, 2)
+    m = FewRouterRows(MuvetarConfig.from_dict(dict(cfg, architecture="Muvetar")), dtype="bfloat16", max_ctx=64, max_batch=2)
+    m.load_weights(sd.items())
+    m.buf["moe_logits"].fill_(float("nan"))
+    toks = list(range(5))
+    got = m.step_tokens([(0, toks, toks)]).double().cpu()
+    want = F.forward(cfg, sd, toks).double()
+    assert float((got - want).norm() / want.norm()) < 2e-4
+    assert bool(m.buf["moe_logits"].view(-1)[:experts].isfinite().all()) == own
