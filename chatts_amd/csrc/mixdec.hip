@@ -44,9 +44,10 @@ struct ChattsMixDecoder {
   ChattsMixBuffers b;
   std::vector<ChattsMixLayer> layers;
   std::vector<ChattsMixRun> runs;
+  bool mid_planes = false;      // 17 .. 95 rows on planes: no bias of a layer is one that the plane path refuses and the float32 path takes (not 16-byte aligned)
 };
 
-static bool mix_planes(const ChattsMixConfig& c, int m, int k) { return !c.exact && k % 64 == 0 && (m >= 96 || (m >= 2 && (m <= 16 || k >= kMidPlanesK))); }
+static bool mix_planes(const ChattsMixDecoder* d, int m, int k) { return !d->c.exact && k % 64 == 0 && (m >= 96 || (m >= 2 && (m <= 16 || (d->mid_planes && k >= kMidPlanesK)))); }
 
 static int mix_equal_blocks(const ChattsMixLayer& l, int i) {      // how many operand blocks from i on have the size of block i
   const int rows = l.mix_row[i + 1] - l.mix_row[i];
@@ -159,6 +160,8 @@ extern "C" ChattsMixDecoder* chatts_mixdec_create(const ChattsMixConfig* c, cons
   d->b = *b;
   d->layers.assign(layers, layers + c->n_layers);
   d->runs.assign(runs, runs + c->n_runs);
+  d->mid_planes = true;
+  for (const ChattsMixLayer& l : d->layers) d->mid_planes = d->mid_planes && (uintptr_t)l.in_bias % 16 == 0;
   return d;
 }
 
@@ -168,7 +171,7 @@ extern "C" void chatts_mixdec_destroy(ChattsMixDecoder* d) { delete d; }
 static ChattsOperand operand(const ChattsMixDecoder* d, bool second, int m, int k) {
   ChattsOperand o{};
   o.ld = k;
-  if (mix_planes(d->c, m, k)) {
+  if (mix_planes(d, m, k)) {
     o.hi = second ? d->b.b_hi : d->b.a_hi;
     o.lo = second ? d->b.b_lo : d->b.a_lo;
   } else {
@@ -318,7 +321,7 @@ static int mix_delta(const ChattsMixDecoder* d, const ChattsMixLayer& l, const C
 static ChattsOperand second_norm(const ChattsMixDecoder* d, const ChattsMixLayer& l, int m) {
   ChattsOperand o{};
   o.ld = d->c.width_p;
-  const bool planes = mix_planes(d->c, m, o.ld);
+  const bool planes = mix_planes(d, m, o.ld);
   if (planes || (l.ff_kind == CHATTS_FF_MOE && !d->c.exact)) { o.hi = d->b.n_hi; o.lo = d->b.n_lo; }      // (experts take planes, the router what its kernel wants)
   if (!planes) o.f32 = d->b.n_f32;
   return o;
@@ -332,7 +335,7 @@ static ChattsOperand shift_operand(const ChattsMixDecoder* d, int m, int block) 
   ChattsOperand o{};
   o.ld = d->c.width_p;
   const int64_t at = block * d->b.mix_stride;
-  if (mix_planes(d->c, m, o.ld)) { o.hi = d->b.m_hi + at; o.lo = d->b.m_lo + at; }
+  if (mix_planes(d, m, o.ld)) { o.hi = d->b.m_hi + at; o.lo = d->b.m_lo + at; }
   else o.f32 = d->b.m_f32 + at;
   return o;
 }
@@ -511,7 +514,7 @@ static int mix_parallel_forward(ChattsMixDecoder* d, const int64_t* tokens, int 
 static ChattsOperand stream_operand(const ChattsMixDecoder* d, int m, bool experts) {
   ChattsOperand o{};
   o.ld = d->c.width_p;
-  const bool planes = mix_planes(d->c, m, o.ld);
+  const bool planes = mix_planes(d, m, o.ld);
   if (planes || (experts && !d->c.exact)) { o.hi = d->b.a_hi; o.lo = d->b.a_lo; }
   if (!planes) o.f32 = d->b.x;
   return o;
@@ -585,7 +588,7 @@ static int mix_select(const ChattsMixDecoder* d, const ChattsMixLayer& l, const 
   a.rows = b.rows; a.n_rows = t; a.spans = b.spans; a.n_spans = single ? 0 : n_spans;
   a.u.f32 = b.sel_u; a.u.ld = l.sel_k;
   ChattsOperand in = f32_out(b.sel_u, l.sel_k);
-  if (mix_planes(d->c, t, l.sel_k)) {
+  if (mix_planes(d, t, l.sel_k)) {
     a.u.hi = b.sel_u_hi; a.u.lo = b.sel_u_lo;
     in.f32 = nullptr; in.hi = b.sel_u_hi; in.lo = b.sel_u_lo;
   }
@@ -601,7 +604,7 @@ static int mix_select(const ChattsMixDecoder* d, const ChattsMixLayer& l, const 
     if ((rc = chatts_select_steps(&a, s)) != 0) return rc;
     return chatts_select_scan(&a, s);
   }
-  if (mix_planes(d->c, t, a.rank)) {
+  if (mix_planes(d, t, a.rank)) {
     if ((rc = chatts_split_bf16x2(dt.f32, t, a.rank, a.ld_low, b.sel_dt_hi, b.sel_dt_lo, a.rank, s)) != 0) return rc;
     dt.f32 = nullptr; dt.hi = b.sel_dt_hi; dt.lo = b.sel_dt_lo; dt.ld = a.rank;
   }
