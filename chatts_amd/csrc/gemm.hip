@@ -983,6 +983,20 @@ static int pick_stream_sk(int m, int n, int k, bool w8) {
   return sk;
 }
 
+// Does the prefill kernel, with W and planes in its blocks, beat the weight stream at 65 .. 128 rows?  The stream has one workgroup a CU there, and as many of them as fit: the prefill kernel is faster
+// where these leave more than a twentieth of the CUs idle, and not where they fill them; with fewer than three quarters (short K: a split ends at four K-steps) neither fills them.  Four
+// layers of H columns and the first one, weights from HBM (800 MB of encoders in turn), us, stream / prefill kernel, 65 | 96 | 128 rows:
+//   2560 .78 of the CUs 65.2 / 65.2 | 72.2 / 68.9 | 81.0 / 76.3    3072 .94 73.2 / 69.4 | 81.1 / 76.7 | 87.7 / 82.8     4736 .87 100.7 / 98.1 | 108.4 / 101.3 | 113.5 / 110.0
+//   5120 .94 111.0 / 103.3 | 116.6 / 114.6 | 121.7 / 122.0         6144 .94 136.9 / 120.9 | 138.7 / 135.9 | 147.0 / 144.3  6656 .81 146.3 / 129.3 | 155.3 / 146.2 | 167.7 / 163.5
+//   3584 .98 79.2 / 80.5 | 85.5 / 88.2 | 91.9 / 87.0               4096 1.0 85.5 / 88.3 | 91.9 / 93.9 | 96.5 / 101.9     4608 .98 97.1 / 93.1 | 105.1 / 106.6 | 110.8 / 117.9
+//   8192 1.0 187.2 / 186.2 | 196.6 / 204.6 | 213.6 / 225.6         1536 .28 52.3 / 57.9 | 56.8 / 59.8 | 61.9 / 61.6      2304 .63 60.6 / 62.0 | 66.8 / 70.5 | 74.7 / 72.7
+// On the wrong side: 4224 and 4352 (2 to 7 % slower), 7168 from 80 rows on (1 to 5 %), 3712 up to 80 rows (5 to 7 %); 3584 from 104 rows on would be 2 to 5 % faster.  An encoder that runs again at once,
+// its weights in the Infinity Cache, is 5 to 30 % faster in the prefill kernel at any width from 2048 to 5120; a request's decoder has evicted them.
+bool stream_leaves_cus(int m, int n, int k) {
+  const int cus = device_cus(), wgs = (n + kStreamBN - 1) / kStreamBN * pick_stream_sk(m, n, k, false);
+  return 4 * wgs >= 3 * cus && 20 * wgs < 19 * cus;
+}
+
 // Do more workgroups than CUs come out of 128 columns each, where 160 would fit?  A workgroup streams at the rate of its CU, so the launch lasts as long as the CUs that have two.
 // The K ranges, and with them the bits, stay.  16 rows bf16, us with the epilogue, 128 / 160 columns: 7168 x 5120 22.4 / 17.8, 7168 x 8192 32.1 / 24.6,
 // 9216 x 4096 22.4 / 17.8, 11264 x 4096 26.6 / 20.4, 7168 x 2048 11.3 / 10.8, 11776 x 1024 10.8 / 10.2.  (A range less for each tile instead: 7168 x 5120 18.0, 9216 x 4096 16.9, but

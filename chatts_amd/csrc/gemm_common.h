@@ -103,6 +103,7 @@ struct PlaneTiles {
 // 11.2 / 8.0; 48 rows 7168 x 5120 30.2 / 22.6, 27648 x 5120 gated 85.9 / 64.1; 80 rows 5120 x 13824 57.0 / 44.1, 8192 x 2048 23.7 / 20.5.  Shorter K is not the weight stream's.
 constexpr int kMidPlanesK = 1024;
 bool planes_tiled_for(int m, int n, int k);      // (gemm.hip: of the A of an m x n x k product)
+bool stream_leaves_cus(int m, int n, int k);     // (gemm.hip: 65 .. 128 rows with W in tiles are the prefill kernel's)
 int linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles);      // chatts_linear on such planes (decoder.hip)
 
 constexpr int kRingPanel = 256;      // W rows per panel of the prefill kernel

@@ -492,13 +492,12 @@ static int ts_encode(const float* series, const int32_t* lengths, int32_t* row_o
   // Plane path (P > 1 and every K a multiple of 64): each activation matrix lives as bf16 hi / lo planes inside the caller's
   // float32 scratch of the same byte size (4 B per element = 2 + 2) - patchify writes the planes of layer 0's operand, every
   // GELU epilogue writes the planes of the next layer's, and the GEMMs stage all operands with whole-line LDS-DMA
-  // (gemm_stream_kernel for P <= 16: the 213 MB of MLP weights are streamed once; gemm_dma_kernel above).  The values are
+  // (gemm_stream_kernel for few rows: the 213 MB of MLP weights are streamed once; gemm_ring_kernel above).  The values are
   // the splits of exactly the float32 numbers the float32 path would hold, so both paths give the same result.
   const int P = total_patches, H = w->hidden;
   const bool planes = P > 1 && w->in_features_pad % 64 == 0 && H % 64 == 0 && opt_get(OPT_TS_F32_PATH, 0) == 0;
-  // The prefill kernel from 65 rows on, where the weights lie in its blocks (us a layer, weight stream / prefill kernel: 66 rows 5120 x 5120 25.1 / 20.8, 4096 x 4096 20.1 / 18.6; 96 rows
-  // 28.3 / 23.8, 22.3 / 19.8; 128 rows 29.2 / 27.2, 23.5 / 23.9); without, up to 128 rows the weight stream.  Activations between its layers in blocks, too.
-  const bool mid = planes && w_tiled && P > 64 && P <= 128;
+  // The prefill kernel from 65 rows on, where the weights lie in its blocks and stream_leaves_cus; else, up to 128 rows, the weight stream.  Activations between its layers in blocks, too.
+  const bool mid = planes && w_tiled && P > 64 && P <= 128 && stream_leaves_cus(P, H, H);
   const bool tile = planes && (mid ? opt_get(OPT_PLANE_TILES, 1) != 0 : planes_tiled_for(P, H, H));
   // The weights in blocks likewise, where the caller has them so: a 1 KB piece of the loader is 1 KB of memory.  1036 rows of 5120 x 5120, us a layer: 88.6 -> 82.4.
   auto hi_of = [&](float* buf) { return reinterpret_cast<chatts_bf16*>(buf); };

@@ -65,3 +65,26 @@ def test_the_encoder_and_its_series_alone(name, patches):
     got = e(x.view(2, -1, 1), valid_lengths=lengths)[0].clone()
     want = torch.cat([e(x[i:i + 1].view(1, -1, 1), valid_lengths=[n])[0].clone() for i, n in enumerate(lengths)])
     assert got.shape == want.shape and got.shape[0] == patches and rel(got, want) < 5e-6
+
+
+# where the weight stream's workgroups fill the CUs (32 x 8, 36 x 7) or three quarters of them at most (18 x 9), it runs whether the weights lie in tiles or not; where they leave some idle (24 x 10,
+# 40 x 6, 52 x 4 of 256), weights in tiles are the prefill kernel's, whose sums run in another order
+@pytest.mark.parametrize("width,prefill_kernel", [(2304, False), (3072, True), (4096, False), (4608, False), (5120, True), (6656, True)])
+def test_which_kernel_an_encoder_of_some_rows_takes(width, prefill_kernel):
+    ts = dict(preset("chatts-8b").ts, hidden_size=width, num_layers=3)
+    e = TimeSeriesEmbedding(ts, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(width)
+    e.load_tensor("position_embedding.weight", torch.randn((ts["max_sequence_length"] + 1, ts["embedding_dim"]), generator=g, device="cuda"))
+    k = ts["patch_size"] * (1 + ts["embedding_dim"])
+    for l in range(3):
+        e.load_tensor(f"mlp.{2 * l}.weight", (torch.randn((width, k), generator=g, device="cuda") * k ** -0.5).bfloat16())
+        e.load_tensor(f"mlp.{2 * l}.bias", torch.randn(width, generator=g, device="cuda") * 0.1)
+        k = width
+    for patches in (65, 100, 128):
+        x = torch.randn((1, patches * 16, 2), generator=g, device="cuda")
+        x[..., 1] = 1.0
+        rows = e(x.view(1, -1, 1), valid_lengths=[patches * 16])[0].clone()
+        e._tsw_tiled = None
+        plain = e.replay_last().clone()
+        e._tsw = None
+        assert rel(rows, plain) < 5e-6 and torch.equal(rows, plain) != prefill_kernel, patches
