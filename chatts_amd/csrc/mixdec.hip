@@ -642,9 +642,11 @@ static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, co
     e.x = d->b.x; e.x0 = d->b.streams; e.width = c.width; e.pos_fine = d->b.pos_fine; e.pos_coarse = d->b.pos_coarse;
     if ((rc = chatts_embed_pair(&e, s)) != 0) return rc;
   }
-  // A in tiles where a step of K is short beside the whole: prompts of 200, 2 x 350, 2048 rows of 4096 columns row-major / in tiles 5.04 / 4.92, 6.96 / 6.77, 16.9 / 16.8 ms; at 2048 columns 1 % slower.
-  // (The second norm's planes and the activation in tiles gave nothing.)
-  auto tiles_for = [&](const ChattsMixLayer& l) { return wp >= 4096 && !A.f32 && planes_tiled_for(t, l.in_n, wp); };
+  // A in tiles where rows are long.  Whole prompts of four layers, ms, row-major / in tiles, 100, 200, 2 x 350, 1024, 2048 rows: 2048 columns 1.03 / 1.04, 1.22 / 1.23, 1.77 / 1.76, 2.15 / 2.15,
+  // 3.46 / 3.46; 2560 1.32 / 1.33, 1.62 / 1.61, 2.44 / 2.41, 2.77 / 2.76, 4.56 / 4.54; 3072 1.53 / 1.53, 1.86 / 1.85, 2.85 / 2.83, 3.40 / 3.40, 5.67 / 5.67; 3584 1.86 / 1.86, 2.22 / 2.22,
+  // 3.36 / 3.33, 4.33 / 4.26, 7.06 / 6.98; 4096 2.13 / 2.12, 2.59 / 2.57, 4.02 / 4.02, 5.21 / 5.16, 8.69 / 8.72; 5120 2.99 / 2.99, 3.58 / 3.55, 6.09 / 5.96, 7.54 / 7.48, 13.5 / 13.4; 1024 columns up
+  // to 1 % slower.  (The second norm's planes and the activation in tiles gave nothing.)
+  auto tiles_for = [&](const ChattsMixLayer& l) { return wp >= 3072 && !A.f32 && planes_tiled_for(t, l.in_n, wp); };
   bool tiles = tiles_for(d->layers[d->runs[0].layer]);
   if ((rc = mix_depth_norm(d, t, nullptr, nullptr, nullptr, 0, d->layers[d->runs[0].layer].norm1, A, s, tiles)) != 0) return rc;
   for (int r = 0; r < c.n_runs; ++r) {

@@ -1,4 +1,4 @@
-"""The first norm's planes in the prefill kernel's blocks (PLANE_TILES), decoders with norms before their sublayers and rows of 4096 columns and more: the same bits as row-major planes, for
+"""The first norm's planes in the prefill kernel's blocks (PLANE_TILES), decoders with norms before their sublayers and rows of 3072 columns and more: the same bits as row-major planes, for
 rows that end with a whole block of 16, one row later and one row earlier, one prompt and several, at the smallest number of rows that travels so and above."""
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ from tests.muvetar_models import _gru, _moe, _par
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("width", [4050, 4160])
+@pytest.mark.parametrize("width", [3072, 4050, 4160])
 def test_the_same_bits(width):
     cfg = {"vocab": 96, "width": width, "norm": {"eps": 1e-6}, "residual_mult": 0.5, "logit_softcap": 40.0,
            "layers": [_moe(_par(4, 2, 32, 32, 0.25, 64, 4, 8, 2, (1.0, 0.5)), 64, 7.0, 4, 2, 1.0, (64, 7.0)), dict(_gru(2100), mlp=None), _moe(_gru(64), 64, 7.0, 4, 2, 1.0)]}
