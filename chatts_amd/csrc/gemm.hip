@@ -11,9 +11,9 @@
 // bit-identical results at equal split-K:
 //   gemm_bf16x2_kernel  register-staged, BM x 128 x 32 tiles, A split on the VALU while staging; any M, float32 A;
 //                       callers with float32 A and rows for which planes do not pay (kMidPlanesK)
-//   gemm_ring_kernel    (gemm_ring.hip) prefill (M > 16) on pre-split planes: persistent workgroups, balanced M-tiles x 256 columns,
+//   gemm_ring_kernel    (gemm_ring.hip) prefill (M > 16, where the next one does not run) on pre-split planes: persistent workgroups, balanced M-tiles x 256 or 192 columns,
 //                       4 loader waves feeding a ring of four 32-deep half-stages by LDS-DMA, 8 compute waves
-//   gemm_stream_kernel  batched decode (2 <= M <= 16) on planes: 16 x 128 x 64 (128 for fp8 W), weight-streaming shape
+//   gemm_stream_kernel  batched decode (2 <= M <= 16) on planes: 16 x 128 x 64 (128 for fp8 W), weight-streaming shape; in several row blocks 17 .. 64 or 128 rows (stream_multiblock)
 // The comments above each kernel say which measurement made it look the way it does.
 //
 // Register-staged kernel geometry: 256 threads = 4 waves (WM x WN), double-buffered LDS, global loads issued one
@@ -252,7 +252,7 @@ __device__ __forceinline__ int lds_off128(int r, int c) { return r * 128 + ((c ^
 // fetching W in the MFMA fragment pattern (16 rows x 64 B per wave instruction - what a BK = 32 tile does, in registers
 // or through LDS) tops out near 4.0-4.5 TB/s, the same bytes as 8 rows x 128 B (whole lines) stream at 5.2-5.7 TB/s
 // (profiles/r1_probe_weight_stream_patterns.txt, DBG=1 vs DBG=3).  So: tile 16 x 128 x 64, every operand staged by
-// LDS-DMA in whole-line pieces (the same 128-byte-row, XOR-swizzled layout as gemm_dma_kernel), a ring of NSTAGE
+// LDS-DMA in whole-line pieces (128-byte rows, their 16-byte chunks XOR-swizzled), a ring of NSTAGE
 // 20 KB stages so that 2 workgroups per CU keep 60-80 KB of W in flight, split-K over workgroups to fill the chip
 // (52 MB of o_proj weights are only 40 N-tiles).  A comes as bf16 hi / lo planes ([M, K], M <= 16).
 constexpr int kStreamBN = 128;
@@ -991,7 +991,7 @@ static int pick_stream_sk(int m, int n, int k, bool w8) {
 //   3584 .98 79.2 / 80.5 | 85.5 / 88.2 | 91.9 / 87.0               4096 1.0 85.5 / 88.3 | 91.9 / 93.9 | 96.5 / 101.9     4608 .98 97.1 / 93.1 | 105.1 / 106.6 | 110.8 / 117.9
 //   8192 1.0 187.2 / 186.2 | 196.6 / 204.6 | 213.6 / 225.6         1536 .28 52.3 / 57.9 | 56.8 / 59.8 | 61.9 / 61.6      2304 .63 60.6 / 62.0 | 66.8 / 70.5 | 74.7 / 72.7
 // On the wrong side: 4224 and 4352 (2 to 7 % slower), 7168 from 80 rows on (1 to 5 %), 3712 up to 80 rows (5 to 7 %); 3584 from 104 rows on would be 2 to 5 % faster.  An encoder that runs again at once,
-// its weights in the Infinity Cache, is 5 to 30 % faster in the prefill kernel at any width from 2048 to 5120; a request's decoder has evicted them.
+// its weights in the Infinity Cache, is 5 to 30 % faster in the prefill kernel at any width from 2048 to 5120 (a request's decoder has evicted them); right behind a copy of 512 MB 5120 columns are 3 to 5 % slower.
 bool stream_leaves_cus(int m, int n, int k) {
   const int cus = device_cus(), wgs = (n + kStreamBN - 1) / kStreamBN * pick_stream_sk(m, n, k, false);
   return 4 * wgs >= 3 * cus && 20 * wgs < 19 * cus;
