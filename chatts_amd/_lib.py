@@ -324,6 +324,10 @@ SIGNATURES = {
     "chatts_decoder_set_prefill_f16q": (c_int, [c_void_p, c_int]),
     "chatts_tile_bf16_elems": (c_size_t, [c_int, c_int]),
     "chatts_tile_bf16": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p]),
+    "chatts_tile_w4_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "chatts_tile_w4": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
+    "chatts_decoder_set_w4_tiles": (c_int, [c_void_p, C.POINTER(c_void_p), c_int]),
+    "chatts_linear_w4_tiles": (c_int, [C.POINTER(LinearArgs), c_void_p, c_void_p]),
     "chatts_split_bf16x2": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p]),
     "chatts_embed_merge": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int, c_void_p, c_int, c_int64,
                                    c_void_p, c_void_p, c_void_p, c_void_p]),

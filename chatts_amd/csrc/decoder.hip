@@ -58,7 +58,9 @@ struct ChattsDecoder {
   bool prefill_fp8 = false; // SPEED MODE (chatts_decoder_set_prefill_fp8): prefill chunks of >= 16 rows multiply fp8 x fp8 (gemm_fp8.hip)
   bool fuse_tp = false;     // set by chatts_decoder_decode_step: the M == 1 o_proj / down_proj GEMVs carry the exchange in their own launch
   bool tp_fused = false;    // ... and whether the last layer part's projection did (otherwise the caller launches chatts_allreduce)
+  std::vector<const void*> w4_tiles;      // [n_layers][qkv, o, gate_up, down]: 4-bit codes in chatts_tile_w4's order (chatts_decoder_set_w4_tiles); empty or null: the layer's row-major codes
 };
+enum { kProjQkv, kProjO, kProjGateUp, kProjDown };
 
 static int64_t embed_rows(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_rows : d->cfg.vocab_local; }
 static int64_t embed_offset(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_offset : d->cfg.vocab_offset; }
@@ -239,6 +241,27 @@ extern "C" void chatts_decoder_destroy(ChattsDecoder* d) { delete d; }
 
 static size_t seq_stride(const ChattsDecoder* d) {      // floats between the caches of consecutive sequences
   return (size_t)d->cfg.n_layers * d->cfg.n_kv * d->cfg.max_ctx * kHeadDim;
+}
+
+extern "C" int chatts_decoder_set_w4_tiles(ChattsDecoder* d, const void* const* tiles, int n) {
+  CHATTS_REQUIRE(d && (tiles || n == 0), CHATTS_E_BADARG, "decoder_set_w4_tiles: null argument");
+  CHATTS_REQUIRE(n == 0 || n == 4 * d->cfg.n_layers, CHATTS_E_SHAPE, "decoder_set_w4_tiles: %d pointers for %d layers", n, d->cfg.n_layers);
+  for (int i = 0; i < n; ++i) {
+    const ChattsLayerWeights& lw = d->layers[i / 4];
+    const uint8_t* const w4[4] = {lw.qkv4, lw.o4, lw.gate_up4, lw.down4};
+    CHATTS_REQUIRE(!tiles[i] || (w4[i % 4] && ((uintptr_t)tiles[i] % 16) == 0), CHATTS_E_BADARG, "decoder_set_w4_tiles: layer %d, projection %d has no 4-bit codes", i / 4, i % 4);
+  }
+  try {
+    d->w4_tiles.assign(tiles, tiles + n);
+  } catch (const std::bad_alloc&) {
+    CHATTS_REQUIRE(false, CHATTS_E_BADARG, "decoder_set_w4_tiles: out of host memory");
+  }
+  return CHATTS_OK;
+}
+// a projection of one row: on the tiled 4-bit codes where there are some
+static int linear_one_row(const ChattsDecoder* d, int layer, int proj, const ChattsLinearArgs* la, chatts_stream_t stream) {
+  const void* t = la->w4 && !d->w4_tiles.empty() ? d->w4_tiles[4 * layer + proj] : nullptr;
+  return t ? chatts_linear_w4_tiles(la, t, stream) : chatts_linear(la, stream);
 }
 
 static ChattsKvCache layer_cache(const ChattsDecoder* d, int layer, int seq) {
@@ -596,7 +619,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
                                   &rf)) != 0) return rc;
       rope_done.want_planes = prefill_on_planes(t, c.n_kv, pos0, pos0_dev, out_planes, ks, d->b.workspace, d->b.workspace_bytes);
       if ((rc = linear_impl(&la, stream, &rf, &rope_done, nullptr, {tile_h, false, false})) != 0) return rc;
-    } else if ((rc = linear_tiled(&la, stream, {tile_h, false, false})) != 0) {
+    } else if ((rc = t == 1 ? linear_one_row(d, layer, kProjQkv, &la, stream) : linear_tiled(&la, stream, {tile_h, false, false})) != 0) {
       return rc;
     }
     bool attn_out_planes = false;
@@ -638,7 +661,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
     } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
     else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
     request_post_norm(d, &la, lw.post_norm, 2 * c.inter, false);
-    return linear_tiled(&la, stream, after(d, la, tile_attn));
+    return t == 1 ? linear_one_row(d, layer, kProjO, &la, stream) : linear_tiled(&la, stream, after(d, la, tile_attn));
   }
   // part 1: RMSNorm -> gate_up + SwiGLU -> down (+ residual / partial)
   la = ChattsLinearArgs{};
@@ -654,7 +677,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   }
   const bool act_planes = t > 1 && planes_path(d, t, c.inter), tile_act = act_planes && !la.a && tiles_path(d, t, 2 * c.inter, H) && tiles_path(d, t, H, c.inter);   // SwiGLU output goes straight into down_proj's operand format
   if (act_planes) { la.c = nullptr; la.c_hi = d->b.planes2_hi; la.c_lo = d->b.planes2_lo; la.ld_cplanes = c.inter; }
-  if ((rc = linear_tiled(&la, stream, {tile_h, tile_act, false})) != 0) return rc;
+  if ((rc = t == 1 ? linear_one_row(d, layer, kProjGateUp, &la, stream) : linear_tiled(&la, stream, {tile_h, tile_act, false})) != 0) return rc;
   la = ChattsLinearArgs{};
   la.a = d->b.act; la.w = lw.down; la.w_tiled = lw.down_t; la.m = t; la.n = H; la.k = c.inter;
   la.lda = c.inter; la.ldw = c.inter; la.ldc = H;
@@ -671,7 +694,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
   else { la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; }
   request_post_norm(d, &la, layer + 1 < c.n_layers ? d->layers[layer + 1].input_norm : nullptr, (c.n_q + 2 * c.n_kv) * kHeadDim, false);
-  return linear_tiled(&la, stream, after(d, la, tile_act));
+  return t == 1 ? linear_one_row(d, layer, kProjDown, &la, stream) : linear_tiled(&la, stream, after(d, la, tile_act));
 }
 
 extern "C" int chatts_decoder_layer_part_add(ChattsDecoder* d, int add_delta, int layer, int part, int t, int pos0,
@@ -899,7 +922,7 @@ static int layer_last_row(ChattsDecoder* d, int layer, int t, int pos0, chatts_s
   const bool tp = c.tp_world > 1;
   if (tp && !la.w4) la.tp_reduce = d->tp;                  // row 0 of x += the sum over the ranks, inside the GEMV launch
   else if (tp) { la.c = d->b.delta; la.resid = nullptr; la.epilogue = CHATTS_EPI_NONE; }
-  if ((rc = chatts_linear(&la, stream)) != 0) return rc;
+  if ((rc = linear_one_row(d, layer, kProjO, &la, stream)) != 0) return rc;
   if (tp && !la.tp_reduce && (rc = chatts_allreduce(d->tp, d->b.delta, d->b.x, d->b.x, H, stream)) != 0) return rc;
   d->fuse_tp = tp;
   rc = chatts_decoder_layer_part(d, layer, 1, 1, 0, nullptr, 1, stream);      // MLP on row 0: the decode path's GEMVs

@@ -17,35 +17,13 @@
 // x = hi + lo bf16 (2^-17), products exact, float32 sums: the accuracy of the kernel it replaces.
 #include <type_traits>
 
-#include "common.h"
-#include "gemv_common.h"
+#include "gemv4.h"
 
 namespace chatts {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
-struct Gemv4Params {
-  const uint8_t* w4;
-  const float2* sz;
-  const float* x;
-  const float* norm_w;
-  const float* bias;
-  const float* resid;
-  float* out;
-  float eps;
-  int n, k, ldw4, gshift, ng;
-  int quads_each, quads_more;      // every workgroup has quads_each quads, the first quads_more of them one more
-  unsigned parts_inv;              // ceil(2^32 / parts of K), 0 where there is one: a quotient without a division
-};
-
 // Units of the ring: more of them only cost code and registers.  us with 8 / 6 / 4 / 3 / 2: 7168 x 5120 9.9 / 9.1 / 9.0 / 8.4 / 9.3, 5120 x 5120 8.5 / 8.2 / 7.4 / 7.4 / 7.7, 27648 x 5120 gated
 // 21.5 / 20.3 / 20.2 / 19.9 / 22.4, 5120 x 13824 13.9 / 12.6 / 12.6 / 12.2 / 13.7, 24576 x 4096 gated 17.0 / 16.4 / 15.3 / 15.2 / 16.4, 4096 x 12288 11.5 / 10.3 / 9.9 / 10.0 / 10.8.
-constexpr int kQ4Waves = 8, kQ4Threads = 64 * kQ4Waves, kQ4Turns = 4, kQ4Bufs = 3, kQ4Ahead = kQ4Bufs - 1, kQ4Early = 1;
-constexpr int kQ4Piece = 512 + 32;      // bytes of an operand: (k group) x (part, hi / lo) x 16; the 32 keep the writes of x apart
-constexpr unsigned kQ4Far = 0x7ffffff0u;
-__host__ __device__ constexpr int q4_parts(int k) { return (k + 511) >> 9; }
-static size_t q4_lds(int k, int quads) { return (size_t)q4_parts(k) * 4 * kQ4Piece + (size_t)quads * kQ4Waves * 128; }
+constexpr int kQ4Bufs = 3, kQ4Ahead = kQ4Bufs - 1;
 
 template <int EPI, bool NORM>
 __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
@@ -66,10 +44,7 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
   // (up to the last code of the last row: units of 512 codes run past the end of a row)
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)p.w4, 0, (int)((unsigned)(p.n - 1) * (unsigned)p.ldw4 + (unsigned)K / 2u), 0x00020000);
   const unsigned lane_off = (unsigned)(GLU ? (r >> 1) + (r & 1) * 16 : r) * (unsigned)p.ldw4 + pos * 16;
-  auto first_row = [&](int q) __attribute__((always_inline)) {           // of quad q of this workgroup (gated: gates 2 u, 2 u + 1 and their up rows, 16 further on)
-    const int at = (q0 + q) * (GLU ? 2 : 4);
-    return GLU ? (at >> 4) * 32 + (at & 15) : at;
-  };
+  auto first_row = [&](int q) __attribute__((always_inline)) { return q4_first_row<GLU>(q0 + q); };
   // scale and zero of this lane's 32 codes: they lie in one group, and 512 s is a whole number of groups or inside one
   const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc((void*)p.sz, 0, (int)((unsigned)p.n * (unsigned)p.ng * 8u), 0x00020000);
   const unsigned lane_sz = ((unsigned)(GLU ? (r >> 1) + (r & 1) * 16 : r) * (unsigned)p.ng + (unsigned)((pos * 32) >> p.gshift)) * 8u;
@@ -103,8 +78,7 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
       }
     }
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int b = 0; b < kQ4Early; ++b) request(b);
+  request(0);
   __builtin_amdgcn_sched_barrier(0);
   float ss = 0.f;
 #pragma unroll
@@ -137,7 +111,7 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
     if (lane == 0) red[wave] = ss;
   }
 #pragma unroll
-  for (int b = kQ4Early; b < kQ4Ahead; ++b) request(b);
+  for (int b = 1; b < kQ4Ahead; ++b) request(b);
   __syncthreads();
 
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -190,43 +164,7 @@ __global__ __launch_bounds__(64 * kQ4Waves) void gemv4_kernel(Gemv4Params p) {
   }
   __syncthreads();
 
-  float rstd = 1.f;
-  if (NORM) {
-    float t = 0.f;
-#pragma unroll
-    for (int i = 0; i < kQ4Waves; ++i) t += red[i];
-    rstd = rsqrtf(t / (float)K + p.eps);
-  }
-  // eight lanes a quad: the vectors of the waves that had a share of it, in wave order, then over the lanes
-  for (int i = tid; i < (nq * 8 + 63) / 64 * 64; i += kQ4Threads) {
-    const int qq = i >> 3, e = i & 7;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (qq < nq) {
-      const int a = qq * S, z = a + S;
-      // from the wave before the one that a 1 / items in floating point names: its share may end at a
-      int w = (int)((float)(a * kQ4Waves) * __builtin_amdgcn_rcpf((float)items)) - 1;
-      for (w = w < 0 ? 0 : w; w < kQ4Waves && w * items / kQ4Waves < z; ++w) {
-        const int to = (w + 1) * items / kQ4Waves;
-        if (to > a && w * items / kQ4Waves < to) v += part[(qq * kQ4Waves + w) * 8 + e];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { v[j] += lane_xor1(v[j]); v[j] += lane_xor2(v[j]); v[j] += half_mirror(v[j]); if (NORM) v[j] *= rstd; }
-    if (qq >= nq) continue;
-    const int row = first_row(qq);
-    if (GLU) {
-      if (e < 2) {
-        float g = e ? v[2] : v[0], u = e ? v[3] : v[1];
-        if (p.bias) { g += p.bias[row + e]; u += p.bias[row + e + 16]; }
-        p.out[(q0 + qq) * 2 + e] = silu_f(g) * u;
-      }
-    } else if (e < 4) {
-      float o = e == 0 ? v[0] : (e == 1 ? v[1] : (e == 2 ? v[2] : v[3]));
-      if (p.bias) o += p.bias[row + e];
-      if (EPI == CHATTS_EPI_RESID) o = p.resid[row + e] + o;
-      p.out[row + e] = o;
-    }
-  }
+  q4_finish<EPI, NORM, kQ4Waves>(p, part, red, tid, q0, nq, S, items);
 #endif
 }
 
@@ -256,7 +194,7 @@ int launch_gemv4(const ChattsLinearArgs* a, hipStream_t s, bool* done) {
   const int quads = a->n / 4, cus = device_cus(), grid = quads < cus ? quads : cus, parts = q4_parts(a->k);
   p.quads_each = quads / grid; p.quads_more = quads % grid;
   p.parts_inv = parts > 1 ? (unsigned)((0x100000000ull + parts - 1) / parts) : 0u;      // (units of a workgroup stay below 65536)
-  const size_t lds = q4_lds(a->k, (quads + grid - 1) / grid);
+  const size_t lds = q4_lds(a->k, (quads + grid - 1) / grid, kQ4Waves);
   // Short rows of few codes stay with gemv4_ldsx_kernel: laying x out as operands and the reduction over the waves cost 4.3 us before any code is read, its batches
   // 3 us and a step for every 1024 codes a row.  us there / here: 1024 x 512 3.0 / 4.3, 4096 x 1024 3.8 / 4.4, 8192 x 1024 4.55 / 4.8, 6144 x 2048 5.1 / 5.9, 1536 x 2560 4.7 / 5.2,
   // 4096 x 2560 5.2 / 5.45; but 7168 x 1536 1 to 8 % less here, 9728 x 896 6.4 / 5.3, 16384 x 1024 6.5 / 5.6, 3072 x 2560 with the norm 7 % less, and from 3073 codes a row on

@@ -339,6 +339,30 @@ class ChatTSForCausalLM(SlotModel):
             self.int4_group = q.shape[1] // sc.shape[1]
             L[k + "4"], L[k + "4_sz"] = pack_int4(q, sc, z)
 
+    def _tile_int4(self):
+        """4-bit codes once more in the order the matrix pipe takes them in (chatts_tile_w4), for the projections of one row; those of a shape or with scales that have no such form, and
+        those there is no memory for, keep the row-major codes."""
+        lib, names = self.lib, ("qkv", "o", "gate_up", "down")
+        self._int4_tiles = {}
+        bad = torch.zeros(4 * len(self.layers), dtype=torch.int32, device=self.device)
+        for i, lw in enumerate(self.layers):
+            for j, name in enumerate(names):
+                if name + "4" not in lw:
+                    continue
+                rows, k = lw[name].shape
+                need = int(lib.chatts_tile_w4_bytes(rows, k, self.int4_group))
+                if need == 0 or torch.cuda.mem_get_info(self.device)[0] < need + (8 << 30):
+                    continue
+                out = torch.empty(need, dtype=torch.uint8, device=self.device)
+                _lib.check(lib.chatts_tile_w4(lw[name + "4"].data_ptr(), lw[name + "4_sz"].data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", out.data_ptr(),
+                                              bad[4 * i + j:].data_ptr(), _lib.stream_ptr()))
+                self._int4_tiles[4 * i + j] = out
+        if self._int4_tiles:
+            for n in bad.nonzero().flatten().tolist():
+                del self._int4_tiles[n]
+            ptrs = (C.c_void_p * len(bad))(*[_lib.ptr(self._int4_tiles.get(n)) for n in range(len(bad))])
+            _lib.check(lib.chatts_decoder_set_w4_tiles(self._decoder, ptrs, len(bad)))
+
     def _finalize(self):
         """Allocate activations / KV cache and create the C-side decoder handle (borrowing all pointers)."""
         cfg, plan, dev, lib = self.config, self.plan, self.device, self.lib
@@ -507,6 +531,7 @@ class ChatTSForCausalLM(SlotModel):
         if not h:
             raise _lib.ChattsError(-1, lib.chatts_last_error().decode())
         self._decoder = C.c_void_p(h)
+        self._tile_int4()
         self._graph = None
         self._graph_batched = None
         if self.precision == "fp8":              # speed mode: prefill chunks and the TS encoder on the fp8 matrix pipe

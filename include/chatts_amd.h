@@ -296,6 +296,14 @@ int chatts_split_bf16x2(const float* x, int m, int k, int ldx, chatts_bf16* hi, 
  * block of a ragged row count) repeat the last row.  dst holds chatts_tile_bf16_elems(rows, k) = ceil(rows / 16) * 16 * k elements. */
 size_t chatts_tile_bf16_elems(int rows, int k);
 int chatts_tile_bf16(const chatts_bf16* src, int rows, int k, int ld, chatts_bf16* dst, chatts_stream_t stream);
+/* 4-bit codes (ChattsLinearArgs.w4 / w4_sz, groups of 128 and more) -> the order the matrix pipe takes them in (csrc/gemv4_tiles.hip): for every four rows
+ * (gated != 0: rows for SWIGLU, two gates and their up rows) and 512 K-values 1 KB of codes, behind all of them 64 bytes of scales and zeros each (float16).  dst holds
+ * chatts_tile_w4_bytes(rows, k, group) bytes, 16-byte aligned; 0 = this shape has no such form (the row-major codes serve it as well or better).  *bad (device) grows by
+ * the number of groups whose scale float16 does not hold exactly, or whose zero is no whole number up to 64 (a GPTQ checkpoint has none): with any the copy may not be used. */
+size_t chatts_tile_w4_bytes(int rows, int k, int group);
+int chatts_tile_w4(const uint8_t* w4, const float* w4_sz, int rows, int k, int ldw4, int group, int gated, void* dst, int32_t* bad, chatts_stream_t stream);
+/* chatts_linear for M == 1 and EPI_NONE / RESID / SWIGLU on such a copy (`gated` as SWIGLU is); `w`, `w4` and `w8` of the arguments are not read. */
+int chatts_linear_w4_tiles(const ChattsLinearArgs* args, const void* tiles, chatts_stream_t stream);
 /* Dispatch: M == 1       -> weight-streaming GEMV (exact f32 VALU products, x staged in LDS, HBM-bound): gemv_ring_kernel for long rows
  *                           (chatts_gemv_ring), gemv4_kernel for 4-bit codes, else gemv_ldsx_kernel and its K-split form;
  *           2 <= M <= 16 -> with pre-split planes: gemm_cols_kernel (chatts_linear_cols), gemm_rows_kernel (chatts_linear_few_rows) or
@@ -719,6 +727,9 @@ typedef struct ChattsDecoder ChattsDecoder;  /* opaque; host memory only */
 ChattsDecoder* chatts_decoder_create(const ChattsDecoderConfig*, const ChattsDecoderWeights*,
                                      const ChattsDecoderBuffers*);
 void chatts_decoder_destroy(ChattsDecoder*);
+/* Copies of the layers' 4-bit codes in chatts_tile_w4's order (gate_up: gated), borrowed like the weights: host array [n_layers][qkv, o, gate_up, down], n = 4 * n_layers (0: none).
+ * Projections of one row stream them instead of qkv4 / o4 / gate_up4 / down4, which stay for the entries that are NULL. */
+int chatts_decoder_set_w4_tiles(ChattsDecoder*, const void* const* tiles, int n);
 size_t chatts_decoder_workspace(const ChattsDecoderConfig*, int t_max, int n_splits_max);
 
 /* One layer, split at the two tensor-parallel exchange points (vLLM: all-reduce after o_proj and
