@@ -114,6 +114,13 @@ struct RingGeom {
   int units;          // T * P * sk, ordered (split, panel, M-tile): the M-tiles of a panel are adjacent
   int wpx;            // workgroups per XCD (grid = 8 * wpx)
   int nf;             // a panel is 64 nf rows (3 or 4)
+  int fbase, frem;    // fragments of an M-tile, the first frem tiles one more
+  unsigned inv_t, inv_p;      // ceil(2^32 / T), / P, 0 for 1: a unit's place without divisions (units * T and * P are below 2^32)
+  void finish() {
+    fbase = F / T; frem = F % T;
+    inv_t = T > 1 ? (unsigned)((0x100000000ull + T - 1) / T) : 0u;
+    inv_p = P > 1 ? (unsigned)((0x100000000ull + P - 1) / P) : 0u;
+  }
 };
 void ring_pick(int m, int n, int k, int cus, int force_t, int force_sk, int force_nf, RingGeom& g);
 // the same kernel over lists of rows with weights of their own (experts): tiles [count][4] = {matrix, first place, places, -}, places of a tile

@@ -687,7 +687,9 @@ void f16q_pick(int m, int n, int k, int cus, int force_t, int force_sk, RingGeom
   g.wpx = wpx;
 }
 
-int launch_f16q(const F16qGemm& q, const RingGeom& g, hipStream_t s) {
+int launch_f16q(const F16qGemm& q, const RingGeom& geom, hipStream_t s) {
+  RingGeom g = geom;
+  g.finish();
   static bool configured = false;
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f16q_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, kQLds);

@@ -88,10 +88,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
   const int ubeg = xcd * share + (xcd < rem ? xcd : rem), ucnt = share + (xcd < rem);
   if (local >= ucnt) return;                                   // padding workgroup (fewer units than workgroups): uniform exit
   const int uend = ubeg + ucnt, u0 = ubeg + local, ustep = g.wpx;
-  int G = 0;                                                   // half-steps of this workgroup = barriers after the first
-  if constexpr (GROUPED) G = (uend - u0 + ustep - 1) / ustep * (p.k >> 5);
-  else
-    for (int u = u0; u < uend; u += ustep) G += ring_unit(p, g, u).nh;
+  const int G = GROUPED ? (uend - u0 + ustep - 1) / ustep * (p.k >> 5) : 0;      // half-steps of this workgroup = barriers after the first
 
   if (wave >= kRingCompute) {
     // ---- loader wave L: pieces of 16 rows x 64 bytes (1 KB per wave instruction).  W pieces {L, L + 4, L + 8, L + 12}; of the unit's
@@ -104,6 +101,101 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
     const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64, astep = alltiled ? 1024 : 64;
     // three fragments do not hold whole (gate, up) pairs of 16 columns: there a gated product's W block is 8 gates and their 8 up rows
     const bool mixed = NF == 3 && p.direct && epi_is_glu(p.epilogue);
+    if constexpr (!GROUPED) {
+      // A launch's first bytes wait for what stands here: places by multiplication, bases in scalar registers, one offset a lane (as divisions and 64-bit addresses a lane they took 1.4 to
+      // 2.0 us of a launch).  As many pieces a half-stage for the whole launch (a shorter tile asks for one of its pieces twice): one loop, straight down, whose waits are constants (a branch
+      // a piece and the choice of the wait at run time: 1 us).
+      const int fmax = g.fbase + (g.frem > 0), na_max = SINGLE ? fmax : 2 * fmax, more = na_max > L ? (na_max - L + 3) >> 2 : 0;
+      const int wl = mixed ? (L & 1) * 8 + (prow & 7) : prow;      // this lane's row of a tiled block of W
+      unsigned lane_w = wtiled ? (mixed ? (unsigned)(prow >> 3) * (unsigned)nkt * 1024u : 0u) + (wl * 4 + (gchunk ^ ((wl >> 3) << 1))) * 16
+                                     : (unsigned)(mixed ? (prow >> 3) * 16 + (prow & 7) : prow) * (unsigned)p.ldw * 2u + gchunk * 16;
+      auto run = [&](auto n_c) __attribute__((always_inline)) {
+        constexpr int N = decltype(n_c)::value, NA = N - NF;
+        const char* wb[NF];
+        const char* ab[NA > 0 ? NA : 1];
+        unsigned lane_a[NA > 0 ? NA : 1];
+        int to[NA > 0 ? NA : 1], ashift[NA > 0 ? NA : 1];
+        char* base = smem;
+        int left = 3;                                          // half-stages that are asked for before the first barrier
+        for (int u = u0; u < uend; u += ustep) {
+          const RingUnit r = ring_unit(p, g, u);
+          const int kb = r.kbeg >> 5, na = SINGLE ? r.f : 2 * r.f;
+#pragma unroll
+          for (int h = 0; h < NF; ++h) {                       // (n is a multiple of 16, of 32 where it is gated: a block is there or not)
+            if (mixed) {
+              int unit8 = r.panel * (BN / 16) + L + 4 * h;     // eights of units
+              if (unit8 > (p.n >> 4) - 1) unit8 -= ((unit8 - ((p.n >> 4) - 1) + 1) >> 1) << 1;      // (its parity is in lane_w)
+              wb[h] = wtiled ? reinterpret_cast<const char*>(p.wt) + ((size_t)(unit8 >> 1) * 2 * nkt + kb) * 1024
+                             : reinterpret_cast<const char*>(p.w) + ((size_t)((unit8 >> 1) * 32 + (unit8 & 1) * 8) * p.ldw + r.kbeg) * 2;
+            } else {
+              int rb = r.panel * (BN / 16) + L + 4 * h;
+              if (rb > (p.n >> 4) - 1) rb = (p.n >> 4) - 1;
+              wb[h] = wtiled ? reinterpret_cast<const char*>(p.wt) + ((size_t)rb * nkt + kb) * 1024 : reinterpret_cast<const char*>(p.w) + ((size_t)rb * 16 * p.ldw + r.kbeg) * 2;
+            }
+          }
+#pragma unroll
+          for (int h = 0; h < NA; ++h) {
+            int q = L + 4 * h;
+            if (q >= na) q = h > 0 ? q - 4 : na - 1;             // (two fewer than the most)
+            const int plane = q >= r.f, frag = plane ? q - r.f : q, row = r.m0 + frag * 16;
+            const bool atiled = TILES ? alltiled || row < p.a_tiled : alltiled;
+            ashift[h] = atiled ? 10 : 6;
+            to[h] = plane * kRingAPlane + frag * 1024;
+            const char* pl = reinterpret_cast<const char*>(plane ? a_lo : a_hi);
+            if (atiled) {
+              ab[h] = pl + ((size_t)(row >> 4) * nkt + kb) * 1024;
+              lane_a[h] = lane * 16;
+            } else {
+              ab[h] = pl + ((size_t)row * ldp + r.kbeg) * 2;
+              const int last = p.m - 1 - row;
+              lane_a[h] = (unsigned)(prow < last ? prow : last) * (unsigned)ldp * 2u + gchunk * 16;
+            }
+          }
+          for (int t = 0; t < r.nh; ++t) {
+            if (left > 0) {
+              --left;
+            } else {
+              ring_wait_vmcnt_c<2 * N>();                      // the half-stage before the two youngest has landed
+              __builtin_amdgcn_s_barrier();                    // publishes it; every read of the slot that is asked for next has returned
+            }
+            asm("" : "+v"(lane_w));                            // (the sum of base and offset is not one to be carried along in vector registers)
+#pragma unroll
+            for (int h = 0; h < NA; ++h) asm("" : "+v"(lane_a[h]));
+#pragma unroll
+            for (int h = 0; h < NF; ++h) {
+              __builtin_amdgcn_global_load_lds((gptr_t)(wb[h] + lane_w), (lptr_t)(base + kRingWOff + (L + 4 * h) * 1024), 16, 0, 0);
+              wb[h] += wstep;
+            }
+#pragma unroll
+            for (int h = 0; h < NA; ++h) {
+              __builtin_amdgcn_global_load_lds((gptr_t)(ab[h] + lane_a[h]), (lptr_t)(base + to[h]), 16, 0, 0);
+              ab[h] += TILES ? 1 << ashift[h] : astep;
+            }
+            base = base == smem + (kRingSlots - 1) * kRingHalf ? smem : base + kRingHalf;
+          }
+        }
+        // (a launch has two half-steps at least)
+        if (left > 0) ring_wait_vmcnt_c<N>();
+        else ring_wait_vmcnt_c<2 * N>();
+        __builtin_amdgcn_s_barrier();
+        if (left == 0) {
+          ring_wait_vmcnt_c<N>();
+          __builtin_amdgcn_s_barrier();
+        }
+        ring_wait_vmcnt_c<0>();
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();
+      };
+      switch (more) {
+        case 0: run(std::integral_constant<int, NF>{}); break;
+        case 1: run(std::integral_constant<int, NF + 1>{}); break;
+        case 2: run(std::integral_constant<int, NF + 2>{}); break;
+        case 3: run(std::integral_constant<int, NF + 3>{}); break;
+        case 4: run(std::integral_constant<int, NF + 4>{}); break;
+        default: run(std::integral_constant<int, NF + 5>{}); break;
+      }
+      return;
+    }
     const char* src[NF + 5];
     int dst[NF + 5], ashift[TILES ? 5 : 1];
     int np = 0, nh_cur = 0, hh = 0, ucur = u0;
@@ -386,7 +478,9 @@ int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t*
   CHATTS_CHECK_LAUNCH("gemm_ring_group");
   return CHATTS_OK;
 }
-int launch_ring(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& g, bool single, hipStream_t s) {
+int launch_ring(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGeom& geom, bool single, hipStream_t s) {
+  RingGeom g = geom;
+  g.finish();
   if (g.nf == 3) return single ? launch_ring_t<true, 3>(p, a_hi, a_lo, ldp, g, s) : launch_ring_t<false, 3>(p, a_hi, a_lo, ldp, g, s);
   return single ? launch_ring_t<true, 4>(p, a_hi, a_lo, ldp, g, s) : launch_ring_t<false, 4>(p, a_hi, a_lo, ldp, g, s);
 }

@@ -18,17 +18,19 @@ __device__ __forceinline__ void ring_wait_vmcnt(int n) {      // wave-uniform n:
 #undef CHATTS_VM
 }
 
+template <int N>
+__device__ __forceinline__ void ring_wait_vmcnt_c() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+
 struct RingUnit {
   int panel, split, m0, f, f0, kbeg, nh;      // f0 = fragments of wave row 0 (ceil(f / 2)); nh = half-steps (K / 32) of this unit
 };
 __device__ __forceinline__ RingUnit ring_unit(const GemmParams& p, const RingGeom& g, int u) {
   RingUnit r;
-  const int mt = u % g.T, rest = u / g.T;
-  r.panel = rest % g.P;
-  r.split = rest / g.P;
-  const int base = g.F / g.T, rem = g.F % g.T;
-  r.f = base + (mt < rem);
-  r.m0 = (mt * base + (mt < rem ? mt : rem)) * 16;
+  const int rest = g.inv_t ? (int)__umulhi((unsigned)u, g.inv_t) : u, mt = u - rest * g.T;
+  r.split = g.inv_p ? (int)__umulhi((unsigned)rest, g.inv_p) : rest;
+  r.panel = rest - r.split * g.P;
+  r.f = g.fbase + (mt < g.frem);
+  r.m0 = (mt * g.fbase + (mt < g.frem ? mt : g.frem)) * 16;
   r.f0 = (r.f + 1) >> 1;
   r.kbeg = r.split * p.k_per_split;
   int kend = r.kbeg + p.k_per_split;
