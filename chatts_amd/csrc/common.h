@@ -88,6 +88,21 @@ __device__ __forceinline__ float rows4_sum(float v) {
   return (readlane_bits(v, 0) + readlane_bits(v, 16)) + (readlane_bits(v, 32) + readlane_bits(v, 48));
 }
 
+// The first N bytes of a kernel's arguments, a word of every 64: all their lines are asked for at once when a launch starts.  The compiler loads an argument where it is used, behind
+// branches and other waits, and each line is a round trip to memory of its own the first time.
+template <size_t N>
+__device__ __forceinline__ void kernarg_touch() {
+#ifdef __HIP_DEVICE_COMPILE__
+  const __attribute__((address_space(4))) uint32_t* k = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int LINES = (int)((N + 63) / 64);
+  uint32_t v[LINES];
+#pragma unroll
+  for (int i = 0; i < LINES; ++i) v[i] = k[i * 16];
+#pragma unroll
+  for (int i = 0; i < LINES; ++i) asm volatile("" :: "s"(v[i]));
+#endif
+}
+
 __device__ __forceinline__ float wave_sum(float v) { return rows4_sum(row16_sum(v)); }   // every lane gets the total
 __device__ __forceinline__ float wave_max(float v) { return rows4_max(row16_max(v)); }
 __device__ __forceinline__ int wave_sum_i(int v) {

@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
                                                                  const uint16_t* __restrict__ a_lo, int ldp, RingGeom g, RingGroup gr) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int BN = 64 * NF;
+  kernarg_touch<sizeof(GemmParams) + 2 * sizeof(void*) + 8 + sizeof(RingGeom) + (GROUPED ? sizeof(RingGroup) : 0)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // this workgroup's units: XCD x (= blockIdx % 8, observed; speed only) owns a contiguous eighth of the unit sequence and its
