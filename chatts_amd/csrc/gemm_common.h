@@ -62,14 +62,16 @@ __device__ __forceinline__ void store_planes4(uint16_t* hi, uint16_t* lo, f32x4 
   *reinterpret_cast<bf16x4_t*>(lo) = lv;
 }
 
-// eight 8-bit weights as bf16: both steps are exact
+// eight 8-bit weights as bf16, exactly: two a instruction (by way of float32 it took two for that, and they are most of what a few-rows kernel issues).
 __device__ __forceinline__ bf16x8_t widen_fp8(u32x2 q8) {
-  typedef float f32x2_t __attribute__((ext_vector_type(2)));
-  const f32x2_t f0 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, false), f1 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.x, true);
-  const f32x2_t f2 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, false), f3 = __builtin_amdgcn_cvt_pk_f32_fp8(q8.y, true);
-  bf16x8_t bv;
-  bv[0] = (__bf16)f0.x; bv[1] = (__bf16)f0.y; bv[2] = (__bf16)f1.x; bv[3] = (__bf16)f1.y;
-  bv[4] = (__bf16)f2.x; bv[5] = (__bf16)f2.y; bv[6] = (__bf16)f3.x; bv[7] = (__bf16)f3.y;
+  bf16x8_t bv = {};
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q8[i], 1.f, false), hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q8[i], 1.f, true);
+    bv[4 * i] = lo[0]; bv[4 * i + 1] = lo[1]; bv[4 * i + 2] = hi[0]; bv[4 * i + 3] = hi[1];
+  }
+#endif
   return bv;
 }
 __device__ __forceinline__ bf16x8_t widen_i8(u32x2 q8) {
