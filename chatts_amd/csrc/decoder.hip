@@ -15,7 +15,7 @@ int launch_gemv(const ChattsLinearArgs* a, hipStream_t s);
 int launch_gemm_f32(const ChattsLinearArgs* a, hipStream_t s);
 bool gemm_batched_stream(const ChattsLinearArgs* a);
 size_t gemm_workspace_batch(int m, int n, int k, int batch);
-int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles);
+int launch_gemm(const ChattsLinearArgs* a, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles, SplitSums* leave);
 int gemm_post_ss_parts(const ChattsLinearArgs* a);
 int gemm_few_rows(const ChattsLinearArgs* a, const ChattsNormChain* chain);
 bool gemm_takes_cols(const ChattsLinearArgs* a);
@@ -65,7 +65,8 @@ enum { kProjQkv, kProjO, kProjGateUp, kProjDown };
 static int64_t embed_rows(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_rows : d->cfg.vocab_local; }
 static int64_t embed_offset(const ChattsDecoder* d) { return d->cfg.embed_rows > 0 ? d->cfg.embed_offset : d->cfg.vocab_offset; }
 
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain = nullptr, PlaneTiles tiles = {});
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain = nullptr, PlaneTiles tiles = {},
+                       SplitSums* leave = nullptr);
 extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream) {
   CHATTS_REQUIRE(a && ch, CHATTS_E_BADARG, "linear_chain: null args");
   CHATTS_REQUIRE(!ch->row_ss || (((uintptr_t)ch->row_ss % 16) == 0 && a->a_hi && a->a_lo && a->m >= 2 && a->m <= 16 && a->batch <= 1 && !a->exact_f32 && ch->row_ss_parts >= 1 &&
@@ -107,11 +108,11 @@ extern "C" size_t chatts_linear_workspace_batch(int m, int n, int k, int batch) 
 }
 
 extern "C" int chatts_linear(const ChattsLinearArgs* a, chatts_stream_t stream) { return linear_impl(a, stream, nullptr, nullptr); }
-int chatts::linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles) { return linear_impl(a, stream, nullptr, nullptr, nullptr, tiles); }
+int chatts::linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles, SplitSums* leave) { return linear_impl(a, stream, nullptr, nullptr, nullptr, tiles, leave); }
 
 // rope / rope_done: the qkv projection of a prefill chunk may carry rope_kv_kernel's work in its split-K epilogue (*rope_done says
 // whether it did, and the planes of K and V with it; otherwise rope_attention_impl does both)
-static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
+static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles, SplitSums* leave) {
   CHATTS_REQUIRE(a != nullptr, CHATTS_E_BADARG, "linear: null args");
   CHATTS_REQUIRE(a->m >= 0 && a->n > 0 && a->k > 0, CHATTS_E_BADARG, "linear: bad sizes m=%d n=%d k=%d", a->m, a->n, a->k);
   if (a->m == 0) return CHATTS_OK;
@@ -174,7 +175,7 @@ static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const 
     return launch_gemm_f32(a, as_stream(stream));
   }
   CHATTS_REQUIRE(a->norm_w == nullptr, CHATTS_E_BADARG, "linear: fused RMSNorm is only available for M == 1");
-  return launch_gemm(a, as_stream(stream), rope, rope_done, chain, tiles);
+  return launch_gemm(a, as_stream(stream), rope, rope_done, chain, tiles, leave);
 }
 
 extern "C" int chatts_split_bf16x2(const float* x, int m, int k, int ldx, chatts_bf16* hi, chatts_bf16* lo, int ld_planes,

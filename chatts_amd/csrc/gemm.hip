@@ -1079,7 +1079,7 @@ size_t gemm_workspace(int m, int n, int k) {
   return sk > 1 ? (size_t)sk * m * n * sizeof(float) : 0;
 }
 
-int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles) {
+int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain, PlaneTiles tiles, SplitSums* leave) {
   int bm, sk;
   ChattsLinearArgs a_copy;
   const ChattsLinearArgs* a = a_in;
@@ -1201,6 +1201,11 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     }
   }
   CHATTS_CHECK_LAUNCH("gemm_bf16x2");
+  if (leave && stream && sk > 1 && sk <= kMostSplitSums && a->m <= 16 && batch == 1 && !chain && a->epilogue == CHATTS_EPI_NONE && !a->post_norm_w && !a->c_hi && !a->w8 &&
+      (((uintptr_t)a->workspace | (uintptr_t)a->bias) % 16) == 0) {
+    *leave = SplitSums{reinterpret_cast<const float*>(a->workspace), a->bias, (size_t)a->m * a->n, sk, a->n};
+    return CHATTS_OK;
+  }
   if (ch.post_ss) {
     const int groups = a->n / 4, parts = rows_grid(a->n, a->epilogue);
     hipLaunchKernelGGL(splitk_epilogue_ss_kernel, dim3(parts), dim3(64 * (((groups + parts - 1) / parts + 3) / 4)), 0, s, reinterpret_cast<const float*>(a->workspace), sk, a->m, a->n, a->bias, a->resid, a->c, a->ldc,

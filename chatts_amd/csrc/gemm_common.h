@@ -106,7 +106,34 @@ struct PlaneTiles {
 constexpr int kMidPlanesK = 1024;
 bool planes_tiled_for(int m, int n, int k);      // (gemm.hip: of the A of an m x n x k product)
 bool stream_leaves_cus(int m, int n, int k);     // (gemm.hip: 65 .. 128 rows with W in tiles are the prefill kernel's)
-int linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles);      // chatts_linear on such planes (decoder.hip)
+// The sums that a projection of few rows left in the workspace, [sk][rows][n], for a reader that adds them up itself (sk == 0: none were left, c is written).  A launch of a captured graph
+// takes 1.7 us before it does anything, and the sums' own launch does 0.3 us of work on 16 rows.
+struct SplitSums {
+  const float* slabs;
+  const float* bias;
+  size_t plane;         // floats of a split
+  int sk, n;
+};
+constexpr int kMostSplitSums = 8;
+// four neighbours, in splitk_epilogue_v4_kernel's order: the same bits
+template <int S>
+__device__ __forceinline__ f32x4 split_sum4(const SplitSums& p, int row, int col) {
+  const float* at = p.slabs + (size_t)row * p.n + col;
+  f32x4 t[S], b = {0.f, 0.f, 0.f, 0.f}, v = b;
+#pragma unroll
+  for (int s = 0; s < S; ++s) t[s] = *reinterpret_cast<const f32x4*>(at + (s < p.sk ? s : p.sk - 1) * p.plane);
+  if (p.bias) b = *reinterpret_cast<const f32x4*>(p.bias + col);
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < p.sk) v += t[s];
+  if (p.bias) v += b;
+  return v;
+}
+int linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles, SplitSums* leave = nullptr);      // chatts_linear on such planes (decoder.hip)
+int gru_decode(const ChattsGruArgs* a, const SplitSums& in, hipStream_t s);      // chatts_gru_decode on what a projection left (gru.hip)
+// what attention and a selective scan that read one projection do before their own launches, one token per row, and the rest of its sums into proj (window.hip)
+bool window_select_can_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c);
+int window_select_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c, const SplitSums& in, float* proj, hipStream_t s);
 
 constexpr int kRingPanel = 256;      // W rows per panel of the prefill kernel
 // gemm_ring.hip: the prefill kernel's decomposition (M-tiles per panel, K splits) and launcher

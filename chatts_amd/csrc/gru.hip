@@ -4,21 +4,25 @@
 //   gru_scan_kernel    segments of several tokens: every step is an affine map S -> a S + b and maps compose, so a workgroup owns 16 channels and walks the
 //                      tokens in tiles: a thread composes its four tokens, a wave and then the workgroup put the threads' maps together, and every thread
 //                      runs its tokens again from the state it then knows.  Every input is read once.
-#include "common.h"
+#include "gemm_common.h"
 
 namespace chatts {
 
 __device__ __forceinline__ float gru_candidate(float x) { return x >= 0.f ? x + 0.5f : sigmoid_f(x); }
 __device__ __forceinline__ float silu4(float g) { return g * sigmoid_f(g); }
 
-// grid (width / 1024, rows): a thread owns four channels
-__global__ __launch_bounds__(256) void gru_decode_kernel(ChattsGruArgs p) {
-  const int row = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
+// grid (width / four a thread, rows): a thread owns four channels.  S_IN: the projection left up to so many splits, their sums are taken here
+template <int S_IN>
+__global__ __launch_bounds__(256) void gru_decode_kernel(ChattsGruArgs p, SplitSums in) {
+  const int row = blockIdx.y, c = (int)(blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const ChattsRow R = p.rows[row];
   const int w4 = (p.width + 3) & ~3;
   if (R.pos < 0 || c >= w4) return;
-  const float* pr = p.proj + (size_t)row * p.ld_proj + c;
-  const f32x4 z = *reinterpret_cast<const f32x4*>(pr + p.off_z), x = *reinterpret_cast<const f32x4*>(pr + p.off_x), g = *reinterpret_cast<const f32x4*>(pr + p.off_g);
+  auto input = [&](int off) __attribute__((always_inline)) {
+    if constexpr (S_IN > 0) return split_sum4<S_IN>(in, row, off + c);
+    else return *reinterpret_cast<const f32x4*>(p.proj + (size_t)row * p.ld_proj + c + off);
+  };
+  const f32x4 z = input(p.off_z), x = input(p.off_x), g = input(p.off_g);
   float* st = p.state + (size_t)R.slot * w4 + c;
   f32x4 S = {0.f, 0.f, 0.f, 0.f};
   if (R.pos > 0) S = *reinterpret_cast<const f32x4*>(st);
@@ -132,7 +136,17 @@ using namespace chatts;
 extern "C" int chatts_gru_decode(const ChattsGruArgs* a, chatts_stream_t stream) {
   if (const int rc = check_gru(a, "gru_decode")) return rc;
   if (a->n_rows == 0) return CHATTS_OK;
-  hipLaunchKernelGGL(gru_decode_kernel, dim3((a->width + 1023) / 1024, a->n_rows), dim3(256), 0, as_stream(stream), *a);
+  hipLaunchKernelGGL(gru_decode_kernel<0>, dim3((a->width + 1023) / 1024, a->n_rows), dim3(256), 0, as_stream(stream), *a, SplitSums{});
+  CHATTS_CHECK_LAUNCH("gru_decode");
+  return CHATTS_OK;
+}
+int chatts::gru_decode(const ChattsGruArgs* a, const SplitSums& in, hipStream_t s) {
+  if (const int rc = check_gru(a, "gru_decode")) return rc;
+  CHATTS_REQUIRE(in.sk >= 1 && in.sk <= kMostSplitSums && in.n == a->ld_proj, CHATTS_E_SHAPE, "gru_decode: %d splits of %d columns", in.sk, in.n);
+  if (a->n_rows == 0) return CHATTS_OK;
+  const dim3 grid((a->width + 255) / 256, a->n_rows), block(64);      // (single waves: all of a launch's loads are one round trip)
+  if (in.sk <= 4) hipLaunchKernelGGL(gru_decode_kernel<4>, grid, block, 0, s, *a, in);
+  else hipLaunchKernelGGL(gru_decode_kernel<kMostSplitSums>, grid, block, 0, s, *a, in);
   CHATTS_CHECK_LAUNCH("gru_decode");
   return CHATTS_OK;
 }

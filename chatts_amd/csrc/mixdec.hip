@@ -181,7 +181,7 @@ static ChattsOperand operand(const ChattsMixDecoder* d, bool second, int m, int 
 }
 
 static int mix_linear(const ChattsMixDecoder* d, const ChattsOperand& in, const chatts_bf16* w, const chatts_bf16* w_t, int m, int n, int k, int epilogue,
-                      const ChattsOperand& out, chatts_stream_t s, float limit = 0.f, float alpha = 0.f, const float* bias = nullptr, bool a_tiles = false) {
+                      const ChattsOperand& out, chatts_stream_t s, float limit = 0.f, float alpha = 0.f, const float* bias = nullptr, bool a_tiles = false, SplitSums* leave = nullptr) {
   ChattsLinearArgs a{};
   a.bias = bias;
   a.glu_limit = limit; a.glu_alpha = alpha;
@@ -195,7 +195,7 @@ static int mix_linear(const ChattsMixDecoder* d, const ChattsOperand& in, const 
   if (!out.f32) { a.c_hi = out.hi; a.c_lo = out.lo; a.ld_cplanes = out.ld; }
   a.exact_f32 = d->c.exact;
   a.workspace = d->b.workspace; a.workspace_bytes = d->b.workspace_bytes;
-  return linear_tiled(&a, s, {a_tiles, false, false});
+  return linear_tiled(&a, s, {a_tiles, false, false}, leave);
 }
 static ChattsOperand f32_out(float* p, int ld) {
   ChattsOperand o{};
@@ -362,9 +362,8 @@ static int mix_recur(const ChattsMixDecoder* d, const ChattsMixLayer& l, const C
   return chatts_recur_out(&a, s);
 }
 
-static int mix_window(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, const ChattsSpan* spans, int n_spans, bool single,
-                      const ChattsOperand& out, chatts_stream_t s) {
-  StageRange stage("chatts.mix.window");
+static ChattsWindowArgs mix_window_args(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, const ChattsSpan* spans, int n_spans, bool single,
+                                        const ChattsOperand& out) {
   ChattsWindowArgs a = l.window;
   a.proj = d->b.proj; a.ld_proj = l.in_n; a.eps = d->c.eps;
   a.kcache = run.cache; a.vcache = run.vcache; a.cache_f32 = d->c.exact;
@@ -378,7 +377,15 @@ static int mix_window(const ChattsMixDecoder* d, const ChattsMixLayer& l, const 
   a.out = out; a.n_splits = 1; a.longest = 0;
   for (int i = 0; !single && i < n_spans; ++i)
     if (spans[i].t > a.longest) a.longest = spans[i].t;
-  if (const int rc = chatts_window_prep(&a, s)) return rc;
+  return a;
+}
+// prepared: queries, keys and values are in their places
+static int mix_window(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, const ChattsSpan* spans, int n_spans, bool single,
+                      const ChattsOperand& out, chatts_stream_t s, bool prepared = false) {
+  StageRange stage("chatts.mix.window");
+  ChattsWindowArgs a = mix_window_args(d, l, run, t, spans, n_spans, single, out);
+  if (!prepared)
+    if (const int rc = chatts_window_prep(&a, s)) return rc;
   if (a.longest >= 8 && !d->c.exact && chatts_window_can_prefill(a.dim_p, a.vdim_p)) return chatts_window_prefill(&a, s);
   if (!d->c.exact) {      // few rows: a row's tiles (32 keys a wave, 4 waves) are spread over workgroups, about three per CU, the same number to every wave
     const int group = a.heads / a.kv_heads, wgs = a.kv_heads * ((group + 15) / 16) * t;
@@ -569,32 +576,40 @@ static int mix_post_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, c
 }
 
 // ---- norms before the sublayers only ----
-static int mix_gru(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, int n_spans, bool single, const ChattsOperand& out, chatts_stream_t s) {
+// in: the projection's sums, where it left them
+static int mix_gru(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, int n_spans, bool single, const ChattsOperand& out, chatts_stream_t s,
+                   const SplitSums& in) {
   StageRange stage("chatts.mix.gru");
   ChattsGruArgs a = l.gru;
   a.proj = d->b.proj; a.ld_proj = l.in_n;
   a.state = run.gru_state;
   a.rows = d->b.rows; a.n_rows = t; a.spans = d->b.spans; a.n_spans = n_spans;
   a.out = out;
+  if (in.sk) return gru_decode(&a, in, as_stream(s));
   return single ? chatts_gru_decode(&a, s) : chatts_gru_scan(&a, s);
 }
 
-static int mix_select(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, int n_spans, bool single, const ChattsOperand& out, chatts_stream_t s) {
-  StageRange stage("chatts.mix.select");
+static ChattsSelectArgs mix_select_args(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, int n_spans, bool single, const ChattsOperand& out) {
   const ChattsMixBuffers& b = d->b;
   ChattsSelectArgs a = l.select;
   a.proj = b.proj; a.ld_proj = l.in_n;
   a.s = run.sel_state; a.ring = run.sel_ring;
   a.rows = b.rows; a.n_rows = t; a.spans = b.spans; a.n_spans = single ? 0 : n_spans;
   a.u.f32 = b.sel_u; a.u.ld = l.sel_k;
-  ChattsOperand in = f32_out(b.sel_u, l.sel_k);
-  if (mix_planes(d, t, l.sel_k)) {
-    a.u.hi = b.sel_u_hi; a.u.lo = b.sel_u_lo;
-    in.f32 = nullptr; in.hi = b.sel_u_hi; in.lo = b.sel_u_lo;
-  }
+  if (mix_planes(d, t, l.sel_k)) { a.u.hi = b.sel_u_hi; a.u.lo = b.sel_u_lo; }
   a.low = b.sel_low; a.out = out;
+  return a;
+}
+// prepared: the convolution has run
+static int mix_select(const ChattsMixDecoder* d, const ChattsMixLayer& l, const ChattsMixRun& run, int t, int n_spans, bool single, const ChattsOperand& out, chatts_stream_t s,
+                      bool prepared = false) {
+  StageRange stage("chatts.mix.select");
+  const ChattsMixBuffers& b = d->b;
+  ChattsSelectArgs a = mix_select_args(d, l, run, t, n_spans, single, out);
+  ChattsOperand in = a.u;
+  if (in.hi) in.f32 = nullptr;
   int rc;
-  if ((rc = chatts_select_conv(&a, s)) != 0) return rc;
+  if (!prepared && (rc = chatts_select_conv(&a, s)) != 0) return rc;
   if ((rc = mix_linear(d, in, l.sel_low, l.sel_low_t, t, a.ld_low, l.sel_k, CHATTS_EPI_NONE, f32_out(b.sel_low, a.ld_low), s)) != 0) return rc;
   if (single) return chatts_select_decode(&a, s);
   ChattsOperand dt = f32_out(b.sel_low + a.off_dt, a.ld_low);
@@ -613,9 +628,9 @@ static int mix_select(const ChattsMixDecoder* d, const ChattsMixLayer& l, const 
 }
 
 static int mix_one(const ChattsMixDecoder* d, const ChattsMixLayer& l, int kind, const ChattsMixRun& run, int t, const ChattsSpan* spans, int n_spans, bool single,
-                   const ChattsOperand& out, chatts_stream_t s) {
-  if (kind == CHATTS_MIX_WINDOW) return mix_window(d, l, run, t, spans, n_spans, single, out, s);
-  return kind == CHATTS_MIX_GRU ? mix_gru(d, l, run, t, n_spans, single, out, s) : mix_select(d, l, run, t, n_spans, single, out, s);
+                   const ChattsOperand& out, chatts_stream_t s, const SplitSums& in) {
+  if (kind == CHATTS_MIX_WINDOW) return mix_window(d, l, run, t, spans, n_spans, single, out, s, in.sk > 0);
+  return kind == CHATTS_MIX_GRU ? mix_gru(d, l, run, t, n_spans, single, out, s, in) : mix_select(d, l, run, t, n_spans, single, out, s, in.sk > 0);
 }
 
 // x += mult (y + what the experts of `moe` owe it), averaged over depth after the run number `stream` of a layer with such weights; then the next norm
@@ -653,16 +668,26 @@ static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, co
     const ChattsMixRun& run = d->runs[r];
     const ChattsMixLayer& l = d->layers[run.layer];
     const float* next = r + 1 < c.n_runs ? d->layers[d->runs[r + 1].layer].norm1 : nullptr;
-    if ((rc = mix_linear(d, A, l.in, l.in_t, t, l.in_n, wp, CHATTS_EPI_NONE, f32_out(d->b.proj, l.in_n), s, 0.f, 0.f, l.in_bias, tiles)) != 0) return rc;
-    tiles = next && tiles_for(d->layers[d->runs[r + 1].layer]);
     const ChattsOperand B = operand(d, true, t, l.out_k);
-    if ((rc = mix_one(d, l, l.kind, run, t, spans, n_spans, single, B, s)) != 0) return rc;
-    if (l.beside) {
-      ChattsOperand C = B;
-      if (C.f32) C.f32 += l.beside_col;
-      else { C.hi += l.beside_col; C.lo += l.beside_col; }
-      if ((rc = mix_one(d, l, l.beside, run, t, spans, n_spans, single, C, s)) != 0) return rc;
+    ChattsOperand C = B;      // of the mixer beside the first
+    if (C.f32) C.f32 += l.beside_col;
+    else { C.hi += l.beside_col; C.lo += l.beside_col; }
+    // one token per row: a recurrence takes the sums of its projection's splits itself, and attention beside a scan in the launch that prepares both
+    const bool pair = l.beside && l.kind != l.beside && mix_has(l, CHATTS_MIX_WINDOW) && mix_has(l, CHATTS_MIX_SELECT), window_first = l.kind == CHATTS_MIX_WINDOW;
+    ChattsWindowArgs wa{};
+    ChattsSelectArgs sa{};
+    bool takes_sums = single && l.kind == CHATTS_MIX_GRU && !l.beside;
+    if (single && pair) {
+      wa = mix_window_args(d, l, run, t, spans, n_spans, single, window_first ? B : C);
+      sa = mix_select_args(d, l, run, t, n_spans, single, window_first ? C : B);
+      takes_sums = window_select_can_prep(&wa, &sa);
     }
+    SplitSums left{};
+    if ((rc = mix_linear(d, A, l.in, l.in_t, t, l.in_n, wp, CHATTS_EPI_NONE, f32_out(d->b.proj, l.in_n), s, 0.f, 0.f, l.in_bias, tiles, takes_sums ? &left : nullptr)) != 0) return rc;
+    if (left.sk && pair && (rc = window_select_prep(&wa, &sa, left, d->b.proj, as_stream(s))) != 0) return rc;
+    tiles = next && tiles_for(d->layers[d->runs[r + 1].layer]);
+    if ((rc = mix_one(d, l, l.kind, run, t, spans, n_spans, single, B, s, left)) != 0) return rc;
+    if (l.beside && (rc = mix_one(d, l, l.beside, run, t, spans, n_spans, single, C, s, left)) != 0) return rc;
     if ((rc = mix_linear(d, B, l.out, l.out_t, t, wp, l.out_k, CHATTS_EPI_NONE, Y, s)) != 0) return rc;
     const bool moe = l.ff_kind == CHATTS_FF_MOE;
     if (l.ff_kind == CHATTS_FF_NONE) {

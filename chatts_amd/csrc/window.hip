@@ -3,6 +3,7 @@
 // keeps a sequence's first tokens, chunks, a sink (one more term exp(0) in the denominator); an output gate per value or per head.
 //   window_prep_kernel      per-head work: norms, rotation, values; queries as an operand, keys and values into their pages
 //   window_prep_quads_kernel  the same, four channels a lane
+//   window_select_prep_kernel  one token per row, beside a selective scan: the quads' work, the scan's convolution and the sums of their projection
 //   window_prep_rows_kernel the same for layers with convolutions or norms over all heads: a workgroup owns whole rows
 //   window_ring_kernel      the last convolution inputs of every segment
 //   window_attend_kernel    one row and query head per workgroup, vector units: 32-bit runs, head sizes beyond the matrix kernels
@@ -10,6 +11,8 @@
 //   window_prefill_kernel   flash attention for segments of many rows
 // Pages: keys [page][kv head][token][dim_p], values [page][kv head][token][vdim_p]; a page holds a multiple of 64 tokens, so a tile of up to 64
 // keys of a head is contiguous memory.
+#include <utility>
+
 #include "gemm_common.h"
 
 namespace chatts {
@@ -70,6 +73,8 @@ __device__ __forceinline__ CT to_page(float v) {
   if constexpr (sizeof(CT) == 4) return v;
   else return __builtin_bit_cast(uint16_t, (__bf16)v);
 }
+
+constexpr int kConvRegs = 4;      // taps whose weights stay in registers
 
 // grid (rows, n): the 4 n waves of a row take heads [q | k | v] in turn
 template <typename CT>
@@ -144,17 +149,16 @@ __device__ __forceinline__ void store_page4(CT* dst, const f32x4& v) {
   if constexpr (sizeof(CT) == 4) *reinterpret_cast<f32x4*>(dst) = v;
   else *reinterpret_cast<w16x4*>(dst) = (w16x4){(short)to_page<CT>(v[0]), (short)to_page<CT>(v[1]), (short)to_page<CT>(v[2]), (short)to_page<CT>(v[3])};
 }
-template <typename CT, int LPH>
-__global__ __launch_bounds__(256) void window_prep_quads_kernel(ChattsWindowArgs p) {
+template <typename CT, int LPH, class Input>
+__device__ __forceinline__ void window_quads(const ChattsWindowArgs& p, int row, int part, int parts, Input input) {      // input(column): four of the row's projected values
   constexpr int PER = 64 / LPH;
-  const int row = blockIdx.x, lane = threadIdx.x & 63, H = p.heads, G = p.kv_heads, c = (lane & (LPH - 1)) * 4;
+  const int lane = threadIdx.x & 63, H = p.heads, G = p.kv_heads, c = (lane & (LPH - 1)) * 4;
   const ChattsRow R = p.rows[row];
   if (R.pos < 0) return;
-  const float* pr = p.proj + (size_t)row * p.ld_proj;
   const size_t page = window_tile(p, R.slot, 0, R.pos);      // head e of the page: e << log_block rows further
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  const int stride = 4 * PER * gridDim.y;
-  for (int e0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * PER + lane / LPH; e0 - lane / LPH < H + 2 * G; e0 += 2 * stride) {      // (uniform)
+  const int stride = 4 * PER * parts;
+  for (int e0 = (part * 4 + (threadIdx.x >> 6)) * PER + lane / LPH; e0 - lane / LPH < H + 2 * G; e0 += 2 * stride) {      // (uniform)
     f32x4 x[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -162,7 +166,7 @@ __global__ __launch_bounds__(256) void window_prep_quads_kernel(ChattsWindowArgs
       const bool value = e >= H + G;
       const int n = value ? p.vdim : p.dim;
       x[u] = zero;
-      if (e < H + 2 * G && c < n) x[u] = *reinterpret_cast<const f32x4*>(pr + (e < H ? p.off_q + e * n : (value ? p.off_v + (e - H - G) * n : p.off_k + (e - H) * n)) + c);
+      if (e < H + 2 * G && c < n) x[u] = input((e < H ? p.off_q + e * n : (value ? p.off_v + (e - H - G) * n : p.off_k + (e - H) * n)) + c);
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -204,9 +208,60 @@ __global__ __launch_bounds__(256) void window_prep_quads_kernel(ChattsWindowArgs
   }
 }
 
+template <typename CT, int LPH>
+__global__ __launch_bounds__(256) void window_prep_quads_kernel(ChattsWindowArgs p) {
+  const float* pr = p.proj + (size_t)blockIdx.x * p.ld_proj;
+  window_quads<CT, LPH>(p, blockIdx.x, blockIdx.y, gridDim.y, [&](int col) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(pr + col); });
+}
+
+// One token per row, a layer of attention beside a selective scan: this kernel's work, select_conv_kernel's and the sums of their projection, which it left as splits, in one launch of
+// three kinds of workgroups (three launches of two round trips each before: with the recurrences that take their sums themselves, 16 rows of 2048 columns, eight layers, 951 -> 928 us).
+// rest: ranges of columns that later launches read from proj (gates).  At most kConvRegs taps.
+struct RestCols { int n, from[5], quads[5], total; };
+template <int LPH, int S>
+__global__ __launch_bounds__(256) void window_select_prep_kernel(ChattsWindowArgs p, ChattsSelectArgs q, SplitSums in, RestCols rest, float* proj, int parts, int conv_parts) {
+  const int row = blockIdx.x;
+  int part = blockIdx.y;
+  if (part < parts) {
+    window_quads<uint16_t, LPH>(p, row, part, parts, [&](int col) __attribute__((always_inline)) { return split_sum4<S>(in, row, col); });
+    return;
+  }
+  part -= parts;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (part < conv_parts) {
+    const int c = (part * 256 + (int)threadIdx.x) * 4, taps = q.taps;
+    const ChattsRow R = q.rows[row];
+    if (R.pos < 0 || c >= ((q.inner + 3) & ~3)) return;
+    f32x4 w[kConvRegs], x[kConvRegs];      // [tokens back]
+#pragma unroll
+    for (int g = kConvRegs - 1; g >= 0; --g) {
+      const int at = R.pos - g;
+      w[g] = g < taps ? *reinterpret_cast<const f32x4*>(q.conv_w + (size_t)(taps - 1 - g) * q.conv_ch + c) : zero;
+      if (g > 0) x[g] = g < taps && at >= 0 ? *reinterpret_cast<const f32x4*>(q.ring + ((size_t)R.slot * taps + at % taps) * q.conv_ch + c) : zero;
+    }
+    f32x4 y = *reinterpret_cast<const f32x4*>(q.conv_b + c);
+    x[0] = split_sum4<S>(in, row, q.off_x + c);
+#pragma unroll
+    for (int g = kConvRegs - 1; g >= 0; --g)
+      if (g < taps) y += w[g] * x[g];
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = y[k] * sigmoid_f(y[k]);
+    store_operand4(q.u, row, c, v);
+    *reinterpret_cast<f32x4*>(q.ring + ((size_t)R.slot * taps + R.pos % taps) * q.conv_ch + c) = x[0];
+    return;
+  }
+  int i = (part - conv_parts) * 256 + (int)threadIdx.x, col = -1;
+#pragma unroll
+  for (int r = 0; r < 5; ++r) {
+    if (r < rest.n && col < 0 && i < rest.quads[r]) col = rest.from[r] + 4 * i;
+    if (r < rest.n) i -= rest.quads[r];
+  }
+  if (col >= 0) *reinterpret_cast<f32x4*>(proj + (size_t)row * p.ld_proj + col) = split_sum4<S>(in, row, col);
+}
+
 // A workgroup owns ROWS rows, a thread quads of channels of [q | k | v]: convolutions over a window of rows in registers (inputs before a segment come from
 // the ring), norms over all heads, mixed values.
-constexpr int kConvRegs = 4;      // taps whose weights stay in registers
 template <typename CT, int NT, int NV, int ROWS>
 __global__ __launch_bounds__(NT, 4) void window_prep_rows_kernel(ChattsWindowArgs p) {
   __shared__ float red[NT / 64][2 * ROWS];
@@ -991,6 +1046,46 @@ extern "C" int chatts_window_prep(const ChattsWindowArgs* a, chatts_stream_t str
   if (a->cache_f32) hipLaunchKernelGGL(window_prep_kernel<float>, dim3(a->n_rows, per_row), dim3(256), 0, as_stream(stream), *a);
   else hipLaunchKernelGGL(window_prep_kernel<uint16_t>, dim3(a->n_rows, per_row), dim3(256), 0, as_stream(stream), *a);
   CHATTS_CHECK_LAUNCH("window_prep");
+  return CHATTS_OK;
+}
+
+// Where the quads' kernel serves the attention, and a scan's taps fit the registers.
+bool chatts::window_select_can_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c) {
+  return !w->taps && !w->norm_whole && !w->cache_f32 && c->n_spans == 0 && c->taps <= kConvRegs && (w->dim | w->vdim | w->off_q | w->off_k | w->off_v) % 4 == 0 &&
+         ((uintptr_t)w->q_norm | (uintptr_t)w->k_norm) % 16 == 0 && w->ld_proj == c->ld_proj && w->n_rows == c->n_rows;
+}
+int chatts::window_select_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c, const SplitSums& in, float* proj, hipStream_t s) {
+  if (const int rc = check_window(w, "window_select_prep")) return rc;
+  CHATTS_REQUIRE(window_select_can_prep(w, c) && c->conv_w && c->conv_b && c->ring && c->u.f32 && (c->off_x | c->conv_ch | c->u.ld) % 4 == 0 && c->conv_ch >= ((c->inner + 3) & ~3) &&
+                     c->off_x >= 0 && c->off_x + ((c->inner + 3) & ~3) <= c->ld_proj && c->u.ld >= ((c->inner + 3) & ~3) && in.sk >= 1 && in.sk <= kMostSplitSums && in.n == w->ld_proj &&
+                     ((uintptr_t)proj % 16) == 0 && (((uintptr_t)c->conv_w | (uintptr_t)c->conv_b | (uintptr_t)c->ring | (uintptr_t)c->u.f32) % 16) == 0 &&
+                     (((uintptr_t)c->u.hi | (uintptr_t)c->u.lo) % 8) == 0, CHATTS_E_SHAPE, "window_select_prep: %d splits of %d columns for %d", in.sk, in.n, w->ld_proj);
+  if (w->n_rows == 0) return CHATTS_OK;
+  // the columns between what is read here, in order
+  int taken[5][2] = {{w->off_q, w->off_q + w->heads * w->dim}, {w->off_k, w->off_k + w->kv_heads * w->dim}, {w->off_v, w->off_v + w->kv_heads * w->vdim},
+                     {c->off_x, c->off_x + ((c->inner + 3) & ~3)}, {w->ld_proj, w->ld_proj}};
+  for (int i = 1; i < 5; ++i)
+    for (int j = i; j > 0 && taken[j][0] < taken[j - 1][0]; --j) { std::swap(taken[j][0], taken[j - 1][0]); std::swap(taken[j][1], taken[j - 1][1]); }
+  RestCols rest{};
+  for (int i = 0, at = 0; i < 5; ++i) {
+    if (taken[i][0] > at) {
+      rest.from[rest.n] = at;
+      rest.quads[rest.n] = (taken[i][0] - at) / 4;
+      rest.total += rest.quads[rest.n++];
+    }
+    if (taken[i][1] > at) at = taken[i][1];
+  }
+  const int heads = w->heads + 2 * w->kv_heads, widest = w->dim > w->vdim ? w->dim : w->vdim, lph = widest <= 64 ? 16 : (widest <= 128 ? 32 : 64), parts = (heads * lph + 255) / 256;
+  const int conv_parts = (c->inner + 1023) / 1024;
+  const dim3 g(w->n_rows, parts + conv_parts + (rest.total + 255) / 256), b(256);
+#define CHATTS_PREP(L)                                                                                                                              \
+  if (in.sk <= 4) hipLaunchKernelGGL((window_select_prep_kernel<L, 4>), g, b, 0, s, *w, *c, in, rest, proj, parts, conv_parts);                       \
+  else hipLaunchKernelGGL((window_select_prep_kernel<L, kMostSplitSums>), g, b, 0, s, *w, *c, in, rest, proj, parts, conv_parts)
+  if (lph == 16) { CHATTS_PREP(16); }
+  else if (lph == 32) { CHATTS_PREP(32); }
+  else { CHATTS_PREP(64); }
+#undef CHATTS_PREP
+  CHATTS_CHECK_LAUNCH("window_select_prep");
   return CHATTS_OK;
 }
 
