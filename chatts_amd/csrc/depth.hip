@@ -18,6 +18,7 @@ struct DepthChoose {
 // for all rows and made lists of them were three launches: 12.5 us a layer of 32 experts at 16 rows of 2048, now 1.  The router's first K-steps are requested before the row is there.
 template <int NT, int NV, int NR = 0>
 __global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch, int tiled) {
+  kernarg_touch<sizeof(ChattsDepthNormArgs) + sizeof(DepthChoose) + 4>();
   __shared__ float red[NT / 64];
   constexpr int NW = NT / 64, NX = NV * NT * 4;
   __shared__ __attribute__((aligned(16))) uint16_t xh[NR ? NX : 1], xl[NR ? NX : 1];

@@ -14,6 +14,7 @@ __device__ __forceinline__ float silu4(float g) { return g * sigmoid_f(g); }
 // grid (width / four a thread, rows): a thread owns four channels.  S_IN: the projection left up to so many splits, their sums are taken here
 template <int S_IN>
 __global__ __launch_bounds__(256) void gru_decode_kernel(ChattsGruArgs p, SplitSums in) {
+  kernarg_touch<sizeof(ChattsGruArgs) + sizeof(SplitSums)>();
   const int row = blockIdx.y, c = (int)(blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const ChattsRow R = p.rows[row];
   const int w4 = (p.width + 3) & ~3;

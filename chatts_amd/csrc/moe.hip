@@ -283,6 +283,7 @@ __device__ __forceinline__ void moe_relu2_4(const ChattsOperand& o, size_t row, 
 // TILED: weights from the chatts_tile_bf16 copy: a fragment's 64 pieces are 1 KB of consecutive memory
 template <int STEP, bool TILED, int NW, int RF>
 __global__ __launch_bounds__(64 * NW) void moe_stream_kernel(ChattsMoeArgs p, MoeBeside sh, int sh_blocks, int nx) {
+  kernarg_touch<sizeof(ChattsMoeArgs) + sizeof(MoeBeside) + 8>();
   __shared__ f32x4 red[NW][RF][64];
   static_assert(!moe_pairs(STEP) || RF == 2, "a pair of fragments");
   constexpr bool IN = STEP != kDown;

@@ -124,6 +124,7 @@ __device__ __forceinline__ void states_store(float* dst, int l, int n4, const fl
 // grid (channels / (256 / LPC), rows / NR): NR sequences share what a workgroup reads of W_dt
 template <int SPL, int LPC, int NR>
 __global__ __launch_bounds__(256) void select_decode_kernel(ChattsSelectArgs p) {
+  kernarg_touch<sizeof(ChattsSelectArgs)>();
   constexpr int CH = 256 / LPC;
   const int row0 = blockIdx.y * NR, l = threadIdx.x & (LPC - 1), c = blockIdx.x * CH + threadIdx.x / LPC, n4 = (p.state + 3) & ~3;
   const bool live = c < p.inner;

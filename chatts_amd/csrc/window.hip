@@ -220,6 +220,7 @@ __global__ __launch_bounds__(256) void window_prep_quads_kernel(ChattsWindowArgs
 struct RestCols { int n, from[5], quads[5], total; };
 template <int LPH, int S>
 __global__ __launch_bounds__(256) void window_select_prep_kernel(ChattsWindowArgs p, ChattsSelectArgs q, SplitSums in, RestCols rest, float* proj, int parts, int conv_parts) {
+  kernarg_touch<sizeof(ChattsWindowArgs) + sizeof(ChattsSelectArgs) + sizeof(SplitSums) + sizeof(RestCols) + 16>();
   const int row = blockIdx.x;
   int part = blockIdx.y;
   if (part < parts) {
@@ -517,6 +518,7 @@ __global__ __launch_bounds__(256) void window_attend_kernel(ChattsWindowArgs p) 
 // fragment IS the 8 probabilities of the lane (K slot 8 g + j = key 4 g + j, j < 4, or 16 + 4 g + j - 4, on both sides).  The waves' softmaxes meet once.
 template <int NK, int NV, int SCORE>      // dim_p <= 32 NK, vdim_p <= 16 NV
 __global__ __launch_bounds__(256, NV <= 4 ? 4 : (NV <= 8 ? 3 : 1)) void window_decode_kernel(ChattsWindowArgs p) {
+  kernarg_touch<sizeof(ChattsWindowArgs)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int split = blockIdx.x, row = blockIdx.z, tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -667,6 +669,7 @@ __global__ __launch_bounds__(256, NV <= 4 ? 4 : (NV <= 8 ? 3 : 1)) void window_d
 
 // merge of the splits: grid (heads, rows)
 __global__ __launch_bounds__(128) void window_merge_kernel(ChattsWindowArgs p) {
+  kernarg_touch<sizeof(ChattsWindowArgs)>();
   __shared__ float w[64];
   const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, ld = p.vdim_p + 4;
   if (p.rows[row].pos < 0) return;
