@@ -23,6 +23,7 @@ namespace chatts {
 
 }  // namespace chatts
 #include "attn_decode.h"
+#include "gemm_common.h"
 namespace chatts {
 
 // ---------------------------------------------------------------------------------------------------
@@ -31,13 +32,13 @@ namespace chatts {
 // ---------------------------------------------------------------------------------------------------
 // TWO: groups of 7 and 8 heads, whose sums do not fit the registers of two waves per SIMD: two waves a slot, four heads and the rest, next to each other on one XCD (a row of the
 // cache comes from memory once).  One wave per SIMD with all heads was 1.1 .. 1.4 times slower from 12 sequences on, spilling 10 registers 1.1 .. 1.3 times nearly everywhere.
-template <int GMAX, bool EXACT, bool TWO = false>
+template <int GMAX, bool EXACT, bool TWO = false, int SPLITS = 0>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void attn_decode_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) float q_s[GMAX * kHeadDim];
   __shared__ __attribute__((aligned(16))) float knew_s[kHeadDim];
   __shared__ __attribute__((aligned(16))) float vnew_s[kHeadDim];
   const int group = EXACT ? GMAX : p.n_q / p.n_kv, g0 = TWO ? ((int)blockIdx.y & 1) * GMAX : 0;
-  attn_decode_wave<GMAX, EXACT>(p, blockIdx.x, TWO ? blockIdx.y >> 1 : blockIdx.y, blockIdx.z, threadIdx.x, q_s, knew_s, vnew_s, g0, group - g0 < GMAX ? group - g0 : GMAX, p.part_o,
+  attn_decode_wave<GMAX, EXACT, SPLITS>(p, blockIdx.x, TWO ? blockIdx.y >> 1 : blockIdx.y, blockIdx.z, threadIdx.x, q_s, knew_s, vnew_s, g0, group - g0 < GMAX ? group - g0 : GMAX, p.part_o,
                                 p.part_ml, (size_t)blockIdx.z * p.n_q + blockIdx.x * group);
 }
 
@@ -1431,13 +1432,14 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
 }
 
 namespace chatts {
+bool attn_takes_splits(int n_q, int n_kv) { return n_kv > 0 && (n_q == 4 * n_kv || n_q == 5 * n_kv) && opt_get(OPT_ATTN_EXACT, 1) != 0; }
 // chatts_attention_decode_batched with an optional plane output (internal: the decoder's batched step feeds o_proj's
 // weight-streaming kernel directly from the combine)
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w,
                                   const float* k_norm_w, float norm_eps, const float* cos_tab, const float* sin_tab, int pos,
                                   const int32_t* pos_dev, const ChattsKvCache* cache, size_t seq_stride, float* out,
                                   uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes,
-                                  chatts_stream_t stream) {
+                                  chatts_stream_t stream, const SplitSums* in) {
   CHATTS_REQUIRE(batch >= 1 && n_q > 0 && n_kv > 0 && n_splits >= 1 && n_splits <= kMaxSlots, CHATTS_E_BADARG,
                  "attention_decode: bad sizes (batch >= 1, 1 <= n_splits <= %d)", kMaxSlots);
   CHATTS_REQUIRE(qkv_raw && (out || (out_hi && out_lo)) && cos_tab && sin_tab && cache && cache->k && cache->v, CHATTS_E_BADARG,
@@ -1458,11 +1460,25 @@ int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int 
   const int rc = bind_workspace(p, workspace, workspace_bytes);
   if (rc) return rc;
   const dim3 grid(n_kv, n_splits, batch);
+  const dim3 wave(64);
+  if (in) {
+    CHATTS_REQUIRE(attn_takes_splits(n_q, n_kv) && in->sk >= 1 && in->sk <= kMostSplitSums && in->n == (n_q + 2 * n_kv) * kHeadDim, CHATTS_E_SHAPE, "attention_decode: %d splits of %d columns", in->sk, in->n);
+    p.qkv = in->slabs; p.qkv_plane = in->plane; p.qkv_splits = in->sk; p.qkv_scale = in->scale; p.qkv_bias = in->bias;
+#define CHATTS_ATTN_IN(G, S) hipLaunchKernelGGL((attn_decode_kernel<G, true, false, S>), grid, wave, 0, as_stream(stream), p)
+    switch ((n_q / n_kv == 5 ? 8 : 0) + (in->sk <= 4 ? 0 : in->sk - 4 < 2 ? 1 : 2)) {
+      case 0: CHATTS_ATTN_IN(4, 4); break;
+      case 1: CHATTS_ATTN_IN(4, 5); break;
+      case 2: CHATTS_ATTN_IN(4, kMostSplitSums); break;
+      case 8: CHATTS_ATTN_IN(5, 4); break;
+      case 9: CHATTS_ATTN_IN(5, 5); break;
+      default: CHATTS_ATTN_IN(5, kMostSplitSums); break;
+    }
+#undef CHATTS_ATTN_IN
+  }
   // registers sized for the group (every head's arithmetic is the same in all instantiations); the groups of the shipped models
   // (Qwen2.5-14B: 5, Qwen3-8B: 4) get the form with the head count known to the compiler; option ATTN_EXACT=0: the run-time form
   const bool exact = opt_get(OPT_ATTN_EXACT, 1) != 0;
-  const dim3 wave(64);
-  switch (n_q / n_kv) {
+  if (!in) switch (n_q / n_kv) {
     case 4: if (exact) { hipLaunchKernelGGL((attn_decode_kernel<4, true>), grid, wave, 0, as_stream(stream), p); break; }
     case 1: case 2: case 3: hipLaunchKernelGGL((attn_decode_kernel<4, false>), grid, wave, 0, as_stream(stream), p); break;
     case 5: if (exact) hipLaunchKernelGGL((attn_decode_kernel<5, true>), grid, wave, 0, as_stream(stream), p);
@@ -1488,7 +1504,7 @@ extern "C" int chatts_attention_decode_batched(const float* qkv_raw, int batch, 
                                                void* workspace, size_t workspace_bytes, chatts_stream_t stream) {
   return chatts::attention_decode_batched_impl(qkv_raw, batch, n_q, n_kv, q_norm_w, k_norm_w, norm_eps, cos_tab, sin_tab, pos,
                                                pos_dev, cache, seq_stride, out, nullptr, nullptr, n_splits, workspace,
-                                               workspace_bytes, stream);
+                                               workspace_bytes, stream, nullptr);
 }
 
 extern "C" int chatts_attention_decode_fused(const float* qkv_raw, int n_q, int n_kv, const float* q_norm_w,

@@ -45,6 +45,10 @@ struct AttnParams {
   // attn_prefill_planes_kernel's 1-D grid: query tiles per head and, when n_kv divides 8, the number of XCDs that share one kv head
   // (8 / n_kv; 0 = no XCD-aware order) - see the kernel
   int units, xcd_share;
+  // decode: qkv points at the splits that the projection left (SplitSums), qkv_splits of them, floats qkv_plane apart; their sums times qkv_scale plus qkv_bias (either may be NULL)
+  size_t qkv_plane;
+  const float *qkv_scale, *qkv_bias;
+  int qkv_splits;
 };
 
 // rotate one 128-wide head held as (a = x[lane], b = x[lane+64]) by the wave; optional RMSNorm first
@@ -157,7 +161,10 @@ __device__ __forceinline__ bool attn_decode_preload(const AttnParams& p, const i
 // other, so the split does not change a single operation of any head.  The wave with g0 == 0 stores the new K / V row.
 // EXACT: the group IS GMAX heads - `g < gn` is decided by the compiler and the tile body is one straight-line block (the
 // run-time form compiled to ~400 basic blocks, every head's every step behind a scalar branch, no load / FMA interleaving across them).
-template <int GMAX, bool EXACT>
+// SPLITS: up to so many splits of qkv are summed here (splitk_epilogue_v4_kernel's order: the same bits), 0: qkv is whole
+// (a wave reads so many times 3.5 KB instead of 3.5, all of them requested at once, and a launch of 2.5 us that only sums falls away: a step of ChatTS-14B, fp8, 16 sequences at 1204, four
+// splits: 5300 -> 5170 us.)
+template <int GMAX, bool EXACT, int SPLITS>
 __device__ __forceinline__ void attn_decode_finish(const AttnParams& p, const int hk, const int slot, const int seq, const int lane,
                                                    AttnTileRegs& t, float* q_s, float* knew_s, float* vnew_s, const int g0, const int gn_rt,
                                                    float* part_o, float* part_ml, const size_t head_base) {
@@ -167,7 +174,39 @@ __device__ __forceinline__ void attn_decode_finish(const AttnParams& p, const in
   const int ntiles = pos / kDTile + 1, NS = p.n_splits, walk = attn_slots(ntiles, NS);
   const int qkv_n = (p.n_q + 2 * p.n_kv) * kHeadDim;
   const float* qkv = p.qkv + (size_t)seq * qkv_n;
-  auto qkv_at = [&](const int col) __attribute__((always_inline)) -> float { return qkv[col]; };
+  // a head of 128 as (x[lane], x[lane + 64]): what is requested for it, and its values once that is there
+  struct Head { float a[SPLITS ? SPLITS : 1], b[SPLITS ? SPLITS : 1], fa, fb, ba, bb; };
+  auto request = [&](Head& h, const int col) __attribute__((always_inline)) {
+    const float* at = qkv + col + lane;
+    if constexpr (SPLITS == 0) {
+      h.a[0] = at[0];
+      h.b[0] = at[64];
+    } else {
+#pragma unroll
+      for (int i = 0; i < SPLITS; ++i) {
+        const float* split = at + (i < p.qkv_splits ? i : p.qkv_splits - 1) * p.qkv_plane;
+        h.a[i] = split[0];
+        h.b[i] = split[64];
+      }
+      h.fa = h.fb = 1.f;
+      h.ba = h.bb = 0.f;
+      if (p.qkv_scale) { h.fa = p.qkv_scale[col + lane]; h.fb = p.qkv_scale[col + lane + 64]; }
+      if (p.qkv_bias) { h.ba = p.qkv_bias[col + lane]; h.bb = p.qkv_bias[col + lane + 64]; }
+    }
+  };
+  auto value = [&](const Head& h, float& a, float& b) __attribute__((always_inline)) {
+    if constexpr (SPLITS == 0) {
+      a = h.a[0];
+      b = h.b[0];
+    } else {
+      a = b = 0.f;
+#pragma unroll
+      for (int i = 0; i < SPLITS; ++i)
+        if (i < p.qkv_splits) { a += h.a[i]; b += h.b[i]; }
+      a *= h.fa; b *= h.fb;
+      if (p.qkv_bias) { a += h.ba; b += h.bb; }
+    }
+  };
   float* kcache = p.kc + (p.table ? 0 : (size_t)seq * p.seq_stride);
   float* vcache = p.vc + (p.table ? 0 : (size_t)seq * p.seq_stride);
   const KvLayout kvl{p.table ? p.table + (size_t)seq * p.table_stride : nullptr, p.n_kv, p.max_ctx, p.log_block};
@@ -180,19 +219,26 @@ __device__ __forceinline__ void attn_decode_finish(const AttnParams& p, const in
 
   {
     const float c = t.c, s = t.s;
+    Head q[GMAX];
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g)
+      if (g < gn) request(q[g], (hk * G + g0 + g) * kHeadDim);
 #pragma unroll
     for (int g = 0; g < GMAX; ++g) {
       if (g < gn) {
-        const int src = (hk * G + g0 + g) * kHeadDim;
-        float a = qkv_at(src + lane), b = qkv_at(src + lane + 64);
+        float a, b;
+        value(q[g], a, b);
         norm_rope(a, b, p.q_norm_w, p.eps, c, s, lane);
         q_s[g * kHeadDim + lane] = a;
         q_s[g * kHeadDim + lane + 64] = b;
       }
     }
     if (owner) {                                // the new K/V row: to the cache and to LDS
-      const int ks = (p.n_q + hk) * kHeadDim;
-      float a = qkv_at(ks + lane), b = qkv_at(ks + lane + 64);
+      Head kh, vh;
+      request(kh, (p.n_q + hk) * kHeadDim);
+      request(vh, (p.n_q + p.n_kv + hk) * kHeadDim);
+      float a, b;
+      value(kh, a, b);
       norm_rope(a, b, p.k_norm_w, p.eps, c, s, lane);
       a = kv_round_f(a, p.kv_round); b = kv_round_f(b, p.kv_round);
       knew_s[lane] = a;
@@ -200,8 +246,10 @@ __device__ __forceinline__ void attn_decode_finish(const AttnParams& p, const in
       const size_t noff = kv_tile_off(kvl, hk, pos);      // row of the new token
       float* kd = kcache + noff;
       if (g0 == 0) { kd[lane] = a; kd[lane + 64] = b; }
-      const int vs = (p.n_q + p.n_kv + hk) * kHeadDim;
-      const float va = kv_round_f(qkv_at(vs + lane), p.kv_round), vb = kv_round_f(qkv_at(vs + lane + 64), p.kv_round);
+      float va, vb;
+      value(vh, va, vb);
+      va = kv_round_f(va, p.kv_round);
+      vb = kv_round_f(vb, p.kv_round);
       vnew_s[lane] = va;
       vnew_s[lane + 64] = vb;
       float* vd = vcache + noff;
@@ -347,13 +395,13 @@ __device__ __forceinline__ void attn_decode_finish(const AttnParams& p, const in
 
 
 // GMAX >= the heads of this wave: the per-head registers are sized by it
-template <int GMAX, bool EXACT>
+template <int GMAX, bool EXACT, int SPLITS>
 __device__ __forceinline__ void attn_decode_wave(const AttnParams& p, const int hk, const int slot, const int seq, const int lane,
                                                  float* q_s, float* knew_s, float* vnew_s, const int g0, const int gn, float* part_o, float* part_ml,
                                                  const size_t head_base) {
   AttnTileRegs t;
   if (!attn_decode_preload(p, hk, slot, seq, lane, t)) return;
-  attn_decode_finish<GMAX, EXACT>(p, hk, slot, seq, lane, t, q_s, knew_s, vnew_s, g0, gn, part_o, part_ml, head_base);
+  attn_decode_finish<GMAX, EXACT, SPLITS>(p, hk, slot, seq, lane, t, q_s, knew_s, vnew_s, g0, gn, part_o, part_ml, head_base);
 }
 
 // out[h] = sum_s e^{m_s - M} o_s / sum_s e^{m_s - M} l_s over the slots that saw keys (<= CAP of them).

@@ -22,7 +22,8 @@ bool gemm_takes_cols(const ChattsLinearArgs* a);
 int attention_decode_batched_impl(const float* qkv_raw, int batch, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w,
                                   float norm_eps, const float* cos_tab, const float* sin_tab, int pos, const int32_t* pos_dev,
                                   const ChattsKvCache* cache, size_t seq_stride, float* out, uint16_t* out_hi, uint16_t* out_lo,
-                                  int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream);
+                                  int n_splits, void* workspace, size_t workspace_bytes, chatts_stream_t stream, const SplitSums* in);
+bool attn_takes_splits(int n_q, int n_kv);
 int rope_attention_impl(float* qkv, int t, int n_q, int n_kv, const float* q_norm_w, const float* k_norm_w, float norm_eps, const float* cos_tab, const float* sin_tab, int pos0,
                         const int32_t* pos0_dev, const ChattsKvCache* cache, float* out, uint16_t* out_hi, uint16_t* out_lo, int n_splits, void* workspace, size_t workspace_bytes,
                         chatts_stream_t stream, int out_tiled = 0);
@@ -67,7 +68,7 @@ static int64_t embed_offset(const ChattsDecoder* d) { return d->cfg.embed_rows >
 
 static int linear_impl(const ChattsLinearArgs* a, chatts_stream_t stream, const RopeFuse* rope, RopeDone* rope_done, const ChattsNormChain* chain = nullptr, PlaneTiles tiles = {},
                        SplitSums* leave = nullptr);
-extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream) {
+static int linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream, SplitSums* leave) {
   CHATTS_REQUIRE(a && ch, CHATTS_E_BADARG, "linear_chain: null args");
   CHATTS_REQUIRE(!ch->row_ss || (((uintptr_t)ch->row_ss % 16) == 0 && a->a_hi && a->a_lo && a->m >= 2 && a->m <= 16 && a->batch <= 1 && !a->exact_f32 && ch->row_ss_parts >= 1 &&
                                  ch->row_ss_parts <= 256), CHATTS_E_SHAPE,
@@ -81,8 +82,9 @@ extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormCh
   if (ch->post_ss || ch->row_ss)
     for (const chatts_bf16* plane : {a->post_hi, a->post_lo}) meet = meet || in.meets(matrix_range(plane, a->m, a->ld_post, a->n, 2)) || out.meets(matrix_range(plane, a->m, a->ld_post, a->n, 2));
   CHATTS_REQUIRE(!meet, CHATTS_E_SHAPE, "linear_chain: the sums of squares overlap each other, a result or A (M=%d N=%d K=%d)", a->m, a->n, a->k);
-  return linear_impl(a, stream, nullptr, nullptr, ch);
+  return linear_impl(a, stream, nullptr, nullptr, ch, {}, leave);
 }
+extern "C" int chatts_linear_chain(const ChattsLinearArgs* a, const ChattsNormChain* ch, chatts_stream_t stream) { return linear_chain(a, ch, stream, nullptr); }
 extern "C" int chatts_linear_post_ss_parts(const ChattsLinearArgs* a) {
   const bool ok = a && a->w && a->m >= 2 && a->m <= 16 && a->n > 0 && a->n % 16 == 0 && a->k > 0 && a->ldc >= a->n && a->ldw >= a->k && (!a->w8 || a->ldw8 >= a->k) &&
                   a->post_norm_w && ((uintptr_t)a->post_norm_w % 16) == 0 && a->post_hi && a->post_lo && a->ld_post >= a->n && a->ld_post % 4 == 0 &&
@@ -735,13 +737,18 @@ extern "C" int chatts_decoder_layer_part_batched(ChattsDecoder* d, int layer, in
     la.w8 = lw.qkv8; la.w8_scale = lw.qkv8_scale; la.ldw8 = H; la.w8_format = d->cfg.w8_format;
     la.workspace = d->b.workspace; la.workspace_bytes = d->b.workspace_bytes;
     if ((rc = norm_into(d, lw.input_norm, &la, stream, &chain)) != 0) return rc;
-    if ((rc = chatts_linear_chain(&la, &chain, stream)) != 0) return rc;
+    // the attention takes the sums of qkv's splits itself, where its partials find room behind them
+    const size_t in_most = ((size_t)kMostSplitSums * batch * qkv_n * sizeof(float) + 255) & ~(size_t)255;
+    SplitSums in{};
+    const bool takes = attn_takes_splits(c.n_q, c.n_kv) && in_most + chatts_attn_workspace(batch, c.n_q, n_splits) <= d->b.workspace_bytes;
+    if ((rc = linear_chain(&la, &chain, stream, takes ? &in : nullptr)) != 0) return rc;
+    const size_t in_bytes = in.sk ? in_most : 0;
     ChattsKvCache kc = layer_cache(d, layer, 0);
     const bool attn_planes = planes_path(d, batch, c.n_q * kHeadDim, lw.o8 != nullptr);   // the combine writes o_proj's operand format
     if ((rc = attention_decode_batched_impl(d->b.qkv, batch, c.n_q, c.n_kv, lw.q_norm, lw.k_norm, c.rms_eps, d->w.cos_tab, d->w.sin_tab, 0,
                                             pos_dev, &kc, seq_stride(d), d->b.attn, attn_planes ? d->b.planes_hi : nullptr,
-                                            attn_planes ? d->b.planes_lo : nullptr, n_splits, d->b.workspace, d->b.workspace_bytes,
-                                            stream)) != 0) return rc;
+                                            attn_planes ? d->b.planes_lo : nullptr, n_splits, static_cast<char*>(d->b.workspace) + in_bytes, d->b.workspace_bytes - in_bytes,
+                                            stream, in.sk ? &in : nullptr)) != 0) return rc;
     la = ChattsLinearArgs{};
     la.a = d->b.attn; la.w = lw.o; la.w_tiled = lw.o_t; la.m = batch; la.n = H; la.k = c.n_q * kHeadDim;
     la.lda = la.k; la.ldw = la.k; la.ldc = H;

@@ -110,7 +110,7 @@ bool stream_leaves_cus(int m, int n, int k);     // (gemm.hip: 65 .. 128 rows wi
 // takes 1.7 us before it does anything, and the sums' own launch does 0.3 us of work on 16 rows.
 struct SplitSums {
   const float* slabs;
-  const float* bias;
+  const float *scale, *bias;      // per column, or NULL
   size_t plane;         // floats of a split
   int sk, n;
 };
@@ -119,13 +119,15 @@ constexpr int kMostSplitSums = 8;
 template <int S>
 __device__ __forceinline__ f32x4 split_sum4(const SplitSums& p, int row, int col) {
   const float* at = p.slabs + (size_t)row * p.n + col;
-  f32x4 t[S], b = {0.f, 0.f, 0.f, 0.f}, v = b;
+  f32x4 t[S], f, b, v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < S; ++s) t[s] = *reinterpret_cast<const f32x4*>(at + (s < p.sk ? s : p.sk - 1) * p.plane);
+  if (p.scale) f = *reinterpret_cast<const f32x4*>(p.scale + col);
   if (p.bias) b = *reinterpret_cast<const f32x4*>(p.bias + col);
 #pragma unroll
   for (int s = 0; s < S; ++s)
     if (s < p.sk) v += t[s];
+  if (p.scale) v *= f;
   if (p.bias) v += b;
   return v;
 }
