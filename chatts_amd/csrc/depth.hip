@@ -16,9 +16,10 @@ struct DepthChoose {
 // a thread keeps its columns in registers.  NT: threads (more of them for a few rows: then every load of a row is in flight at once)
 // NR > 0 (2 to 16 rows): the same launch multiplies the row by the router, as the planes that it writes, and chooses its experts.  A projection, its split's epilogue and a workgroup that chose
 // for all rows and made lists of them were three launches: 12.5 us a layer of 32 experts at 16 rows of 2048, now 1.  The router's first K-steps are requested before the row is there.
-template <int NT, int NV, int NR = 0>
-__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch, int tiled) {
-  kernarg_touch<sizeof(ChattsDepthNormArgs) + sizeof(DepthChoose) + 4>();
+// S_IN: y is what its projection left, up to so many splits, all requested with the row (16 rows of 2048, eight splits or sixteen: a layer's launch less, 921 -> 911 us a step of eight layers)
+template <int NT, int NV, int NR = 0, int S_IN = 0>
+__global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, DepthChoose ch, int tiled, SplitSums y_in) {
+  kernarg_touch<sizeof(ChattsDepthNormArgs) + sizeof(DepthChoose) + (S_IN ? 8 + sizeof(SplitSums) : 4)>();
   __shared__ float red[NT / 64];
   constexpr int NW = NT / 64, NX = NV * NT * 4;
   __shared__ __attribute__((aligned(16))) uint16_t xh[NR ? NX : 1], xl[NR ? NX : 1];
@@ -45,7 +46,8 @@ __global__ __launch_bounds__(NT) void depth_norm_kernel(ChattsDepthNormArgs p, D
   for (int i = 0; i < NV; ++i) {
     const int c = (i * NT + tid) * 4;
     x[i] = c < p.ldx ? *reinterpret_cast<const f32x4*>(p.x + row * p.ldx + c) : zero;
-    add[i] = p.y && c < p.ldx ? *reinterpret_cast<const f32x4*>(p.y + row * p.ldx + c) : zero;
+    if constexpr (S_IN > 0) add[i] = c < p.ldx ? split_sum4<S_IN>(y_in, (int)row, c) : zero;
+    else add[i] = p.y && c < p.ldx ? *reinterpret_cast<const f32x4*>(p.y + row * p.ldx + c) : zero;
   }
   if (p.ey) {
     for (int j0 = 0; j0 < p.top; j0 += U) {
@@ -218,13 +220,13 @@ int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t
   const DepthChoose none{};
   const dim3 g(a->t);
   hipStream_t s = as_stream(stream);
-  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a, none, tiled);
-  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a, none, tiled);
-  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a, none, tiled);
-  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a, none, tiled);
-  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a, none, tiled);
-  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a, none, tiled);
-  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a, none, tiled);
+  if (a->ldx <= 1024) hipLaunchKernelGGL((depth_norm_kernel<256, 1>), g, dim3(256), 0, s, *a, none, tiled, SplitSums{});
+  else if (a->t <= 64 && a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<1024, 1>), g, dim3(1024), 0, s, *a, none, tiled, SplitSums{});
+  else if (a->t <= 64 && a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<1024, 2>), g, dim3(1024), 0, s, *a, none, tiled, SplitSums{});
+  else if (a->ldx <= 2048) hipLaunchKernelGGL((depth_norm_kernel<256, 2>), g, dim3(256), 0, s, *a, none, tiled, SplitSums{});
+  else if (a->ldx <= 4096) hipLaunchKernelGGL((depth_norm_kernel<256, 4>), g, dim3(256), 0, s, *a, none, tiled, SplitSums{});
+  else if (a->ldx <= 8192) hipLaunchKernelGGL((depth_norm_kernel<256, 8>), g, dim3(256), 0, s, *a, none, tiled, SplitSums{});
+  else hipLaunchKernelGGL((depth_norm_kernel<1024, 4>), g, dim3(1024), 0, s, *a, none, tiled, SplitSums{});
   CHATTS_CHECK_LAUNCH("depth_norm");
   return CHATTS_OK;
 }
@@ -234,13 +236,24 @@ int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t
 static int router_blocks(int outputs) { return outputs <= 32 ? 2 : 4; }
 bool chatts::depth_norm_can_choose(int ldx, int router_rows, int outputs) { return ldx % 64 == 0 && ldx <= 4096 && outputs <= 64 && router_rows >= 16 * router_blocks(outputs); }
 int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream) {
+  return depth_norm_choose_sums(a, moe, router, router_t, router_rows, nullptr, stream);
+}
+int chatts::depth_norm_choose_sums(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
+                                   chatts_stream_t stream) {
   if (const int rc = check_depth_norm(a)) return rc;
   CHATTS_REQUIRE(moe && router && a->w && a->out.hi && a->out.lo && depth_norm_can_choose(a->ldx, router_rows, moe->experts + moe->identity) && moe_takes_choice(moe) &&
                      moe->n_rows == a->t && moe->ids && moe->place && moe->weight && moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);
   if (a->t == 0) return CHATTS_OK;
   const DepthChoose ch{router_t ? router_t : router, router_t ? 16 : 1, *moe};
-  if (router_blocks(moe->experts + moe->identity) == 2) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 2>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
-  else hipLaunchKernelGGL((depth_norm_kernel<1024, 1, 4>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0);
+  CHATTS_REQUIRE(!y || (a->y && y->sk >= 1 && y->sk <= kMostNormSums && y->n == a->ldx), CHATTS_E_SHAPE, "depth_norm: %d splits of %d columns", y->sk, y->n);
+  const SplitSums in = y ? *y : SplitSums{};
+#define CHATTS_CHOOSE(R, S) hipLaunchKernelGGL((depth_norm_kernel<1024, 1, R, S>), dim3(a->t), dim3(1024), 0, as_stream(stream), *a, ch, 0, in)
+  if (router_blocks(moe->experts + moe->identity) == 2) {
+    if (!y) CHATTS_CHOOSE(2, 0); else if (in.sk <= 8) CHATTS_CHOOSE(2, 8); else CHATTS_CHOOSE(2, kMostNormSums);
+  } else {
+    if (!y) CHATTS_CHOOSE(4, 0); else if (in.sk <= 8) CHATTS_CHOOSE(4, 8); else CHATTS_CHOOSE(4, kMostNormSums);
+  }
+#undef CHATTS_CHOOSE
   CHATTS_CHECK_LAUNCH("depth_norm_choose");
   return CHATTS_OK;
 }

@@ -108,13 +108,14 @@ bool planes_tiled_for(int m, int n, int k);      // (gemm.hip: of the A of an m 
 bool stream_leaves_cus(int m, int n, int k);     // (gemm.hip: 65 .. 128 rows with W in tiles are the prefill kernel's)
 // The sums that a projection of few rows left in the workspace, [sk][rows][n], for a reader that adds them up itself (sk == 0: none were left, c is written).  A launch of a captured graph
 // takes 1.7 us before it does anything, and the sums' own launch does 0.3 us of work on 16 rows.
+constexpr int kMostSplitSums = 8, kMostNormSums = 16;      // splits that a reader takes, and those of a norm
 struct SplitSums {
-  const float* slabs;
-  const float *scale, *bias;      // per column, or NULL
-  size_t plane;         // floats of a split
-  int sk, n;
+  const float* slabs = nullptr;
+  const float *scale = nullptr, *bias = nullptr;      // per column, or NULL
+  size_t plane = 0;         // floats of a split
+  int sk = 0, n = 0;
+  int most = kMostSplitSums;      // asked for: splits that may be left
 };
-constexpr int kMostSplitSums = 8;
 // four neighbours, in splitk_epilogue_v4_kernel's order: the same bits
 template <int S>
 __device__ __forceinline__ f32x4 split_sum4(const SplitSums& p, int row, int col) {
@@ -215,6 +216,8 @@ bool moe_takes_choice(const ChattsMoeArgs* a);
 int depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t stream);      // chatts_depth_norm; tiles: the operand's planes as plane_at has them, whole blocks of 16 rows in tiles
 bool depth_norm_can_choose(int ldx, int router_rows, int outputs);
 int depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream);
+int depth_norm_choose_sums(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
+                           chatts_stream_t stream);      // y: a->y as its projection's splits, or NULL
 int moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, bool direct, chatts_stream_t stream);
 
 typedef const __attribute__((address_space(1))) void* gptr_t;

@@ -637,13 +637,13 @@ static int mix_one(const ChattsMixDecoder* d, const ChattsMixLayer& l, int kind,
 // tiles: out's planes in the prefill kernel's blocks
 // choose: the experts for whose router the norm is (depth_norm_choose)
 static int mix_depth_norm(const ChattsMixDecoder* d, int t, const float* y, const ChattsMixLayer* moe, const float* depth, int stream, const float* w, const ChattsOperand& out,
-                          chatts_stream_t s, bool tiles = false, const ChattsMoeArgs* choose = nullptr, const ChattsMixLayer* router = nullptr) {
+                          chatts_stream_t s, bool tiles = false, const ChattsMoeArgs* choose = nullptr, const ChattsMixLayer* router = nullptr, const SplitSums* y_in = nullptr) {
   ChattsDepthNormArgs a{};
   a.x = d->b.x; a.t = t; a.width = d->c.width; a.ldx = d->c.width_p; a.mult = d->c.mult; a.eps = d->c.eps; a.y = y;
   if (moe) { a.ey = d->b.moe_y; a.place = d->b.moe_place; a.weight = d->b.moe_weight; a.top = moe->moe.top; }
   a.depth = depth; a.streams = d->b.streams; a.stream_stride = d->b.stream_stride; a.n_streams = stream + 1; a.keep = depth && stream + 1 < d->c.n_runs;
   a.w = w; a.out = out;
-  return choose ? depth_norm_choose(&a, choose, router->router, router->router_t, router->router_n, s) : depth_norm(&a, tiles, s);
+  return choose ? depth_norm_choose_sums(&a, choose, router->router, router->router_t, router->router_n, y_in, s) : depth_norm(&a, tiles, s);
 }
 
 static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, const ChattsSpan* spans, int n_spans, bool single, chatts_stream_t s) {
@@ -688,18 +688,20 @@ static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, co
     tiles = next && tiles_for(d->layers[d->runs[r + 1].layer]);
     if ((rc = mix_one(d, l, l.kind, run, t, spans, n_spans, single, B, s, left)) != 0) return rc;
     if (l.beside && (rc = mix_one(d, l, l.beside, run, t, spans, n_spans, single, C, s, left)) != 0) return rc;
-    if ((rc = mix_linear(d, B, l.out, l.out_t, t, wp, l.out_k, CHATTS_EPI_NONE, Y, s)) != 0) return rc;
     const bool moe = l.ff_kind == CHATTS_FF_MOE;
+    const ChattsOperand N = second_norm(d, l, t);
+    const ChattsMoeArgs m = moe ? mix_moe_args(d, l, t, N) : ChattsMoeArgs{};
+    const bool choose = moe && moe_takes_choice(&m) && depth_norm_can_choose(wp, l.router_n, m.experts + m.identity) && (uintptr_t)l.router_t % 16 == 0;
+    SplitSums y;      // the norm that chooses takes the sums of the output projection's splits itself
+    y.most = kMostNormSums;
+    if ((rc = mix_linear(d, B, l.out, l.out_t, t, wp, l.out_k, CHATTS_EPI_NONE, Y, s, 0.f, 0.f, nullptr, false, choose ? &y : nullptr)) != 0) return rc;
     if (l.ff_kind == CHATTS_FF_NONE) {
       if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, l.depth, r, next, next ? A : none, s, tiles)) != 0) return rc;
       continue;
     }
-    const ChattsOperand N = second_norm(d, l, t);
     bool beside = false;
     if (moe) {
-      const ChattsMoeArgs m = mix_moe_args(d, l, t, N);
-      const bool choose = moe_takes_choice(&m) && depth_norm_can_choose(wp, l.router_n, m.experts + m.identity) && (uintptr_t)l.router_t % 16 == 0;
-      if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s, false, choose ? &m : nullptr, &l)) != 0) return rc;
+      if ((rc = mix_depth_norm(d, t, d->b.y, nullptr, nullptr, 0, l.norm2, N, s, false, choose ? &m : nullptr, &l, y.sk ? &y : nullptr)) != 0) return rc;
       StageRange stage("chatts.mix.experts");
       if (!choose) {
         if ((rc = mix_linear(d, linear_form(N), l.router, l.router_t, t, l.router_n, wp, CHATTS_EPI_NONE, f32_out(d->b.moe_logits, l.router_n), s)) != 0) return rc;

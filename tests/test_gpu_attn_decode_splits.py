@@ -9,6 +9,13 @@ from tests.test_gpu_batched_step_rows import model_of, step
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def own_random_numbers():
+    """the tests behind these draw what they would draw without them"""
+    with torch.random.fork_rng():
+        yield
+
+
 @pytest.mark.parametrize("name,form", [("chatts-8b", "bf16"), ("chatts-14b", "bf16"), ("chatts-14b", "fp8"), ("chatts-8b", "int8")])
 def test_splits_left_to_the_attention(name, form):
     m, positions, tokens = model_of(name, form)

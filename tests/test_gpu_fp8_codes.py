@@ -10,6 +10,13 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+@pytest.fixture(autouse=True)
+def own_random_numbers():
+    """the tests behind these draw what they would draw without them"""
+    with torch.random.fork_rng():
+        yield
+
+
 @pytest.mark.parametrize("m", [2, 16])
 @pytest.mark.parametrize("n,k", [(256, 256), (5120, 5120), (24576, 4096)])
 def test_every_code(n, k, m):

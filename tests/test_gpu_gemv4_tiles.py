@@ -10,6 +10,14 @@ from chatts_amd import _lib
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
+
+@pytest.fixture(autouse=True)
+def own_random_numbers():
+    """the tests behind these draw what they would draw without them"""
+    with torch.random.fork_rng():
+        yield
+
+
 # one unit a row that K does not fill; fewer quads than CUs and the largest K; K that ends inside a unit; groups of more than a part; ChatTS shapes
 SHAPES = [(65568, 128, 128), (544, 16384, 128), (2080, 4224, 128), (6176, 2048, 1024), (3296, 2560, 256), (7168, 5120, 128), (5120, 13824, 128), (27648, 5120, 128)]
 

@@ -1,5 +1,6 @@
-"""Muvetar's steps of few rows where the input projection leaves its splits to the layer's own launches (csrc/gru.hip, csrc/window.hip): heads of 48 to 200 channels, one to five taps, sizes
-that no quad fits (those keep the launches of their own), up to eight splits, a place that is not taken - against the plain reference, and against a projection without splits."""
+"""Muvetar's steps of few rows where the input projection leaves its splits to the layer's own launches (csrc/gru.hip, csrc/window.hip) and the output projection to the norm that chooses
+experts (csrc/depth.hip): heads of 48 to 200 channels, one to five taps, sizes that no quad fits (those keep the launches of their own), up to eight splits and sixteen, a place that is not
+taken - against the plain reference, and against projections without splits."""
 import pytest
 import torch
 
@@ -10,6 +11,13 @@ from tests.muvetar_models import CONFIGS, model
 from tests.test_gpu_muvetar import TOL, tokens, worst
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def own_random_numbers():
+    """the tests behind these draw what they would draw without them"""
+    with torch.random.fork_rng():
+        yield
 
 
 def steps(name, n=5):
@@ -33,7 +41,7 @@ def steps(name, n=5):
     return toks, {s: torch.stack(v) for s, v in out.items()}
 
 
-@pytest.mark.parametrize("splits", [2, 3, 5, 8])
+@pytest.mark.parametrize("splits", [2, 3, 5, 8, 12])
 @pytest.mark.parametrize("name", sorted(CONFIGS))
 def test_sums_left_to_the_layer(name, splits):
     cfg, _, sd = model(name, all_experts=True)
