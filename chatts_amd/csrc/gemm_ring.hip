@@ -306,54 +306,57 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
 
     auto k_loop = [&](auto fml_c) {
       constexpr int FML = decltype(fml_c)::value;
-      bf16x8_t wf[2][NF], alo[FML], ahi[FML];
+      bf16x8_t wf[NF], alo[FML], ahi[FML];
       const int a_off = rowblk * 1024 + lane_off, w_off = kRingWOff + wn * NF * 1024 + lane_off;
       auto slot = [&](int h) { return smem + ((gh + h) & (kRingSlots - 1)) * kRingHalf; };
-      auto read_w = [&](const char* base, bf16x8_t (&dst)[NF]) {
-#pragma unroll
-        for (int j = 0; j < NF; ++j) dst[j] = *reinterpret_cast<const bf16x8_t*>(base + w_off + j * 1024);
-      };
-      auto read_a = [&](const char* base, int plane, bf16x8_t (&dst)[FML]) {
+      auto read_a = [&](const char* base, int plane, bf16x8_t (&dst)[FML]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < FML; ++i) dst[i] = *reinterpret_cast<const bf16x8_t*>(base + plane * kRingAPlane + a_off + i * 1024);
       };
-      auto sweep = [&](const bf16x8_t (&af)[FML], const bf16x8_t (&wfr)[NF]) {      // D = W . A^T: operands swapped
+      auto column = [&](int j, const bf16x8_t (&af)[FML]) __attribute__((always_inline)) {      // D = W . A^T: operands swapped
 #pragma unroll
-        for (int i = 0; i < FML; ++i)
-#pragma unroll
-          for (int j = 0; j < NF; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wfr[j], af[i], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < FML; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
       };
-      // half-step h (operands in registers) with the fragments of h + 1 requested behind the barrier
-      auto half = [&](int h, const bf16x8_t (&wcur)[NF], bf16x8_t (&wnxt)[NF], bool more) {
+      // Half-step h (operands in registers).  Behind the barrier the fragments of h + 1 are asked for: lo, then a column of W behind its last product and into its registers, hi behind the
+      // last column.  (Both sweeps row by row, W in two sets and all of it asked for at once with lo: 224 rows 4096 x 4096 26.7 / 26.0 us, 4096 x 12288 53.5 / 52.5, 800 rows
+      // 27648 x 5120 gated 334.6 / 333.5, 2048 rows the same.)
+      auto half = [&](int h, auto more_c) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_c)::value;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!SINGLE) sweep(alo, wcur);
+        if constexpr (!SINGLE) {
+#pragma unroll
+          for (int j = 0; j < NF; ++j) column(j, alo);
+        }
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // every fragment read of half-stage h has returned
         __builtin_amdgcn_s_barrier();                          // h + 1 is published; the loaders refill the slot of h
-        if (more) {
-          const char* nb = slot(h + 1);
-          read_w(nb, wnxt);
-          if constexpr (!SINGLE) read_a(nb, 1, alo);
+        const char* nb = slot(h + 1);
+        if constexpr (MORE && !SINGLE) read_a(nb, 1, alo);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NF; ++j) {
+          column(j, ahi);
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (MORE) wf[j] = *reinterpret_cast<const bf16x8_t*>(nb + w_off + j * 1024);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        sweep(ahi, wcur);
-        __builtin_amdgcn_sched_barrier(0);
-        if (more) read_a(slot(h + 1), 0, ahi);
+        if constexpr (MORE) read_a(nb, 0, ahi);
       };
       {
         const char* b0 = slot(0);
-        read_w(b0, wf[0]);
         if constexpr (!SINGLE) read_a(b0, 1, alo);
+#pragma unroll
+        for (int j = 0; j < NF; ++j) wf[j] = *reinterpret_cast<const bf16x8_t*>(b0 + w_off + j * 1024);
         read_a(b0, 0, ahi);
       }
-      // (nh is even: K splits are multiples of 64; the last pair is peeled so that the loop body has no `more` test)
+      // (nh is even: K splits are multiples of 64; the last pair is peeled so that the loop body has no test)
       int h = 0;
       for (; h + 2 < r.nh; h += 2) {
-        half(h, wf[0], wf[1], true);
-        half(h + 1, wf[1], wf[0], true);
+        half(h, std::true_type{});
+        half(h + 1, std::true_type{});
       }
-      half(h, wf[0], wf[1], true);
-      half(h + 1, wf[1], wf[0], false);
+      half(h, std::true_type{});
+      half(h + 1, std::false_type{});
     };
     switch (fml) {
       case 1: k_loop(std::integral_constant<int, 1>{}); break;
