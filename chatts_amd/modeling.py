@@ -343,25 +343,25 @@ class ChatTSForCausalLM(SlotModel):
         """4-bit codes once more in the order the matrix pipe takes them in (chatts_tile_w4), for the projections of one row; those of a shape or with scales that have no such form, and
         those there is no memory for, keep the row-major codes."""
         lib, names = self.lib, ("qkv", "o", "gate_up", "down")
-        self._int4_tiles = {}
-        bad = torch.zeros(4 * len(self.layers), dtype=torch.int32, device=self.device)
+        self._int4_tiles, total, places = None, 0, {}
+        room = torch.cuda.mem_get_info(self.device)[0] - (8 << 30)
         for i, lw in enumerate(self.layers):
             for j, name in enumerate(names):
-                if name + "4" not in lw:
-                    continue
-                rows, k = lw[name].shape
-                need = int(lib.chatts_tile_w4_bytes(rows, k, self.int4_group))
-                if need == 0 or torch.cuda.mem_get_info(self.device)[0] < need + (8 << 30):
-                    continue
-                out = torch.empty(need, dtype=torch.uint8, device=self.device)
-                _lib.check(lib.chatts_tile_w4(lw[name + "4"].data_ptr(), lw[name + "4_sz"].data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", out.data_ptr(),
-                                              bad[4 * i + j:].data_ptr(), _lib.stream_ptr()))
-                self._int4_tiles[4 * i + j] = out
-        if self._int4_tiles:
-            for n in bad.nonzero().flatten().tolist():
-                del self._int4_tiles[n]
-            ptrs = (C.c_void_p * len(bad))(*[_lib.ptr(self._int4_tiles.get(n)) for n in range(len(bad))])
-            _lib.check(lib.chatts_decoder_set_w4_tiles(self._decoder, ptrs, len(bad)))
+                need = -(-int(lib.chatts_tile_w4_bytes(*lw[name].shape, self.int4_group)) // 256) * 256 if name + "4" in lw else 0
+                if 0 < need <= room - total:
+                    places[4 * i + j] = (lw, name, total)
+                    total += need
+        if not places:
+            return
+        bad = torch.zeros(4 * len(self.layers), dtype=torch.int32, device=self.device)
+        self._int4_tiles = torch.empty(total, dtype=torch.uint8, device=self.device)      # (one allocation: 192 of them took as long as the rest of a model's preparation)
+        base = self._int4_tiles.data_ptr()
+        for n, (lw, name, at) in places.items():
+            rows, k = lw[name].shape
+            _lib.check(lib.chatts_tile_w4(lw[name + "4"].data_ptr(), lw[name + "4_sz"].data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", base + at, bad[n:].data_ptr(), _lib.stream_ptr()))
+        bad = bad.tolist()
+        ptrs = (C.c_void_p * len(bad))(*[base + places[n][2] if n in places and not bad[n] else None for n in range(len(bad))])
+        _lib.check(lib.chatts_decoder_set_w4_tiles(self._decoder, ptrs, len(bad)))
 
     def _finalize(self):
         """Allocate activations / KV cache and create the C-side decoder handle (borrowing all pointers)."""
