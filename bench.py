@@ -159,7 +159,10 @@ def roofline_gate_up(model, reps=2, m=1):
 
     def sweep():
         for lw in model.layers:
-            _lib.check(lib.chatts_linear(args(lw), stream.cuda_stream))
+            if m == 1 and "gate_up4_tiles" in lw:
+                _lib.check(lib.chatts_linear_w4_tiles(args(lw), lw["gate_up4_tiles"].data_ptr(), stream.cuda_stream))
+            else:
+                _lib.check(lib.chatts_linear(args(lw), stream.cuda_stream))
 
     sweep()
     torch.cuda.synchronize()
@@ -173,17 +176,18 @@ def roofline_gate_up(model, reps=2, m=1):
     avg_s = e0.elapsed_time(e1) * 1e-3 / launches
     # algorithmic bytes per launch: bf16 weights + f32 x in + norm weights + f32 out (SURVEY.md 8d per-unit figure)
     fp8 = "gate_up8" in model.layers[0]
-    int4 = m == 1 and "gate_up4" in model.layers[0]
+    int4_tiles = m == 1 and "gate_up4_tiles" in model.layers[0]
+    int4 = int4_tiles or (m == 1 and "gate_up4" in model.layers[0])
     bytes_per_launch = n * H * (1 if fp8 else 2) + (n * 4 if fp8 else 0) + m * (H * 4 + H * 4 + plan.inter * 4)
     if int4:
-        bytes_per_launch = n * H // 2 + n * (H // model.int4_group) * 8 + H * 4 + H * 4 + plan.inter * 4
+        bytes_per_launch = (model.layers[0]["gate_up4_tiles"].numel() if int4_tiles else n * H // 2 + n * (H // model.int4_group) * 8) + H * 4 + H * 4 + plan.inter * 4
     first = args(model.layers[0])
     weights = "int8" if fp8 and fmt == _lib.W8_INT8 else "fp8" if fp8 else "bf16"
     if m > 1:
         name = "gemm_cols_kernel" if lib.chatts_linear_cols(first) else "gemm_rows_kernel" if lib.chatts_linear_few_rows(ctypes.byref(first), None) else "gemm_stream_kernel"
         what = f"gate_up_proj + SwiGLU, {weights}, M = {m} sequences, bf16 planes in/out"
     else:
-        name = "gemv4_kernel" if int4 else "gemv_ring_kernel" if lib.chatts_gemv_ring(first) else "gemv8_ldsx_kernel" if fp8 else "gemv_ldsx_kernel"
+        name = "gemv4_tiles_kernel" if int4_tiles else "gemv4_kernel" if int4 else "gemv_ring_kernel" if lib.chatts_gemv_ring(first) else "gemv8_ldsx_kernel" if fp8 else "gemv_ldsx_kernel"
         what = f"gate_up_proj + fused RMSNorm + SwiGLU, {'int4' if int4 else weights}"
     return dict(kernel=f"{name} ({what})", launches=launches, avg_us=avg_s * 1e6, bytes_per_launch=bytes_per_launch, gbs=bytes_per_launch / avg_s / 1e9)
 

@@ -59,7 +59,7 @@ struct ChattsDecoder {
   bool prefill_fp8 = false; // SPEED MODE (chatts_decoder_set_prefill_fp8): prefill chunks of >= 16 rows multiply fp8 x fp8 (gemm_fp8.hip)
   bool fuse_tp = false;     // set by chatts_decoder_decode_step: the M == 1 o_proj / down_proj GEMVs carry the exchange in their own launch
   bool tp_fused = false;    // ... and whether the last layer part's projection did (otherwise the caller launches chatts_allreduce)
-  std::vector<const void*> w4_tiles;      // [n_layers][qkv, o, gate_up, down]: 4-bit codes in chatts_tile_w4's order (chatts_decoder_set_w4_tiles); empty or null: the layer's row-major codes
+  std::vector<const void*> w4_tiles;      // [n_layers][qkv, o, gate_up, down]: 4-bit codes in chatts_tile_w4's order (chatts_decoder_set_w4_tiles); empty or null: row-major codes or other weights
 };
 enum { kProjQkv, kProjO, kProjGateUp, kProjDown };
 
@@ -249,11 +249,11 @@ static size_t seq_stride(const ChattsDecoder* d) {      // floats between the ca
 extern "C" int chatts_decoder_set_w4_tiles(ChattsDecoder* d, const void* const* tiles, int n) {
   CHATTS_REQUIRE(d && (tiles || n == 0), CHATTS_E_BADARG, "decoder_set_w4_tiles: null argument");
   CHATTS_REQUIRE(n == 0 || n == 4 * d->cfg.n_layers, CHATTS_E_SHAPE, "decoder_set_w4_tiles: %d pointers for %d layers", n, d->cfg.n_layers);
-  for (int i = 0; i < n; ++i) {
-    const ChattsLayerWeights& lw = d->layers[i / 4];
-    const uint8_t* const w4[4] = {lw.qkv4, lw.o4, lw.gate_up4, lw.down4};
-    CHATTS_REQUIRE(!tiles[i] || (w4[i % 4] && ((uintptr_t)tiles[i] % 16) == 0), CHATTS_E_BADARG, "decoder_set_w4_tiles: layer %d, projection %d has no 4-bit codes", i / 4, i % 4);
-  }
+  const ChattsDecoderConfig& c = d->cfg;
+  const int shape[4][2] = {{(c.n_q + 2 * c.n_kv) * kHeadDim, c.hidden}, {c.hidden, c.n_q * kHeadDim}, {2 * c.inter, c.hidden}, {c.hidden, c.inter}};      // (in kProj*'s order)
+  for (int i = 0; i < n; ++i)
+    CHATTS_REQUIRE(!tiles[i] || (((uintptr_t)tiles[i] % 16) == 0 && chatts_tile_w4_bytes(shape[i % 4][0], shape[i % 4][1], 128) != 0), CHATTS_E_BADARG,
+                   "decoder_set_w4_tiles: layer %d, projection %d has no tiled form, or its copy is not 16-byte aligned", i / 4, i % 4);
   try {
     d->w4_tiles.assign(tiles, tiles + n);
   } catch (const std::bad_alloc&) {
@@ -262,8 +262,9 @@ extern "C" int chatts_decoder_set_w4_tiles(ChattsDecoder* d, const void* const* 
   return CHATTS_OK;
 }
 // a projection of one row: on the tiled 4-bit codes where there are some
+static const void* w4_tiles_of(const ChattsDecoder* d, int layer, int proj) { return d->w4_tiles.empty() ? nullptr : d->w4_tiles[4 * layer + proj]; }
 static int linear_one_row(const ChattsDecoder* d, int layer, int proj, const ChattsLinearArgs* la, chatts_stream_t stream) {
-  const void* t = la->w4 && !d->w4_tiles.empty() ? d->w4_tiles[4 * layer + proj] : nullptr;
+  const void* t = w4_tiles_of(d, layer, proj);
   return t ? chatts_linear_w4_tiles(la, t, stream) : chatts_linear(la, stream);
 }
 
@@ -658,7 +659,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
       la.a_hi = d->b.planes_hi; la.a_lo = d->b.planes_lo; la.ld_planes = la.k;
     }
     d->tp_fused = false;
-    if (tp && t == 1 && d->fuse_tp && d->tp && !la.w4) {      // x += sum over the ranks, inside the GEMV launch (ChattsLinearArgs.tp_reduce)
+    if (tp && t == 1 && d->fuse_tp && d->tp && !la.w4 && !w4_tiles_of(d, layer, kProjO)) {      // x += sum over the ranks, inside the GEMV launch (ChattsLinearArgs.tp_reduce)
       la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; la.tp_reduce = d->tp;
       d->tp_fused = true;
     } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
@@ -691,7 +692,7 @@ extern "C" int chatts_decoder_layer_part(ChattsDecoder* d, int layer, int part, 
   }
   if (act_planes) { la.a = nullptr; la.a_hi = d->b.planes2_hi; la.a_lo = d->b.planes2_lo; la.ld_planes = c.inter; }
   d->tp_fused = false;
-  if (tp && t == 1 && d->fuse_tp && d->tp && !la.w4) {
+  if (tp && t == 1 && d->fuse_tp && d->tp && !la.w4 && !w4_tiles_of(d, layer, kProjDown)) {
     la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID; la.tp_reduce = d->tp;
     d->tp_fused = true;
   } else if (tp) { la.c = d->b.delta; la.epilogue = CHATTS_EPI_NONE; }
@@ -928,7 +929,8 @@ static int layer_last_row(ChattsDecoder* d, int layer, int t, int pos0, chatts_s
   la.w4 = lw.o4; la.w4_sz = lw.o4_sz; la.ldw4 = la.k / 2; la.w4_group = lw.w4_group;
   la.c = d->b.x; la.resid = d->b.x; la.epilogue = CHATTS_EPI_RESID;
   const bool tp = c.tp_world > 1;
-  if (tp && !la.w4) la.tp_reduce = d->tp;                  // row 0 of x += the sum over the ranks, inside the GEMV launch
+  const bool w4 = la.w4 || w4_tiles_of(d, layer, kProjO);
+  if (tp && !w4) la.tp_reduce = d->tp;                  // row 0 of x += the sum over the ranks, inside the GEMV launch
   else if (tp) { la.c = d->b.delta; la.resid = nullptr; la.epilogue = CHATTS_EPI_NONE; }
   if ((rc = linear_one_row(d, layer, kProjO, &la, stream)) != 0) return rc;
   if (tp && !la.tp_reduce && (rc = chatts_allreduce(d->tp, d->b.delta, d->b.x, d->b.x, H, stream)) != 0) return rc;

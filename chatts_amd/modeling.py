@@ -337,31 +337,21 @@ class ChatTSForCausalLM(SlotModel):
                  "gate_up": tuple(interleave_gate_up(c[names[4]][i], c[names[5]][i]) for i in range(3))}
         for k, (q, sc, z) in fused.items():
             self.int4_group = q.shape[1] // sc.shape[1]
-            L[k + "4"], L[k + "4_sz"] = pack_int4(q, sc, z)
+            self._keep_int4(L, k, q, sc, z)
 
-    def _tile_int4(self):
-        """4-bit codes once more in the order the matrix pipe takes them in (chatts_tile_w4), for the projections of one row; those of a shape or with scales that have no such form, and
-        those there is no memory for, keep the row-major codes."""
-        lib, names = self.lib, ("qkv", "o", "gate_up", "down")
-        self._int4_tiles, total, places = None, 0, {}
-        room = torch.cuda.mem_get_info(self.device)[0] - (8 << 30)
-        for i, lw in enumerate(self.layers):
-            for j, name in enumerate(names):
-                need = -(-int(lib.chatts_tile_w4_bytes(*lw[name].shape, self.int4_group)) // 256) * 256 if name + "4" in lw else 0
-                if 0 < need <= room - total:
-                    places[4 * i + j] = (lw, name, total)
-                    total += need
-        if not places:
-            return
-        bad = torch.zeros(4 * len(self.layers), dtype=torch.int32, device=self.device)
-        self._int4_tiles = torch.empty(total, dtype=torch.uint8, device=self.device)      # (one allocation: 192 of them took as long as the rest of a model's preparation)
-        base = self._int4_tiles.data_ptr()
-        for n, (lw, name, at) in places.items():
-            rows, k = lw[name].shape
-            _lib.check(lib.chatts_tile_w4(lw[name + "4"].data_ptr(), lw[name + "4_sz"].data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", base + at, bad[n:].data_ptr(), _lib.stream_ptr()))
-        bad = bad.tolist()
-        ptrs = (C.c_void_p * len(bad))(*[base + places[n][2] if n in places and not bad[n] else None for n in range(len(bad))])
-        _lib.check(lib.chatts_decoder_set_w4_tiles(self._decoder, ptrs, len(bad)))
+    def _keep_int4(self, lw, name, codes, scale, zero):
+        """4-bit codes of a projection, for one row (more rows take the bf16 weights): in the order the matrix pipe takes them in (chatts_tile_w4), or row-major where the shape or a scale
+        has no such form.  Never both, and free memory has no say: the two sum in different orders."""
+        lib, (rows, k) = self.lib, codes.shape
+        w4, sz = pack_int4(codes, scale, zero)
+        need = int(lib.chatts_tile_w4_bytes(rows, k, self.int4_group))
+        if need and (name != "gate_up" or rows % 32 == 0):
+            tiles, bad = torch.empty(need, dtype=torch.uint8, device=self.device), torch.zeros(1, dtype=torch.int32, device=self.device)
+            _lib.check(lib.chatts_tile_w4(w4.data_ptr(), sz.data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", tiles.data_ptr(), bad.data_ptr(), _lib.stream_ptr()))
+            if not int(bad):
+                lw[name + "4_tiles"] = tiles
+                return
+        lw[name + "4"], lw[name + "4_sz"] = w4, sz
 
     def _finalize(self):
         """Allocate activations / KV cache and create the C-side decoder handle (borrowing all pointers)."""
@@ -382,12 +372,12 @@ class ChatTSForCausalLM(SlotModel):
             T["lm_head"] = deq
             if tied:
                 T["embed"] = deq
-        if self.weight_format == "int4" and self.layers and "qkv4" not in self.layers[0]:
+        if self.weight_format == "int4" and self.layers and not {"qkv4", "qkv4_tiles"} & self.layers[0].keys():
             # round-to-nearest 4-bit codes of every decoder projection; the bf16 tensors are REPLACED by the dequantised values
             for lw in self.layers:
                 for name in ("qkv", "o", "gate_up", "down"):
                     q, sc, z, lw[name] = quantize_int4_rows(lw[name], self.int4_group)
-                    lw[name + "4"], lw[name + "4_sz"] = pack_int4(q, sc, z)
+                    self._keep_int4(lw, name, q, sc, z)
         # decode attention: one wave per 16-key tile; slots beyond the live context exit immediately
         self.n_splits = max(1, min(64, (self.max_ctx + 15) // 16))
         dc = _lib.DecoderConfig(hidden=H, n_layers=cfg.num_hidden_layers, n_q=plan.nq, n_kv=plan.nkv, head_dim=d,
@@ -531,7 +521,9 @@ class ChatTSForCausalLM(SlotModel):
         if not h:
             raise _lib.ChattsError(-1, lib.chatts_last_error().decode())
         self._decoder = C.c_void_p(h)
-        self._tile_int4()
+        tiles = [_lib.ptr(lw.get(name + "4_tiles")) for lw in self.layers for name in ("qkv", "o", "gate_up", "down")]
+        if any(tiles):
+            _lib.check(lib.chatts_decoder_set_w4_tiles(self._decoder, (C.c_void_p * len(tiles))(*tiles), len(tiles)))
         self._graph = None
         self._graph_batched = None
         if self.precision == "fp8":              # speed mode: prefill chunks and the TS encoder on the fp8 matrix pipe
@@ -591,7 +583,7 @@ class ChatTSForCausalLM(SlotModel):
         n = 0
         for lw in self.layers:
             for k, t in lw.items():
-                if k + "8" in lw or k + "4" in lw:
+                if any(k + form in lw for form in ("8", "4", "4_tiles")):
                     continue                       # the fp8 / 4-bit copy is the one the decode GEMV reads
                 n += t.numel() * t.element_size()
         T = self._tensors

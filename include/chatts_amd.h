@@ -727,8 +727,8 @@ typedef struct ChattsDecoder ChattsDecoder;  /* opaque; host memory only */
 ChattsDecoder* chatts_decoder_create(const ChattsDecoderConfig*, const ChattsDecoderWeights*,
                                      const ChattsDecoderBuffers*);
 void chatts_decoder_destroy(ChattsDecoder*);
-/* Copies of the layers' 4-bit codes in chatts_tile_w4's order (gate_up: gated), borrowed like the weights: host array [n_layers][qkv, o, gate_up, down], n = 4 * n_layers (0: none).
- * Projections of one row stream them instead of qkv4 / o4 / gate_up4 / down4, which stay for the entries that are NULL. */
+/* The layers' 4-bit codes in chatts_tile_w4's order (gate_up: gated), borrowed like the weights: host array [n_layers][qkv, o, gate_up, down], n = 4 * n_layers (0: none).
+ * Projections of one row stream them; entries that are NULL stream qkv4 / o4 / gate_up4 / down4, which a projection with an entry need not have. */
 int chatts_decoder_set_w4_tiles(ChattsDecoder*, const void* const* tiles, int n);
 size_t chatts_decoder_workspace(const ChattsDecoderConfig*, int t_max, int n_splits_max);
 
