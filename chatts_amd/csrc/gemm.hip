@@ -1201,7 +1201,7 @@ int launch_gemm(const ChattsLinearArgs* a_in, hipStream_t s, const RopeFuse* rop
     }
   }
   CHATTS_CHECK_LAUNCH("gemm_bf16x2");
-  if (leave && stream && sk > 1 && sk <= leave->most && a->m <= 16 && batch == 1 && a->epilogue == CHATTS_EPI_NONE && !a->post_norm_w && !ch.post_ss && !a->c_hi &&
+  if (leave && opt_get(OPT_SPLIT_SUMS, 1) != 0 && stream && sk > 1 && sk <= leave->most && a->m <= 16 && batch == 1 && a->epilogue == CHATTS_EPI_NONE && !a->post_norm_w && !ch.post_ss && !a->c_hi &&
       (((uintptr_t)a->workspace | (uintptr_t)a->bias | (uintptr_t)(a->w8 ? a->w8_scale : nullptr)) % 16) == 0) {
     leave->slabs = reinterpret_cast<const float*>(a->workspace); leave->plane = (size_t)a->m * a->n; leave->sk = sk; leave->n = a->n;
     leave->scale = a->w8 ? a->w8_scale : nullptr; leave->bias = a->bias;

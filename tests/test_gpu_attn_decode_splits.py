@@ -21,8 +21,10 @@ def test_splits_left_to_the_attention(name, form):
     m, positions, tokens = model_of(name, form)
     for splits in (2, 4, 5, 6, 8):
         got = []
-        for exact in (1, 0):      # (0: heads counted at run time, which reads whole rows)
-            with _lib.options(GEMM_SK=splits, ATTN_EXACT=exact):
+        for exact, left in ((1, 1), (1, 0), (0, 1)):      # (heads counted at run time read whole rows)
+            with _lib.options(GEMM_SK=splits, ATTN_EXACT=exact, SPLIT_SUMS=left):
+                m.buf["qkv"].fill_(float("nan"))
                 first = step(m, positions, tokens, 16)
+                assert bool(torch.isnan(m.buf["qkv"][:16]).all()) == bool(exact and left), splits      # (the sums were left, or not)
                 got.append((first, step(m, positions + 1, tokens.flip(0), 16)))
-        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), splits
+        assert all(torch.equal(a, b) for other in got[1:] for a, b in zip(got[0], other)), splits

@@ -1,13 +1,13 @@
 """Muvetar's steps of few rows where the input projection leaves its splits to the layer's own launches (csrc/gru.hip, csrc/window.hip) and the output projection to the norm that chooses
 experts (csrc/depth.hip): heads of 48 to 200 channels, one to five taps, sizes that no quad fits (those keep the launches of their own), up to eight splits and sixteen, a place that is not
-taken - against the plain reference, and against projections without splits."""
+taken - against the plain reference, against projections without splits, and bit for bit against sums in launches of their own; that the sums are left at all."""
 import pytest
 import torch
 
 from chatts_amd import _lib
 from chatts_amd.muvetar import MuvetarConfig, MuvetarForCausalLM
 from oracle import muvetar as F
-from tests.muvetar_models import CONFIGS, model
+from tests.muvetar_models import CONFIGS, _gru, _moe, _par, model
 from tests.test_gpu_muvetar import TOL, tokens, worst
 
 pytestmark = pytest.mark.gpu
@@ -47,8 +47,39 @@ def test_sums_left_to_the_layer(name, splits):
     cfg, _, sd = model(name, all_experts=True)
     with _lib.options(GEMM_SK=splits):      # (the workspace is sized for them, too)
         toks, got = steps(name)
+    with _lib.options(GEMM_SK=splits, SPLIT_SUMS=0):
+        _, apart = steps(name)
     with _lib.options(GEMM_SK=1):
         _, whole = steps(name)
     for s, t in toks.items():
         assert worst(got[s], F.forward(cfg, sd, t)[-len(got[s]):]) < TOL[name, "bfloat16"]
         assert worst(got[s], whole[s].cpu()) < TOL[name, "bfloat16"]
+        assert torch.equal(got[s], apart[s])
+
+
+# one layer of each kind whose sums are left, nothing behind it that writes what its projections would have written; K of 1024 for both
+ALONE = {"recurrence": _moe(_gru(1024), 64, 7.0, 4, 4, 1.0), "attention beside a scan": _moe(_par(8, 2, 64, 64, 0.2, 512, 16, 16, 4, (0.9, 0.5)), 64, 7.0, 4, 4, 1.0)}
+
+
+@pytest.mark.parametrize("splits", [2, 8, 16])
+@pytest.mark.parametrize("kind", sorted(ALONE))
+def test_the_sums_are_left(kind, splits):
+    public = {"vocab": 96, "width": 1024, "norm": {"eps": 1e-5}, "residual_mult": 0.5, "logit_softcap": 30.0, "layers": [ALONE[kind]], "architecture": "Muvetar"}
+    sd = F.random_model({k: v for k, v in public.items() if k != "architecture"}, 1)
+    got = {}
+    for on in (1, 0):
+        with _lib.options(GEMM_SK=splits, SPLIT_SUMS=on):
+            m = MuvetarForCausalLM(MuvetarConfig.from_dict(public), dtype="bfloat16", max_ctx=128, max_batch=4)
+            m.load_weights(sd.items())
+            for s in range(4):
+                m.step_tokens([(s, tokens("plain", 5 + s, s), [])])
+                m.reserve_kv(s, 100)
+            m.buf["pos_all"].copy_(torch.arange(5, 9, dtype=torch.int32))
+            m.buf["token_all"].copy_(torch.tensor([3, 50, 7, 90]))
+            m.buf["proj"].fill_(5.0)
+            m.buf["y"].fill_(5.0)
+            m.batched_step()
+            got[on] = [m.buf[n].clone() for n in ("logits_all", "proj", "y")]
+    assert torch.equal(got[1][0], got[0][0])
+    written = {on: [int((t != 5.0).sum()) for t in got[on][1:]] for on in got}
+    assert (written[1][0] < written[0][0]) == (splits <= 8) and written[1][1] == 0 < written[0][1]      # (the mixers take eight splits, the norm sixteen)
