@@ -60,6 +60,81 @@ __device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const R
   return r;
 }
 
+// Loader wave L over lists of rows: how many pieces a tile has is only known on the device, so a piece is a branch and a wait a choice at run time.  Planes row-major, four column fragments.
+constexpr int kGroupNF = 4;
+__device__ __forceinline__ void ring_group_load(const GemmParams& p, const RingGroup& gr, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, int T, int P, int u0, int uend, int ustep, int L,
+                                                int lane, char* smem) {
+  const int prow = lane >> 2, gchunk = (lane & 3) ^ ((lane >> 5) << 1);
+  const bool wtiled = p.wt != nullptr;
+  const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64;
+  const char* src[kGroupNF + 5];
+  int dst[kGroupNF + 5];
+  int np = 0, hh = 0, ucur = u0;
+  auto setup = [&](int u) {
+    int matrix = 0, places = 0;
+    const RingUnit r = ring_group_unit(p, gr, T, P, u, matrix, places);
+    const int n0 = r.panel * kRingBN;
+    const size_t skip = (size_t)matrix * gr.w_stride;
+#pragma unroll
+    for (int h = 0; h < kGroupNF; ++h) {
+      int wr = n0 + (L + 4 * h) * 16 + prow;
+      if (wr > p.n - 1) wr = p.n - 1;
+      if (wtiled) {
+        const int rr = wr & 15;
+        src[h] = reinterpret_cast<const char*>(p.wt + skip + (size_t)(wr >> 4) * nkt * 512) + (rr * 4 + (gchunk ^ ((rr >> 3) << 1))) * 16;
+      } else {
+        src[h] = reinterpret_cast<const char*>(p.w + skip + (size_t)wr * p.ldw + gchunk * 8);
+      }
+      dst[h] = kRingWOff + (L + 4 * h) * 1024;
+    }
+    np = kGroupNF;
+#pragma unroll
+    for (int h = 0; h < 5; ++h) {
+      const int q = L + 4 * h;
+      if (q < 2 * r.f) {
+        const int plane = q >= r.f, frag = plane ? q - r.f : q;
+        int am = r.m0 + frag * 16 + prow;
+        if (am > r.m0 + places - 1) am = r.m0 + places - 1;
+        if (gr.order) am = gr.order[am] / gr.top;
+        src[kGroupNF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + (size_t)am * ldp + gchunk * 8);
+        dst[kGroupNF + h] = plane * kRingAPlane + frag * 1024;
+        np = kGroupNF + 1 + h;
+      }
+    }
+  };
+  int gi = 0;                                                // global index of the next half-stage to request
+  auto issue = [&]() -> int {                                // request the next half-stage (if any); -> its piece count
+    if (ucur >= uend) return 0;
+    char* base = smem + (gi & (kRingSlots - 1)) * kRingHalf;
+    const size_t koffw = (size_t)hh * wstep, koffa = (size_t)hh * 64;
+#pragma unroll
+    for (int h = 0; h < kGroupNF + 5; ++h)
+      if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < kGroupNF ? koffw : koffa)), (lptr_t)(base + dst[h]), 16, 0, 0);
+    const int n = np;
+    ++gi;
+    if (++hh == nkt) {
+      ucur += ustep;
+      hh = 0;
+      if (ucur < uend) setup(ucur);
+    }
+    return n;
+  };
+  const int G = (uend - u0 + ustep - 1) / ustep * nkt;       // half-steps of this workgroup = barriers after the first
+  setup(u0);
+  issue();
+  int q1 = issue(), q2 = issue();
+  ring_wait_vmcnt(q1 + q2);                                  // half-stage 0 landed
+  __builtin_amdgcn_s_barrier();                              // ... published
+  int q3 = issue();                                          // (slot 3 has never been read)
+  for (int gh = 0; gh < G; ++gh) {
+    ring_wait_vmcnt(q2 + q3);                                // half-stage gh + 1 landed; gh + 2, gh + 3 stay in flight
+    __builtin_amdgcn_s_barrier();                            // publishes it; every read of half-stage gh has returned
+    const int q4 = issue();                                  // gh + 4 -> the slot of gh
+    q1 = q2; q2 = q3; q3 = q4;
+  }
+  (void)q1;
+}
+
 // SINGLE: the "bf16" speed mode - the lo plane is neither staged nor multiplied (activations rounded to bf16: NOT parity grade)
 // NF: column fragments of a compute wave - a panel is 64 NF rows of W
 // TILES: planes of A or of the result whose whole blocks lie in tiles and whose last rows do not (a_tiled, c_tiled).  An instance of its own: the choice a piece cost row-major planes up
@@ -68,6 +143,7 @@ __device__ __forceinline__ RingUnit ring_group_unit(const GemmParams& p, const R
 template <bool SINGLE, bool GROUPED = false, int NF = 4, bool TILES = false>
 __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, const uint16_t* __restrict__ a_hi,
                                                                  const uint16_t* __restrict__ a_lo, int ldp, RingGeom g, RingGroup gr) {
+  static_assert(!GROUPED || (!SINGLE && NF == 4 && !TILES), "what the loader of lists knows");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int BN = 64 * NF;
   kernarg_touch<sizeof(GemmParams) + 2 * sizeof(void*) + 8 + sizeof(RingGeom) + (GROUPED ? sizeof(RingGroup) : 0)>();
@@ -89,20 +165,21 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
   const int ubeg = xcd * share + (xcd < rem ? xcd : rem), ucnt = share + (xcd < rem);
   if (local >= ucnt) return;                                   // padding workgroup (fewer units than workgroups): uniform exit
   const int uend = ubeg + ucnt, u0 = ubeg + local, ustep = g.wpx;
-  const int G = GROUPED ? (uend - u0 + ustep - 1) / ustep * (p.k >> 5) : 0;      // half-steps of this workgroup = barriers after the first
 
   if (wave >= kRingCompute) {
     // ---- loader wave L: pieces of 16 rows x 64 bytes (1 KB per wave instruction).  W pieces {L, L + 4, L + 8, L + 12}; of the unit's
     // A pieces q = 0 .. 2 f - 1 (q < f: hi plane fragment q, else lo plane fragment q - f) those with q % 4 == L.
     const int L = wave - kRingCompute;
-    const int prow = lane >> 2, gchunk = (lane & 3) ^ ((lane >> 5) << 1);
-    // tiled operands (chatts_tile_bf16): piece (16-row block b, half-stage t) is the 1 KB at ((b * K / 32) + t) * 1 KB, already in LDS
-    // order - whole cache lines per request instead of 16 half lines (profiles/r6_feed_probe.txt)
-    const bool wtiled = p.wt != nullptr, alltiled = p.planes_tiled != 0;
-    const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64, astep = alltiled ? 1024 : 64;
-    // three fragments do not hold whole (gate, up) pairs of 16 columns: there a gated product's W block is 8 gates and their 8 up rows
-    const bool mixed = NF == 3 && p.direct && epi_is_glu(p.epilogue);
-    if constexpr (!GROUPED) {
+    if constexpr (GROUPED) {
+      ring_group_load(p, gr, a_hi, a_lo, ldp, g.T, g.P, u0, uend, ustep, L, lane, smem);
+    } else {
+      const int prow = lane >> 2, gchunk = (lane & 3) ^ ((lane >> 5) << 1);
+      // tiled operands (chatts_tile_bf16): piece (16-row block b, half-stage t) is the 1 KB at ((b * K / 32) + t) * 1 KB, already in LDS
+      // order - whole cache lines per request instead of 16 half lines (profiles/r6_feed_probe.txt)
+      const bool wtiled = p.wt != nullptr, alltiled = p.planes_tiled != 0;
+      const int nkt = p.k >> 5, wstep = wtiled ? 1024 : 64, astep = alltiled ? 1024 : 64;
+      // three fragments do not hold whole (gate, up) pairs of 16 columns: there a gated product's W block is 8 gates and their 8 up rows
+      const bool mixed = NF == 3 && p.direct && epi_is_glu(p.epilogue);
       // A launch's first bytes wait for what stands here: places by multiplication, bases in scalar registers, one offset a lane (as divisions and 64-bit addresses a lane they took 1.4 to
       // 2.0 us of a launch).  As many pieces a half-stage for the whole launch (a shorter tile asks for one of its pieces twice): one loop, straight down, whose waits are constants (a branch
       // a piece and the choice of the wait at run time: 1 us).
@@ -195,90 +272,7 @@ __global__ __launch_bounds__(kRingThreads) void gemm_ring_kernel(GemmParams p, c
         case 4: run(std::integral_constant<int, NF + 4>{}); break;
         default: run(std::integral_constant<int, NF + 5>{}); break;
       }
-      return;
     }
-    const char* src[NF + 5];
-    int dst[NF + 5], ashift[TILES ? 5 : 1];
-    int np = 0, nh_cur = 0, hh = 0, ucur = u0;
-    auto setup = [&](int u) {
-      int matrix = 0, places = 0;
-      const RingUnit r = unit(u, matrix, places);
-      nh_cur = r.nh;
-      np = 0;
-      const int n0 = r.panel * BN;
-      const size_t skip = GROUPED ? (size_t)matrix * gr.w_stride : 0;
-#pragma unroll
-      for (int h = 0; h < NF; ++h) {
-        int wr = n0 + (L + 4 * h) * 16 + prow;
-        if (mixed) {
-          const int u = (n0 >> 1) + (L + 4 * h) * 8;
-          wr = (u >> 4) * 32 + (u & 15) + (prow & 7) + (prow >> 3) * 16;
-        }
-        if (wr > p.n - 1) wr = p.n - 1;
-        if (wtiled) {
-          const int rr = wr & 15;
-          src[h] = reinterpret_cast<const char*>(p.wt + skip + ((size_t)(wr >> 4) * nkt + (r.kbeg >> 5)) * 512) + (rr * 4 + (gchunk ^ ((rr >> 3) << 1))) * 16;
-        } else {
-          src[h] = reinterpret_cast<const char*>(p.w + skip + (size_t)wr * p.ldw + r.kbeg + gchunk * 8);
-        }
-        dst[h] = kRingWOff + (L + 4 * h) * 1024;
-      }
-      np = NF;
-      const int na = SINGLE ? r.f : 2 * r.f;
-#pragma unroll
-      for (int h = 0; h < 5; ++h) {
-        const int q = L + 4 * h;
-        if (q < na) {
-          const int plane = q >= r.f, frag = plane ? q - r.f : q;
-          const bool atiled = TILES ? alltiled || r.m0 + frag * 16 < p.a_tiled : alltiled;
-          if constexpr (TILES) ashift[h] = atiled ? 10 : 6;
-          if (atiled) {
-            src[NF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + ((size_t)((r.m0 >> 4) + frag) * nkt + (r.kbeg >> 5)) * 512) + lane * 16;
-          } else {
-            int am = r.m0 + frag * 16 + prow;
-            if constexpr (GROUPED) {
-              if (am > r.m0 + places - 1) am = r.m0 + places - 1;
-              if (gr.order) am = gr.order[am] / gr.top;
-            } else if (am > p.m - 1) {
-              am = p.m - 1;
-            }
-            src[NF + h] = reinterpret_cast<const char*>((plane ? a_lo : a_hi) + (size_t)am * ldp + r.kbeg + gchunk * 8);
-          }
-          dst[NF + h] = plane * kRingAPlane + frag * 1024;
-          np = NF + 1 + h;
-        }
-      }
-    };
-    int gi = 0;                                                // global index of the next half-stage to request
-    auto issue = [&]() -> int {                                // request the next half-stage (if any); -> its piece count
-      if (ucur >= uend) return 0;
-      char* base = smem + (gi & (kRingSlots - 1)) * kRingHalf;
-      const size_t koffw = (size_t)hh * wstep, koffa = (size_t)hh * astep;
-#pragma unroll
-      for (int h = 0; h < NF + 5; ++h)
-        if (h < np) __builtin_amdgcn_global_load_lds((gptr_t)(src[h] + (h < NF ? koffw : (TILES ? (size_t)((unsigned)hh << ashift[h < NF ? 0 : h - NF]) : koffa))), (lptr_t)(base + dst[h]), 16, 0, 0);
-      const int n = np;
-      ++gi;
-      if (++hh == nh_cur) {
-        ucur += ustep;
-        hh = 0;
-        if (ucur < uend) setup(ucur);
-      }
-      return n;
-    };
-    setup(u0);
-    issue();
-    int q1 = issue(), q2 = issue();
-    ring_wait_vmcnt(q1 + q2);                                  // half-stage 0 landed
-    __builtin_amdgcn_s_barrier();                              // ... published
-    int q3 = issue();                                          // (slot 3 has never been read)
-    for (int gh = 0; gh < G; ++gh) {
-      ring_wait_vmcnt(q2 + q3);                                // half-stage gh + 1 landed; gh + 2, gh + 3 stay in flight
-      __builtin_amdgcn_s_barrier();                            // publishes it; every read of half-stage gh has returned
-      const int q4 = issue();                                  // gh + 4 -> the slot of gh
-      q1 = q2; q2 = q3; q3 = q4;
-    }
-    (void)q1;
     return;
   }
 
@@ -467,6 +461,7 @@ static int launch_ring_t(const GemmParams& p, const uint16_t* a_hi, const uint16
 }
 int launch_ring_group(const GemmParams& p, const uint16_t* a_hi, const uint16_t* a_lo, int ldp, const RingGroup& gr, int most_tiles, hipStream_t s) {
   static_assert(kRingTile == kRingMaxF * 16, "a tile's places");
+  CHATTS_REQUIRE(!p.planes_tiled && !p.a_tiled && !p.c_tiled && p.direct && p.k % 64 == 0, CHATTS_E_SHAPE, "gemm_ring_group: row-major planes, K in one piece of whole steps (K=%d)", p.k);
   static bool configured = false;
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<false, true>), hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);
