@@ -1,5 +1,5 @@
-"""Build a VARIANT of libchatts_amd.so next to the shipped one: same sources, extra -D flags (A/B arms), or a source swapped for a
-diagnostic twin (--replace gemm_ring.hip=tools/probes/gemm_ring_probe.hip: the prefill kernel with its timeline probe and ablations).
+"""Build a VARIANT of libchatts_amd.so next to the shipped one: same sources, extra -D flags (A/B arms), or a source swapped for
+another (--replace x.hip=path).
     python tools/build_variant.py NAME [-DFOO=1 ...] [--only a.hip,b.hip] [--replace x.hip=path]   ->  chatts_amd/lib/variants/libchatts_amd_NAME.so
 Point the Python side at it with CHATTS_AMD_LIB=<that path>.  Variant libraries are git-ignored like the shipped build and travel
 with the gpurun snapshot."""
