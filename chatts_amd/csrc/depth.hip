@@ -235,8 +235,11 @@ int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t
 // (a router of router_rows x ldx, outputs of them in use: the kernel reads 32 rows or 64)
 static int router_blocks(int outputs) { return outputs <= 32 ? 2 : 4; }
 bool chatts::depth_norm_can_choose(int ldx, int router_rows, int outputs) { return ldx % 64 == 0 && ldx <= 4096 && outputs <= 64 && router_rows >= 16 * router_blocks(outputs); }
-int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
-                              chatts_stream_t stream) {
+int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream) {
+  return depth_norm_choose_sums(a, moe, router, router_t, router_rows, nullptr, stream);
+}
+int chatts::depth_norm_choose_sums(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
+                                   chatts_stream_t stream) {
   if (const int rc = check_depth_norm(a)) return rc;
   CHATTS_REQUIRE(moe && router && a->w && a->out.hi && a->out.lo && depth_norm_can_choose(a->ldx, router_rows, moe->experts + moe->identity) && moe_takes_choice(moe) &&
                      moe->n_rows == a->t && moe->ids && moe->place && moe->weight && moe->kept && moe->rows && ((uintptr_t)router % 16) == 0 && ((uintptr_t)router_t % 16) == 0, CHATTS_E_BADARG, "depth_norm: a choice behind %d rows of %d", a->t, a->ldx);

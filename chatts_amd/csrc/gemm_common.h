@@ -215,8 +215,9 @@ bool moe_takes_beside(const ChattsMoeArgs* a, const MoeBeside& sh);
 bool moe_takes_choice(const ChattsMoeArgs* a);
 int depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t stream);      // chatts_depth_norm; tiles: the operand's planes as plane_at has them, whole blocks of 16 rows in tiles
 bool depth_norm_can_choose(int ldx, int router_rows, int outputs);
-int depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
-                      chatts_stream_t stream);      // y: a->y as its projection's splits, or NULL
+int depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream);
+int depth_norm_choose_sums(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, const SplitSums* y,
+                           chatts_stream_t stream);      // y: a->y as its projection's splits, or NULL
 int moe_experts(const ChattsMoeArgs* a, const MoeBeside& sh, bool direct, chatts_stream_t stream);
 
 typedef const __attribute__((address_space(1))) void* gptr_t;

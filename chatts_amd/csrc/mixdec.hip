@@ -643,7 +643,7 @@ static int mix_depth_norm(const ChattsMixDecoder* d, int t, const float* y, cons
   if (moe) { a.ey = d->b.moe_y; a.place = d->b.moe_place; a.weight = d->b.moe_weight; a.top = moe->moe.top; }
   a.depth = depth; a.streams = d->b.streams; a.stream_stride = d->b.stream_stride; a.n_streams = stream + 1; a.keep = depth && stream + 1 < d->c.n_runs;
   a.w = w; a.out = out;
-  return choose ? depth_norm_choose(&a, choose, router->router, router->router_t, router->router_n, y_in, s) : depth_norm(&a, tiles, s);
+  return choose ? depth_norm_choose_sums(&a, choose, router->router, router->router_t, router->router_n, y_in, s) : depth_norm(&a, tiles, s);
 }
 
 static int mix_pre_forward(ChattsMixDecoder* d, const int64_t* tokens, int t, const ChattsSpan* spans, int n_spans, bool single, chatts_stream_t s) {
