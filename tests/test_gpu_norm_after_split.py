@@ -23,10 +23,11 @@ def test_norm_after_a_split(lib, form, m, h, k, n2):
     x, w1, _, resid, q1, s1 = problem(m, h, k, form, h)
     _, w2, _, _, q2, s2 = problem(m, n2, h, form, n2)
     resid *= 10.0 ** torch.linspace(-3, 3, m, device=DEV)[:, None]
-    nw = 1 + 0.1 * torch.randn(h, device=DEV)
+    nw = 1 + 0.1 * torch.randn(h, generator=torch.Generator(device=DEV).manual_seed(m + h), device=DEV)
     hi, lo = planes(lib, x)
     new = resid.double() + x.double() @ w1.double().T
-    want = (new * torch.rsqrt((new * new).mean(1, keepdim=True) + 1e-6) * nw.double()) @ w2.double().T
+    normed = new * torch.rsqrt((new * new).mean(1, keepdim=True) + 1e-6) * nw.double()
+    want = normed @ w2.double().T
     plain = torch.empty_like(resid)
     run(lib, args(m, h, k, hi, lo, w1, q1, s1, form, plain, resid=resid.data_ptr(), ldc=h, epilogue=_lib.EPI_RESID), m, h, k)
     ph, pl = (torch.empty((m, h), dtype=torch.bfloat16, device=DEV) for _ in range(2))
@@ -43,15 +44,17 @@ def test_norm_after_a_split(lib, form, m, h, k, n2):
     assert bool(((ss[:m, :parts].double().sum(1) / (c.double() ** 2).sum(1) - 1).abs() < (6 + h / 16 / parts + 1) * 2.0 ** -24).all())
     out = torch.full((m, n2), float("nan"), device=DEV)
     run(lib, args(m, n2, h, ph, pl, w2, q2, s2, form, out, ldc=n2, epilogue=_lib.EPI_NONE), m, n2, h, _lib.NormChain(row_ss=ss.data_ptr(), row_ss_parts=parts, row_eps=1e-6))
-    for i in range(m):
-        assert rel(out[i], want[i]) < 2e-5                # (x to 2^-17, sums in 32 bits)
+    # Two splits into two parts, each to 2^-18 of a value, the first halfway hidden behind resid; sums in 32 bits.  They are measured against the size that the terms' squares give, not that of the
+    # result: 8-bit weights have one column of forty times the others' size, and where its terms happen to cancel, the result is small and the errors are not.
+    size = (normed ** 2 @ (w2.double() ** 2).T).sum(1).sqrt()
+    assert bool(((out.double() - want).norm(dim=1) < 2e-5 * size).all())
 
 
 @pytest.mark.parametrize("form,few", [("bf16", 8), ("bf16", 3), ("fp8", 4), ("int8", 2)])
 @pytest.mark.parametrize("h,k", [(5120, 5120), (4096, 4096), (1152, 2048)])
 def test_a_row_does_not_depend_on_the_number_of_rows(lib, form, few, h, k):
     x, w, _, resid, q, s = problem(16, h, k, form, h)
-    nw = 1 + 0.1 * torch.randn(h, device=DEV)
+    nw = 1 + 0.1 * torch.randn(h, generator=torch.Generator(device=DEV).manual_seed(h), device=DEV)
     got = []
     for m in (16, few):
         hi, lo = planes(lib, x[:m].contiguous())
