@@ -135,6 +135,7 @@ __device__ __forceinline__ f32x4 split_sum4(const SplitSums& p, int row, int col
 int linear_tiled(const ChattsLinearArgs* a, chatts_stream_t stream, PlaneTiles tiles, SplitSums* leave = nullptr);      // chatts_linear on such planes (decoder.hip)
 int gru_decode(const ChattsGruArgs* a, const SplitSums& in, hipStream_t s);      // chatts_gru_decode on what a projection left (gru.hip)
 // what attention and a selective scan that read one projection do before their own launches, one token per row, and the rest of its sums into proj (window.hip)
+int check_select_conv(const ChattsSelectArgs* a, const char* who);      // what chatts_select_conv takes (select.hip)
 bool window_select_can_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c);
 int window_select_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c, const SplitSums& in, float* proj, hipStream_t s);
 

@@ -574,10 +574,14 @@ static void launch_select_conv(const ChattsSelectArgs* a, hipStream_t s) {
 
 using namespace chatts;
 
-extern "C" int chatts_select_conv(const ChattsSelectArgs* a, chatts_stream_t stream) {
-  if (const int rc = check_select(a, "select_conv")) return rc;
+int chatts::check_select_conv(const ChattsSelectArgs* a, const char* who) {
+  if (const int rc = check_select(a, who)) return rc;
   CHATTS_REQUIRE(a->conv_w && a->conv_b && a->ring && (a->n_spans == 0 || a->spans) && (((uintptr_t)a->conv_w | (uintptr_t)a->conv_b | (uintptr_t)a->ring) % 16) == 0 &&
-                     (((uintptr_t)a->u.hi | (uintptr_t)a->u.lo) % 8) == 0, CHATTS_E_BADARG, "select_conv: bad arguments");
+                     (((uintptr_t)a->u.hi | (uintptr_t)a->u.lo) % 8) == 0, CHATTS_E_BADARG, "%s: bad arguments", who);
+  return CHATTS_OK;
+}
+extern "C" int chatts_select_conv(const ChattsSelectArgs* a, chatts_stream_t stream) {
+  if (const int rc = check_select_conv(a, "select_conv")) return rc;
   if (a->n_rows == 0) return CHATTS_OK;
   hipStream_t s = as_stream(stream);
   switch (a->taps) {

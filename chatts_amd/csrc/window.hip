@@ -1058,11 +1058,11 @@ bool chatts::window_select_can_prep(const ChattsWindowArgs* w, const ChattsSelec
          ((uintptr_t)w->q_norm | (uintptr_t)w->k_norm) % 16 == 0 && w->ld_proj == c->ld_proj && w->n_rows == c->n_rows;
 }
 int chatts::window_select_prep(const ChattsWindowArgs* w, const ChattsSelectArgs* c, const SplitSums& in, float* proj, hipStream_t s) {
-  if (const int rc = check_window(w, "window_select_prep")) return rc;
-  CHATTS_REQUIRE(window_select_can_prep(w, c) && c->conv_w && c->conv_b && c->ring && c->u.f32 && (c->off_x | c->conv_ch | c->u.ld) % 4 == 0 && c->conv_ch >= ((c->inner + 3) & ~3) &&
-                     c->off_x >= 0 && c->off_x + ((c->inner + 3) & ~3) <= c->ld_proj && c->u.ld >= ((c->inner + 3) & ~3) && in.sk >= 1 && in.sk <= kMostSplitSums && in.n == w->ld_proj &&
-                     ((uintptr_t)proj % 16) == 0 && (((uintptr_t)c->conv_w | (uintptr_t)c->conv_b | (uintptr_t)c->ring | (uintptr_t)c->u.f32) % 16) == 0 &&
-                     (((uintptr_t)c->u.hi | (uintptr_t)c->u.lo) % 8) == 0, CHATTS_E_SHAPE, "window_select_prep: %d splits of %d columns for %d", in.sk, in.n, w->ld_proj);
+  // what the launches of their own refuse is refused here, before anything is launched
+  if (const int rc = check_window(w, "window_prep")) return rc;
+  if (const int rc = check_select_conv(c, "select_conv")) return rc;
+  CHATTS_REQUIRE(window_select_can_prep(w, c) && in.sk >= 1 && in.sk <= kMostSplitSums && in.n == w->ld_proj && ((uintptr_t)proj % 16) == 0, CHATTS_E_SHAPE,
+                 "window_select_prep: %d splits of %d columns for %d", in.sk, in.n, w->ld_proj);
   if (w->n_rows == 0) return CHATTS_OK;
   // the columns between what is read here, in order
   int taken[5][2] = {{w->off_q, w->off_q + w->heads * w->dim}, {w->off_k, w->off_k + w->kv_heads * w->dim}, {w->off_v, w->off_v + w->kv_heads * w->vdim},
