@@ -1,4 +1,5 @@
-"""Few rows on fp8 weights: every finite code arrives as the number it stands for, bit for bit, in each kernel that widens them (csrc/gemm_rows.hip, gemm_cols.hip, gemm.hip)."""
+"""Few rows on fp8 weights: every finite code arrives as the number it stands for, bit for bit, and both codes of no number as none, in each kernel that widens them (csrc/gemm_rows.hip,
+gemm_cols.hip, gemm.hip)."""
 import ctypes as C
 
 import pytest
@@ -22,7 +23,8 @@ def own_random_numbers():
 def test_every_code(n, k, m):
     lib = _lib.load()
     codes = ((torch.arange(n, device=DEV)[:, None] * 3 + torch.arange(k, device=DEV)[None]) % 256).to(torch.uint8)
-    codes[(codes & 0x7f) == 0x7f] = 0                              # (NaN)
+    codes[(codes & 0x7f) == 0x7f] = 0                              # (no number)
+    codes[5, 3], codes[n - 1, k - 1] = 0x7f, 0xff
     scale = 2.0 ** (torch.arange(n, device=DEV) % 7 - 3).float()
     w = codes.view(torch.float8_e4m3fn).float() * scale[:, None]
     deq = w.bfloat16()
@@ -36,4 +38,8 @@ def test_every_code(n, k, m):
                         w8_scale=scale.data_ptr(), ldw8=k, a_hi=hi.data_ptr(), a_lo=lo.data_ptr(), ld_planes=k)
     _lib.check(lib.chatts_linear(C.byref(a), _lib.stream_ptr()))
     torch.cuda.synchronize()
-    assert torch.equal(out, w[:, at].T.contiguous())
+    rows = [5, n - 1]                                              # (nothing times no number is none, too)
+    assert bool(torch.isnan(out[:, rows]).all())
+    finite = torch.ones(n, dtype=torch.bool, device=DEV)
+    finite[rows] = False
+    assert torch.equal(out[:, finite], w[:, at].T[:, finite])
