@@ -1432,6 +1432,12 @@ int chatts::attention_impl(const float* qkv, int t, int n_q, int n_kv, int pos0,
 }
 
 namespace chatts {
+// Which qkv projections of 2 .. 16 rows leave their splits to the attention: those of two to eight, for groups of four and five heads.  Every wave of every slot reads them, and still no
+// measured cell lost: us a layer that the launch of their own cost more, contexts 100 / 400 / 1200 / 2000 / 4000, 16 rows, all slots taken:
+//   the projection's own number of splits: ChatTS-14B bf16 2.2 / 1.9 / 1.2 / 1.5 / 1.4, fp8 2.5 / 2.5 / 2.0 / 2.5 / 2.6;   ChatTS-8B bf16 2.4 / 1.9 / 1.4 / 1.6 / 1.7, int8 2.1 / 1.8 / 1.3 / 1.7 / 1.5
+//   ChatTS-14B bf16, two 2.2 / 1.8 / 2.0 / 2.3 / 2.5, five 2.2 / 1.7 / 1.2 / 1.5 / 1.2, eight 2.1 / 1.2 / 0.8 / 1.0 / 1.0;   ChatTS-8B int8, six 2.1 / 1.0 / 0.6 / 0.8 / 0.9, eight 2.6 / 1.2 / 0.7 / 0.9 / 0.9
+// 5 and 8 (8-bit weights), 9 and 12 rows 0.8 to 2.4; half of ChatTS-14B's heads in fp8, 9 and 16 rows 1.1 to 1.5 (the other shards of two, four and eight ranks leave none).
+// Other groups keep it, too: the forms whose heads are counted at run time read a head behind a branch, so a head's splits would be a round trip each.  Instances for them are not measured.
 bool attn_takes_splits(int n_q, int n_kv) { return n_kv > 0 && (n_q == 4 * n_kv || n_q == 5 * n_kv) && opt_get(OPT_ATTN_EXACT, 1) != 0; }
 // chatts_attention_decode_batched with an optional plane output (internal: the decoder's batched step feeds o_proj's
 // weight-streaming kernel directly from the combine)

@@ -235,6 +235,7 @@ int chatts::depth_norm(const ChattsDepthNormArgs* a, bool tiles, chatts_stream_t
 // (a router of router_rows x ldx, outputs of them in use: the kernel reads 32 rows or 64)
 static int router_blocks(int outputs) { return outputs <= 32 ? 2 : 4; }
 bool chatts::depth_norm_can_choose(int ldx, int router_rows, int outputs) { return ldx % 64 == 0 && ldx <= 4096 && outputs <= 64 && router_rows >= 16 * router_blocks(outputs); }
+// (rows that are there already; the tests call it)
 int chatts::depth_norm_choose(const ChattsDepthNormArgs* a, const ChattsMoeArgs* moe, const chatts_bf16* router, const chatts_bf16* router_t, int router_rows, chatts_stream_t stream) {
   return depth_norm_choose_sums(a, moe, router, router_t, router_rows, nullptr, stream);
 }

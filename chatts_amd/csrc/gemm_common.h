@@ -108,6 +108,10 @@ bool planes_tiled_for(int m, int n, int k);      // (gemm.hip: of the A of an m 
 bool stream_leaves_cus(int m, int n, int k);     // (gemm.hip: 65 .. 128 rows with W in tiles are the prefill kernel's)
 // The sums that a projection of few rows left in the workspace, [sk][rows][n], for a reader that adds them up itself (sk == 0: none were left, c is written).  A launch of a captured graph
 // takes 1.7 us before it does anything, and the sums' own launch does 0.3 us of work on 16 rows.
+// Where the line lies: splits are left wherever a reader takes them, as no measured cell lost.  Attention: see attn_takes_splits.  Mixed layers, steps of eight layers with the same tokens on
+// every route, us with all sums in launches of their own / those of the mixers left / those of the norm, too: width 2048, 9, 10, 12, 16 rows 810 / 788 / 772, 829 / 804 / 789, 858 / 831 / 816,
+// 893 / 868 / 854 (runs of one route differ by 1 to 4); width 4096, 9 to 16 rows 0 to 6 us for the mixers and 3 to 24 for the norm (of 1900 to 2190; runs differ by 5 to 20); 8 rows and
+// fewer take kernels without splits.  More than eight (mixers, attention) or sixteen (norm) splits keep their launch: a reader asks for all of them at once, in registers.
 constexpr int kMostSplitSums = 8, kMostNormSums = 16;      // splits that a reader takes, and those of a norm
 struct SplitSums {
   const float* slabs = nullptr;

@@ -3,13 +3,17 @@
 // The weight is DEFINED as bf16_rne(code * scale - scale * zero).  gemv4_kernel (gemv4.hip) forms it on the vector pipe: v_fma_mix and v_cvt_pk issue at half rate, 3.6 issue slots a
 // code, 13 of 20 us of a gate_up projection.  Here the matrix pipe multiplies by the scale, too:
 //   * D = A . B + C with A = codes as float16 denormals (a mask makes two of them: code * 2^-24, or * 2^-20 for the nibble above), 16 places of K x 16 row slots, B = the slots' scales
-//     on the diagonal, C = -(scale * zero): D holds weight * 2^-24 exactly (11 + 5 bits), one v_cvt_pk rounds two, and what is left are 1.6 slots a code.  The power of two is
-//     applied to the sums.
+//     on the diagonal (sixteen times them for the lower nibbles), C = -(scale * zero) * 2^-20: D holds weight * 2^-20 exactly (11 bits of a scale, 7 of code - zero), one v_cvt_pk rounds
+//     two, and what is left are 1.6 slots a code.  The power of two is applied to the sums.
 //   * a lane of A holds the codes of four rows at ONE place of K, which no row-major layout gives: the codes are stored in that order, units of four rows x 512 k = 1 KB that a wave
 //     reads as one piece, and their 16 scales and zeros as 64 bytes.
 //   * D is the operand of the second product as it lies: slots (4 rows x 4 parts of 128 k) x 8 places, against x as columns (part, hi / lo), as in gemv4_kernel.
-// us there / here, weights from HBM, with the norm: 27648 x 5120 gated 19.9 / 17.4 (4.3 TB/s with scales; 75 MB are 11.7 at the rate of a stream), 5120 x 13824 12.2 / 11.8, 7168 x 5120 8.4 / 7.3,
-// 5120 x 5120 7.4 / 6.7.  Weights that lie in L2 or the Infinity Cache already are 0.2 to 0.9 faster: what is left is the launch, x and the conversion.
+// us there / here, both in one run, copies of the weights in turn (600 MB and more, so that they come from memory), the norm where the model has it, at 12 waves and a ring of four:
+//   27648 x 5120 gated 22.5 / 17.5   24576 x 4096 gated 17.5 / 12.9   13824 x 5120 gated 12.7 / 10.2   16384 x 2048 gated 7.6 / 6.8   65536 x 8192 gated 78.3 / 53.2
+//   5120 x 13824 13.4 / 10.9   4096 x 12288 11.3 / 8.6   5120 x 6912 7.5 / 7.3   2560 x 8192 7.2 / 6.9   2048 x 8192 5.7 / 5.8
+//   7168 x 5120 8.7 / 7.3   6144 x 4096 6.7 / 6.2   3584 x 5120 6.5 / 5.9   5120 x 5120 6.9 / 6.4   4096 x 4096 5.5 / 5.1   5120 x 2560 5.2 / 4.8
+// Another run of the same had up to 12 % more (27648 x 5120 18.4, 24576 x 4096 14.5): figures of one line belong together, those of different lines do not.  75 MB of 27648 x 5120 are 11.7 us
+// at the rate of a stream; weights that lie in L2 or the Infinity Cache already are 0.2 to 0.9 faster: what is left is the launch, x and the conversion.
 #include "common.h"
 #include "gemv4.h"
 
@@ -60,6 +64,7 @@ __global__ __launch_bounds__(256) void tile_w4_kernel(W4TileParams p) {
       const _Float16 h = (_Float16)z.x;
       const float zero = z.x == 0.f ? 0.f : rintf(z.y / z.x);
       const _Float16 zh = (_Float16)(-zero * 0x1p-20f);
+      // (4000: sixteen times a scale has to be a float16 number)
       if (!(__builtin_isfinite(z.x) && (float)h == z.x && fabsf(zero) <= 64.f && (float)zh * z.x == -z.y * 0x1p-20f && fabsf(z.x) <= 4000.f)) atomicAdd(p.bad, 1);
       e = (uint32_t)__builtin_bit_cast(uint16_t, h) | (uint32_t)__builtin_bit_cast(uint16_t, zh) << 16;
     }
@@ -67,11 +72,15 @@ __global__ __launch_bounds__(256) void tile_w4_kernel(W4TileParams p) {
   }
 }
 
-// us by waves / units of the ring, 27648 x 5120 gated, 5120 x 13824, 5120 x 5120, 7168 x 5120: 8 / 3 20.3, 11.7, 6.6, 7.8; 8 / 8 21.4, 13.8, 7.4, 8.8 (every line of the unrolled loop is fetched
-// by each launch); 12 / 3 18.8, 11.45, 6.45, 7.55; 12 / 4 18.1, 11.4, 6.7, 7.7; 16 / 3 18.0, 11.6, 6.9, 8.1.  More than one unit before x is there costs 0.2 to 0.9.
+// us by waves / units of the ring, 8 / 3, 8 / 4, 12 / 3, 12 / 4, 16 / 3, one run:
+//   65536 x 8192 gated 60.2, 58.4, 52.8, 52.5, no room   27648 x 5120 gated 19.3, 18.6, 17.8, 18.4, 17.5   13824 x 5120 gated 11.1, 11.2, 10.7, 10.5, 12.5   7168 x 5120 7.9, 7.8, 7.5, 7.5, 7.9
+//   24576 x 4096 gated 14.0, 13.7, 14.3, 14.5, 14.2   5120 x 13824 11.6, 11.4, 11.7, 12.2, 12.3   4096 x 12288 9.2, 9.2, 9.1, 9.5, 9.9   5120 x 5120 6.2, 6.3, 6.0, 6.4, 6.8
+//   16384 x 2048 gated 6.4, 6.8, 6.8, 7.0, 7.2   6144 x 4096 5.7, 5.8, 6.1, 6.2, 6.6   4096 x 4096 4.7, 4.8, 5.0, 5.1, 5.7   2560 x 8192 6.4, 6.4, 6.7, 6.9, 7.1   2048 x 8192 5.2, 5.2, 5.8, 5.9, 6.2
+// Twelve are for K of 5120 and gated rows, where most of a ChatTS-14B step is; below 40 million codes eight are 3 to 12 % faster, and there is no rule between them yet.  A ring of eight units
+// with eight waves takes 1 to 2 us more (every line of the unrolled loop is fetched by each launch).  More than one unit before x is there costs 0.2 to 0.9.
 constexpr int kT4Bufs = 4, kT4Ahead = kT4Bufs - 1, kT4Waves = 12, kT4Threads = 64 * kT4Waves, kT4Turns = (16384 / 8 + kT4Threads - 1) / kT4Threads;
 
-// weights of a unit, times 2^-24 (even) and 2^-20 (odd): the operands of four products of 32 k.  place 8 quad .. of product p: k = 16 ma + 4 quad .. + 3 and 32 further on, of this
+// weights of a unit, times 2^-20: the operands of four products of 32 k.  place 8 quad .. of product p: k = 16 ma + 4 quad .. + 3 and 32 further on, of this
 // lane's part, ma = (p & 1) * 4 + (p >> 1)
 struct W4Diag { uint32_t m0, m1; };
 __device__ __forceinline__ W4Diag w4_diag(int lane) {
@@ -193,8 +202,9 @@ __global__ __launch_bounds__(64 * kT4Waves) void gemv4_tiles_kernel(Gemv4Params 
     acc0 = acc1 = (f32x4){0.f, 0.f, 0.f, 0.f};
   };
   const char* xl = xs + (kq * 8 + (lane & 7)) * 16;
-  // A SIMD issues for its oldest wave first: of three waves with equal shares the first was done at 12.5 us, the last at 21.  A wave that is ahead lets the others go first: 15.1 and 18.6
-  // (27648 x 5120: 20.6 -> 19.4 us).
+  // A SIMD issues for its oldest wave first: of three waves with equal shares of 27648 x 5120 the first was done at 12.5 us, the last at 21.  A wave that is ahead lets the others go first:
+  // 15.1 and 18.6.  us without / with, one run: 27648 x 5120 gated 19.8 / 18.4, 65536 x 8192 gated 55.6 / 52.5, 13824 x 5120 gated 11.4 / 10.5, 5120 x 13824 12.6 / 12.2, 7168 x 5120 7.7 / 7.5,
+  // nothing for shares of few units (0.1 to either side).
   int calm = 0, level = 3;
   for (int t = 0; t < cnt; t += kT4Bufs) {
     if (t >= calm) {

@@ -299,7 +299,8 @@ int chatts_tile_bf16(const chatts_bf16* src, int rows, int k, int ld, chatts_bf1
 /* 4-bit codes (ChattsLinearArgs.w4 / w4_sz, groups of 128 and more) -> the order the matrix pipe takes them in (csrc/gemv4_tiles.hip): for every four rows
  * (gated != 0: rows for SWIGLU, two gates and their up rows) and 512 K-values 1 KB of codes, behind all of them 64 bytes of scales and zeros each (float16).  dst holds
  * chatts_tile_w4_bytes(rows, k, group) bytes, 16-byte aligned; 0 = this shape has no such form (the row-major codes serve it as well or better).  *bad (device) grows by
- * the number of groups whose scale float16 does not hold exactly, or whose zero is no whole number up to 64 (a GPTQ checkpoint has none): with any the copy may not be used. */
+ * the number of groups whose scale float16 does not hold exactly or is beyond +-4000 (sixteen times it has to be a float16 number, too), or whose zero is no whole number up to 64 (a GPTQ
+ * checkpoint has none): with any the copy may not be used. */
 size_t chatts_tile_w4_bytes(int rows, int k, int group);
 int chatts_tile_w4(const uint8_t* w4, const float* w4_sz, int rows, int k, int ldw4, int group, int gated, void* dst, int32_t* bad, chatts_stream_t stream);
 /* chatts_linear for M == 1 and EPI_NONE / RESID / SWIGLU on such a copy (`gated` as SWIGLU is); `w`, `w4` and `w8` of the arguments are not read. */
