@@ -335,23 +335,33 @@ class ChatTSForCausalLM(SlotModel):
         cat = lambda ns: tuple(torch.cat([c[n][i] for n in ns], dim=0).contiguous() for i in range(3))
         fused = {"qkv": cat(names[:3]), "o": c[names[3]], "down": c[names[6]],
                  "gate_up": tuple(interleave_gate_up(c[names[4]][i], c[names[5]][i]) for i in range(3))}
-        for k, (q, sc, z) in fused.items():
-            self.int4_group = q.shape[1] // sc.shape[1]
-            self._keep_int4(L, k, q, sc, z)
+        q, sc, _ = fused["qkv"]
+        self.int4_group = q.shape[1] // sc.shape[1]
+        self._keep_int4(L, {k: pack_int4(*f) for k, f in fused.items()})
 
-    def _keep_int4(self, lw, name, codes, scale, zero):
-        """4-bit codes of a projection, for one row (more rows take the bf16 weights): in the order the matrix pipe takes them in (chatts_tile_w4), or row-major where the shape or a scale
-        has no such form.  Never both, and free memory has no say: the two sum in different orders."""
-        lib, (rows, k) = self.lib, codes.shape
-        w4, sz = pack_int4(codes, scale, zero)
-        need = int(lib.chatts_tile_w4_bytes(rows, k, self.int4_group))
-        if need and (name != "gate_up" or rows % 32 == 0):
-            tiles, bad = torch.empty(need, dtype=torch.uint8, device=self.device), torch.zeros(1, dtype=torch.int32, device=self.device)
-            _lib.check(lib.chatts_tile_w4(w4.data_ptr(), sz.data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", tiles.data_ptr(), bad.data_ptr(), _lib.stream_ptr()))
-            if not int(bad):
-                lw[name + "4_tiles"] = tiles
-                return
-        lw[name + "4"], lw[name + "4_sz"] = w4, sz
+    def _keep_int4(self, lw, packed):
+        """packed: projection -> what pack_int4 gives, of a layer's four.  The codes serve one row (more rows take the bf16 weights) and stay in the order the matrix pipe takes them in
+        (chatts_tile_w4), or row-major where the shape or a scale has no such form.  Never both, and free memory has no say: the two sum in different orders."""
+        lib, at, total = self.lib, {}, 0      # at: first byte and bytes of a projection's tiles
+        for name in packed:
+            rows, k = lw[name].shape
+            need = 0 if name == "gate_up" and rows % 32 else int(lib.chatts_tile_w4_bytes(rows, k, self.int4_group))
+            if need:
+                at[name] = (total, need)
+                total += -(-need // 256) * 256
+        refused = {}
+        if at:      # (an allocation and a wait a layer; ms to load ChatTS-8B from device memory: so 204, one for every projection 215, one for all layers, which holds both forms meanwhile, 190)
+            tiles, bad = torch.empty(total, dtype=torch.uint8, device=self.device), torch.zeros(len(at), dtype=torch.int32, device=self.device)
+            for i, (name, (first, need)) in enumerate(at.items()):
+                (rows, k), (w4, sz) = lw[name].shape, packed[name]
+                _lib.check(lib.chatts_tile_w4(w4.data_ptr(), sz.data_ptr(), rows, k, k // 2, self.int4_group, name == "gate_up", tiles[first:].data_ptr(), bad[i:].data_ptr(), _lib.stream_ptr()))
+            refused = dict(zip(at, bad.tolist()))
+        for name, (w4, sz) in packed.items():
+            if name in at and not refused[name]:
+                kept = tiles[at[name][0]:sum(at[name])]
+                lw[name + "4_tiles"] = kept.clone() if any(refused.values()) else kept
+            else:
+                lw[name + "4"], lw[name + "4_sz"] = w4, sz
 
     def _finalize(self):
         """Allocate activations / KV cache and create the C-side decoder handle (borrowing all pointers)."""
@@ -375,9 +385,11 @@ class ChatTSForCausalLM(SlotModel):
         if self.weight_format == "int4" and self.layers and not {"qkv4", "qkv4_tiles"} & self.layers[0].keys():
             # round-to-nearest 4-bit codes of every decoder projection; the bf16 tensors are REPLACED by the dequantised values
             for lw in self.layers:
+                packed = {}
                 for name in ("qkv", "o", "gate_up", "down"):
                     q, sc, z, lw[name] = quantize_int4_rows(lw[name], self.int4_group)
-                    self._keep_int4(lw, name, q, sc, z)
+                    packed[name] = pack_int4(q, sc, z)
+                self._keep_int4(lw, packed)
         # decode attention: one wave per 16-key tile; slots beyond the live context exit immediately
         self.n_splits = max(1, min(64, (self.max_ctx + 15) // 16))
         dc = _lib.DecoderConfig(hidden=H, n_layers=cfg.num_hidden_layers, n_q=plan.nq, n_kv=plan.nkv, head_dim=d,

@@ -89,6 +89,30 @@ def test_a_refused_scale_keeps_its_projection_row_major(monkeypatch):
     assert rel(got, want) < BOUND and not torch.equal(got, want)
 
 
+def test_codes_of_a_checkpoint(monkeypatch):
+    """(codes that come with the weights of q, k, v, gate and up one by one)"""
+    quantize, made = modeling.quantize_int4_rows, []
+    with monkeypatch.context() as p:
+        p.setattr(modeling, "quantize_int4_rows", lambda w, group=128: made.append(quantize(w, group)) or made[-1])
+        want = model_of("chatts-8b")
+    c = want.config
+    d, pairs = c.head_dim, {"model.embed_tokens.weight": want._tensors["embed"], "model.norm.weight": want._tensors["final_norm"], "lm_head.weight": want._tensors["lm_head"]}
+    rows = [n * d for n in (c.num_attention_heads, c.num_key_value_heads, c.num_key_value_heads)]
+    for l, lw in enumerate(want.layers):
+        qkv, o, gate_up, down = made[4 * l:4 * l + 4]
+        halves = [t.view(-1, 2, 16, t.shape[1]) for t in gate_up]
+        parts = dict(zip(("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj"), zip(*(t.split(rows) for t in qkv))))
+        parts |= {"self_attn.o_proj": o, "mlp.down_proj": down, "mlp.gate_proj": [t[:, 0].reshape(-1, t.shape[3]) for t in halves], "mlp.up_proj": [t[:, 1].reshape(-1, t.shape[3]) for t in halves]}
+        for name, (codes, scale, zero, deq) in parts.items():
+            pairs[f"model.layers.{l}.{name}.weight"], pairs[f"model.layers.{l}.{name}.gptq_codes"] = deq, (codes, scale, zero)
+        for name, key in (("input_layernorm", "input_norm"), ("post_attention_layernorm", "post_norm"), ("self_attn.q_norm", "q_norm"), ("self_attn.k_norm", "k_norm")):
+            pairs[f"model.layers.{l}.{name}.weight"] = lw[key]
+    m = ChatTSForCausalLM(c, max_ctx=256, max_prefill_tokens=128)
+    m.load_weights(pairs.items())
+    assert all(torch.equal(a[n + "4_tiles"], b[n + "4_tiles"]) and n + "4" not in a for a, b in zip(m.layers, want.layers) for n in NAMES)
+    assert torch.equal(logits(m), logits(want))
+
+
 def test_free_memory_does_not_choose_the_form(monkeypatch):
     want = logits(model_of("chatts-14b", prefill_tiled_weights=False))
     before = torch.cuda.memory_allocated()
