@@ -56,3 +56,31 @@ def test_panels_agree(monkeypatch, m, n, k, sk, t, epi, planes, tiled):
         return
     for p, q in zip(*got):
         assert torch.isfinite(p.float()).all() and torch.equal(p, q)
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("m,n,k,sk,t", [(5, 64, 64, 1, 1), (17, 384, 64, 1, 1), (97, 400, 64, 1, 1), (160, 1024, 64, 1, 1), (223, 1024, 128, 2, 2), (145, 800, 64, 1, 1)])
+def test_two_half_steps(m, n, k, sk, t, tiled):
+    """the fewest that a workgroup walks: its loaders never come to their loop's wait (one unit a workgroup, one to ten fragments, tiles of unequal length)"""
+    lib = _lib.load()
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)
+    x, w, bias = r(m, k), (r(n, k) * k ** -0.5).bfloat16(), r(n)
+    hi, lo = torch.empty(2, m, k, dtype=torch.bfloat16, device=DEV)
+    _lib.check(lib.chatts_split_bf16x2(x.data_ptr(), m, k, k, hi.data_ptr(), lo.data_ptr(), k, _lib.stream_ptr()))
+    wt = torch.empty(int(lib.chatts_tile_bf16_elems(n, k)), dtype=torch.bfloat16, device=DEV)
+    _lib.check(lib.chatts_tile_bf16(w.data_ptr(), n, k, k, wt.data_ptr(), _lib.stream_ptr()))
+    want = x.double() @ w.double().T + bias.double()
+    # x = hi + lo loses 2^-18 of each term; float32 sums of K terms and the bias
+    bound = x.double().abs() @ w.double().abs().T * (2.0 ** -18 + (k + 2) * 2.0 ** -24) + want.abs() * 2.0 ** -24
+    for panel in (256, 192):
+        with _lib.options(GEMM_SK=sk, GEMM_T=t, GEMM_STREAM=0, GEMM_PANEL=panel):
+            size = max(16, int(lib.chatts_linear_workspace(m, n, k)))
+            ws, out = torch.empty(size, dtype=torch.uint8, device=DEV), torch.full((m, n), float("nan"), device=DEV)
+            a = _lib.LinearArgs(w=w.data_ptr(), bias=bias.data_ptr(), c=out.data_ptr(), m=m, n=n, k=k, lda=k, ldw=k, ldc=n, epilogue=_lib.EPI_NONE, workspace=ws.data_ptr(), workspace_bytes=size,
+                                a_hi=hi.data_ptr(), a_lo=lo.data_ptr(), ld_planes=k)
+            if tiled:
+                a.w_tiled = wt.data_ptr()
+            _lib.check(lib.chatts_linear(C.byref(a), _lib.stream_ptr()))
+            torch.cuda.synchronize()
+        assert bool(((out.double() - want).abs() <= bound).all()), panel
