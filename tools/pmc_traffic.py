@@ -18,9 +18,9 @@ import sys
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 OUT = os.environ.get("PMC_TRAFFIC_OUT") or os.path.join(ROOT, "profiles", "pmc_traffic.json")      # (a GPU-box job writes under gpurun_out/)
 GEMV_FILES = ["chatts_amd/csrc/gemv.hip", "chatts_amd/csrc/gemv_ring.hip", "chatts_amd/csrc/gemv_common.h", "chatts_amd/csrc/tp_common.h", "chatts_amd/csrc/common.h"]
-TS_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_ring.hip", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/ts_frontend.hip",
+TS_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_ring.hip", "chatts_amd/csrc/ring_store.h", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/ts_frontend.hip",
             "chatts_amd/csrc/common.h"]
-BATCHED_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/attention.hip", "chatts_amd/csrc/attn_decode.h",
+BATCHED_FILES = ["chatts_amd/csrc/gemm.hip", "chatts_amd/csrc/gemm_cols.hip", "chatts_amd/csrc/gemm_common.h", "chatts_amd/csrc/attention.hip", "chatts_amd/csrc/attn_decode.h",
                  "chatts_amd/csrc/common.h"]
 
 
@@ -61,7 +61,7 @@ def headline(db, cmd, src):
     name, grid, wg, n, kib, us = max(rows, key=lambda r: r[4])            # gate_up: the SwiGLU GEMV with the most bytes
     inter = 13824
     d = load()
-    d.update({"source": f"{src} ({cmd}, MI355X, round 6)", "code_digest": code_digest(GEMV_FILES), "code_files": GEMV_FILES,
+    d.update({"source": f"{src} ({cmd}, MI355X)", "code_digest": code_digest(GEMV_FILES), "code_files": GEMV_FILES,
               "kernel": f"{'gemv_ring_kernel' if 'gemv_ring' in name else 'gemv_ldsx_kernel'}<SWIGLU,NORM> (gate_up_proj, grid {grid} = {grid // wg} workgroups x {wg} threads)",
               "launches_counted": n, "fetch_size_kib_per_launch": round(kib, 1), "gfx950_fetch_correction": 2.0,
               "write_bytes_per_launch": inter * 4, "hbm_bytes_per_launch": int(kib * 1024 * 2 + inter * 4), "avg_us_under_pmc": round(us, 2)})
@@ -74,14 +74,14 @@ def ts(db, cmd, src):
     calls = int(os.environ.get("TS_CALLS", "20")) + 1
     per_kernel, total = [], 0.0
     for name, grid, wg, n, kib, us in rows:
-        if "fill_hash" in name:
+        if "fill_hash" in name or "tile_bf16" in name:      # (weights, laid out once)
             continue
         b = kib * 1024 * 2 * n / calls
         total += b
         per_kernel.append({"kernel": name.split("(")[0].replace("void chatts::", "")[:80], "grid": grid, "launches_per_call": round(n / calls, 2),
                            "fetch_bytes_per_call": int(b), "avg_us_under_pmc": round(us, 2)})
     d = load()
-    d["ts_encoder"] = {"source": f"{src} ({cmd}, MI355X, round 6)", "code_digest": code_digest(TS_FILES), "code_files": TS_FILES,
+    d["ts_encoder"] = {"source": f"{src} ({cmd}, MI355X)", "code_digest": code_digest(TS_FILES), "code_files": TS_FILES,
                        "workload": "8 series x 256 steps (P = 128 patches), chatts_ts_encode", "calls_counted": calls,
                        "hbm_fetch_bytes_per_call": int(total), "algorithmic_bytes_per_call": 215257152,
                        "ratio": round(total / 215257152, 3), "per_kernel": per_kernel}
@@ -94,12 +94,12 @@ def ts(db, cmd, src):
 def batched(db, cmd, src, key="14b_8x1024_fp8_b16"):
     rows = counter_rows(db)
     # gate_up: the per-layer weight stream with the most bytes (>= 40 launches: lm_head runs once per step and is larger)
-    gu = max((r for r in rows if "gemm_stream_kernel" in r[0] and r[3] >= 40), key=lambda r: r[4])
+    gu = max((r for r in rows if ("gemm_stream_kernel" in r[0] or "gemm_cols_kernel" in r[0]) and r[3] >= 40), key=lambda r: r[4])
     at = max((r for r in rows if "attn_decode_kernel" in r[0]), key=lambda r: r[4])
     d = load()
     inter, B = 13824, 16
     d.setdefault("batched", {})[key] = {
-        "source": f"{src} ({cmd}, MI355X, round 6)", "code_digest": code_digest(BATCHED_FILES), "code_files": BATCHED_FILES,
+        "source": f"{src} ({cmd}, MI355X)", "code_digest": code_digest(BATCHED_FILES), "code_files": BATCHED_FILES,
         "kernel": f"{gu[0].split('(')[0].replace('void chatts::', '')} (gate_up_proj + SwiGLU, M = {B}, grid {gu[1]})",
         "fetch_size_kib_per_launch": round(gu[4], 1), "gfx950_fetch_correction": 2.0, "write_bytes_per_launch": B * inter * 2 * 2,
         "hbm_bytes_per_launch": int(gu[4] * 1024 * 2 + B * inter * 4), "algorithmic_bytes_per_launch": 143208448,
