@@ -143,3 +143,21 @@ def test_shards_of_two_ranks(monkeypatch):
     (tp, got), (plain, want) = run(), without_tiles(monkeypatch, run)
     assert all(n + "4_tiles" in lw for m in tp.ms for lw in m.layers for n in NAMES) and "qkv4" in plain.ms[0].layers[0]
     assert rel(got, want) < BOUND and not torch.equal(got, want)
+
+
+def test_tiles_that_are_refused():
+    """shapes without a tiled form, copies off 16 bytes, lists of another length"""
+    import ctypes as C
+    tiny, m = ChatTSForCausalLM.from_synthetic("tiny-qwen2", max_ctx=64, max_prefill_tokens=64, weight_format="int4"), model_of("chatts-8b")
+    assert all(n + "4" in lw and n + "4_tiles" not in lw for lw in tiny.layers for n in NAMES)
+    want = logits(m)
+    at = m.layers[0]["qkv4_tiles"].data_ptr()
+
+    def give(model, entries):
+        return model.lib.chatts_decoder_set_w4_tiles(model._decoder, (C.c_void_p * len(entries))(*entries), len(entries))
+
+    assert give(tiny, [at] + [None] * (4 * len(tiny.layers) - 1)) != 0 and give(tiny, [None] * (4 * len(tiny.layers))) == 0
+    assert give(m, [at + 8] + [None] * 7) != 0 and give(m, [at] * 7) != 0 and give(m, [None] * 9) != 0
+    assert m.lib.chatts_decoder_set_w4_tiles(m._decoder, None, 8) != 0 and m.lib.chatts_decoder_set_w4_tiles(None, None, 0) != 0
+    m._graph = None
+    assert torch.equal(logits(m), want)                   # (what was refused changed nothing)
